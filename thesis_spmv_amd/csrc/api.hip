@@ -379,6 +379,36 @@ static CrsDev crs_of(const pwm_matrix* h) {
     return A;
 }
 
+// The CRS arrays the one-workgroup power method reads: the handle's own, or
+// the copy a blocked format keeps of a small matrix.
+static CrsDev small_crs_of(const pwm_matrix* h) {
+    CrsDev A = crs_of(h);
+    if (h->format == PWM_FORMAT_CSB || h->format == PWM_FORMAT_BLOCKCOH) {
+        A.rs = h->sm_rs.as<int32_t>();
+        A.ci = h->sm_ci.as<int32_t>();
+        A.val = h->sm_val.p;
+    }
+    return A;
+}
+
+// Whether the power method of the handle about to be planned runs in one
+// workgroup (k_power.hip): the matrix fits it, and the caller chose no kernel,
+// layout or partition count, which a power step would otherwise have to run.
+static bool wants_power_small(const pwm_matrix* h) {
+    bool chosen = false;
+    switch (h->format) {
+        case PWM_FORMAT_CRS: chosen = h->crs_kernel || h->group_opt || h->vec_blocks_opt || h->long_row || h->crs_nt >= 0; break;
+        case PWM_FORMAT_CRS_MERGE: chosen = h->threads > 0 || h->ipt != 8; break;
+        case PWM_FORMAT_CSB:
+            chosen = h->csb_bits_override || h->csb_groups || h->csb_layout || h->csb_window_bits || h->csb_unroll ||
+                     h->csb_nt >= 0;
+            break;
+        case PWM_FORMAT_BLOCKCOH: chosen = h->threads > 0 || h->coh_occ8 >= 0; break;
+    }
+    CrsDev A = crs_of(h);
+    return !chosen && pwmk::power_small_fits(A, h->stats.row_max);
+}
+
 static int pow2_ceil(int64_t v) {
     int g = 1;
     while (g < v && g < 64) g <<= 1;
@@ -785,9 +815,14 @@ extern "C" int pwm_set_option(pwm_matrix* h, const char* key, int64_t value) {
     }
     if (h->loaded && (k == "group_size" || k == "vec_blocks" || k == "long_row" || k == "long_chunk" || k == "crs_kernel" ||
                       k == "crs_nt") &&
-        h->format == PWM_FORMAT_CRS)
+        h->format == PWM_FORMAT_CRS) {
+        h->power_small = wants_power_small(h);
         return plan_crs(h);
-    if (h->loaded && k == "items_per_thread" && h->format == PWM_FORMAT_CRS_MERGE) return plan_merge(h);
+    }
+    if (h->loaded && k == "items_per_thread" && h->format == PWM_FORMAT_CRS_MERGE) {
+        h->power_small = wants_power_small(h);
+        return plan_merge(h);
+    }
     return PWM_OK;
 }
 
@@ -824,11 +859,38 @@ static void reset_matrix(pwm_matrix* h) {
     h->crs_used = 1;
     h->csb.clear();
     h->coh.clear();
+    h->power_small = false;
+    h->sm_rs.release();
+    h->sm_ci.release();
+    h->sm_val.release();
+}
+
+// A blocked format drops the CRS arrays once it is built; the one-workgroup
+// power method of a small matrix keeps its own copy (at most 200 KB).
+static int keep_small_crs(pwm_matrix* h) {
+    const size_t vb = value_size(h->vtype);
+    hipError_t e;
+    if ((e = h->sm_rs.alloc((h->nor + 1) * 4)) != hipSuccess ||
+        (e = h->sm_ci.alloc(std::max<int64_t>(h->nnz, 1) * 4)) != hipSuccess ||
+        (e = h->sm_val.alloc(std::max<int64_t>(h->nnz, 1) * vb)) != hipSuccess)
+        return hip_fail(h, e, "small-matrix copy");
+    e = hipMemcpyAsync(h->sm_rs.p, h->rs.p, (h->nor + 1) * 4, hipMemcpyDeviceToDevice, h->stream);
+    if (e == hipSuccess && h->nnz)
+        e = hipMemcpyAsync(h->sm_ci.p, h->ci.p, h->nnz * 4, hipMemcpyDeviceToDevice, h->stream);
+    if (e == hipSuccess && h->nnz)
+        e = hipMemcpyAsync(h->sm_val.p, h->val.p, h->nnz * vb, hipMemcpyDeviceToDevice, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);  // before the build frees the originals
+    if (e != hipSuccess) return hip_fail(h, e, "small-matrix copy");
+    return PWM_OK;
 }
 
 static int finish_load(pwm_matrix* h, const int32_t* hrs, const int32_t* hci, const double* hval) {
     int rc = compute_matrix_stats(h);
     if (rc != PWM_OK) return rc;
+    h->power_small = wants_power_small(h);
+    if (h->power_small && (h->format == PWM_FORMAT_CSB || h->format == PWM_FORMAT_BLOCKCOH) &&
+        (rc = keep_small_crs(h)) != PWM_OK)
+        return rc;
     switch (h->format) {
         case PWM_FORMAT_CRS: rc = plan_crs(h); break;
         case PWM_FORMAT_CRS_MERGE: rc = plan_merge(h); break;
@@ -1045,7 +1107,7 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
                                       &h->csb.soff, &h->csb.srows, &h->csb.sweep_start,
                                       &h->coh.row_jump, &h->coh.col_jump, &h->coh.data, &h->coh.row_jump_block,
                                       &h->coh.col_jump_block, &h->coh.block_nnz, &h->coh.block_coords,
-                                      &h->coh.band_table, &h->coh.tasks, &h->pw_ctrl, &h->pw_rec, &h->pw_partials,
+                                      &h->coh.band_table, &h->coh.tasks, &h->sm_rs, &h->sm_ci, &h->sm_val, &h->pw_ctrl, &h->pw_rec, &h->pw_partials,
                                       &h->hx, &h->hy};
     int64_t b = 0;
     for (auto* d : bufs) b += (int64_t)d->bytes;
@@ -1185,6 +1247,33 @@ struct PowerWs {
     double* partials;
 };
 
+// The power loop of a small matrix in one workgroup (k_power.hip), at most
+// kSmallSteps steps (a few ms) per launch; the last launch leaves the vectors
+// as the general loop's finish does.
+static int run_power_small(pwm_matrix* h, const PowerArgs& pw, int64_t* steps, double* lambda, double* ynorm) {
+    constexpr int64_t kSmallSteps = 4096;
+    struct {
+        int ctrl[2];
+        double pad, lambda, yy;  // PowerArgs::ctrl + 4 ints: the result
+    } out = {};
+    static_assert(sizeof(out) == 32, "step control and result are read back as one record");
+    const CrsDev A = small_crs_of(h);
+    hipError_t e;
+    for (int64_t k = 0; k < pw.max_it; k += kSmallSteps) {
+        e = pwmk::launch_power_small(A, h->stats.row_max, pw, k, kSmallSteps, (double*)(pw.ctrl + 4), h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "power loop");
+        if (pw.tol < 0 && k + kSmallSteps < pw.max_it) continue;
+        e = hipMemcpyAsync(&out, pw.ctrl, sizeof(out), hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "power loop");
+        if (out.ctrl[1]) break;
+    }
+    if (steps) *steps = out.ctrl[0];
+    if (lambda) *lambda = out.lambda;
+    if (ynorm) *ynorm = sqrt(out.yy);
+    return PWM_OK;
+}
+
 // Runs the device power loop on buf0 (start vector) / buf1 with workspace ws
 // (NULL: the handle's own, allocated on first use); returns steps done.
 static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, double tol, int64_t* steps,
@@ -1210,6 +1299,7 @@ static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, doub
     pw.partials = ws->partials;
     pw.max_it = max_it;
     pw.tol = tol;
+    if (h->power_small) return run_power_small(h, pw, steps, lambda, ynorm);
     hipError_t e = pwmk::launch_power_reset(pw, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "power reset");
     const int64_t chunk = tol < 0 ? max_it : 32;

@@ -216,6 +216,11 @@ struct pwm_matrix {
     pwm_impl::CsbDev csb;
     pwm_impl::CohDev coh;
 
+    // small matrices: the power loop runs in one workgroup (k_power.hip); the
+    // blocked formats keep a copy of their CRS arrays for it
+    bool power_small = false;
+    pwm_impl::DevBuf sm_rs, sm_ci, sm_val;
+
     // power-method workspace
     pwm_impl::DevBuf pw_ctrl, pw_rec, pw_partials;
     int64_t pw_rec_cap = 0;

@@ -76,6 +76,13 @@ inline int merge_fix_blocks(int64_t P) {
     return (int)(b < 1 ? 1 : (b > 256 ? 256 : b));
 }
 
+// ---- power method of a small matrix in one workgroup (k_power.hip) ----------
+// Steps [k0, min(k0 + nsteps, pw.max_it)) of the power loop; writes the step
+// control, the last step's record, and its lambda and |y|^2 to result[0..1].
+bool power_small_fits(const CrsDev& A, int64_t row_max);
+hipError_t launch_power_small(const CrsDev& A, int64_t row_max, const PowerArgs& pw, int64_t k0, int64_t nsteps,
+                              double* result, hipStream_t s);
+
 // ---- utilities (k_util.hip) -------------------------------------------------
 // Util/Poisson.hpp:32-83 on the device, one thread per row.
 hipError_t launch_fill_poisson(int64_t m, int64_t n, int32_t* rs, int32_t* ci, void* val, int vtype,
