@@ -1247,33 +1247,6 @@ struct PowerWs {
     double* partials;
 };
 
-// The power loop of a small matrix in one workgroup (k_power.hip), at most
-// kSmallSteps steps (a few ms) per launch; the last launch leaves the vectors
-// as the general loop's finish does.
-static int run_power_small(pwm_matrix* h, const PowerArgs& pw, int64_t* steps, double* lambda, double* ynorm) {
-    constexpr int64_t kSmallSteps = 4096;
-    struct {
-        int ctrl[2];
-        double pad, lambda, yy;  // PowerArgs::ctrl + 4 ints: the result
-    } out = {};
-    static_assert(sizeof(out) == 32, "step control and result are read back as one record");
-    const CrsDev A = small_crs_of(h);
-    hipError_t e;
-    for (int64_t k = 0; k < pw.max_it; k += kSmallSteps) {
-        e = pwmk::launch_power_small(A, h->stats.row_max, pw, k, kSmallSteps, (double*)(pw.ctrl + 4), h->stream);
-        if (e != hipSuccess) return hip_fail(h, e, "power loop");
-        if (pw.tol < 0 && k + kSmallSteps < pw.max_it) continue;
-        e = hipMemcpyAsync(&out, pw.ctrl, sizeof(out), hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        if (e != hipSuccess) return hip_fail(h, e, "power loop");
-        if (out.ctrl[1]) break;
-    }
-    if (steps) *steps = out.ctrl[0];
-    if (lambda) *lambda = out.lambda;
-    if (ynorm) *ynorm = sqrt(out.yy);
-    return PWM_OK;
-}
-
 // Runs the device power loop on buf0 (start vector) / buf1 with workspace ws
 // (NULL: the handle's own, allocated on first use); returns steps done.
 static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, double tol, int64_t* steps,
@@ -1299,39 +1272,47 @@ static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, doub
     pw.partials = ws->partials;
     pw.max_it = max_it;
     pw.tol = tol;
-    if (h->power_small) return run_power_small(h, pw, steps, lambda, ynorm);
-    hipError_t e = pwmk::launch_power_reset(pw, h->stream);
-    if (e != hipSuccess) return hip_fail(h, e, "power reset");
-    const int64_t chunk = tol < 0 ? max_it : 32;
-    int64_t issued = 0;
-    int ctrl[2] = {0, 0};
-    while (issued < max_it) {
-        const int64_t n = std::min(chunk, max_it - issued);
-        for (int64_t i = 0; i < n; ++i) {
-            rc = spmv_launch(h, nullptr, nullptr, &pw, nullptr);
-            if (rc != PWM_OK) return rc;
-        }
-        issued += n;
-        if (tol >= 0) {
-            e = hipMemcpyAsync(ctrl, ws->ctrl, 8, hipMemcpyDeviceToHost, h->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-            if (e != hipSuccess) return hip_fail(h, e, "power loop");
-            if (ctrl[1]) break;
-        }
-    }
-    e = pwmk::launch_power_finish(pw, h->nor, h->vtype == PWM_VALUES_F64, 0, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(ctrl, ws->ctrl, 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return hip_fail(h, e, "power finish");
-    if (steps) *steps = ctrl[0];
-    if ((lambda || ynorm) && ctrl[0] > 0) {
-        double rec[4];
-        e = hipMemcpyAsync(rec, ws->rec + 4 * (ctrl[0] - 1), 32, hipMemcpyDeviceToHost, h->stream);
+    pw.k = 0;
+    // what the loop leaves in ctrl: the step count, the done flag, and the
+    // last step's lambda and |y|^2
+    struct {
+        int steps, done;
+        double pad, lambda, yy;
+    } out = {};
+    static_assert(sizeof(out) == 32, "step control and result are read back as one record");
+    hipError_t e = hipSuccess;
+    auto read_back = [&] {
+        e = hipMemcpyAsync(&out, ws->ctrl, sizeof(out), hipMemcpyDeviceToHost, h->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        if (e != hipSuccess) return hip_fail(h, e, "power record");
-        if (lambda) *lambda = rec[3];
-        if (ynorm) *ynorm = sqrt(rec[0]);
+        return e == hipSuccess;
+    };
+    // Steps issued between looks at the stop test (none: all at once).  A
+    // small matrix runs its steps in one workgroup (k_power.hip), at most 4096
+    // (a few ms) per launch, and leaves the vectors finished.
+    const CrsDev small = small_crs_of(h);
+    const int64_t chunk = h->power_small ? 4096 : tol < 0 ? max_it : 32;
+    while (pw.k < max_it) {
+        const int64_t end = std::min(max_it, pw.k + chunk);
+        if (h->power_small) {
+            e = pwmk::launch_power_small(small, h->stats.row_max, pw, pw.k, chunk, h->stream);
+            if (e != hipSuccess) return hip_fail(h, e, "power loop");
+            pw.k = end;
+        }
+        for (; pw.k < end; ++pw.k)
+            if ((rc = spmv_launch(h, nullptr, nullptr, &pw, nullptr)) != PWM_OK) return rc;
+        if (tol >= 0 && end < max_it) {
+            if (!read_back()) return hip_fail(h, e, "power loop");
+            if (out.done) break;
+        }
     }
+    if (!h->power_small) {
+        e = pwmk::launch_power_finish(pw, h->nor, h->vtype == PWM_VALUES_F64, h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "power finish");
+    }
+    if (!read_back()) return hip_fail(h, e, "power finish");
+    if (steps) *steps = out.steps;
+    if (lambda) *lambda = out.lambda;
+    if (ynorm) *ynorm = sqrt(out.yy);
     return PWM_OK;
 }
 

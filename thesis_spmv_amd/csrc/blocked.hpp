@@ -122,7 +122,5 @@ hipError_t launch_csb(const CsbArgs& a, const void* x, void* y, const pwmk::Powe
 int csb_reduce_blocks(int64_t nor);
 hipError_t launch_coh(const CohArgs& a, const int32_t* atomic_bands, int n_atomic, const void* x, void* y,
                       const pwmk::PowerArgs* pw, hipStream_t s);
-// FP64 reduction of the per-workgroup power-method partials (one workgroup).
-hipError_t launch_blocked_finalize(int vtype, int n_partials, const pwmk::PowerArgs& pw, hipStream_t s);
 
 }  // namespace blocked

@@ -847,7 +847,7 @@ hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     a.sstart = h->csb.sweep_start.as<int32_t>();
     hipError_t e = blocked::launch_csb(a, x, y, pw, h->stream, part);
     if (e == hipSuccess && pw && part != 1)
-        e = blocked::launch_blocked_finalize(h->vtype, (int)csb_partials(h), *pw, h->stream);
+        e = pwmk::launch_power_reduce(*pw, csb_partials(h), h->stream);
     return e;
 }
 
@@ -869,7 +869,7 @@ hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     a.occ8 = h->coh.occ8;
     hipError_t e = blocked::launch_coh(a, h->coh.atomic_bands.as<int32_t>(), (int)h->coh.n_atomic, x, y, pw, h->stream);
     if (e == hipSuccess && pw)
-        e = blocked::launch_blocked_finalize(h->vtype, (int)coh_partials(h), *pw, h->stream);
+        e = pwmk::launch_power_reduce(*pw, coh_partials(h), h->stream);
     return e;
 }
 

@@ -188,8 +188,8 @@ __global__ __launch_bounds__(kBS) void k_csb(CsbArgs a, const typename Arith<VT>
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
@@ -294,8 +294,8 @@ __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename A
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
@@ -369,8 +369,8 @@ __global__ __launch_bounds__(kBS) void k_csb_reduce(CsbArgs a, typename Arith<VT
     const X* __restrict__ x = nullptr;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
@@ -488,8 +488,8 @@ __global__ __launch_bounds__(kSwBS) void k_csb_sweep(CsbArgs a, const typename A
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
@@ -609,8 +609,8 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
@@ -778,8 +778,8 @@ __global__ __launch_bounds__(kBS) void k_coh_zero(CohArgs a, const int32_t* __re
     using X = typename Arith<VT>::X;
     X* y = y_arg;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (pwmk::power_done(pw)) return;
+        const int64_t k = pw.k;
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
     }
     const CohBand band = a.bands[atomic_bands[blockIdx.x]];
@@ -799,8 +799,8 @@ template <typename VT>
 __global__ __launch_bounds__(kBS) void k_coh_stats(CohArgs a, const int32_t* __restrict__ atomic_bands, PowerArgs pw) {
     using X = typename Arith<VT>::X;
     __shared__ double red[16];
-    if (pw.ctrl[1]) return;
-    const int k = pw.ctrl[0];
+    if (pwmk::power_done(pw)) return;
+    const int64_t k = pw.k;
     const X* x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
     const X* y = (const X*)((k & 1) ? pw.buf0 : pw.buf1);
     const double scale = pwmk::step_scale(pw, k);
@@ -926,13 +926,6 @@ hipError_t launch_coh(const CohArgs& a, const int32_t* atomic_bands, int n_atomi
         case 2: return coh_t<bf16_t>(a, atomic_bands, n_atomic, x, y, pw, s);
     }
     return hipErrorInvalidValue;
-}
-
-hipError_t launch_blocked_finalize(int vtype, int n_partials, const PowerArgs& pw, hipStream_t s) {
-    pwmk::CrsDev A;
-    A.vtype = vtype;
-    pwmk::LongRows none;
-    return pwmk::launch_crs_finalize(A, n_partials, none, nullptr, &pw, s);
 }
 
 }  // namespace blocked

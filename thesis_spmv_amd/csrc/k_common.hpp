@@ -142,21 +142,47 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nblocks) {
     return xcd * per + (xcd < extra ? xcd : extra) + slot;
 }
 
-// Per-iteration control block of the device-side power method.
+// One step of the device-side power method.  The host issues the steps in
+// order and passes each its number, so that a step's vectors are known without
+// reading device memory; only a stop test (tol >= 0) can end the loop early.
 struct PowerArgs {
     void* buf0;        // ping-pong vectors: step k reads buf[k&1], writes buf[(k+1)&1]
     void* buf1;
-    int* ctrl;         // ctrl[0] = step k, ctrl[1] = done flag
+    int* ctrl;         // ctrl[0] = steps done, ctrl[1] = done flag, then (ctrl + 4) lambda and |y|^2 of the last step
     double* rec;       // rec[4k..4k+3] = |y|^2, x^T y, x^T x, lambda of step k
     double* partials;  // per-block FP64 partial sums (3 per block)
     int64_t max_it;
     double tol;        // < 0: never stop early
+    int64_t k;         // this step
 };
+
+// An earlier step met the stop test: this one does nothing.
+__device__ __forceinline__ bool power_done(const PowerArgs& p) { return p.tol >= 0.0 && p.k > 0 && p.ctrl[1]; }
 
 // FP64 scale applied to step k's output: 1/|y_{k-1}| (1 for the first step,
 // which multiplies the caller's unnormalised start vector).
-__device__ __forceinline__ double step_scale(const PowerArgs& p, int k) {
+__device__ __forceinline__ double step_scale(const PowerArgs& p, int64_t k) {
     return k == 0 ? 1.0 : 1.0 / sqrt(p.rec[4 * (k - 1)]);
+}
+
+// Step k's record, stop test and step count, from its |y|^2, x^T y and x^T x
+// (one thread).
+__device__ __forceinline__ void power_record(const PowerArgs& pw, int64_t k, double yy, double xy, double xx) {
+    const double lam = xy / xx;
+    pw.rec[4 * k + 0] = yy;
+    pw.rec[4 * k + 1] = xy;
+    pw.rec[4 * k + 2] = xx;
+    pw.rec[4 * k + 3] = lam;
+    int done = (k + 1 >= pw.max_it);
+    if (pw.tol >= 0.0 && k >= 1) {
+        const double prev = pw.rec[4 * (k - 1) + 3];
+        if (fabs(lam - prev) <= pw.tol * fabs(lam)) done = 1;
+    }
+    pw.ctrl[0] = (int)(k + 1);
+    pw.ctrl[1] = done;
+    double* result = (double*)(pw.ctrl + 4);
+    result[0] = lam;
+    result[1] = yy;
 }
 
 }  // namespace pwmk

@@ -39,8 +39,8 @@ __global__ __launch_bounds__(kBS) void k_crs_vector(CrsDev A, int n_vec_blocks, 
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = step_scale(pw, k);
@@ -161,8 +161,8 @@ __global__ __launch_bounds__(kBS) void k_crs_vector(CrsDev A, int n_vec_blocks, 
 constexpr int kFinBS = 1024;
 
 // Long rows: y[row] = sum of the row's chunk partials in chunk order.  Power
-// mode: FP64 reduction of the block partials (fixed order), then step k's
-// record, the convergence test and k+1.
+// mode (only with long rows; otherwise launch_power_reduce): FP64 reduction of
+// the block partials (fixed order) and step k's record.
 template <typename VT, bool POWER>
 __global__ __launch_bounds__(kFinBS) void k_crs_finalize(CrsDev A, int n_partials, LongRows lr,
                                                          typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
@@ -171,10 +171,10 @@ __global__ __launch_bounds__(kFinBS) void k_crs_finalize(CrsDev A, int n_partial
     X* __restrict__ y = y_arg;
     const X* __restrict__ x = nullptr;
     double scale = 1.0;
-    int k = 0;
+    int64_t k = 0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        k = pw.ctrl[0];
+        if (power_done(pw)) return;
+        k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = step_scale(pw, k);
@@ -203,20 +203,7 @@ __global__ __launch_bounds__(kFinBS) void k_crs_finalize(CrsDev A, int n_partial
         const double a = block_sum<kFinBS>(yy, red);
         const double b = block_sum<kFinBS>(xy, red);
         const double c = block_sum<kFinBS>(xx, red);
-        if (threadIdx.x == 0) {
-            const double lam = b / c;
-            pw.rec[4 * k + 0] = a;
-            pw.rec[4 * k + 1] = b;
-            pw.rec[4 * k + 2] = c;
-            pw.rec[4 * k + 3] = lam;
-            int done = (k + 1 >= pw.max_it);
-            if (pw.tol >= 0.0 && k >= 1) {
-                const double prev = pw.rec[4 * (k - 1) + 3];
-                if (fabs(lam - prev) <= pw.tol * fabs(lam)) done = 1;
-            }
-            pw.ctrl[0] = k + 1;
-            pw.ctrl[1] = done;
-        }
+        if (threadIdx.x == 0) power_record(pw, k, a, b, c);
     }
 }
 

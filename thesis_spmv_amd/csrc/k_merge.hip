@@ -55,8 +55,8 @@ __global__ __launch_bounds__(kMBS) void k_merge_spmv(CrsDev A, MergePlan mp, con
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = step_scale(pw, k);
@@ -97,20 +97,24 @@ __global__ void k_merge_fixup(int64_t nrows, MergePlan mp, typename Arith<VT>::X
 }
 
 constexpr int kFixBS = 256;
+constexpr int kFixOneBS = 1024;
 
 // Power mode, pass 1: workgroup b owns tiles [b*per, (b+1)*per): it adds the
 // carries of the runs whose head tile it owns (a run of tiles p..q-1 carrying
 // into row r is summed in tile order and added to y[r] once, by the thread of
 // the run's head, which follows the run past its own range) and sums, in a
 // fixed order, its tiles' FP64 partials plus the completed rows'
-// contributions, into the second-level slot after the tile partials.
-template <typename VT>
-__global__ __launch_bounds__(kFixBS) void k_merge_fixup_power1(CrsDev A, MergePlan mp, PowerArgs pw, int64_t per) {
+// contributions, into the second-level slot after the tile partials, or, as
+// the only workgroup (ONE), straight into step k's record.
+template <typename VT, bool ONE>
+__global__ __launch_bounds__(ONE ? kFixOneBS : kFixBS) void k_merge_fixup_power1(CrsDev A, MergePlan mp, PowerArgs pw,
+                                                                                int64_t per) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
+    constexpr int BS = ONE ? kFixOneBS : kFixBS;
     __shared__ double red[48];
-    if (pw.ctrl[1]) return;
-    const int k = pw.ctrl[0];
+    if (power_done(pw)) return;
+    const int64_t k = pw.k;
     const X* __restrict__ x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
     X* __restrict__ y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
     const double scale = step_scale(pw, k);
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(kFixBS) void k_merge_fixup_power1(CrsDev A, MergePl
     const int64_t p0 = (int64_t)blockIdx.x * per;
     const int64_t p1 = p0 + per < mp.P ? p0 + per : mp.P;
     double yy = 0.0, xy = 0.0, xx = 0.0;
-    for (int64_t p = p0 + threadIdx.x; p < p1; p += kFixBS) {
+    for (int64_t p = p0 + threadIdx.x; p < p1; p += BS) {
         yy += pw.partials[3 * p + 0];
         xy += pw.partials[3 * p + 1];
         xx += pw.partials[3 * p + 2];
@@ -139,42 +143,16 @@ __global__ __launch_bounds__(kFixBS) void k_merge_fixup_power1(CrsDev A, MergePl
         xy += xd * yd;
         xx += xd * xd;
     }
-    block_sum3<kFixBS>(yy, xy, xx, red);
+    block_sum3<BS>(yy, xy, xx, red);
     if (threadIdx.x == 0) {
-        double* q2 = pw.partials + 3 * mp.P + 3 * (int64_t)blockIdx.x;
-        q2[0] = yy;
-        q2[1] = xy;
-        q2[2] = xx;
-    }
-}
-
-// Power mode, pass 2 (one workgroup): the second-level sums in workgroup
-// order, then step k's record and k+1.
-__global__ __launch_bounds__(kFixBS) void k_merge_fixup_power2(MergePlan mp, PowerArgs pw, int nblk) {
-    __shared__ double red[48];
-    if (pw.ctrl[1]) return;
-    const int k = pw.ctrl[0];
-    double a = 0.0, b = 0.0, c = 0.0;
-    for (int i = threadIdx.x; i < nblk; i += kFixBS) {
-        const double* q2 = pw.partials + 3 * mp.P + 3 * (int64_t)i;
-        a += q2[0];
-        b += q2[1];
-        c += q2[2];
-    }
-    block_sum3<kFixBS>(a, b, c, red);
-    if (threadIdx.x == 0) {
-        const double lam = b / c;
-        pw.rec[4 * k + 0] = a;
-        pw.rec[4 * k + 1] = b;
-        pw.rec[4 * k + 2] = c;
-        pw.rec[4 * k + 3] = lam;
-        int done = (k + 1 >= pw.max_it);
-        if (pw.tol >= 0.0 && k >= 1) {
-            const double prev = pw.rec[4 * (k - 1) + 3];
-            if (fabs(lam - prev) <= pw.tol * fabs(lam)) done = 1;
+        if constexpr (ONE) {
+            power_record(pw, k, yy, xy, xx);
+        } else {
+            double* q2 = pw.partials + 3 * mp.P + 3 * (int64_t)blockIdx.x;
+            q2[0] = yy;
+            q2[1] = xy;
+            q2[2] = xx;
         }
-        pw.ctrl[0] = k + 1;
-        pw.ctrl[1] = done;
     }
 }
 
@@ -225,10 +203,17 @@ template <typename VT>
 static hipError_t launch_fix_t(const CrsDev& A, const MergePlan& mp, void* y, const PowerArgs* pw, hipStream_t s) {
     using X = typename Arith<VT>::X;
     if (pw) {
+        // one tile per thread of one workgroup: the second launch costs more
+        // (a step of 706 tiles 14.5 against 15.6 us); with three or four tiles
+        // per thread their chains of loads do (45 against 33 us)
+        if (mp.P <= kFixOneBS) {
+            hipLaunchKernelGGL((k_merge_fixup_power1<VT, true>), dim3(1), dim3(kFixOneBS), 0, s, A, mp, *pw, mp.P);
+            return hipGetLastError();
+        }
         const int nblk = merge_fix_blocks(mp.P);
         const int64_t per = (mp.P + nblk - 1) / nblk;
-        hipLaunchKernelGGL((k_merge_fixup_power1<VT>), dim3(nblk), dim3(kFixBS), 0, s, A, mp, *pw, per);
-        hipLaunchKernelGGL(k_merge_fixup_power2, dim3(1), dim3(kFixBS), 0, s, mp, *pw, nblk);
+        hipLaunchKernelGGL((k_merge_fixup_power1<VT, false>), dim3(nblk), dim3(kFixBS), 0, s, A, mp, *pw, per);
+        return launch_power_final(*pw, pw->partials + 3 * mp.P, nblk, 1, s);
     } else
         hipLaunchKernelGGL((k_merge_fixup<VT>), dim3((unsigned)((mp.P + 255) / 256)), dim3(256), 0, s, A.nrows, mp,
                            (X*)y);

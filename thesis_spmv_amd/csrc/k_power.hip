@@ -21,6 +21,8 @@
 // accumulator type, out = sum / |y_previous| and the norms in FP64, every sum
 // in a fixed order.  A step takes 1.1 us at 10 x 10, 1.7 us at 37 x 29 (15.9
 // before) and 2.6 us at 52 x 51, FP64; 100 steps at 37 x 29 take 0.20 ms.
+#include <algorithm>
+
 #include "kernels.hpp"
 
 namespace pwmk {
@@ -31,8 +33,7 @@ constexpr int kPsWaves = kPsBS / 64;
 constexpr int64_t kPsLds = 160 * 1024 - 2048;
 
 template <typename VT, int E>
-__global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArgs pw, int64_t k0, int64_t nsteps,
-                                                       double* __restrict__ result) {
+__global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArgs pw, int64_t k0, int64_t nsteps) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     extern __shared__ __align__(16) unsigned char ps_smem[];
@@ -136,6 +137,7 @@ __global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArg
                     pw.rec[4 * k + 3] = lam;
                     pw.ctrl[0] = (int)(k + 1);
                     pw.ctrl[1] = done;
+                    double* result = (double*)(pw.ctrl + 4);
                     result[0] = lam;
                     result[1] = yy;
                 }
@@ -161,6 +163,81 @@ __global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArg
         if (k > 0) gx[i] = done ? (X)((double)x[i] * scale) : x[i];
     }
 }
+
+// ---------------------------------------------------------------- norms of a step
+
+constexpr int kFinBS = 1024;
+constexpr int kSumBS = 256;
+constexpr int kPsU = 4;  // slots a thread loads together
+
+// Sum of the slots i0, i0 + stride, ... < end of this thread, in that order.
+__device__ __forceinline__ void slot_sum(const double* slots, int64_t i0, int64_t stride, int64_t end, double& yy,
+                                         double& xy, double& xx) {
+    for (int64_t i = i0; i < end; i += kPsU * stride) {
+        double a[kPsU], b[kPsU], c[kPsU];
+#pragma unroll
+        for (int u = 0; u < kPsU; ++u) {
+            const int64_t j = i + u * stride;
+            const bool ok = j < end;
+            a[u] = ok ? slots[3 * j + 0] : 0.0;
+            b[u] = ok ? slots[3 * j + 1] : 0.0;
+            c[u] = ok ? slots[3 * j + 2] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kPsU; ++u) {
+            yy += a[u];
+            xy += b[u];
+            xx += c[u];
+        }
+    }
+}
+
+// Many slots: workgroup b leaves the sum of slots [b*per, (b+1)*per) in slot
+// b*per.
+__global__ __launch_bounds__(kSumBS) void k_power_sum(PowerArgs pw, int64_t n, int64_t per) {
+    __shared__ double red[48];
+    if (power_done(pw)) return;
+    const int64_t i0 = (int64_t)blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
+    double yy = 0.0, xy = 0.0, xx = 0.0;
+    slot_sum(pw.partials, i0 + threadIdx.x, kSumBS, i1, yy, xy, xx);
+    block_sum3<kSumBS>(yy, xy, xx, red);
+    if (threadIdx.x == 0) {
+        pw.partials[3 * i0 + 0] = yy;
+        pw.partials[3 * i0 + 1] = xy;
+        pw.partials[3 * i0 + 2] = xx;
+    }
+}
+
+// One workgroup: slots 0, step, 2*step, ... (n of them) into step k's record.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_power_final(PowerArgs pw, const double* slots, int64_t n, int64_t step) {
+    __shared__ double red[48];
+    if (power_done(pw)) return;
+    double yy = 0.0, xy = 0.0, xx = 0.0;
+    slot_sum(slots, threadIdx.x * step, BS * step, n * step, yy, xy, xx);
+    block_sum3<BS>(yy, xy, xx, red);
+    if (threadIdx.x == 0) power_record(pw, pw.k, yy, xy, xx);
+}
+
+hipError_t launch_power_final(const PowerArgs& pw, const double* slots, int64_t n, int64_t step, hipStream_t s) {
+    if (n <= kPsU * kSumBS)
+        hipLaunchKernelGGL(k_power_final<kSumBS>, dim3(1), dim3(kSumBS), 0, s, pw, slots, n, step);
+    else
+        hipLaunchKernelGGL(k_power_final<kFinBS>, dim3(1), dim3(kFinBS), 0, s, pw, slots, n, step);
+    return hipGetLastError();
+}
+
+// One workgroup reads kPsU slots per thread in one go; beyond two such rounds
+// a launch that spreads the reading costs less than a third.
+hipError_t launch_power_reduce(const PowerArgs& pw, int64_t n, hipStream_t s) {
+    if (n <= 2 * kPsU * kFinBS) return launch_power_final(pw, pw.partials, n, 1, s);
+    const int64_t per = std::max<int64_t>(kPsU * kSumBS, (n + kFinBS - 1) / kFinBS);
+    const int64_t nb = (n + per - 1) / per;
+    hipLaunchKernelGGL(k_power_sum, dim3((unsigned)nb), dim3(kSumBS), 0, s, pw, n, per);
+    return launch_power_final(pw, pw.partials, nb, per, s);
+}
+
+// ---------------------------------------------------------------- the one-workgroup loop
 
 // Entries per thread: the smallest instance that holds all nonzeros.  FP64
 // entries take 3 registers each and FP32 ones 2, of the 128 a thread of a
@@ -203,34 +280,32 @@ bool power_small_fits(const CrsDev& A, int64_t row_max) {
 }
 
 template <typename VT, int E>
-static hipError_t launch_ps(const CrsDev& A, int G, const PowerArgs& pw, int64_t k0, int64_t nsteps, double* result,
-                            hipStream_t s) {
-    hipLaunchKernelGGL((k_power_small<VT, E>), dim3(1), dim3(kPsBS), (size_t)ps_lds(A), s, A, G, pw, k0, nsteps, result);
+static hipError_t launch_ps(const CrsDev& A, int G, const PowerArgs& pw, int64_t k0, int64_t nsteps, hipStream_t s) {
+    hipLaunchKernelGGL((k_power_small<VT, E>), dim3(1), dim3(kPsBS), (size_t)ps_lds(A), s, A, G, pw, k0, nsteps);
     return hipGetLastError();
 }
 
 template <typename VT>
-static hipError_t launch_ps_t(const CrsDev& A, int G, const PowerArgs& pw, int64_t k0, int64_t nsteps, double* result,
-                              hipStream_t s) {
+static hipError_t launch_ps_t(const CrsDev& A, int G, const PowerArgs& pw, int64_t k0, int64_t nsteps, hipStream_t s) {
     switch (ps_entries(A.vtype, A.nnz)) {
-        case 2: return launch_ps<VT, 2>(A, G, pw, k0, nsteps, result, s);
-        case 4: return launch_ps<VT, 4>(A, G, pw, k0, nsteps, result, s);
-        case 8: return launch_ps<VT, 8>(A, G, pw, k0, nsteps, result, s);
-        case 16: return launch_ps<VT, 16>(A, G, pw, k0, nsteps, result, s);
+        case 2: return launch_ps<VT, 2>(A, G, pw, k0, nsteps, s);
+        case 4: return launch_ps<VT, 4>(A, G, pw, k0, nsteps, s);
+        case 8: return launch_ps<VT, 8>(A, G, pw, k0, nsteps, s);
+        case 16: return launch_ps<VT, 16>(A, G, pw, k0, nsteps, s);
         case 24:
-            if constexpr (sizeof(typename Arith<VT>::A) == 4) return launch_ps<VT, 24>(A, G, pw, k0, nsteps, result, s);
+            if constexpr (sizeof(typename Arith<VT>::A) == 4) return launch_ps<VT, 24>(A, G, pw, k0, nsteps, s);
             return hipErrorInvalidValue;
         default: return hipErrorInvalidValue;
     }
 }
 
 hipError_t launch_power_small(const CrsDev& A, int64_t row_max, const PowerArgs& pw, int64_t k0, int64_t nsteps,
-                              double* result, hipStream_t s) {
+                              hipStream_t s) {
     const int G = ps_lanes(A.nrows, row_max);
     switch (A.vtype) {
-        case VT_F64: return launch_ps_t<double>(A, G, pw, k0, nsteps, result, s);
-        case VT_F32: return launch_ps_t<float>(A, G, pw, k0, nsteps, result, s);
-        case VT_BF16: return launch_ps_t<bf16_t>(A, G, pw, k0, nsteps, result, s);
+        case VT_F64: return launch_ps_t<double>(A, G, pw, k0, nsteps, s);
+        case VT_F32: return launch_ps_t<float>(A, G, pw, k0, nsteps, s);
+        case VT_BF16: return launch_ps_t<bf16_t>(A, G, pw, k0, nsteps, s);
         default: return hipErrorInvalidValue;
     }
 }

@@ -29,8 +29,8 @@ __global__ __launch_bounds__(kTBS) void k_tiles_spmv(CrsDev A, const ETile* __re
     X* __restrict__ y = y_arg;
     double scale = 1.0;
     if constexpr (POWER) {
-        if (pw.ctrl[1]) return;
-        const int k = pw.ctrl[0];
+        if (power_done(pw)) return;
+        const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = step_scale(pw, k);

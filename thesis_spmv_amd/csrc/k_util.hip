@@ -130,20 +130,8 @@ __global__ void k_power_finish(PowerArgs pw, int64_t n, int is_f64) {
     }
 }
 
-hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, int64_t, hipStream_t s) {
+hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, hipStream_t s) {
     hipLaunchKernelGGL(k_power_finish, dim3(grid_for(n)), dim3(256), 0, s, pw, n, is_f64);
-    return hipGetLastError();
-}
-
-__global__ void k_power_reset(int* ctrl) {
-    if (threadIdx.x == 0) {
-        ctrl[0] = 0;
-        ctrl[1] = 0;
-    }
-}
-
-hipError_t launch_power_reset(const PowerArgs& pw, hipStream_t s) {
-    hipLaunchKernelGGL(k_power_reset, dim3(1), dim3(64), 0, s, pw.ctrl);
     return hipGetLastError();
 }
 

@@ -43,7 +43,7 @@ struct LongRows {
 hipError_t launch_crs_vector(const CrsDev& A, int G, int n_vec_blocks, const LongRows& lr, const void* x,
                              void* y, const PowerArgs* pw, hipStream_t s);
 // Finishes long rows (sum of chunk partials, in chunk order) and, for the
-// power method, reduces the per-block partials into rec[k] and advances k.
+// power method, reduces the per-block partials into step k's record.
 hipError_t launch_crs_finalize(const CrsDev& A, int n_partials, const LongRows& lr, void* y,
                                const PowerArgs* pw, hipStream_t s);
 
@@ -76,12 +76,17 @@ inline int merge_fix_blocks(int64_t P) {
     return (int)(b < 1 ? 1 : (b > 256 ? 256 : b));
 }
 
-// ---- power method of a small matrix in one workgroup (k_power.hip) ----------
-// Steps [k0, min(k0 + nsteps, pw.max_it)) of the power loop; writes the step
-// control, the last step's record, and its lambda and |y|^2 to result[0..1].
+// ---- power method: norms of a step, and small matrices (k_power.hip) --------
+// The n partial-sum slots of step pw.k into its record (slots are overwritten).
+hipError_t launch_power_reduce(const PowerArgs& pw, int64_t n, hipStream_t s);
+// The slots 0, step, 2 step, ... (n of them) of `slots`, by one workgroup.
+hipError_t launch_power_final(const PowerArgs& pw, const double* slots, int64_t n, int64_t step, hipStream_t s);
+// The whole loop of a small matrix in one workgroup:
+// Steps [k0, min(k0 + nsteps, pw.max_it)) of the power loop; leaves the last
+// one's record and step control.
 bool power_small_fits(const CrsDev& A, int64_t row_max);
 hipError_t launch_power_small(const CrsDev& A, int64_t row_max, const PowerArgs& pw, int64_t k0, int64_t nsteps,
-                              double* result, hipStream_t s);
+                              hipStream_t s);
 
 // ---- utilities (k_util.hip) -------------------------------------------------
 // Util/Poisson.hpp:32-83 on the device, one thread per row.
@@ -95,8 +100,7 @@ hipError_t launch_fill(void* p, int64_t n, int is_f64, double v, hipStream_t s);
 hipError_t launch_copy_vec(const void* src_f64_or_f32, int src_f64, void* dst, int dst_f64, int64_t n,
                            hipStream_t s);
 // Final normalisation of the power method (see api.cpp).
-hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, int64_t steps, hipStream_t s);
-hipError_t launch_power_reset(const PowerArgs& pw, hipStream_t s);
+hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, hipStream_t s);
 // Rewrite a buffer (Infinity-Cache flush for the roofline timing).
 hipError_t launch_flush(void* p, int64_t bytes, hipStream_t s);
 // Plain streaming copy (profiler counter calibration).
