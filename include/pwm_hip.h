@@ -173,9 +173,10 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * device), "coh_build" (BlockCOH layout built on the device, 0, or on the
  * host, 1; both give the same arrays), "coh_occ8" (BlockCOH kernel instance
  * with registers capped for 8 waves per SIMD: 1, the compiler's budget: 0,
- * or -1 = time both at load, the default), "crs_kernel" (CRS: 0 = time the vector kernel at
+ * or -1 = time both at load, the default), "crs_kernel" (CRS: 0 = one wave per tile of short
+ * rows when no row has more than 64 entries, else time the vector kernel at
  * three lane counts and the row-aligned tiles kernel at load and keep the
- * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernel: 1 =
+ * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =
  * non-temporal col_ind/value loads, 0 = plain, -1 = time both at load, the
  * default).  Must be set before the matrix is loaded unless noted. */
 int pwm_set_option(pwm_matrix* h, const char* key, int64_t value);

@@ -82,3 +82,32 @@ def test_small_power_method(kind, n, values):
         x3, y3 = pw.DeviceVector.from_array(x0, vt), pw.DeviceVector(A.nor, vt)
         lam3 = m.power_method_device(x3, y3, k - 1)[0]
         assert abs(lam2 - lam3) <= 1.1e-5 * abs(lam2)
+
+
+# The general loop's norms: partial-sum slots of every kernel within one
+# workgroup's reach, and more of them than that (wave tiles: one slot per 8
+# tiles of about 250 entries; merge path and tiles: one slot a tile)
+GENERAL = [("crs", pw.CRSHip, {}), ("tiles", pw.CRSHip, {"crs_kernel": 2}), ("vector", pw.CRSHip, {"crs_kernel": 1}),
+           ("merge", pw.CRSMergeHip, {}), ("csb", pw.CSBHip, {}), ("coh", pw.BlockCOHHip, {})]
+
+
+@pytest.mark.parametrize("side", [(80, 77), (331, 300), (2100, 2000)], ids=str)
+@pytest.mark.parametrize("name,cls,opt", GENERAL, ids=[g[0] for g in GENERAL])
+def test_power_steps(name, cls, opt, side):
+    A = _matrix("poisson", side)
+    x0 = np.random.default_rng(4).uniform(0.5, 1.5, A.nor)
+    m = cls(**opt)
+    m.loadCRS(A.nor, A.noc, A.row_start, A.col_ind, A.data)
+    its, u = 5, 2.0 ** -53
+    xr, yr = oracle.crs_power_iteration(A, x0, its)
+    x, y = pw.DeviceVector.from_array(x0), pw.DeviceVector(A.nor)
+    lam, yn, k = m.power_method_device(x, y, its)
+    bound = 2 * (9 * its + 8) * u + 2 * A.nor * u  # the norms: N squares added in any order
+    assert k == its
+    for got, ref in ((x.download(), xr), (y.download(), yr)):
+        assert np.max(np.abs(got - ref) / ref) <= bound
+    w = oracle.crs_mv(A, xr)
+    assert abs(lam - xr @ w / (xr @ xr)) <= 4 * bound * lam
+    assert abs(yn - np.linalg.norm(w)) <= 4 * bound * yn
+    lam2, yn2, k2 = m.power_method_device(*(pw.DeviceVector.from_array(v) for v in (x0, x0)), 40, 1e-3)
+    assert 2 <= k2 <= 40 and abs(lam2 - lam) <= 0.05 * lam

@@ -355,9 +355,10 @@ class SparseMatrixHip:
 
 
 class CRSHip(SparseMatrixHip):
-    """CRS (beside CRS / CRSOMP, Matrix/CRS.hpp, Env_Implementations/CRSOMP.hpp): the
-    vector kernel or the row-aligned tiles kernel, whichever timed faster at
-    load (option crs_kernel: 1 vector, 2 tiles)."""
+    """CRS (beside CRS / CRSOMP, Matrix/CRS.hpp, Env_Implementations/CRSOMP.hpp): one
+    wave per tile of short rows (no row above 64 entries), else the vector
+    kernel or the row-aligned tiles kernel, whichever timed faster at load
+    (option crs_kernel: 1 vector, 2 tiles)."""
     FORMAT = FORMAT_CRS
 
 

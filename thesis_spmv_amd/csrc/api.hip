@@ -457,6 +457,11 @@ static int plan_crs_tiles(pwm_matrix* h) {
 static hipError_t crs_kernel_launch(pwm_matrix* h, int which, const void* x, void* y, const PowerArgs* pw) {
     const CrsDev A = crs_of(h);
     hipError_t e;
+    if (which == 3) {
+        e = pwmk::launch_rows(A, h->rp, x, y, pw, h->stream);
+        if (e == hipSuccess && pw) e = pwmk::launch_power_reduce(*pw, pwmk::rows_power_blocks(h->rp.nt), h->stream);
+        return e;
+    }
     if (which == 2) {
         // a plain SpMV whose tiles are all row-aligned stream tiles has no
         // carries to add; power steps always finish in the fix-up (norms)
@@ -552,7 +557,41 @@ static int plan_crs_vector(pwm_matrix* h, int G) {
     return PWM_OK;
 }
 
-// CRS planning and the autotuner.  Candidates: the vector kernel with the
+// Wave tiles (k_rows.hip), where every row is short and no tile has too many
+// rows; PWM_OK with rp.nt = 0 where not.
+static int plan_crs_rows(pwm_matrix* h) {
+    h->rp = pwmk::RowsPlan{};
+    h->rows_cut.release();
+    const int64_t step = pwmk::rows_step(h->stats.row_max);
+    if (step <= 0 || h->nnz == 0) return PWM_OK;
+    pwmk::RowsPlan rp;
+    rp.nt = (h->nnz + step - 1) / step;
+    // the cuts and, behind them, the plan kernel's flag
+    hipError_t e = h->rows_cut.alloc((rp.nt + 2) * sizeof(int2));
+    if (e != hipSuccess) return hip_fail(h, e, "wave tile plan");
+    int2* cut = h->rows_cut.as<int2>();
+    int* flag = (int*)(cut + rp.nt + 1);
+    int too_many = 0;
+    e = hipMemsetAsync(flag, 0, 4, h->stream);
+    if (e == hipSuccess) e = pwmk::launch_rows_plan(crs_of(h), step, rp.nt, cut, flag, h->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&too_many, flag, 4, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return hip_fail(h, e, "wave tile plan");
+    if (too_many) {
+        h->rows_cut.release();
+        return PWM_OK;
+    }
+    rp.cut = cut;
+    h->rp = rp;
+    return PWM_OK;
+}
+
+// CRS planning and the autotuner.  Rows of at most 64 entries take the wave
+// tiles (k_rows.hip): the kernels below were slower or equal on every such
+// matrix (FP64, us: Poisson 300 x 301 2.7 against 3.4, 5000 x 5000 332 against
+// 441, 9-point stencil with 2 random entries per row, 1448 x 1448, 100 against
+// 100); only the kind of entry load is timed.  Otherwise, or when the caller
+// named a kernel or set up the vector kernel: candidates are that one with the
 // rows-per-wave heuristic G0 = pow2(avg row length / 2) in [2, 32] and with
 // G0/2 and 2 G0 when the longest row fills them (only G0 when the caller
 // fixed group_size), and the tiles kernel (unless crs_kernel excludes
@@ -572,11 +611,23 @@ int plan_crs(pwm_matrix* h) {
                 if (g >= 1 && g <= 64 && (g == G0 || g <= std::max<int64_t>(1, h->stats.row_max))) gs.push_back(g);
         }
     }
-    const bool tiles = h->crs_kernel != 1;
     int rc;
+    h->rp = pwmk::RowsPlan{};
+    const bool vector_options = h->group_opt > 0 || h->vec_blocks_opt > 0 || h->long_row > 0;
+    if (h->crs_kernel == 0 && !vector_options && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
+    const bool rows = h->rp.nt > 0;
+    const bool tiles = !rows && h->crs_kernel != 1;
+    if (rows) {
+        gs.clear();
+        h->lr = pwmk::LongRows{};
+    }
     if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
     h->crs_nt_used = h->crs_nt > 0 ? 1 : 0;
-    if ((int)gs.size() + (tiles ? 1 : 0) == 1 && (!tiles || h->crs_nt >= 0)) {
+    if (rows && h->crs_nt >= 0) {
+        h->crs_used = 3;
+        return PWM_OK;
+    }
+    if (!rows && (int)gs.size() + (tiles ? 1 : 0) == 1 && (!tiles || h->crs_nt >= 0)) {
         h->crs_used = tiles ? 2 : 1;
         return plan_crs_vector(h, tiles ? G0 : gs[0]);
     }
@@ -590,16 +641,17 @@ int plan_crs(pwm_matrix* h) {
     if (e != hipSuccess) return hip_fail(h, e, "CRS autotune vectors");
     float best = -1.0f;
     int best_kernel = 1, best_g = G0, best_nt = 0;
-    if (tiles) {
+    if (rows || tiles) {
         // entry loads plain or non-temporal: the caller's choice, else both
+        const int kernel = rows ? 3 : 2;
         for (int nt : {0, 1}) {
             if (h->crs_nt >= 0 && nt != h->crs_nt) continue;
             h->crs_nt_used = nt;
             float ms = 0.0f;
-            if ((e = time_crs_kernel(h, 2, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
+            if ((e = time_crs_kernel(h, kernel, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
             if (best < 0.0f || ms < best) {
                 best = ms;
-                best_kernel = 2;
+                best_kernel = kernel;
                 best_nt = nt;
             }
         }
@@ -616,6 +668,7 @@ int plan_crs(pwm_matrix* h) {
         }
     }
     h->crs_used = best_kernel;
+    if (rows) return PWM_OK;
     return plan_crs_vector(h, best_kernel == 1 ? best_g : G0);
 }
 
@@ -656,7 +709,9 @@ int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw, int*
     switch (h->format) {
         case PWM_FORMAT_CRS:
             e = crs_kernel_launch(h, h->crs_used, x, y, pw);
-            np = h->crs_used == 2 ? (int)h->mp.P : h->vec_blocks;
+            np = h->crs_used == 3   ? (int)pwmk::rows_power_blocks(h->rp.nt)
+                 : h->crs_used == 2 ? (int)h->mp.P
+                                    : h->vec_blocks;
             break;
         case PWM_FORMAT_CRS_MERGE:
             e = pwmk::launch_merge_spmv(A, h->mp, x, y, pw, h->stream);
@@ -682,6 +737,7 @@ int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw, int*
 static int64_t partials_needed(const pwm_matrix* h) {
     switch (h->format) {
         case PWM_FORMAT_CRS:
+            if (h->crs_used == 3) return pwmk::rows_power_blocks(h->rp.nt);
             return std::max<int64_t>(h->vec_blocks, h->tiles.p ? h->mp.P + pwmk::merge_fix_blocks(h->mp.P) : 0);
         case PWM_FORMAT_CRS_MERGE: return h->mp.P + pwmk::merge_fix_blocks(h->mp.P);
         case PWM_FORMAT_CSB: return csb_partials(h);
@@ -856,6 +912,8 @@ static void reset_matrix(pwm_matrix* h) {
     h->lr = pwmk::LongRows{};
     h->mp = pwmk::MergePlan{};
     h->tiles.release();
+    h->rp = pwmk::RowsPlan{};
+    h->rows_cut.release();
     h->crs_used = 1;
     h->csb.clear();
     h->coh.clear();
@@ -1074,13 +1132,14 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
     out->nnz = h->nnz;
     out->format = h->format;
     out->value_type = h->vtype;
-    // CRS: the lanes per row of the vector kernel, 0 when the tiles kernel runs
+    // CRS: the lanes per row of the vector kernel, 0 when a tiles kernel runs
     out->group_size = h->format == PWM_FORMAT_CSB ? h->csb.groups
-                      : (h->format == PWM_FORMAT_CRS && h->crs_used == 2) ? 0
+                      : (h->format == PWM_FORMAT_CRS && h->crs_used >= 2) ? 0
                                                                            : h->group;
     out->long_rows = h->lr.n_rows;
     out->threads = (h->format == PWM_FORMAT_CRS_MERGE || (h->format == PWM_FORMAT_CRS && h->crs_used == 2))
                        ? (int32_t)h->mp.P
+                   : h->format == PWM_FORMAT_CRS && h->crs_used == 3 ? (int32_t)h->rp.nt
                    : h->format == PWM_FORMAT_BLOCKCOH ? (int32_t)h->coh.bands.size()
                    : h->format == PWM_FORMAT_CSB      ? (int32_t)h->csb.n_tasks
                                                       : h->vec_blocks;
@@ -1099,11 +1158,11 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
     if (h->format == PWM_FORMAT_CSB && h->csb.n_tasks <= 0) out->kernels = 0;
     out->high_occupancy = h->format == PWM_FORMAT_BLOCKCOH ? h->coh.occ8 : 0;
     out->non_temporal = h->format == PWM_FORMAT_CSB                         ? h->csb.nt
-                        : (h->format == PWM_FORMAT_CRS && h->crs_used == 2) ? h->crs_nt_used
+                        : (h->format == PWM_FORMAT_CRS && h->crs_used >= 2) ? h->crs_nt_used
                                                                            : 0;
     const pwm_impl::DevBuf* bufs[] = {&h->rs, &h->ci, &h->val, &h->lr_chunks, &h->lr_rows, &h->lr_begin,
                                       &h->lr_partial, &h->split_a, &h->split_b, &h->carry_row, &h->carry_val, &h->tiles,
-                                      &h->csb.ind, &h->csb.data, &h->csb.blk_ptr, &h->csb.work, &h->csb.ypart,
+                                      &h->rows_cut, &h->csb.ind, &h->csb.data, &h->csb.blk_ptr, &h->csb.work, &h->csb.ypart,
                                       &h->csb.soff, &h->csb.srows, &h->csb.sweep_start,
                                       &h->coh.row_jump, &h->coh.col_jump, &h->coh.data, &h->coh.row_jump_block,
                                       &h->coh.col_jump_block, &h->coh.block_nnz, &h->coh.block_coords,
@@ -1604,6 +1663,11 @@ static int launch_marked(pwm_matrix* h, const void* x, void* y, hipEvent_t mid) 
     hipError_t e = hipSuccess;
     switch (h->format) {
         case PWM_FORMAT_CRS:
+            if (h->crs_used == 3) {
+                e = pwmk::launch_rows(A, h->rp, x, y, nullptr, h->stream);
+                (void)hipEventRecord(mid, h->stream);
+                break;
+            }
             if (h->crs_used == 2) {
                 e = pwmk::launch_tiles_spmv(A, h->tiles.as<pwmk::ETile>(), h->mp, x, y, nullptr, h->stream);
                 (void)hipEventRecord(mid, h->stream);

@@ -184,13 +184,16 @@ struct pwm_matrix {
     int chunk = 4096;
     pwmk::LongRows lr;
     pwm_impl::DevBuf lr_chunks, lr_rows, lr_begin, lr_partial;
-    // CRS kernel: 0 = time the vector and tiles kernels at load and keep the
-    // faster, 1 = vector, 2 = tiles (row-aligned tiles, carries through the
-    // merge fix-up; the tiles plan lives in mp / split_* / carry_*)
+    // CRS kernel: 0 = wave tiles when the rows are short, else time the vector
+    // and tiles kernels at load and keep the faster, 1 = vector, 2 = tiles
+    // (row-aligned tiles, carries through the merge fix-up; the tiles plan
+    // lives in mp / split_* / carry_*).  crs_used: 1, 2, or 3 for wave tiles
     int crs_kernel = 0;
     int crs_used = 1;
+    pwmk::RowsPlan rp;
+    pwm_impl::DevBuf rows_cut;
     pwm_impl::DevBuf tiles;
-    int crs_nt = -1;          // tiles kernel: non-temporal entry loads (-1 = timed at load)
+    int crs_nt = -1;          // tiles and wave tiles: non-temporal entry loads (-1 = timed at load)
     int crs_nt_used = 0;
     bool tiles_carry = true;  // some tile is a merge tile (its carry needs the fix-up)
 

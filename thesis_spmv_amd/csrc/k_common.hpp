@@ -142,6 +142,17 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nblocks) {
     return xcd * per + (xcd < extra ? xcd : extra) + slot;
 }
 
+// Renumbering in stretches of 8 C blocks: inside a stretch XCD j works on the
+// j-th run of C consecutive items, so the chip reads one front of 8 C items
+// while neighbouring items still meet in an L2.  The blocks beyond the last
+// whole stretch are spread over the XCDs by xcd_remap.
+__device__ __forceinline__ int64_t xcd_chunked(int64_t b, int64_t nblocks, int64_t C) {
+    const int64_t stretch = 8 * C, s0 = b / stretch * stretch;
+    if (s0 + stretch > nblocks) return s0 + xcd_remap(b - s0, nblocks - s0);
+    const int64_t r = b - s0;
+    return s0 + (r % 8) * C + r / 8;
+}
+
 // One step of the device-side power method.  The host issues the steps in
 // order and passes each its number, so that a step's vectors are known without
 // reading device memory; only a stop test (tol >= 0) can end the loop early.

@@ -18,7 +18,7 @@ struct CrsDev {
     const int32_t* ci = nullptr;
     const void* val = nullptr;
     int vtype = VT_F64;
-    int nt = 0;  // tiles kernel: non-temporal col_ind / value loads
+    int nt = 0;  // tiles kernels: non-temporal col_ind / value loads
 };
 
 // A slice of one long row handled by one workgroup: entries [k0, k1) of row
@@ -68,6 +68,20 @@ struct ETile;
 int tiles_items_per_thread();
 hipError_t launch_tiles_spmv(const CrsDev& A, const ETile* tiles, const MergePlan& mp, const void* x, void* y,
                              const PowerArgs* pw, hipStream_t s);
+
+// CRS over wave tiles (k_rows.hip), for matrices of short rows: tile t holds
+// the rows [cut[t].x, cut[t+1].x) and entries [cut[t].y, cut[t+1].y).
+struct RowsPlan {
+    int64_t nt = 0;             // tiles (0: no plan)
+    const int2* cut = nullptr;  // [nt + 1]
+};
+// Entries between cuts for this longest row, 0 when it is too long.
+int64_t rows_step(int64_t row_max);
+int64_t rows_power_blocks(int64_t nt);  // workgroups (partial-sum slots) of a power step
+// Cuts of nt = ceil(nnz / step) tiles; sets *too_many_rows when one has more
+// rows than the kernel takes.
+hipError_t launch_rows_plan(const CrsDev& A, int64_t step, int64_t nt, int2* cut, int* too_many_rows, hipStream_t s);
+hipError_t launch_rows(const CrsDev& A, const RowsPlan& rp, const void* x, void* y, const PowerArgs* pw, hipStream_t s);
 
 // Power-mode carry fix-up runs in this many workgroups (each sums its share
 // of the tile partials into a second-level slot after the P tile slots).
