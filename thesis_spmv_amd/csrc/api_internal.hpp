@@ -94,6 +94,7 @@ struct CsbDev {
     int32_t sweep_wb = 0;
     int64_t sweep_W = 0;
     int32_t sweep_rows = 0;      // LDS rows of a slab (the largest slab)
+    int32_t sweep_acc32 = 0;     // FP32 LDS sums (FP32 storage whose slabs do not fit in FP64)
     DevBuf sweep_start;
     // sweep_order 1: inside a run the entries are in column order, the run
     // is padded to whole blocks of 256 (index 0xffffffff, value 0) and each
@@ -118,6 +119,7 @@ struct CsbDev {
         sweep_wb = 0;
         sweep_W = 0;
         sweep_rows = 0;
+        sweep_acc32 = 0;
         sweep_order = 0;
         sweep_len.clear();
         wide = 0;

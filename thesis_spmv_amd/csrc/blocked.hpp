@@ -8,10 +8,13 @@
 
 namespace blocked {
 
-// Rows of y one workgroup accumulates in LDS (FP64: 32 KB, FP32: 32 KB).
-inline int lds_rows(int vtype) { return vtype == 0 ? 4096 : 8192; }
-constexpr int kLdsRowsF64 = 4096;
-constexpr int kLdsRowsF32 = 8192;
+// Rows of y are summed in LDS in FP64 whatever the storage type: an LDS atomic
+// add of 64 lanes takes 21 clocks in FP64 and 193 in FP32 (ds_add_f32 serves
+// one lane after the other; both measured on random rows), which held every
+// FP32 kernel here to 180 G entries/s.  Rows per workgroup: a CSB slab 32 KB,
+// a BlockCOH band up to 32 KB (FP64 storage) or 64 KB.
+constexpr int kCsbLdsRows = 4096;
+inline int coh_lds_rows(int vtype) { return vtype == 0 ? 4096 : 8192; }
 
 // A contiguous run [start, end) of CSB entries: the part of one block that
 // falls into one workgroup's row slab.
@@ -60,13 +63,14 @@ struct CsbArgs {
     int32_t wb = 0;
     int64_t W = 0;
     int32_t max_rows = 0;
+    int32_t acc32 = 0;       // 1: FP32 LDS sums (FP32 storage whose slabs do not fit in FP64)
     int32_t sync_every = 1;  // windows between workgroup barriers (a power of two)
     const int32_t* sstart = nullptr;
 };
 
 // Swept slabs: workgroups of the sweep kernel one CU holds at once with
-// `rows` LDS rows of the value type's accumulator (0 if none fit).
-int csb_sweep_blocks_per_cu(int vtype, int rows);
+// `rows` LDS rows, FP64 or (acc32) FP32 (0 if none fit).
+int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32);
 
 
 // One BlockCOH block (offsets are relative to its band's arrays).

@@ -68,7 +68,7 @@ hipError_t upload(DevBuf& d, const void* src, size_t bytes) {
 // A swept-slab layout set aside while the other layouts are built and timed.
 struct SweptSave {
     DevBuf ind, data, soff, start;
-    int32_t wb = 0, rows = 0, nt = 1, order = 0;
+    int32_t wb = 0, rows = 0, nt = 1, order = 0, acc32 = 0;
     int64_t W = 0, T = 0;
     std::vector<int32_t> len;
     void take(CsbDev& c) {
@@ -82,6 +82,7 @@ struct SweptSave {
         wb = c.sweep_wb;
         W = c.sweep_W;
         rows = c.sweep_rows;
+        acc32 = c.sweep_acc32;
         T = c.n_tasks;
         nt = c.nt;
         c.sweep = 0;
@@ -100,6 +101,7 @@ struct SweptSave {
         c.sweep_wb = wb;
         c.sweep_W = W;
         c.sweep_rows = rows;
+        c.sweep_acc32 = acc32;
         c.n_tasks = T;
         c.nt = nt;
         c.stream = 0;
@@ -198,21 +200,28 @@ static int build_swept(pwm_matrix* h, const int32_t* rs) {
     hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, 0);
     if (e != hipSuccess) return hip_fail(h, e, "CSB swept slabs: device attributes");
-    const int acc = h->vtype == PWM_VALUES_F64 ? 8 : 4;
+    const int xb = h->vtype == PWM_VALUES_F64 ? 8 : 4;
     const int64_t slabs = (int64_t)std::max(1, cus) * h->csb_sweep_waves;
     int wb = h->csb_window_bits;
     if (wb == 0) {
         wb = 10;
-        while (((int64_t)acc << (wb + 1)) <= ((int64_t)1 << 20)) ++wb;
+        while (((int64_t)xb << (wb + 1)) <= ((int64_t)1 << 20)) ++wb;
         // the packed index keeps 32 - wb bits for the row in the slab: narrow
         // the window while the slabs' expected rows (a fifth of slack) need more
         const int64_t rows_needed = (h->nor + slabs - 1) / slabs * 6 / 5;
         while (wb > 12 && (((int64_t)1 << (32 - wb)) - 1) < rows_needed) --wb;
     }
-    const int64_t rows_cap = std::min<int64_t>(((lds_cu - 1024) / acc) & ~(int64_t)63, ((int64_t)1 << (32 - wb)) - 1);
-    if (rows_cap <= 0 || blocked::csb_sweep_blocks_per_cu(h->vtype, (int)rows_cap) < 1)
-        return fail(h, PWM_ERR_UNSUPPORTED, "CSB swept slabs: no workgroup with LDS rows fits a CU");
-    const int rc = csb_sweep_device(h, rs, slabs, rows_cap, slabs, wb);
+    // FP64 sums in LDS; FP32 storage whose slabs need more rows than that
+    // holds takes (slower) FP32 sums
+    int64_t rows_cap = 0;
+    int rc = PWM_ERR_UNSUPPORTED;
+    for (int acc = 8; acc >= xb && rc == PWM_ERR_UNSUPPORTED; acc -= 4) {
+        c.sweep_acc32 = acc == 4;
+        rows_cap = std::min<int64_t>(((lds_cu - 1024) / acc) & ~(int64_t)63, ((int64_t)1 << (32 - wb)) - 1);
+        if (rows_cap <= 0 || blocked::csb_sweep_blocks_per_cu(h->vtype, (int)rows_cap, acc == 4) < 1)
+            return fail(h, PWM_ERR_UNSUPPORTED, "CSB swept slabs: no workgroup with LDS rows fits a CU");
+        rc = csb_sweep_device(h, rs, slabs, rows_cap, slabs, wb);
+    }
     if (rc == PWM_ERR_UNSUPPORTED)
         return fail(h, rc, "CSB swept slabs: the rows do not fit " + std::to_string(slabs) + " slabs of at most " +
                                std::to_string(rows_cap) + " rows (the LDS of one workgroup per CU)");
@@ -261,7 +270,8 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
     // key (slab, block column, Z-Morton code) would need more than 64 bits;
     // they are sorted on the device too (key: block, Z-Morton code), or
     // built on the host with csb_build = 1.
-    const int lds_bits = blocked::lds_rows(h->vtype) == 8192 ? 13 : 12;
+    const int lds_bits = 12;
+    static_assert(blocked::kCsbLdsRows == 1 << 12, "slabs of 2^lds_bits rows fill the LDS rows");
     int cb = 0;
     while (((int64_t)1 << cb) < noc) ++cb;
     // no longer than needed for about 4096 slabs (16 workgroups per CU),
@@ -308,7 +318,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
         if (rc != PWM_OK) return rc;
     } else if (h->csb_build != 1 && csb_key_bits(V * H, bits) <= 64) {
         // slab pieces over the stored order, sorted on the device
-        const int64_t lds_rows = (int64_t)blocked::lds_rows(h->vtype);
+        const int64_t lds_rows = blocked::kCsbLdsRows;
         int k = 0;
         while ((beta >> k) > lds_rows) ++k;
         rc = csb_pieces_device(h, k);
@@ -362,7 +372,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
         // lives in LDS).  With slab = beta >> k, the entries of one block whose
         // top k row bits equal s form 2^(k-1) contiguous Z-order runs (one per
         // value of the top k-1 column bits), or the whole block when k = 0.
-        const int64_t lds_rows = (int64_t)blocked::lds_rows(h->vtype);
+        const int64_t lds_rows = blocked::kCsbLdsRows;
         int k = 0;
         while ((beta >> k) > lds_rows) ++k;
         const int64_t slab = beta >> k;
@@ -587,7 +597,7 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
     int rc = PWM_OK;
     if (!device) check_bf16(h, vals, nnz, &rc);
     if (rc != PWM_OK) return rc;
-    const int64_t lds_rows = blocked::lds_rows(h->vtype);
+    const int64_t lds_rows = blocked::coh_lds_rows(h->vtype);
     std::vector<int64_t> bstart, bnnz;
     int threads = h->threads;
     auto clamp = [&](int t) {  // BlockCOH.hpp:325-328 (kept >= 1)
@@ -842,6 +852,7 @@ hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     a.wb = h->csb.sweep_wb;
     a.W = h->csb.sweep_W;
     a.max_rows = h->csb.sweep_rows;
+    a.acc32 = h->csb.sweep_acc32;
     a.sync_every = h->csb_sync_every;
     if (a.sweep) a.unroll = h->csb_sweep_unroll;
     a.sstart = h->csb.sweep_start.as<int32_t>();

@@ -1,7 +1,8 @@
 // CSB and BlockCOH SpMV kernels for gfx950.
 //
 // Both formats are processed by workgroups that own a slab of rows and keep
-// its y-slice in LDS (FP64 or FP32 atomic adds, ds_add_*): every entry of a
+// its y-slice in LDS (FP64 atomic adds, ds_add_f64, for every storage type:
+// products are formed in the vectors' type and summed in FP64): every entry of a
 // slab, wherever its block sits in the block row or band, adds into LDS and
 // the slab is written to y once with coalesced stores.
 //
@@ -39,11 +40,6 @@ using pwmk::widen;
 constexpr int kBS = kBlockedBS;
 constexpr int kWaves = kBS / 64;
 constexpr int kWin = 2 * kBS;  // CSB pieces staged per window
-
-template <typename Acc>
-struct LdsRows;
-template <> struct LdsRows<double> { static constexpr int v = kLdsRowsF64; };
-template <> struct LdsRows<float> { static constexpr int v = kLdsRowsF32; };
 
 // Block-wide exclusive scan of one int per thread; returns the prefix and
 // writes the total to *total.  `tmp` holds kWaves ints.
@@ -131,7 +127,7 @@ __device__ __forceinline__ void csb_task(const CsbArgs& a, int& g, int64_t& t) {
 // Writes a slab's LDS sums: to ypart[g] with several column groups, else to
 // y (POWER: scaled, with the slab's |y|^2, x.y, x.x in partial slot t).
 template <typename X, typename Acc, int BS, bool POWER, bool NT = false>
-__device__ __forceinline__ void csb_write_slab(const CsbArgs& a, const Acc* ylds, int h, int64_t row0, int g, int64_t t,
+__device__ __forceinline__ void csb_write_slab(const CsbArgs& a, const double* ylds, int h, int64_t row0, int g, int64_t t,
                                                const X* __restrict__ x, X* __restrict__ y, double scale,
                                                const PowerArgs& pw, double* red) {
     const int tid = threadIdx.x;
@@ -141,9 +137,9 @@ __device__ __forceinline__ void csb_write_slab(const CsbArgs& a, const Acc* ylds
             const int64_t row = row0 + i;
             if (row >= a.nor) break;
             if constexpr (NT)
-                __builtin_nontemporal_store(ylds[i], &yp[row]);
+                __builtin_nontemporal_store((Acc)ylds[i], &yp[row]);
             else
-                yp[row] = ylds[i];
+                yp[row] = (Acc)ylds[i];
         }
         return;
     }
@@ -152,7 +148,7 @@ __device__ __forceinline__ void csb_write_slab(const CsbArgs& a, const Acc* ylds
         const int64_t row = row0 + i;
         if (row >= a.nor) break;
         if constexpr (POWER) {
-            const X out = (X)((double)ylds[i] * scale);
+            const X out = (X)(ylds[i] * scale);
             y[row] = out;
             const double yd = (double)out, xd = (double)x[row] * scale;
             yy += yd * yd;
@@ -177,8 +173,7 @@ __global__ __launch_bounds__(kBS) void k_csb(CsbArgs a, const typename Arith<VT>
                                              typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
-    constexpr int LR = LdsRows<Acc>::v;
-    __shared__ Acc ylds[LR];
+    __shared__ double ylds[kCsbLdsRows];
     __shared__ int32_t p_start[kWin];
     __shared__ int32_t p_pre[kWin + 1];
     __shared__ int scan_tmp[kWaves];
@@ -264,7 +259,7 @@ __global__ __launch_bounds__(kBS) void k_csb(CsbArgs a, const typename Arith<VT>
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                if (ok[u]) atomicAdd(&ylds[(int)(w[u] >> 16) - slab_base], vv[u] * xv[u]);
+                if (ok[u]) atomicAdd(&ylds[(int)(w[u] >> 16) - slab_base], (double)(vv[u] * xv[u]));
         }
     }
     __syncthreads();
@@ -287,7 +282,7 @@ __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename A
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     extern __shared__ __align__(16) unsigned char csb_smem[];
-    Acc* ylds = (Acc*)csb_smem;
+    double* ylds = (double*)csb_smem;
     __shared__ double red[48];
 
     const X* __restrict__ x = x_arg;
@@ -348,7 +343,7 @@ __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename A
                     row = ((j < 2 ? r[u].x : r[u].y) >> (16 * (j & 1))) & 0xffffu;
                 else
                     row = (uint32_t)w[u][j] >> cb;
-                if (k >= e0 && k < e1) atomicAdd(&ylds[row], (Acc)v[u].get(j) * (Acc)xv[u][j]);
+                if (k >= e0 && k < e1) atomicAdd(&ylds[row], (double)((Acc)v[u].get(j) * (Acc)xv[u][j]));
             }
     }
     __syncthreads();
@@ -448,9 +443,10 @@ struct SweepChunk {
     }
 };
 
-template <typename VT, int kSU, bool NT, typename X, typename Acc>
+template <typename VT, int kSU, bool NT, typename X, typename LAcc>
 __device__ __forceinline__ void sweep_add(const SweepChunk<VT, kSU, NT>& c, int32_t qb, int lane, int32_t e0, int32_t e1,
-                                          const X* __restrict__ xw, uint32_t wmask, int wb, Acc* ylds) {
+                                          const X* __restrict__ xw, uint32_t wmask, int wb, LAcc* ylds) {
+    using Acc = typename Arith<VT>::A;
     // an entry outside [e0, e1) belongs to a neighbouring run (its column is
     // in another window), and an index 0xffffffff pads a column-ordered run:
     // such an entry gathers the window's first column, which exists, and
@@ -469,19 +465,20 @@ __device__ __forceinline__ void sweep_add(const SweepChunk<VT, kSU, NT>& c, int3
     for (int u = 0; u < kSU; ++u)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (ok[u][j]) atomicAdd(&ylds[(uint32_t)c.w[u][j] >> wb], (Acc)c.v[u].get(j) * (Acc)xv[u][j]);
+            if (ok[u][j]) atomicAdd(&ylds[(uint32_t)c.w[u][j] >> wb], (LAcc)((Acc)c.v[u].get(j) * (Acc)xv[u][j]));
 }
 
-template <typename VT, bool POWER, bool NT, int SU = 2>
+// LAcc: the LDS sums' type (float only for FP32 storage whose slabs have more
+// rows than fit in FP64).
+template <typename VT, bool POWER, bool NT, typename LAcc, int SU = 2>
 __global__ __launch_bounds__(kSwBS) void k_csb_sweep(CsbArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
                                                      typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
-    using Acc = typename Arith<VT>::A;
     constexpr int kSU = SU;  // groups of 4 entries per lane per chunk
     constexpr int kWv = kSwBS / 64;
     constexpr int kChunk = 64 * kSU;  // groups of 4 entries per wave per chunk
     extern __shared__ __align__(16) unsigned char csb_smem[];
-    Acc* ylds = (Acc*)csb_smem;
+    LAcc* ylds = (LAcc*)csb_smem;
     __shared__ double red[48];
 
     const X* __restrict__ x = x_arg;
@@ -554,23 +551,22 @@ __global__ __launch_bounds__(kSwBS) void k_csb_sweep(CsbArgs a, const typename A
     }
 }
 
-template <typename VT>
+template <typename VT, typename LAcc>
 static int sweep_blocks_t(int rows) {
-    using Acc = typename Arith<VT>::A;
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_csb_sweep<VT, false, true>, kSwBS,
-                                                     (size_t)rows * sizeof(Acc)) != hipSuccess) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_csb_sweep<VT, false, true, LAcc>, kSwBS,
+                                                     (size_t)rows * sizeof(LAcc)) != hipSuccess) {
         (void)hipGetLastError();
         return 0;
     }
     return nb;
 }
 
-int csb_sweep_blocks_per_cu(int vtype, int rows) {
+int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32) {
     switch (vtype) {
-        case 0: return sweep_blocks_t<double>(rows);
-        case 1: return sweep_blocks_t<float>(rows);
-        case 2: return sweep_blocks_t<bf16_t>(rows);
+        case 0: return sweep_blocks_t<double, double>(rows);
+        case 1: return acc32 ? sweep_blocks_t<float, float>(rows) : sweep_blocks_t<float, double>(rows);
+        case 2: return acc32 ? sweep_blocks_t<bf16_t, float>(rows) : sweep_blocks_t<bf16_t, double>(rows);
     }
     return 0;
 }
@@ -593,9 +589,9 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     // the LDS window holds the rows of the largest band accumulated in LDS
-    // (at most LdsRows<Acc>::v), sized at launch
+    // (at most coh_lds_rows), sized at launch
     extern __shared__ __align__(16) unsigned char coh_smem[];
-    Acc* ylds = (Acc*)coh_smem;
+    double* ylds = (double*)coh_smem;
     __shared__ int32_t bstart[kCohChunk + 2];  // up to kCohChunk+1 blocks and a sentinel
     // the records of the chunk's blocks when there are at most kCohStage of
     // them (the usual case), so the decode reads them from LDS
@@ -727,7 +723,7 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
                     xi = xi < a.noc ? xi : a.noc - 1;
                     const Acc p = vv[j] * (Acc)x[xi];
                     if (lds) {
-                        atomicAdd(&ylds[row], p);
+                        atomicAdd(&ylds[row], (double)p);
                     } else {
                         // atomic tasks add the scaled product: y rows of big
                         // bands are final once every task has finished
@@ -748,7 +744,7 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
     for (int i = tid; i < band.rows; i += kBS) {
         const int64_t row = (int64_t)band.start + i;
         if constexpr (POWER) {
-            const X out = (X)((double)ylds[i] * scale);
+            const X out = (X)(ylds[i] * scale);
             y[row] = out;
             const double yd = (double)out, xd = (double)x[row] * scale;
             yy += yd * yd;
@@ -833,15 +829,17 @@ static hipError_t csb_t(const CsbArgs& a, const void* x, void* y, const PowerArg
     if (a.n_tasks <= 0) return hipSuccess;
     if (a.sweep) {
         if (part == 2) return hipSuccess;  // no column-group reduction
-        const size_t lds = (size_t)a.max_rows * sizeof(Acc);
-        auto pick = [&](auto power) {
+        const bool acc32 = sizeof(Acc) == 4 && a.acc32;
+        const size_t lds = (size_t)a.max_rows * (acc32 ? sizeof(Acc) : sizeof(double));
+        auto pick = [&](auto power, auto acc) {
             constexpr bool P = decltype(power)::value;
-            if (a.unroll == 1) return a.nt ? k_csb_sweep<VT, P, true, 1> : k_csb_sweep<VT, P, false, 1>;
-            if (a.unroll == 4) return a.nt ? k_csb_sweep<VT, P, true, 4> : k_csb_sweep<VT, P, false, 4>;
-            return a.nt ? k_csb_sweep<VT, P, true, 2> : k_csb_sweep<VT, P, false, 2>;
+            using L = decltype(acc);
+            if (a.unroll == 1) return a.nt ? k_csb_sweep<VT, P, true, L, 1> : k_csb_sweep<VT, P, false, L, 1>;
+            if (a.unroll == 4) return a.nt ? k_csb_sweep<VT, P, true, L, 4> : k_csb_sweep<VT, P, false, L, 4>;
+            return a.nt ? k_csb_sweep<VT, P, true, L, 2> : k_csb_sweep<VT, P, false, L, 2>;
         };
-        auto kp = pick(std::true_type{});
-        auto kf = pick(std::false_type{});
+        auto kp = acc32 ? pick(std::true_type{}, Acc{}) : pick(std::true_type{}, 0.0);
+        auto kf = acc32 ? pick(std::false_type{}, Acc{}) : pick(std::false_type{}, 0.0);
         if (pw)
             hipLaunchKernelGGL(kp, dim3((unsigned)a.n_tasks), dim3(kSwBS), lds, s, a, (const X*)nullptr, (X*)nullptr,
                                *pw);
@@ -852,7 +850,7 @@ static hipError_t csb_t(const CsbArgs& a, const void* x, void* y, const PowerArg
     if (part == 2) {
         // the column-group reduction only
     } else if (a.stream) {
-        const size_t lds = (size_t)a.slab_rows * sizeof(Acc);
+        const size_t lds = (size_t)a.slab_rows * sizeof(double);
         const dim3 grid((unsigned)a.n_tasks);
         // kernel instance for (power step, unroll, non-temporal)
         auto pick = [&](auto power, auto wide) {
@@ -897,9 +895,8 @@ template <typename VT>
 static hipError_t coh_t(const CohArgs& a, const int32_t* atomic_bands, int n_atomic, const void* x, void* y,
                         const PowerArgs* pw, hipStream_t s) {
     using X = typename Arith<VT>::X;
-    using Acc = typename Arith<VT>::A;
     if (a.n_tasks <= 0) return hipSuccess;
-    const size_t lds = (size_t)std::max<int32_t>(a.lds_rows, 1) * sizeof(Acc);
+    const size_t lds = (size_t)std::max<int32_t>(a.lds_rows, 1) * sizeof(double);
     if (pw) {
         if (n_atomic > 0)
             hipLaunchKernelGGL((k_coh_zero<VT, true>), dim3(n_atomic), dim3(kBS), 0, s, a, atomic_bands, (X*)nullptr,
