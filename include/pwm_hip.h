@@ -154,7 +154,10 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * stored window by window (1 MB of x per window) and every workgroup
  * walking the windows in order; 0 = automatic: 2 when slabs of at least 256
  * rows pack, else 3, replaced by 4 when x exceeds 2 MB, the slabs fit and 4
- * runs faster in the load-time timing), "csb_window_bits" (swept slabs: log2 of the
+ * runs faster in the load-time timing; on CRS and CRS_MERGE handles: 0 = swept
+ * slabs are kept beside the CRS arrays and swept in a fixed order when x
+ * exceeds 4 MB, the columns are scattered and they run faster in the load-time
+ * timing, 4 = always when they fit, 1 to 3 = never), "csb_window_bits" (swept slabs: log2 of the
  * columns per window, 0 = 1 MB of x), "csb_sync_every" (swept slabs: windows
  * between workgroup barriers, 1, 2, 4 or 8, default 2), "csb_sweep_unroll"
  * (swept slabs: groups of 4 entries per lane per chunk, 1, 2 or 4, default 2),

@@ -457,6 +457,11 @@ static int plan_crs_tiles(pwm_matrix* h) {
 static hipError_t crs_kernel_launch(pwm_matrix* h, int which, const void* x, void* y, const PowerArgs* pw) {
     const CrsDev A = crs_of(h);
     hipError_t e;
+    if (which == 0) {  // CRS_MERGE
+        e = pwmk::launch_merge_spmv(A, h->mp, x, y, pw, h->stream);
+        if (e == hipSuccess) e = pwmk::launch_merge_fixup(A, h->mp, y, pw, h->stream);
+        return e;
+    }
     if (which == 3) {
         e = pwmk::launch_rows(A, h->rp, x, y, pw, h->stream);
         if (e == hipSuccess && pw) e = pwmk::launch_power_reduce(*pw, pwmk::rows_power_blocks(h->rp.nt), h->stream);
@@ -491,6 +496,82 @@ static hipError_t time_crs_kernel(pwm_matrix* h, int which, const void* x, void*
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     return e;
+}
+
+constexpr int64_t kXcdL2 = (int64_t)4 << 20;  // an XCD's L2
+
+// Whether the columns are scattered: x beyond one XCD's L2, and 256
+// consecutive entries touch more than 128 lines of x on average (banded
+// matrices and stencils some 20 to 60, uniformly random columns all 256).  A
+// sweep in row order then fetches about one 128-byte line per entry from
+// beyond the L2.
+static hipError_t columns_scattered(pwm_matrix* h, bool* scattered) {
+    *scattered = false;
+    const int64_t xb = (int64_t)vector_size(h->vtype);
+    if (h->noc * xb <= kXcdL2 || h->nnz < 256) return hipSuccess;
+    const int64_t groups = std::min<int64_t>(h->nnz / 256, 2048);
+    DevBuf lines;
+    unsigned n = 0;
+    hipError_t e = lines.alloc(4);
+    if (e == hipSuccess) e = hipMemsetAsync(lines.p, 0, 4, h->stream);
+    if (e == hipSuccess)
+        e = pwmk::launch_scatter(h->ci.as<int32_t>(), h->nnz, groups, xb == 8 ? 4 : 5, lines.as<unsigned>(), h->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&n, lines.p, 4, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    *scattered = n > 128 * (uint64_t)groups;
+    return e;
+}
+
+// Average time of 5 SpMVs (after 2 warm-up ones) of the swept slabs beside the
+// CRS arrays, entry loads plain or non-temporal, the faster kept.
+static hipError_t time_swept(pwm_matrix* h, const void* x, void* y, float* best) {
+    hipEvent_t a, b;
+    (void)hipEventCreate(&a);
+    (void)hipEventCreate(&b);
+    hipError_t e = hipSuccess;
+    int best_nt = 0;
+    *best = -1.0f;
+    for (int nt = 0; nt < 2 && e == hipSuccess; ++nt) {
+        h->csb.nt = nt;
+        for (int i = 0; i < 2 && e == hipSuccess; ++i) e = csb_launch(h, x, y, nullptr);
+        (void)hipEventRecord(a, h->stream);
+        for (int i = 0; i < 5 && e == hipSuccess; ++i) e = csb_launch(h, x, y, nullptr);
+        (void)hipEventRecord(b, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        float ms = 0.0f;
+        (void)hipEventElapsedTime(&ms, a, b);
+        if (*best < 0.0f || ms < *best) {
+            *best = ms;
+            best_nt = nt;
+        }
+    }
+    h->csb.nt = best_nt;
+    (void)hipEventDestroy(a);
+    (void)hipEventDestroy(b);
+    return e;
+}
+
+// Swept slabs for scattered columns (k_csb_sweep, turns): built beside the CRS
+// arrays and timed into *ms, on a vector of ones x; *ms < 0 when not built.
+// csb_layout = 4 builds them for any columns and returns 0 ms (always the
+// faster), 1 to 3 never.  Power-law rows of 16 entries, warm: FP64 1.2 M rows
+// 228 -> 76 us, 2.1 M 487 -> 161; FP32 3 M 586 -> 159; below 4 MB of x the row
+// order is at most a third slower (FP64 600 000 rows, 4.8 MB: 85 -> 60 us) and
+// the build is not worth its time (8 ms at 1.2 M rows).
+static int plan_swept(pwm_matrix* h, const void* x, void* y, float* ms) {
+    *ms = -1.0f;
+    h->csb.clear();
+    const bool asked = h->csb_layout == 4;
+    bool scattered = asked && h->nnz > 0;
+    hipError_t e = hipSuccess;
+    if (h->csb_layout == 0 && (e = columns_scattered(h, &scattered)) != hipSuccess)
+        return hip_fail(h, e, "column scatter");
+    if (!scattered) return PWM_OK;
+    const int rc = build_swept_beside_crs(h);
+    if (rc != PWM_OK || !h->csb.sweep) return rc;
+    if ((e = time_swept(h, x, y, ms)) != hipSuccess) return hip_fail(h, e, "swept slabs");
+    if (asked) *ms = 0.0f;
+    return PWM_OK;
 }
 
 // CRS vector kernel with G lanes per row: grid size and the long-row chunk
@@ -613,8 +694,9 @@ int plan_crs(pwm_matrix* h) {
     }
     int rc;
     h->rp = pwmk::RowsPlan{};
-    const bool vector_options = h->group_opt > 0 || h->vec_blocks_opt > 0 || h->long_row > 0;
-    if (h->crs_kernel == 0 && !vector_options && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
+    h->csb.clear();
+    const bool automatic = h->crs_kernel == 0 && h->group_opt == 0 && h->vec_blocks_opt == 0 && h->long_row == 0;
+    if (automatic && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
     const bool rows = h->rp.nt > 0;
     const bool tiles = !rows && h->crs_kernel != 1;
     if (rows) {
@@ -639,8 +721,9 @@ int plan_crs(pwm_matrix* h) {
         return hip_fail(h, e, "CRS autotune vectors");
     e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "CRS autotune vectors");
-    float best = -1.0f;
+    float best = -1.0f, swept = -1.0f;
     int best_kernel = 1, best_g = G0, best_nt = 0;
+    if (automatic && h->crs_nt < 0 && (rc = plan_swept(h, x.p, y.p, &swept)) != PWM_OK) return rc;
     if (rows || tiles) {
         // entry loads plain or non-temporal: the caller's choice, else both
         const int kernel = rows ? 3 : 2;
@@ -657,6 +740,9 @@ int plan_crs(pwm_matrix* h) {
         }
     }
     h->crs_nt_used = best_nt;
+    // the vector kernel gathers in row order like the tiles and was never a
+    // third faster than they: it is not timed against a sweep that is
+    if (swept >= 0.0f && swept < 0.7f * best) gs.clear();
     for (int g : gs) {
         if ((rc = plan_crs_vector(h, g)) != PWM_OK) return rc;
         float ms = 0.0f;
@@ -668,7 +754,13 @@ int plan_crs(pwm_matrix* h) {
         }
     }
     h->crs_used = best_kernel;
+    if (swept >= 0.0f && swept >= best) h->csb.clear();
     if (rows) return PWM_OK;
+    if (h->csb.sweep) {
+        h->lr = pwmk::LongRows{};
+        h->vec_blocks = 0;
+        return PWM_OK;
+    }
     return plan_crs_vector(h, best_kernel == 1 ? best_g : G0);
 }
 
@@ -699,43 +791,44 @@ int plan_merge(pwm_matrix* h) {
     e = pwmk::launch_merge_splits(crs_of(h), h->mp, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "merge split search");
+    // scattered columns: swept slabs when they time faster than the merge
+    // kernels (not when the caller chose the partition or the tile size)
+    h->csb.clear();
+    if ((h->threads > 0 && P == h->threads) || h->ipt != 8) return PWM_OK;
+    if (h->csb_layout != 4 && h->noc * (int64_t)vector_size(h->vtype) <= kXcdL2) return PWM_OK;
+    DevBuf x, y;
+    const size_t vs = vector_size(h->vtype);
+    if ((e = x.alloc(h->noc * vs)) != hipSuccess || (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess ||
+        (e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream)) != hipSuccess)
+        return hip_fail(h, e, "merge plan vectors");
+    float swept = -1.0f, ms = 0.0f;
+    const int rc = plan_swept(h, x.p, y.p, &swept);
+    if (rc != PWM_OK || swept < 0.0f) return rc;
+    if ((e = time_crs_kernel(h, 0, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "merge plan");
+    if (swept >= ms) h->csb.clear();
     return PWM_OK;
 }
 
-int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw, int* n_partials_out) {
-    const CrsDev A = crs_of(h);
+// A CRS or CRS_MERGE handle whose SpMV sweeps its slabs.
+static bool swept_crs(const pwm_matrix* h) {
+    return (h->format == PWM_FORMAT_CRS || h->format == PWM_FORMAT_CRS_MERGE) && h->csb.sweep;
+}
+
+int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw) {
     hipError_t e = hipSuccess;
-    int np = 0;
-    switch (h->format) {
-        case PWM_FORMAT_CRS:
-            e = crs_kernel_launch(h, h->crs_used, x, y, pw);
-            np = h->crs_used == 3   ? (int)pwmk::rows_power_blocks(h->rp.nt)
-                 : h->crs_used == 2 ? (int)h->mp.P
-                                    : h->vec_blocks;
-            break;
-        case PWM_FORMAT_CRS_MERGE:
-            e = pwmk::launch_merge_spmv(A, h->mp, x, y, pw, h->stream);
-            if (e == hipSuccess) e = pwmk::launch_merge_fixup(A, h->mp, y, pw, h->stream);
-            np = (int)h->mp.P;
-            break;
-        case PWM_FORMAT_CSB:
-            e = csb_launch(h, x, y, pw);
-            np = (int)csb_partials(h);
-            break;
-        case PWM_FORMAT_BLOCKCOH:
-            e = coh_launch(h, x, y, pw);
-            np = (int)coh_partials(h);
-            break;
-        default:
-            return fail(h, PWM_ERR_INVALID, "unknown format");
+    switch (swept_crs(h) ? PWM_FORMAT_CSB : h->format) {
+        case PWM_FORMAT_CRS: e = crs_kernel_launch(h, h->crs_used, x, y, pw); break;
+        case PWM_FORMAT_CRS_MERGE: e = crs_kernel_launch(h, 0, x, y, pw); break;
+        case PWM_FORMAT_CSB: e = csb_launch(h, x, y, pw); break;
+        case PWM_FORMAT_BLOCKCOH: e = coh_launch(h, x, y, pw); break;
+        default: return fail(h, PWM_ERR_INVALID, "unknown format");
     }
-    if (n_partials_out) *n_partials_out = np;
     if (e != hipSuccess) return hip_fail(h, e, "SpMV launch");
     return PWM_OK;
 }
 
 static int64_t partials_needed(const pwm_matrix* h) {
-    switch (h->format) {
+    switch (swept_crs(h) ? PWM_FORMAT_CSB : h->format) {
         case PWM_FORMAT_CRS:
             if (h->crs_used == 3) return pwmk::rows_power_blocks(h->rp.nt);
             return std::max<int64_t>(h->vec_blocks, h->tiles.p ? h->mp.P + pwmk::merge_fix_blocks(h->mp.P) : 0);
@@ -1134,10 +1227,11 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
     out->value_type = h->vtype;
     // CRS: the lanes per row of the vector kernel, 0 when a tiles kernel runs
     out->group_size = h->format == PWM_FORMAT_CSB ? h->csb.groups
-                      : (h->format == PWM_FORMAT_CRS && h->crs_used >= 2) ? 0
+                      : (h->format == PWM_FORMAT_CRS && (h->crs_used >= 2 || swept_crs(h))) ? 0
                                                                            : h->group;
     out->long_rows = h->lr.n_rows;
-    out->threads = (h->format == PWM_FORMAT_CRS_MERGE || (h->format == PWM_FORMAT_CRS && h->crs_used == 2))
+    out->threads = swept_crs(h) && h->format == PWM_FORMAT_CRS ? (int32_t)h->csb.n_tasks
+                   : (h->format == PWM_FORMAT_CRS_MERGE || (h->format == PWM_FORMAT_CRS && h->crs_used == 2))
                        ? (int32_t)h->mp.P
                    : h->format == PWM_FORMAT_CRS && h->crs_used == 3 ? (int32_t)h->rp.nt
                    : h->format == PWM_FORMAT_BLOCKCOH ? (int32_t)h->coh.bands.size()
@@ -1155,9 +1249,10 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
         case PWM_FORMAT_CSB: out->kernels = h->csb.sweep ? 1 : 1 + (h->csb.groups > 1 ? 1 : 0); break;
         case PWM_FORMAT_BLOCKCOH: out->kernels = 1 + (h->coh.n_atomic > 0 ? 1 : 0); break;
     }
+    if (swept_crs(h)) out->kernels = 1;
     if (h->format == PWM_FORMAT_CSB && h->csb.n_tasks <= 0) out->kernels = 0;
     out->high_occupancy = h->format == PWM_FORMAT_BLOCKCOH ? h->coh.occ8 : 0;
-    out->non_temporal = h->format == PWM_FORMAT_CSB                         ? h->csb.nt
+    out->non_temporal = h->format == PWM_FORMAT_CSB || swept_crs(h)         ? h->csb.nt
                         : (h->format == PWM_FORMAT_CRS && h->crs_used >= 2) ? h->crs_nt_used
                                                                            : 0;
     const pwm_impl::DevBuf* bufs[] = {&h->rs, &h->ci, &h->val, &h->lr_chunks, &h->lr_rows, &h->lr_begin,
@@ -1223,7 +1318,7 @@ extern "C" int pwm_mv_device(pwm_matrix* h, const void* x, void* y) {
     if (xb < yb + h->nor * vs && yb < xb + h->noc * vs)
         return fail(h, PWM_ERR_INVALID, "pwm_mv_device: x and y overlap");
     if (int rc0 = check_device_xy(h, x, h->noc, y, h->nor, "pwm_mv_device")) return rc0;
-    int rc = spmv_launch(h, x, y, nullptr, nullptr);
+    int rc = spmv_launch(h, x, y, nullptr);
     if (rc != PWM_OK) return rc;
     hipError_t e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "pwm_mv_device");
@@ -1277,7 +1372,7 @@ extern "C" int pwm_mv(pwm_matrix* h, const double* x, double* y) {
     if (x < y + h->nor && y < x + h->noc) return fail(h, PWM_ERR_INVALID, "pwm_mv: x and y overlap");
     int rc = stage_vectors(h);
     if (rc == PWM_OK) rc = upload_vec(h, x, h->hx.p, h->noc);
-    if (rc == PWM_OK) rc = spmv_launch(h, h->hx.p, h->hy.p, nullptr, nullptr);
+    if (rc == PWM_OK) rc = spmv_launch(h, h->hx.p, h->hy.p, nullptr);
     if (rc == PWM_OK) rc = download_vec(h, h->hy.p, y, h->nor);
     return rc;
 }
@@ -1358,7 +1453,7 @@ static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, doub
             pw.k = end;
         }
         for (; pw.k < end; ++pw.k)
-            if ((rc = spmv_launch(h, nullptr, nullptr, &pw, nullptr)) != PWM_OK) return rc;
+            if ((rc = spmv_launch(h, nullptr, nullptr, &pw)) != PWM_OK) return rc;
         if (tol >= 0 && end < max_it) {
             if (!read_back()) return hip_fail(h, e, "power loop");
             if (out.done) break;
@@ -1661,7 +1756,7 @@ extern "C" int pwm_gather_rate(const void* x_dev, int64_t x_len, int64_t window,
 static int launch_marked(pwm_matrix* h, const void* x, void* y, hipEvent_t mid) {
     const CrsDev A = crs_of(h);
     hipError_t e = hipSuccess;
-    switch (h->format) {
+    switch (swept_crs(h) ? PWM_FORMAT_CSB : h->format) {
         case PWM_FORMAT_CRS:
             if (h->crs_used == 3) {
                 e = pwmk::launch_rows(A, h->rp, x, y, nullptr, h->stream);
@@ -1690,7 +1785,7 @@ static int launch_marked(pwm_matrix* h, const void* x, void* y, hipEvent_t mid) 
             if (e == hipSuccess) e = csb_launch(h, x, y, nullptr, 2);
             break;
         default: {
-            const int rc = spmv_launch(h, x, y, nullptr, nullptr);
+            const int rc = spmv_launch(h, x, y, nullptr);
             (void)hipEventRecord(mid, h->stream);
             return rc;
         }
@@ -1717,7 +1812,7 @@ extern "C" int pwm_time_mv(pwm_matrix* h, const void* x, void* y, int reps, int6
             return hip_fail(h, e, "event create");
         }
         (void)hipEventRecord(e0, h->stream);
-        for (int r = 0; r < reps && rc == PWM_OK; ++r) rc = spmv_launch(h, x, y, nullptr, nullptr);
+        for (int r = 0; r < reps && rc == PWM_OK; ++r) rc = spmv_launch(h, x, y, nullptr);
         (void)hipEventRecord(e1, h->stream);
         e = hipStreamSynchronize(h->stream);
         if (rc == PWM_OK && e != hipSuccess) rc = hip_fail(h, e, "timed SpMV");
@@ -1790,7 +1885,7 @@ extern "C" int pwm_time_mv_rotating(pwm_matrix* const* hs, const void* const* xs
     if (e != hipSuccess) rc = hip_fail(h0, e, "event create");
     if (rc == PWM_OK && !kernel_ms) {
         (void)hipEventRecord(ev[0], s);
-        for (int i = 0; i < n && rc == PWM_OK; ++i) rc = spmv_launch(hs[i % count], xs[i % count], ys[i % count], nullptr, nullptr);
+        for (int i = 0; i < n && rc == PWM_OK; ++i) rc = spmv_launch(hs[i % count], xs[i % count], ys[i % count], nullptr);
         (void)hipEventRecord(ev[1], s);
     } else if (rc == PWM_OK) {
         for (int i = 0; i < n && rc == PWM_OK; ++i) {

@@ -92,6 +92,7 @@ struct CsbDev {
     // column in window.
     int32_t sweep = 0;
     int32_t sweep_wb = 0;
+    int64_t sweep_ww = 0;        // columns per window, at most 2^sweep_wb
     int64_t sweep_W = 0;
     int32_t sweep_rows = 0;      // LDS rows of a slab (the largest slab)
     int32_t sweep_acc32 = 0;     // FP32 LDS sums (FP32 storage whose slabs do not fit in FP64)
@@ -117,6 +118,7 @@ struct CsbDev {
         sweep_start.release();
         sweep = 0;
         sweep_wb = 0;
+        sweep_ww = 0;
         sweep_W = 0;
         sweep_rows = 0;
         sweep_acc32 = 0;
@@ -189,7 +191,9 @@ struct pwm_matrix {
     // CRS kernel: 0 = wave tiles when the rows are short, else time the vector
     // and tiles kernels at load and keep the faster, 1 = vector, 2 = tiles
     // (row-aligned tiles, carries through the merge fix-up; the tiles plan
-    // lives in mp / split_* / carry_*).  crs_used: 1, 2, or 3 for wave tiles
+    // lives in mp / split_* / carry_*).  crs_used: 1, 2, or 3 for wave tiles.
+    // Swept slabs in csb (csb.sweep = 1) replace any of them, and the merge
+    // kernels of CRS_MERGE, on scattered columns
     int crs_kernel = 0;
     int crs_used = 1;
     pwmk::RowsPlan rp;
@@ -272,7 +276,11 @@ int csb_pieces_device(pwm_matrix* h, int k);
 // rows each), windows of 2^wb columns.  Returns PWM_ERR_UNSUPPORTED, with
 // nothing built, when the cut needs more than `max_slabs` slabs.
 int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int64_t max_rows, int64_t max_slabs,
-                     int wb);
+                     int wb, bool fit);
+// Swept slabs beside the CRS arrays of a CRS or CRS_MERGE handle (their sweep
+// over scattered columns); h->csb.sweep tells whether they were built (not
+// when the rows or the memory do not allow it).
+int build_swept_beside_crs(pwm_matrix* h);
 // BlockCOH layout built on the device from the device CRS arrays
 // (coh_build.hip); h->coh.bands holds the band partition (start, rows, nnz,
 // beta_bits, H, V, off_nz) on entry and the per-band sizes and offsets on
@@ -300,7 +308,7 @@ int plan_merge(pwm_matrix* h);
 int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals);
 int build_blockcoh(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals);
 // one SpMV of the loaded format on device vectors; pw != nullptr: power step
-int spmv_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw, int* n_partials_out);
+int spmv_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw);
 hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw, int part = 0);
 hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw);
 int64_t csb_partials(const pwm_matrix* h);

@@ -61,8 +61,10 @@ struct CsbArgs {
     // packed (row in slab << wb) | column in window.
     int32_t sweep = 0;
     int32_t wb = 0;
+    int64_t ww = 0;          // columns per window, at most 2^wb
     int64_t W = 0;
     int32_t max_rows = 0;
+    int32_t ord = 0;         // 1: FP64 LDS sums in a fixed order (the CRS formats' sweep)
     int32_t acc32 = 0;       // 1: FP32 LDS sums (FP32 storage whose slabs do not fit in FP64)
     int32_t sync_every = 1;  // windows between workgroup barriers (a power of two)
     const int32_t* sstart = nullptr;

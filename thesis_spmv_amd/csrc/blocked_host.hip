@@ -69,7 +69,7 @@ hipError_t upload(DevBuf& d, const void* src, size_t bytes) {
 struct SweptSave {
     DevBuf ind, data, soff, start;
     int32_t wb = 0, rows = 0, nt = 1, order = 0, acc32 = 0;
-    int64_t W = 0, T = 0;
+    int64_t W = 0, T = 0, ww = 0;
     std::vector<int32_t> len;
     void take(CsbDev& c) {
         ind.swap(c.ind);
@@ -80,6 +80,7 @@ struct SweptSave {
         order = c.sweep_order;
         c.sweep_order = 0;
         wb = c.sweep_wb;
+        ww = c.sweep_ww;
         W = c.sweep_W;
         rows = c.sweep_rows;
         acc32 = c.sweep_acc32;
@@ -99,6 +100,7 @@ struct SweptSave {
         c.sweep_order = order;
         c.sweep = 1;
         c.sweep_wb = wb;
+        c.sweep_ww = ww;
         c.sweep_W = W;
         c.sweep_rows = rows;
         c.sweep_acc32 = acc32;
@@ -193,8 +195,9 @@ static int time_csb(pwm_matrix* h, float* ms) {
 // persistent workgroup of 1024 threads each, with all of the CU's LDS for its
 // y-slice), or csb_sweep_waves times as many (the workgroups then run in that
 // many waves), windows of 1 MB of x unless csb_window_bits says otherwise.
-// PWM_ERR_UNSUPPORTED when the slabs' rows cannot fit.
-static int build_swept(pwm_matrix* h, const int32_t* rs) {
+// PWM_ERR_UNSUPPORTED when the slabs' rows cannot fit.  ord: for the CRS
+// formats' sweep (FP64 sums, windows fitted to the rounds of its turns).
+static int build_swept(pwm_matrix* h, const int32_t* rs, bool ord) {
     CsbDev& c = h->csb;
     int cus = 0, lds_cu = 0;
     hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0);
@@ -215,12 +218,12 @@ static int build_swept(pwm_matrix* h, const int32_t* rs) {
     // holds takes (slower) FP32 sums
     int64_t rows_cap = 0;
     int rc = PWM_ERR_UNSUPPORTED;
-    for (int acc = 8; acc >= xb && rc == PWM_ERR_UNSUPPORTED; acc -= 4) {
+    for (int acc = 8; acc >= (ord ? 8 : xb) && rc == PWM_ERR_UNSUPPORTED; acc -= 4) {
         c.sweep_acc32 = acc == 4;
         rows_cap = std::min<int64_t>(((lds_cu - 1024) / acc) & ~(int64_t)63, ((int64_t)1 << (32 - wb)) - 1);
         if (rows_cap <= 0 || blocked::csb_sweep_blocks_per_cu(h->vtype, (int)rows_cap, acc == 4) < 1)
             return fail(h, PWM_ERR_UNSUPPORTED, "CSB swept slabs: no workgroup with LDS rows fits a CU");
-        rc = csb_sweep_device(h, rs, slabs, rows_cap, slabs, wb);
+        rc = csb_sweep_device(h, rs, slabs, rows_cap, slabs, wb, ord && h->csb_window_bits == 0);
     }
     if (rc == PWM_ERR_UNSUPPORTED)
         return fail(h, rc, "CSB swept slabs: the rows do not fit " + std::to_string(slabs) + " slabs of at most " +
@@ -228,6 +231,15 @@ static int build_swept(pwm_matrix* h, const int32_t* rs) {
     if (rc != PWM_OK) return rc;
     c.nt = h->csb_nt >= 0 ? h->csb_nt : 1;
     return PWM_OK;
+}
+
+int build_swept_beside_crs(pwm_matrix* h) {
+    if ((int64_t)h->h_rs.size() != h->nor + 1) return PWM_OK;
+    const int rc = build_swept(h, h->h_rs.data(), true);
+    if (rc == PWM_OK) return PWM_OK;
+    h->csb.clear();
+    (void)hipGetLastError();
+    return rc == PWM_ERR_UNSUPPORTED || rc == PWM_ERR_NOMEM ? PWM_OK : rc;
 }
 
 // rs: host row_start; ci / vals: host CRS arrays, or NULL (values already
@@ -296,7 +308,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
                            (h->csb_layout == 0 && h->csb_groups == 0 && h->csb_unroll == 0 && nnz > 0 &&
                             noc * (int64_t)vector_size(h->vtype) > ((int64_t)2 << 20));
     if (try_sweep) {
-        rc = build_swept(h, rs);
+        rc = build_swept(h, rs, false);
         if (rc == PWM_OK) {
             if (h->csb_layout == 4) {
                 // the CRS arrays are not needed by the CSB kernels
@@ -850,9 +862,11 @@ hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     a.srows = h->csb.srows.as<uint16_t>();
     a.sweep = h->csb.sweep;
     a.wb = h->csb.sweep_wb;
+    a.ww = h->csb.sweep_ww;
     a.W = h->csb.sweep_W;
     a.max_rows = h->csb.sweep_rows;
     a.acc32 = h->csb.sweep_acc32;
+    a.ord = h->format != PWM_FORMAT_CSB;
     a.sync_every = h->csb_sync_every;
     if (a.sweep) a.unroll = h->csb_sweep_unroll;
     a.sstart = h->csb.sweep_start.as<int32_t>();
@@ -1034,7 +1048,7 @@ static int csb_sweep_layout(pwm_matrix* h, uint32_t* ind, double* data, int32_t*
                     const int64_t q =
                         by_col ? woff[r] + (i & ~(int64_t)255) + 4 * (i & 63) + ((i >> 6) & 3) : woff[r] + i;
                     const int64_t row = sstart[t] + (int64_t)(sind[q] >> wb);
-                    const int64_t col = (p << wb) + (int64_t)(sind[q] & wmask);
+                    const int64_t col = p * c.sweep_ww + (int64_t)(sind[q] & wmask);
                     blk[n] = (row / beta) * H + col / beta;
                     lr[n] = (uint32_t)(row % beta);
                     lc[n] = (uint32_t)(col % beta);

@@ -19,15 +19,17 @@
 //
 // The swept-slab layout (csb_sweep_device) cuts the rows into nnz-balanced
 // slabs on the host (one per CU), keys entry k of slab t, column c with
-// cell = t*W + (c >> w) (W windows of 2^w columns) and, in column order (the
-// default), cell << w | (c mod 2^w); sorts stably (equal keys keep CRS
-// order) and packs each index as (row in slab << w) | (c mod 2^w).  In
+// cell = t*W + c/ww (W windows of ww <= 2^w columns) and, in column order (the
+// default), cell << w | (c mod ww); sorts stably (equal keys keep CRS
+// order) and packs each index as (row in slab << w) | (c mod ww).  In
 // column order every (slab, window) run is padded to whole blocks of 256
 // entries (index 0xffffffff, value 0) and each block stores its sorted entry
 // j*64 + L at 4L + j, so that lane L, reading 4 consecutive stored entries,
 // holds sorted entries L, 64 + L, 128 + L and 192 + L: each gather
 // instruction of a wave reads 64 consecutive columns.  soff gives every
 // run's stored start.
+#include <math.h>
+
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "api_internal.hpp"
@@ -123,12 +125,13 @@ __global__ void k_csb_soff(const uint64_t* __restrict__ keys, int64_t nnz, int64
     }
 }
 
-// Swept slabs: entry k of row r, column c gets the key t * W + (c >> wb),
+// Swept slabs: entry k of row r, column c gets the key t * W + c / ww,
 // t the slab holding row r; a stable sort keeps CRS order (rows, then
 // columns, ascending) inside every (slab, window) run.
 struct SweepKeyArgs {
     int64_t nor, nnz, T, W;
     int wb;
+    uint32_t ww;  // columns per window, at most 2^wb
     int order;  // 1: the column in the window joins the key (column order inside a run)
     const int32_t* roff = nullptr;  // order 1: sorted run starts
     const int32_t* poff = nullptr;  // order 1: stored (padded) run starts
@@ -152,8 +155,9 @@ __global__ void k_sweep_keys(SweepKeyArgs a, const int32_t* __restrict__ rs, con
     for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < a.nnz; k += (int64_t)gridDim.x * blockDim.x) {
         const int64_t row = last_at_or_below(rs, a.nor, k);
         const int64_t t = last_at_or_below(sstart, a.T, row);
-        const uint64_t cell = (uint64_t)t * (uint64_t)a.W + (uint64_t)((uint32_t)ci[k] >> a.wb);
-        keys[k] = a.order ? (cell << a.wb) | ((uint32_t)ci[k] & (((uint32_t)1 << a.wb) - 1)) : cell;
+        const uint32_t c = (uint32_t)ci[k], w = c / a.ww;
+        const uint64_t cell = (uint64_t)t * (uint64_t)a.W + w;
+        keys[k] = a.order ? (cell << a.wb) | (c - w * a.ww) : cell;
         pos[k] = (uint32_t)k;
     }
 }
@@ -163,7 +167,6 @@ __global__ void k_sweep_gather(SweepKeyArgs a, const int32_t* __restrict__ rs, c
                                const int32_t* __restrict__ sstart, const uint64_t* __restrict__ keys,
                                const uint32_t* __restrict__ pos, const E* __restrict__ val,
                                uint32_t* __restrict__ sind, E* __restrict__ sdat) {
-    const uint32_t wmask = (uint32_t)(((uint64_t)1 << a.wb) - 1);
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < a.nnz; p += (int64_t)gridDim.x * blockDim.x) {
         const int64_t k = pos[p];
         const uint64_t cell = a.order ? keys[p] >> a.wb : keys[p];
@@ -178,7 +181,7 @@ __global__ void k_sweep_gather(SweepKeyArgs a, const int32_t* __restrict__ rs, c
             const int64_t i = p - a.roff[cell];
             q = a.poff[cell] + (i & ~(int64_t)255) + 4 * (i & 63) + ((i >> 6) & 3);
         }
-        sind[q] = ((uint32_t)(row - sstart[t]) << a.wb) | ((uint32_t)ci[k] & wmask);
+        sind[q] = ((uint32_t)(row - sstart[t]) << a.wb) | (uint32_t)((uint32_t)ci[k] - (uint32_t)(cell % (uint64_t)a.W) * a.ww);
         sdat[q] = val[k];
     }
 }
@@ -367,7 +370,7 @@ int csb_pieces_device(pwm_matrix* h, int k) {
 }
 
 int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int64_t max_rows, int64_t max_slabs,
-                     int wb) {
+                     int wb, bool fit) {
     CsbDev& c = h->csb;
     const int64_t nnz = h->nnz, nor = h->nor, noc = h->noc;
     // nnz-balanced row slabs: a slab closes before the row that would take it
@@ -401,7 +404,22 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
     const int64_t T = (int64_t)sstart.size() - 1;
     int32_t rows_max = 0;
     for (int64_t t = 0; t < T; ++t) rows_max = std::max(rows_max, sstart[t + 1] - sstart[t]);
-    const int64_t W = std::max<int64_t>(1, (noc + ((int64_t)1 << wb) - 1) >> wb);
+    // Columns per window: 2^wb, or (fit) as many less as let a run of evenly
+    // spread columns, three deviations included, fill whole rounds of the
+    // kernel's 16 waves x 512 entries: with turns, a chunk more than that is a
+    // round of one wave while 15 wait (1.2 M power-law rows, FP64: 77.2 us
+    // against 88.5 with 2^17 columns; without turns no difference)
+    int64_t ww = (int64_t)1 << wb;
+    if (fit && nnz > 0) {
+        const double run = (double)target * (double)ww / (double)noc;
+        const double rounds = std::max(1.0, floor(run * 1.25 / 8192.0));
+        const double room = 8192.0 * rounds - 3.0 * sqrt(8192.0 * rounds);
+        if (run > room) {
+            const int64_t w = (int64_t)ceil((double)noc * run / (room * (double)ww));  // windows
+            ww = std::min(ww, ((noc + w - 1) / w + 31) & ~(int64_t)31);
+        }
+    }
+    const int64_t W = std::max<int64_t>(1, (noc + ww - 1) / ww);
     const int64_t cells = T * W;
     const int order = h->csb_sweep_order;
     const size_t vs = value_size(h->vtype);
@@ -419,7 +437,7 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
     c.sweep_len.clear();
     int64_t stored = nnz;  // entries stored (order 1: every run padded to whole blocks of 256)
     if (nnz > 0) {
-        pwmk::SweepKeyArgs a{nor, nnz, T, W, wb, order};
+        pwmk::SweepKeyArgs a{nor, nnz, T, W, wb, (uint32_t)ww, order};
         DevBuf keys, keys_out, pos, pos_out, tmp, roff;
         if ((e = keys.alloc(nnz * 8)) != hipSuccess || (e = keys_out.alloc(nnz * 8)) != hipSuccess ||
             (e = pos.alloc(nnz * 4)) != hipSuccess || (e = pos_out.alloc(nnz * 4)) != hipSuccess)
@@ -512,6 +530,7 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
     c.wide = 0;
     c.sweep = 1;
     c.sweep_wb = wb;
+    c.sweep_ww = ww;
     c.sweep_W = W;
     c.sweep_rows = std::max<int32_t>(rows_max, 1);
     c.slabs = 1;

@@ -183,6 +183,37 @@ __global__ void k_gather_fill(uint32_t* __restrict__ idx, double* __restrict__ v
     }
 }
 
+// Scatter of the column indices: over `groups` groups of 256 consecutive
+// entries spread evenly, the 128-byte x lines each group touches (a hash table
+// of a wave in LDS), summed into *lines.
+constexpr int kScatterSlots = 1024;
+__global__ __launch_bounds__(64) void k_scatter(const int32_t* __restrict__ ci, int64_t nnz, int64_t groups, int shift,
+                                                unsigned* __restrict__ lines) {
+    __shared__ int table[kScatterSlots];
+    for (int i = threadIdx.x; i < kScatterSlots; i += 64) table[i] = -1;
+    __syncthreads();
+    const int64_t k0 = (nnz - 256) * blockIdx.x / groups;  // nnz >= 256
+    int found = 0;
+    for (int j = 0; j < 4; ++j) {
+        const int line = ci[k0 + 64 * j + threadIdx.x] >> shift;
+        unsigned h = ((unsigned)line * 2654435761u) >> 22;
+        // at most 256 of the 1024 slots are taken: a free one or the line itself is met
+        for (;;) {
+            const int old = atomicCAS(&table[h], -1, line);
+            if (old == -1) ++found;
+            if (old == -1 || old == line) break;
+            h = (h + 1) & (kScatterSlots - 1);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) found += __shfl_xor(found, off);
+    if (threadIdx.x == 0) atomicAdd(lines, (unsigned)found);
+}
+
+hipError_t launch_scatter(const int32_t* ci, int64_t nnz, int64_t groups, int shift, unsigned* lines, hipStream_t s) {
+    hipLaunchKernelGGL(k_scatter, dim3((unsigned)groups), dim3(64), 0, s, ci, nnz, groups, shift, lines);
+    return hipGetLastError();
+}
+
 constexpr int kProbeU = 8;
 constexpr int kProbePerBlock = 8192;  // entries per workgroup, a multiple of 256 * kProbeU
 

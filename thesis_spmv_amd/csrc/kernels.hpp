@@ -119,6 +119,9 @@ hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, hipSt
 hipError_t launch_flush(void* p, int64_t bytes, hipStream_t s);
 // Plain streaming copy (profiler counter calibration).
 hipError_t launch_stream_copy(void* dst, const void* src, int64_t bytes, hipStream_t s);
+// Distinct lines of 2^shift columns per group of 256 consecutive entries, over
+// `groups` groups (nnz >= 256), added to *lines.
+hipError_t launch_scatter(const int32_t* ci, int64_t nnz, int64_t groups, int shift, unsigned* lines, hipStream_t s);
 // gather-rate probe: entries rounded down to whole workgroups; out holds
 // (entries / 8192) * 256 doubles
 int64_t gather_probe_entries(int64_t n);
