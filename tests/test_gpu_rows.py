@@ -1,4 +1,4 @@
-"""The CRS format's wave tiles (k_rows): SpMV against the oracle.
+"""Wave tiles (k_rows) of CRS and CRS_MERGE handles: SpMV against the oracle.
 
 A lane sums a row's products left to right in the vector's type, as the
 oracle does in FP64, so FP64 results are equal bit for bit.  FP32: products and
@@ -46,17 +46,19 @@ CASES = list(_cases())
 
 @pytest.mark.parametrize("values", ["f64", "f32"])
 @pytest.mark.parametrize("nt", [0, 1])
+@pytest.mark.parametrize("cls", [pw.CRSHip, pw.CRSMergeHip], ids=lambda c: c.__name__)
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
-def test_wave_tiles(case, nt, values):
+def test_wave_tiles(case, cls, nt, values):
     name, lens, noc, taken = case
     A = _crs(lens, noc)
     x = np.random.default_rng(2).standard_normal(noc).astype(np.float32).astype(np.float64)
-    m = pw.CRSHip(values=values, crs_nt=nt)
+    m = cls(values=values, crs_nt=nt)
     m.loadCRS(A.nor, A.noc, A.row_start, A.col_ind, A.data)
-    step = 253 - (int(np.max(lens)) - 1)
-    tiles = -(-len(A.data) // step)
     info = m.info()
-    assert (info["group_size"] == 0 and info["kernels"] == 1 and info["threads"] == tiles) or not taken, info
+    if cls is pw.CRSHip:
+        step = 253 - (int(np.max(lens)) - 1)
+        assert info["threads"] == -(-len(A.data) // step) or not taken, info
+    assert (info["kernels"] == 1 and info["non_temporal"] == nt and info["group_size"] == 0) or not taken, info
     vt = np.float64 if values == "f64" else np.float32
     xd, yd = pw.DeviceVector.from_array(x, vt), pw.DeviceVector(A.nor, vt)
     yd.fill(3.0)

@@ -574,6 +574,27 @@ static int plan_swept(pwm_matrix* h, const void* x, void* y, float* ms) {
     return PWM_OK;
 }
 
+// The faster of plain and non-temporal entry loads (the caller's choice, else
+// both are timed) for a CRS kernel that has them, and its time.
+static hipError_t time_entry_loads(pwm_matrix* h, int which, const void* x, void* y, float* best) {
+    int best_nt = 0;
+    *best = -1.0f;
+    for (int nt : {0, 1}) {
+        if (which == 0 && nt) continue;  // the merge kernel has only plain ones
+        if (which && h->crs_nt >= 0 && nt != h->crs_nt) continue;
+        h->crs_nt_used = nt;
+        float ms = 0.0f;
+        const hipError_t e = time_crs_kernel(h, which, x, y, &ms);
+        if (e != hipSuccess) return e;
+        if (*best < 0.0f || ms < *best) {
+            *best = ms;
+            best_nt = nt;
+        }
+    }
+    h->crs_nt_used = best_nt;
+    return hipSuccess;
+}
+
 // CRS vector kernel with G lanes per row: grid size and the long-row chunk
 // plan (rows longer than max(1024, 128 G) are cut into chunks).
 static int plan_crs_vector(pwm_matrix* h, int G) {
@@ -722,24 +743,13 @@ int plan_crs(pwm_matrix* h) {
     e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "CRS autotune vectors");
     float best = -1.0f, swept = -1.0f;
-    int best_kernel = 1, best_g = G0, best_nt = 0;
+    int best_kernel = 1, best_g = G0;
     if (automatic && h->crs_nt < 0 && (rc = plan_swept(h, x.p, y.p, &swept)) != PWM_OK) return rc;
     if (rows || tiles) {
-        // entry loads plain or non-temporal: the caller's choice, else both
-        const int kernel = rows ? 3 : 2;
-        for (int nt : {0, 1}) {
-            if (h->crs_nt >= 0 && nt != h->crs_nt) continue;
-            h->crs_nt_used = nt;
-            float ms = 0.0f;
-            if ((e = time_crs_kernel(h, kernel, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
-            if (best < 0.0f || ms < best) {
-                best = ms;
-                best_kernel = kernel;
-                best_nt = nt;
-            }
-        }
+        best_kernel = rows ? 3 : 2;
+        if ((e = time_entry_loads(h, best_kernel, x.p, y.p, &best)) != hipSuccess)
+            return hip_fail(h, e, "CRS autotune");
     }
-    h->crs_nt_used = best_nt;
     // the vector kernel gathers in row order like the tiles and was never a
     // third faster than they: it is not timed against a sweep that is
     if (swept >= 0.0f && swept < 0.7f * best) gs.clear();
@@ -791,21 +801,31 @@ int plan_merge(pwm_matrix* h) {
     e = pwmk::launch_merge_splits(crs_of(h), h->mp, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "merge split search");
-    // scattered columns: swept slabs when they time faster than the merge
-    // kernels (not when the caller chose the partition or the tile size)
+    // Unless the caller chose the partition or the tile size, the SpMV takes
+    // the CRS format's wave tiles when the rows are short (Poisson 80 x 80: 8.0
+    // -> 3.0 us, 1024 x 1024: 23.2 -> 13.8, 5000 x 5000: 405 -> 338, FP64; the
+    // merge of each thread's items is what they save) and its swept slabs when
+    // the columns are scattered and the slabs time faster.
     h->csb.clear();
+    h->rp = pwmk::RowsPlan{};
+    h->crs_used = 0;
     if ((h->threads > 0 && P == h->threads) || h->ipt != 8) return PWM_OK;
-    if (h->csb_layout != 4 && h->noc * (int64_t)vector_size(h->vtype) <= kXcdL2) return PWM_OK;
-    DevBuf x, y;
+    int rc = plan_crs_rows(h);
+    if (rc != PWM_OK) return rc;
+    const bool rows = h->rp.nt > 0;
     const size_t vs = vector_size(h->vtype);
+    const bool sweep = h->csb_layout == 4 || h->noc * (int64_t)vs > kXcdL2;
+    if (!rows && !sweep) return PWM_OK;
+    DevBuf x, y;
     if ((e = x.alloc(h->noc * vs)) != hipSuccess || (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess ||
         (e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream)) != hipSuccess)
         return hip_fail(h, e, "merge plan vectors");
-    float swept = -1.0f, ms = 0.0f;
-    const int rc = plan_swept(h, x.p, y.p, &swept);
-    if (rc != PWM_OK || swept < 0.0f) return rc;
-    if ((e = time_crs_kernel(h, 0, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "merge plan");
-    if (swept >= ms) h->csb.clear();
+    float swept = -1.0f, best = -1.0f;
+    if (sweep && (rc = plan_swept(h, x.p, y.p, &swept)) != PWM_OK) return rc;
+    if (!rows && swept < 0.0f) return PWM_OK;
+    h->crs_used = rows ? 3 : 0;
+    if ((e = time_entry_loads(h, h->crs_used, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "merge plan");
+    if (swept >= 0.0f && swept >= best) h->csb.clear();
     return PWM_OK;
 }
 
@@ -817,8 +837,8 @@ static bool swept_crs(const pwm_matrix* h) {
 int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw) {
     hipError_t e = hipSuccess;
     switch (swept_crs(h) ? PWM_FORMAT_CSB : h->format) {
-        case PWM_FORMAT_CRS: e = crs_kernel_launch(h, h->crs_used, x, y, pw); break;
-        case PWM_FORMAT_CRS_MERGE: e = crs_kernel_launch(h, 0, x, y, pw); break;
+        case PWM_FORMAT_CRS:
+        case PWM_FORMAT_CRS_MERGE: e = crs_kernel_launch(h, h->crs_used, x, y, pw); break;
         case PWM_FORMAT_CSB: e = csb_launch(h, x, y, pw); break;
         case PWM_FORMAT_BLOCKCOH: e = coh_launch(h, x, y, pw); break;
         default: return fail(h, PWM_ERR_INVALID, "unknown format");
@@ -832,7 +852,8 @@ static int64_t partials_needed(const pwm_matrix* h) {
         case PWM_FORMAT_CRS:
             if (h->crs_used == 3) return pwmk::rows_power_blocks(h->rp.nt);
             return std::max<int64_t>(h->vec_blocks, h->tiles.p ? h->mp.P + pwmk::merge_fix_blocks(h->mp.P) : 0);
-        case PWM_FORMAT_CRS_MERGE: return h->mp.P + pwmk::merge_fix_blocks(h->mp.P);
+        case PWM_FORMAT_CRS_MERGE:
+            return h->crs_used == 3 ? pwmk::rows_power_blocks(h->rp.nt) : h->mp.P + pwmk::merge_fix_blocks(h->mp.P);
         case PWM_FORMAT_CSB: return csb_partials(h);
         case PWM_FORMAT_BLOCKCOH: return coh_partials(h);
     }
@@ -1245,7 +1266,7 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
         case PWM_FORMAT_CRS:
             out->kernels = 1 + (h->crs_used == 2 ? (h->tiles_carry ? 1 : 0) : (h->lr.n_rows > 0 ? 1 : 0));
             break;
-        case PWM_FORMAT_CRS_MERGE: out->kernels = 2; break;
+        case PWM_FORMAT_CRS_MERGE: out->kernels = h->crs_used == 3 ? 1 : 2; break;
         case PWM_FORMAT_CSB: out->kernels = h->csb.sweep ? 1 : 1 + (h->csb.groups > 1 ? 1 : 0); break;
         case PWM_FORMAT_BLOCKCOH: out->kernels = 1 + (h->coh.n_atomic > 0 ? 1 : 0); break;
     }
@@ -1253,7 +1274,7 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
     if (h->format == PWM_FORMAT_CSB && h->csb.n_tasks <= 0) out->kernels = 0;
     out->high_occupancy = h->format == PWM_FORMAT_BLOCKCOH ? h->coh.occ8 : 0;
     out->non_temporal = h->format == PWM_FORMAT_CSB || swept_crs(h)         ? h->csb.nt
-                        : (h->format == PWM_FORMAT_CRS && h->crs_used >= 2) ? h->crs_nt_used
+                        : (h->format == PWM_FORMAT_CRS && h->crs_used == 2) || h->crs_used == 3 ? h->crs_nt_used
                                                                            : 0;
     const pwm_impl::DevBuf* bufs[] = {&h->rs, &h->ci, &h->val, &h->lr_chunks, &h->lr_rows, &h->lr_begin,
                                       &h->lr_partial, &h->split_a, &h->split_b, &h->carry_row, &h->carry_val, &h->tiles,
@@ -1775,6 +1796,11 @@ static int launch_marked(pwm_matrix* h, const void* x, void* y, hipEvent_t mid) 
                 e = pwmk::launch_crs_finalize(A, h->vec_blocks, h->lr, y, nullptr, h->stream);
             break;
         case PWM_FORMAT_CRS_MERGE:
+            if (h->crs_used == 3) {
+                e = pwmk::launch_rows(A, h->rp, x, y, nullptr, h->stream);
+                (void)hipEventRecord(mid, h->stream);
+                break;
+            }
             e = pwmk::launch_merge_spmv(A, h->mp, x, y, nullptr, h->stream);
             (void)hipEventRecord(mid, h->stream);
             if (e == hipSuccess) e = pwmk::launch_merge_fixup(A, h->mp, y, nullptr, h->stream);
