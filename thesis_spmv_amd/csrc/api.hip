@@ -51,7 +51,6 @@ void DevBuf::release() {
 // ---- host thread pool behind parallel_for
 namespace {
 constexpr int kMaxWorkers = 16;  // the GPU host grants 16 cores per GPU
-using LoopFn = std::function<void(int64_t, int64_t, int)>;
 
 void run_chunks(std::atomic<int64_t>& next, int64_t n, int64_t chunk, const LoopFn& fn, int worker) {
     for (;;) {
@@ -96,21 +95,24 @@ void pool_worker(HostPool* p, int id) {
     }
 }
 
-void spawn_run(int64_t n, int64_t chunk, const LoopFn& fn, int nt) {
+void spawn_run(int64_t n, int64_t chunk, const LoopFn& fn, int nt, const LeadFn* lead) {
     std::atomic<int64_t> next(0);
     std::vector<std::thread> ts;
     for (int t = 1; t < nt; ++t) ts.emplace_back([&, t]() { run_chunks(next, n, chunk, fn, t); });
+    if (lead) (*lead)(next);
     run_chunks(next, n, chunk, fn, 0);
     for (auto& th : ts) th.join();
 }
 }  // namespace
 
-void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn) {
+void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn, const LeadFn* lead) {
     const unsigned hw = std::thread::hardware_concurrency();
     const int64_t pieces = (n + chunk - 1) / chunk;
     const int nt = (int)std::min<int64_t>(std::min<int64_t>(hw ? hw : 4, kMaxWorkers), pieces);
     if (nt <= 1) {
-        fn(0, n, 0);
+        std::atomic<int64_t> next(0);
+        if (lead) (*lead)(next);
+        run_chunks(next, n, lead ? chunk : n, fn, 0);
         return;
     }
     std::call_once(g_pool_once, [&] {
@@ -130,7 +132,7 @@ void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn) {
     HostPool* p = g_pool;
     std::unique_lock<std::mutex> run(p->run_mu, std::try_to_lock);
     if (!run.owns_lock() || p->nworkers == 0 || p->pid != getpid()) {
-        spawn_run(n, chunk, fn, nt);
+        spawn_run(n, chunk, fn, nt, lead);
         return;
     }
     {
@@ -144,6 +146,7 @@ void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn) {
         ++p->epoch;
     }
     p->cv_work.notify_all();
+    if (lead) (*lead)(p->next);
     run_chunks(p->next, n, chunk, fn, 0);
     std::unique_lock<std::mutex> lk(p->mu);
     p->cv_done.wait(lk, [&] { return p->pending == 0; });
@@ -156,6 +159,8 @@ constexpr size_t kStageBytes = (size_t)64 << 20;
 std::mutex g_stage_mu;
 void* g_stage[2] = {nullptr, nullptr};
 hipEvent_t g_stage_ev[2] = {nullptr, nullptr};
+constexpr size_t kRingChunks = 16;  // most chunks per buffer
+hipEvent_t g_ring_ev[2 * kRingChunks] = {};
 bool g_stage_failed = false;
 }  // namespace
 
@@ -175,8 +180,11 @@ static int64_t stage_piece(size_t chunk) { return std::max<int64_t>((int64_t)(ch
 static bool stage_ready() {
     if (!g_stage[0] && !g_stage_failed) {
         for (int i = 0; i < 2 && !g_stage_failed; ++i)
-            if (hipHostMalloc(&g_stage[i], kStageBytes, hipHostMallocDefault) != hipSuccess ||
+            if (hipHostMalloc(&g_stage[i], kStageBytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess ||
                 hipEventCreateWithFlags(&g_stage_ev[i], hipEventDisableTiming) != hipSuccess)
+                g_stage_failed = true;
+        for (hipEvent_t& v : g_ring_ev)
+            if (!g_stage_failed && hipEventCreateWithFlags(&v, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess)
                 g_stage_failed = true;
         if (g_stage_failed) {
             for (int i = 0; i < 2; ++i) {
@@ -185,16 +193,193 @@ static bool stage_ready() {
                 g_stage[i] = nullptr;
                 g_stage_ev[i] = nullptr;
             }
+            for (hipEvent_t& v : g_ring_ev) {
+                if (v) (void)hipEventDestroy(v);
+                v = nullptr;
+            }
             (void)hipGetLastError();
         }
     }
     return !g_stage_failed;
 }
 
-// Host -> device through the pinned pair: fill(stage, a0, a1) writes bytes
-// [a0, a1) of the transfer into `stage` (called by host threads on pieces of
-// a chunk); host threads fill one buffer while the other is in flight.  The
-// caller holds g_stage_mu and stage_ready() is true.
+// FP64 value k as stored: FP32, or BF16 as the upper half of the FP32 value
+// (exact for values exact in BF16, which the callers check).
+static inline void narrow_value(const double* v, int vt, int64_t k, char* out) {
+    const float f = (float)v[k];
+    if (vt == PWM_VALUES_F32) {
+        memcpy(out, &f, 4);
+    } else {
+        uint32_t u;
+        memcpy(&u, &f, 4);
+        const uint16_t h = (uint16_t)(u >> 16);
+        memcpy(out, &h, 2);
+    }
+}
+
+// What the threads do to a piece, bytes [a0, a1) of the transfer (whole values:
+// pieces are multiples of 64 KB): host arrays into the staging buffers, as they
+// are or in the stored type, and vectors out of them.
+static auto bytes_in(const void* src) {
+    return [src](char* to, size_t a0, size_t a1) { memcpy(to, (const char*)src + a0, a1 - a0); };
+}
+static auto values_in(const double* src, int vt) {
+    return [src, vt](char* to, size_t a0, size_t a1) {
+        if (vt == PWM_VALUES_F32)
+            for (size_t k = a0 / 4; k < a1 / 4; ++k) ((float*)to)[k - a0 / 4] = (float)src[k];
+        else
+            for (size_t k = a0 / 2; k < a1 / 2; ++k) narrow_value(src, vt, (int64_t)k, to + 2 * k - a0);
+    };
+}
+static auto bytes_out(double* dst) {
+    return [dst](const char* from, size_t a0, size_t a1) { memcpy((char*)dst + a0, from, a1 - a0); };
+}
+static auto floats_out(double* dst) {
+    return [dst](const char* from, size_t a0, size_t a1) {
+        const float* f = (const float*)from;
+        for (size_t i = 0; i < (a1 - a0) / 4; ++i) dst[a0 / 4 + i] = f[i];
+    };
+}
+
+// ---- transfers in one parallel loop
+// A transfer goes in windows of one staging buffer (64 MB), in turn through the
+// two: while the threads fill or empty one, the copies of the other run.  A
+// window holds chunks; host threads take pieces of the whole window in order,
+// and the calling thread queues a chunk's copy as soon as its pieces are in
+// (uploads) or hands a chunk to the threads as soon as it has arrived
+// (downloads): the threads are woken once per window, not once per chunk.  Up to
+// one buffer, chunks of 1 to 4 MB copied by kernels that read or write the
+// pinned memory: eight of 1 MB take 183 us up and 185 down, where the copy
+// engine takes 225 and 260 (about 10 us more per copy), and 154 for the 8 MB at
+// once.  Beyond, where the host's copies set the pace, chunks of 16 MB by the
+// copy engine in pieces of 1 MB (2 x 200 MB: 8.16 ms, with chunks of 4 MB 8.27).
+// mv(x, y) on host arrays of a Poisson grid, FP64: 300 x 300 165 -> 75 us, 1000 x
+// 999 575 -> 450, 5000 x 5000 as before; FP32, which used to convert in separate
+// loops, 1000 x 999 590 -> 280 and 4000 x 3000 9300 -> 2170.
+namespace {
+// Short transfers are copied by the calling thread: waking the others costs
+// more (mv of 0.7 MB vectors takes 75 us, through the threads 97; of 1.4 MB 143
+// through the threads, without them 155).
+constexpr size_t kInlineBytes = (size_t)1 << 20;
+
+struct Window {
+    size_t bytes, chunk, piece, nch;
+    int64_t pieces;
+    std::unique_ptr<std::atomic<int>[]> left;  // pieces of a chunk not yet copied
+    Window(size_t n, size_t transfer) : bytes(n) {
+        constexpr size_t KB = 1024, MB = KB * KB;
+        chunk = transfer > kStageBytes ? 16 * MB : MB;
+        piece = transfer > kStageBytes ? MB : 128 * KB;
+        while (chunk < 4 * MB && chunk * 16 < transfer) chunk *= 2;
+        nch = (n + chunk - 1) / chunk;
+        pieces = (int64_t)((n + piece - 1) / piece);
+        left.reset(new std::atomic<int>[nch]);
+        for (size_t k = 0; k < nch; ++k) left[k] = (int)((size(k) + piece - 1) / piece);
+    }
+    size_t size(size_t k) const { return std::min(chunk, bytes - k * chunk); }
+    size_t chunk_of(int64_t p) const { return (size_t)p * piece / chunk; }
+};
+}  // namespace
+
+// Host -> device: fill(stage, a0, a1) writes bytes [a0, a1) of the transfer to
+// `stage`.  The caller holds g_stage_mu and stage_ready() is true.  Without
+// `wait` the last copies are still under way: the caller synchronizes s before
+// it gives the buffers up.
+template <typename Fill>
+static hipError_t window_upload(void* dst, size_t bytes, hipStream_t s, Fill fill, bool wait = true) {
+    hipError_t e = hipSuccess;
+    int b = 0, used = 0;
+    for (size_t off = 0; off < bytes && e == hipSuccess; off += kStageBytes, b ^= 1, ++used) {
+        const size_t n = std::min(kStageBytes, bytes - off);
+        char* stage = (char*)g_stage[b];
+        char* to = (char*)dst + off;
+        if (used >= 2 && (e = hipEventSynchronize(g_stage_ev[b])) != hipSuccess) break;
+        if (n <= kInlineBytes) {
+            fill(stage, off, off + n);
+            e = pwmk::launch_copy_bytes(to, stage, n, false, s);
+        } else {
+            Window W(n, bytes);
+            const LoopFn work = [&](int64_t p0, int64_t p1, int) {
+                for (int64_t p = p0; p < p1; ++p) {
+                    const size_t a0 = (size_t)p * W.piece, a1 = std::min(n, a0 + W.piece);
+                    fill(stage + a0, off + a0, off + a1);
+                    W.left[W.chunk_of(p)].fetch_sub(1, std::memory_order_release);
+                }
+            };
+            const LeadFn lead = [&](std::atomic<int64_t>& next) {
+                for (size_t k = 0; k < W.nch; ++k) {
+                    while (W.left[k].load(std::memory_order_acquire) != 0) {
+                        const int64_t p = next.load() < W.pieces ? next.fetch_add(1) : W.pieces;
+                        if (p < W.pieces)
+                            work(p, p + 1, 0);
+                        else
+                            std::this_thread::yield();
+                    }
+                    if (e == hipSuccess)
+                        e = pwmk::launch_copy_bytes(to + k * W.chunk, stage + k * W.chunk, W.size(k), false, s);
+                }
+            };
+            parallel_run(W.pieces, 1, work, &lead);
+        }
+        if (e == hipSuccess && bytes > 2 * kStageBytes) e = hipEventRecord(g_stage_ev[b], s);
+    }
+    if (!wait && e == hipSuccess) return e;
+    const hipError_t e2 = hipStreamSynchronize(s);  // the buffers are the next transfer's
+    return e != hipSuccess ? e : e2;
+}
+
+// Device -> host: empty(stage, a0, a1) takes bytes [a0, a1) from `stage`.  Waits
+// for the work queued on s.  b: the buffer to begin with.
+template <typename Empty>
+static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, Empty empty, int b = 0) {
+    auto issue = [&](size_t off, int to) {
+        const Window W(std::min(kStageBytes, bytes - off), bytes);
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < W.nch && e == hipSuccess; ++k) {
+            e = pwmk::launch_copy_bytes((char*)g_stage[to] + k * W.chunk, (const char*)src + off + k * W.chunk, W.size(k),
+                                        true, s);
+            if (e == hipSuccess) e = hipEventRecord(g_ring_ev[to * kRingChunks + k], s);
+        }
+        return e;
+    };
+    hipError_t e = issue(0, b);
+    for (size_t off = 0; off < bytes && e == hipSuccess; off += kStageBytes, b ^= 1) {
+        if (off + kStageBytes < bytes && (e = issue(off + kStageBytes, b ^ 1)) != hipSuccess) break;
+        const size_t n = std::min(kStageBytes, bytes - off);
+        const char* stage = (const char*)g_stage[b];
+        if (n <= kInlineBytes) {
+            e = hipEventSynchronize(g_ring_ev[b * kRingChunks]);
+            if (e == hipSuccess) empty(stage, off, off + n);
+            continue;
+        }
+        const Window W(n, bytes);
+        std::atomic<size_t> ready{0};  // chunks that have arrived
+        std::atomic<bool> bad{false};
+        const LoopFn work = [&](int64_t p0, int64_t p1, int) {
+            for (int64_t p = p0; p < p1; ++p) {
+                while (ready.load(std::memory_order_acquire) <= W.chunk_of(p)) std::this_thread::yield();
+                const size_t a0 = (size_t)p * W.piece, a1 = std::min(n, a0 + W.piece);
+                if (!bad) empty(stage + a0, off + a0, off + a1);
+            }
+        };
+        const LeadFn lead = [&](std::atomic<int64_t>&) {
+            for (size_t k = 0; k < W.nch; ++k) {
+                if (e == hipSuccess) e = hipEventSynchronize(g_ring_ev[b * kRingChunks + k]);
+                if (e != hipSuccess) bad = true;
+                ready.store(k + 1, std::memory_order_release);
+            }
+        };
+        parallel_run(W.pieces, 1, work, &lead);
+    }
+    const hipError_t e2 = hipStreamSynchronize(s);
+    return e != hipSuccess ? e : e2;
+}
+
+// Host -> device chunk by chunk (a caller that works between the chunks):
+// fill(stage, a0, a1) writes bytes [a0, a1) of the transfer into `stage`
+// (called by host threads on pieces of a chunk); host threads fill one buffer
+// while the other is in flight.  The caller holds g_stage_mu and stage_ready()
+// is true.
 template <typename Fill>
 static hipError_t staged_upload(void* dst, size_t bytes, hipStream_t s, Fill fill,
                                 const std::function<void()>* between) {
@@ -226,9 +411,8 @@ hipError_t upload_staged(void* dst, const void* src, size_t bytes, hipStream_t s
         hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    const char* from = (const char*)src;
-    return staged_upload(
-        dst, bytes, s, [from](char* to, size_t a0, size_t a1) { memcpy(to, from + a0, a1 - a0); }, between);
+    if (between && *between) return staged_upload(dst, bytes, s, bytes_in(src), between);
+    return window_upload(dst, bytes, s, bytes_in(src));
 }
 
 hipError_t upload_indices_staged(void* dst, const int32_t* src, int64_t n, int64_t bound, bool* out_of_range,
@@ -268,20 +452,6 @@ hipError_t upload_indices_staged(void* dst, const int32_t* src, int64_t n, int64
     return e;
 }
 
-// FP64 value k as stored: FP32, or BF16 as the upper half of the FP32 value
-// (exact for values exact in BF16, which the callers check).
-static inline void narrow_value(const double* v, int vt, int64_t k, char* out) {
-    const float f = (float)v[k];
-    if (vt == PWM_VALUES_F32) {
-        memcpy(out, &f, 4);
-    } else {
-        uint32_t u;
-        memcpy(&u, &f, 4);
-        const uint16_t h = (uint16_t)(u >> 16);
-        memcpy(out, &h, 2);
-    }
-}
-
 hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt, hipStream_t s,
                                 const std::function<void()>* between) {
     if (vt == PWM_VALUES_F64) return upload_staged(dst, src, (size_t)n * 8, s, between);
@@ -297,46 +467,22 @@ hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt,
         hipError_t e = hipMemcpyAsync(dst, o, tmp.size(), hipMemcpyHostToDevice, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    // pieces of a chunk start and end on whole values (chunks and pieces are
-    // multiples of 256 KB, and every range below is split at multiples of es)
-    return staged_upload(
-        dst, (size_t)n * es, s,
-        [src, vt, es](char* to, size_t a0, size_t a1) {
-            for (size_t k = a0 / es; k < a1 / es; ++k) narrow_value(src, vt, (int64_t)k, to + (k - a0 / es) * es);
-        },
-        between);
+    if (between && *between) return staged_upload(dst, (size_t)n * es, s, values_in(src, vt), between);
+    return window_upload(dst, (size_t)n * es, s, values_in(src, vt));
 }
 
-hipError_t download_staged(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes == 0) return hipSuccess;
+hipError_t download_doubles(double* dst, const void* src, int64_t n, bool f64, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    const size_t bytes = (size_t)n * (f64 ? 8 : 4);
     std::lock_guard<std::mutex> lk(g_stage_mu);
-    if (!stage_ready()) {
-        hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
-    }
-    // the copy of chunk k+1 into one buffer runs while host threads empty
-    // chunk k from the other
-    const size_t chunk = stage_chunk(bytes);
-    const int64_t piece = stage_piece(chunk);
-    const size_t nch = (bytes + chunk - 1) / chunk;
-    auto issue = [&](size_t k) {
-        const size_t off = k * chunk, n = std::min(chunk, bytes - off);
-        hipError_t e = hipMemcpyAsync(g_stage[k & 1], (const char*)src + off, n, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(g_stage_ev[k & 1], s);
+    if (!stage_ready()) {  // no pinned memory: a plain copy to pageable memory
+        std::vector<float> f(f64 ? 0 : n);
+        hipError_t e = hipMemcpyAsync(f64 ? (void*)dst : f.data(), src, bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        for (size_t i = 0; i < f.size() && e == hipSuccess; ++i) dst[i] = f[i];
         return e;
-    };
-    hipError_t e = issue(0);
-    for (size_t k = 0; k < nch && e == hipSuccess; ++k) {
-        if (k + 1 < nch && (e = issue(k + 1)) != hipSuccess) break;
-        if ((e = hipEventSynchronize(g_stage_ev[k & 1])) != hipSuccess) break;
-        const size_t off = k * chunk, n = std::min(chunk, bytes - off);
-        const char* stage = (const char*)g_stage[k & 1];
-        char* to = (char*)dst + off;
-        parallel_for((int64_t)n, piece,
-                     [&](int64_t a0, int64_t a1, int) { memcpy(to + a0, stage + a0, (size_t)(a1 - a0)); });
     }
-    const hipError_t e2 = hipStreamSynchronize(s);
-    return e != hipSuccess ? e : e2;
+    return f64 ? window_download(src, bytes, s, bytes_out(dst)) : window_download(src, bytes, s, floats_out(dst));
 }
 
 int fail(pwm_matrix* h, int code, const std::string& msg) {
@@ -1357,33 +1503,34 @@ static int stage_vectors(pwm_matrix* h) {
 
 // Host double vector -> device vector of the handle's type.
 static int upload_vec(pwm_matrix* h, const double* src, void* dst, int64_t n) {
-    hipError_t e;
-    if (h->vtype == PWM_VALUES_F64) {
-        e = upload_staged(dst, src, n * 8, h->stream);
-    } else {
-        std::unique_ptr<float[]> f(new float[std::max<int64_t>(n, 1)]);
-        parallel_for(n, (int64_t)1 << 18, [&](int64_t i0, int64_t i1, int) {
-            for (int64_t i = i0; i < i1; ++i) f[i] = (float)src[i];
-        });
-        e = upload_staged(dst, f.get(), n * 4, h->stream);
-    }
-    if (e != hipSuccess) return hip_fail(h, e, "vector upload");
-    return PWM_OK;
+    const int vt = h->vtype == PWM_VALUES_F64 ? PWM_VALUES_F64 : PWM_VALUES_F32;
+    const hipError_t e = upload_values_staged(dst, src, n, vt, h->stream);
+    return e == hipSuccess ? PWM_OK : hip_fail(h, e, "vector upload");
 }
 static int download_vec(pwm_matrix* h, const void* src, double* dst, int64_t n) {
-    hipError_t e;
-    if (h->vtype == PWM_VALUES_F64) {
-        e = download_staged(dst, src, n * 8, h->stream);
-    } else {
-        std::unique_ptr<float[]> f(new float[std::max<int64_t>(n, 1)]);
-        e = download_staged(f.get(), src, n * 4, h->stream);
-        if (e == hipSuccess)
-            parallel_for(n, (int64_t)1 << 18, [&](int64_t i0, int64_t i1, int) {
-                for (int64_t i = i0; i < i1; ++i) dst[i] = f[i];
-            });
+    const hipError_t e = download_doubles(dst, src, n, h->vtype == PWM_VALUES_F64, h->stream);
+    return e == hipSuccess ? PWM_OK : hip_fail(h, e, "vector download");
+}
+
+// y = A x on host vectors of at most one staging buffer each: x goes through
+// one, y through the other, and the host waits once, for y.
+static int mv_staged(pwm_matrix* h, const double* x, double* y, bool* done) {
+    const bool f64 = h->vtype == PWM_VALUES_F64;
+    const size_t vs = vector_size(h->vtype);
+    if ((size_t)std::max(h->nor, h->noc) * vs > kStageBytes) return PWM_OK;
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    if (!stage_ready()) return PWM_OK;  // no pinned memory: the general path
+    *done = true;
+    hipError_t e = f64 ? window_upload(h->hx.p, (size_t)h->noc * vs, h->stream, bytes_in(x), false)
+                       : window_upload(h->hx.p, (size_t)h->noc * vs, h->stream, values_in(x, PWM_VALUES_F32), false);
+    const int rc = e == hipSuccess ? spmv_launch(h, h->hx.p, h->hy.p, nullptr) : hip_fail(h, e, "vector upload");
+    if (rc != PWM_OK) {
+        (void)hipStreamSynchronize(h->stream);
+        return rc;
     }
-    if (e != hipSuccess) return hip_fail(h, e, "vector download");
-    return PWM_OK;
+    e = f64 ? window_download(h->hy.p, (size_t)h->nor * vs, h->stream, bytes_out(y), 1)
+            : window_download(h->hy.p, (size_t)h->nor * vs, h->stream, floats_out(y), 1);
+    return e == hipSuccess ? PWM_OK : hip_fail(h, e, "vector download");
 }
 
 extern "C" int pwm_mv(pwm_matrix* h, const double* x, double* y) {
@@ -1392,6 +1539,9 @@ extern "C" int pwm_mv(pwm_matrix* h, const double* x, double* y) {
     if (!x || !y) return fail(h, PWM_ERR_INVALID, "pwm_mv: NULL vector");
     if (x < y + h->nor && y < x + h->noc) return fail(h, PWM_ERR_INVALID, "pwm_mv: x and y overlap");
     int rc = stage_vectors(h);
+    bool done = false;
+    if (rc == PWM_OK) rc = mv_staged(h, x, y, &done);
+    if (done) return rc;
     if (rc == PWM_OK) rc = upload_vec(h, x, h->hx.p, h->noc);
     if (rc == PWM_OK) rc = spmv_launch(h, h->hx.p, h->hy.p, nullptr);
     if (rc == PWM_OK) rc = download_vec(h, h->hy.p, y, h->nor);

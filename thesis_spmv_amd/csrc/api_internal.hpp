@@ -26,7 +26,12 @@ namespace pwm_impl {
 // at a time.  A persistent pool of 15 threads plus the caller runs it; a call
 // made while the pool is busy (another thread, or from inside fn) starts its
 // own threads instead.
-void parallel_run(int64_t n, int64_t chunk, const std::function<void(int64_t, int64_t, int)>& fn);
+// `lead`, where given, is run by the calling thread first, while the others
+// work; it may take chunks itself (next.fetch_add(chunk)) and returns when the
+// caller should join the loop.
+using LoopFn = std::function<void(int64_t, int64_t, int)>;
+using LeadFn = std::function<void(std::atomic<int64_t>& next)>;
+void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn, const LeadFn* lead = nullptr);
 template <typename F>
 void parallel_for(int64_t n, int64_t chunk, F fn) {
     if (n <= 0) return;
@@ -34,7 +39,7 @@ void parallel_for(int64_t n, int64_t chunk, F fn) {
         fn((int64_t)0, n, 0);
         return;
     }
-    parallel_run(n, chunk, std::function<void(int64_t, int64_t, int)>(fn));
+    parallel_run(n, chunk, LoopFn(fn));
 }
 
 // Thread-local message for calls without a handle.
@@ -262,8 +267,9 @@ hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt,
 // then complete but must not be used)
 hipError_t upload_indices_staged(void* dst, const int32_t* src, int64_t n, int64_t bound, bool* out_of_range,
                                  hipStream_t s, const std::function<void()>* between = nullptr);
-// Device -> host the same way (after the work queued on s).
-hipError_t download_staged(void* dst, const void* src, size_t bytes, hipStream_t s);
+// n device values (FP64 or FP32), as doubles on the host, the same way (after
+// the work queued on s).
+hipError_t download_doubles(double* dst, const void* src, int64_t n, bool f64, hipStream_t s);
 // CSB slab-stream layout built on the device from the device CRS arrays
 // (csb_build.hip); h->csb.bits/H/V set.  csb_key_bits: bits of its sort key.
 int csb_key_bits(int64_t cells, int bits);

@@ -506,14 +506,7 @@ extern "C" int pwm_batch_vector(pwm_batch* b, int32_t id, double* out, double* y
     const BatchInst& I = b->inst[id];
     const size_t xs = pwm_impl::vector_size(b->vtype);
     const char* src = (const char*)b->arena.at(I.o_vec) + (b->where[id] ? I.n * xs : 0);
-    hipError_t e;
-    if (b->vtype == PWM_VALUES_F64) {
-        e = hipMemcpy(out, src, I.n * 8, hipMemcpyDeviceToHost);
-    } else {
-        std::vector<float> f(I.n);
-        e = hipMemcpy(f.data(), src, I.n * 4, hipMemcpyDeviceToHost);
-        for (int64_t i = 0; i < I.n; ++i) out[i] = f[i];
-    }
+    const hipError_t e = pwm_impl::download_doubles(out, src, I.n, b->vtype == PWM_VALUES_F64, b->stream);
     if (e != hipSuccess) return bhip(b, e, "pwm_batch_vector");
     if (ynorm) *ynorm = b->ynorm[id];
     return PWM_OK;

@@ -183,6 +183,29 @@ __global__ void k_gather_fill(uint32_t* __restrict__ idx, double* __restrict__ v
     }
 }
 
+// Bytes between device and pinned host memory, 16 at a time.  PCIe-bound (57
+// GB/s): 64 blocks read 8 MB of host memory in 163 us and 1024 in 213, 256
+// blocks write it in 162.
+__global__ __launch_bounds__(256) void k_copy_bytes(uint4* __restrict__ dst, const uint4* __restrict__ src, int64_t n16,
+                                                    int tail) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256) dst[i] = src[i];
+    if (blockIdx.x == 0 && (int)threadIdx.x < tail)
+        ((char*)(dst + n16))[threadIdx.x] = ((const char*)(src + n16))[threadIdx.x];
+}
+
+hipError_t launch_copy_bytes(void* dst, const void* src, size_t bytes, bool to_host, hipStream_t s) {
+    if (bytes == 0) return hipSuccess;
+    // From 8 MB on the copy engine's setup no longer counts (160 us either way);
+    // odd addresses (a vector inside a larger buffer) are left to it too.
+    if (bytes >= (size_t)8 << 20 || ((uintptr_t)dst | (uintptr_t)src) % 16)
+        return hipMemcpyAsync(dst, src, bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
+    const int64_t n16 = (int64_t)(bytes / 16);
+    const int64_t most = to_host ? 256 : 64;
+    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(most, (n16 + 255) / 256));
+    hipLaunchKernelGGL(k_copy_bytes, dim3(g), dim3(256), 0, s, (uint4*)dst, (const uint4*)src, n16, (int)(bytes % 16));
+    return hipGetLastError();
+}
+
 // Scatter of the column indices: over `groups` groups of 256 consecutive
 // entries spread evenly, the 128-byte x lines each group touches (a hash table
 // of a wave in LDS), summed into *lines.

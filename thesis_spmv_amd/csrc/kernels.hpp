@@ -119,6 +119,8 @@ hipError_t launch_power_finish(const PowerArgs& pw, int64_t n, int is_f64, hipSt
 hipError_t launch_flush(void* p, int64_t bytes, hipStream_t s);
 // Plain streaming copy (profiler counter calibration).
 hipError_t launch_stream_copy(void* dst, const void* src, int64_t bytes, hipStream_t s);
+// Bytes between device and pinned host memory.
+hipError_t launch_copy_bytes(void* dst, const void* src, size_t bytes, bool to_host, hipStream_t s);
 // Distinct lines of 2^shift columns per group of 256 consecutive entries, over
 // `groups` groups (nnz >= 256), added to *lines.
 hipError_t launch_scatter(const int32_t* ci, int64_t nnz, int64_t groups, int shift, unsigned* lines, hipStream_t s);
