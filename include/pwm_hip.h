@@ -174,9 +174,9 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * "csb_build" (CSB slab-piece layout built on the device, 0, or on the host,
  * 1; both give the same arrays; the slab streams are always built on the
  * device), "coh_build" (BlockCOH layout built on the device, 0, or on the
- * host, 1; both give the same arrays), "coh_occ8" (BlockCOH kernel instance
- * with registers capped for 8 waves per SIMD: 1, the compiler's budget: 0,
- * or -1 = time both at load, the default), "crs_kernel" (CRS: 0 = one wave per tile of short
+ * host, 1; both give the same arrays), "coh_occ8" (-1, 0 or 1, reported
+ * as high_occupancy, -1 as 1; one BlockCOH kernel, at 8 waves per SIMD,
+ * serves all three), "crs_kernel" (CRS: 0 = one wave per tile of short
  * rows when no row has more than 64 entries, else time the vector kernel at
  * three lane counts and the row-aligned tiles kernel at load and keep the
  * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =

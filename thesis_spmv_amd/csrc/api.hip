@@ -1414,7 +1414,7 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
             break;
         case PWM_FORMAT_CRS_MERGE: out->kernels = h->crs_used == 3 ? 1 : 2; break;
         case PWM_FORMAT_CSB: out->kernels = h->csb.sweep ? 1 : 1 + (h->csb.groups > 1 ? 1 : 0); break;
-        case PWM_FORMAT_BLOCKCOH: out->kernels = 1 + (h->coh.n_atomic > 0 ? 1 : 0); break;
+        case PWM_FORMAT_BLOCKCOH: out->kernels = 1 + (h->coh.n_pieces > 0 ? 1 : 0); break;
     }
     if (swept_crs(h)) out->kernels = 1;
     if (h->format == PWM_FORMAT_CSB && h->csb.n_tasks <= 0) out->kernels = 0;
@@ -1426,9 +1426,9 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
                                       &h->lr_partial, &h->split_a, &h->split_b, &h->carry_row, &h->carry_val, &h->tiles,
                                       &h->rows_cut, &h->csb.ind, &h->csb.data, &h->csb.blk_ptr, &h->csb.work, &h->csb.ypart,
                                       &h->csb.soff, &h->csb.srows, &h->csb.sweep_start,
-                                      &h->coh.row_jump, &h->coh.col_jump, &h->coh.data, &h->coh.row_jump_block,
+                                      &h->coh.ent, &h->coh.data, &h->coh.row_jump_block,
                                       &h->coh.col_jump_block, &h->coh.block_nnz, &h->coh.block_coords,
-                                      &h->coh.band_table, &h->coh.tasks, &h->sm_rs, &h->sm_ci, &h->sm_val, &h->pw_ctrl, &h->pw_rec, &h->pw_partials,
+                                      &h->coh.band_table, &h->coh.tasks, &h->coh.ysum, &h->sm_rs, &h->sm_ci, &h->sm_val, &h->pw_ctrl, &h->pw_rec, &h->pw_partials,
                                       &h->hx, &h->hy};
     int64_t b = 0;
     for (auto* d : bufs) b += (int64_t)d->bytes;

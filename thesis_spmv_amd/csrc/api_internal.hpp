@@ -16,6 +16,8 @@
 
 namespace blocked {
 struct CohTask;
+struct CohRows;
+struct CohBand;
 }
 
 namespace pwm_impl {
@@ -144,25 +146,26 @@ struct CsbDev {
 struct CohBandMeta {
     int64_t start, rows, nnz, blocks, row_jumps, block_row_jumps;
     int32_t beta_bits, H, V;
-    int64_t off_nz, off_rj, off_blk, off_rjb;
+    int64_t off_nz, off_blk, off_rjb;
 };
 struct CohDev {
     std::vector<CohBandMeta> bands;
-    DevBuf row_jump, col_jump, data, row_jump_block, col_jump_block, block_nnz;
-    DevBuf block_coords;   // decoded (block_row, block_col, entry offset, row_jump offset) per block
-    DevBuf band_table;     // per band: start, rows, beta_bits, first block, blocks
-    DevBuf tasks;          // per band: chunk -> first block table
+    DevBuf ent, data, row_jump_block, col_jump_block, block_nnz;  // ent: packed positions (coh_pack)
+    DevBuf block_coords;   // first row and column per block
+    DevBuf band_table;     // per band: start, rows, first block, entries, step table
+    DevBuf tasks;          // per band: step -> block table
     DevBuf task_list;      // CohTask per workgroup
-    DevBuf atomic_bands;   // bands accumulated with global atomics
-    int64_t n_tasks = 0, total_blocks = 0, n_atomic = 0;
+    DevBuf row_pieces;     // rows accumulated with global atomics (CohRows)
+    DevBuf ysum;           // their sums
+    int64_t n_tasks = 0, total_blocks = 0, n_pieces = 0;
     int32_t lds_rows = 0;  // rows of the largest band accumulated in LDS (the kernel's LDS window)
-    int32_t occ8 = 0;      // kernel instance with 8 waves per SIMD (timed at load)
+    int32_t occ8 = 0;      // reported: 8 waves per SIMD unless the option coh_occ8 says 0
     void clear() {
         bands.clear();
-        for (DevBuf* b : {&row_jump, &col_jump, &data, &row_jump_block, &col_jump_block, &block_nnz, &block_coords,
-                          &band_table, &tasks, &task_list, &atomic_bands})
+        for (DevBuf* b : {&ent, &data, &row_jump_block, &col_jump_block, &block_nnz, &block_coords, &band_table, &tasks, &task_list, &row_pieces,
+                          &ysum})
             b->release();
-        n_tasks = total_blocks = n_atomic = 0;
+        n_tasks = total_blocks = n_pieces = 0;
         lds_rows = 0;
         occ8 = 0;
     }
@@ -222,7 +225,7 @@ struct pwm_matrix {
     int32_t csb_sweep_unroll = 2; // swept slabs: groups of 4 entries per lane per chunk (1, 2 or 4)
     int32_t csb_sweep_waves = 1;  // swept slabs: slabs per CU (workgroups run in that many waves)
     int32_t csb_sweep_order = 1;  // swept slabs: 0 = rows inside a window's run, 1 = columns (lanes share x lines)
-    int32_t coh_occ8 = -1;        // BlockCOH kernel at 8 waves per SIMD: -1 timed at load, 0 no, 1 yes
+    int32_t coh_occ8 = -1;        // BlockCOH: reported as high_occupancy (-1 or 1: yes); one kernel serves all
     int32_t csb_unroll = 0;  // stream kernel groups of 4 per thread per step (0 = default)
     int32_t csb_nt = -1;     // slab streams: non-temporal entry loads / partial stores (-1 = timed)
     int32_t csb_build = 0;   // CSB slab pieces: 0 = built on the device, 1 = on the host
@@ -290,11 +293,13 @@ int build_swept_beside_crs(pwm_matrix* h);
 // BlockCOH layout built on the device from the device CRS arrays
 // (coh_build.hip); h->coh.bands holds the band partition (start, rows, nnz,
 // beta_bits, H, V, off_nz) on entry and the per-band sizes and offsets on
-// return.  coh_plan_tasks: the kernel's work list for those bands, decode
-// states left zero.
+// return.  coh_plan_tasks: the kernel's work list for those bands.
+// coh_clear_sums: the sums of the rows of atomic bands, zero.
 int coh_layout_device(pwm_matrix* h, int64_t lds_rows);
 void coh_plan_tasks(const std::vector<CohBandMeta>& B, int64_t lds_rows, std::vector<blocked::CohTask>& tasks,
-                    std::vector<int32_t>& atomic_bands, int32_t* max_lds_rows);
+                    std::vector<blocked::CohRows>& pieces, std::vector<blocked::CohBand>& table,
+                    int32_t* max_lds_rows);
+hipError_t coh_clear_sums(pwm_matrix* h, const std::vector<blocked::CohRows>& pieces);
 // Statistics of the loaded CRS arrays (stats.hip) into h->stats; needs the
 // device row_start / col_ind.
 int compute_matrix_stats(pwm_matrix* h);

@@ -75,49 +75,68 @@ struct CsbArgs {
 int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32);
 
 
-// One BlockCOH block (offsets are relative to its band's arrays).
+// Workgroup size of the blocked kernels.
+constexpr int kBlockedBS = 512;
+
+// BlockCOH entries, in the format's order (per band the blocks in Hilbert
+// order, inside a block by rows): (first entry of its block) << 31 | row in the
+// block << 15 | column in the block, both below beta <= 2^15.  The jumps of the
+// format (ICRS inside a block) follow from two neighbours and are formed where
+// they are asked for; stored, they cost the same 4 bytes and every SpMV two
+// scans over the entries to undo them.
+constexpr uint32_t kCohFirst = 0x80000000u;
+inline uint32_t coh_pack(uint32_t row, uint32_t col, bool first) { return (first ? kCohFirst : 0u) | row << 15 | col; }
+
+// A block: its first row (inside the band) and column.
 struct CohBlock {
-    int32_t entry;      // first entry (col_jump / data index)
-    int32_t row_jump;   // first row_jump index
-    int32_t brow, bcol; // block coordinates inside the band
+    int32_t row, col;
 };
 
-// Workgroup size and entries per thread of the blocked kernels; a BlockCOH
-// workgroup decodes kCohChunk consecutive entries of its band per step.
-constexpr int kBlockedBS = 512;
-constexpr int kCohIPT = 4;
-constexpr int kCohChunk = kBlockedBS * kCohIPT;
+// A wave takes kCohStep consecutive entries of a band at a time, 4 per lane.
+// The steps of a band begin at its first entry rounded down to a multiple of 4,
+// so that a lane's 4 entries are aligned.
+constexpr int kCohStep = 256;
+__host__ __device__ inline int64_t coh_steps(int64_t entry, int64_t nnz) {
+    return nnz > 0 ? (nnz + (entry & 3) + kCohStep - 1) / kCohStep : 0;
+}
 
 struct CohBand {
-    int32_t start, rows, beta_bits, first_block, blocks, entry, nnz;
-    int32_t chunk_table;  // offset of the band's chunk -> first-block table
+    int32_t start, rows, first_block, blocks, entry, nnz;
+    int32_t step_table;  // offset of the band's step -> block table
+    int32_t sum;         // atomic bands: the first row's place in CohArgs::ysum
 };
 
-// Unit of work of the BlockCOH kernel: chunks [chunk0, chunk0+nchunks) of one
+// Unit of work of the BlockCOH kernel: steps [step0, step0+nsteps) of one
 // band.  A band whose rows fit the LDS window and whose entries fit one task
-// accumulates in LDS (atomic = 0); larger bands are cut into several tasks
-// that add into y with global atomics (atomic = 1), each starting from the
-// decode state (carry_s, carry_r) the build computed for its first entry.
-constexpr int kCohTaskChunks = 16;
+// accumulates in LDS (atomic = 0); larger bands are cut into several tasks of
+// two steps per wave that add into ysum with global atomics (atomic = 1).
+constexpr int kCohTaskSteps = 128;
+constexpr int kCohAtomicSteps = 16;
 struct CohTask {
-    int32_t band, chunk0, nchunks, atomic;
-    int32_t carry_s, carry_r;
+    int32_t band, step0, nsteps, atomic;
+};
+
+// Rows of atomic bands in pieces, one per workgroup of the kernel that finishes
+// them; sum: the first row's place in CohArgs::ysum.
+constexpr int kCohPieceRows = 2048;
+struct CohRows {
+    int32_t start, rows, sum;
 };
 
 struct CohArgs {
-    int64_t nor = 0, noc = 0;
-    int64_t n_bands = 0;
+    int64_t nor = 0;
     int64_t n_tasks = 0;
     const CohTask* tasks = nullptr;
     const CohBand* bands = nullptr;
     const CohBlock* blocks = nullptr;
-    const int32_t* chunk_block = nullptr;  // per band: block holding entry c*kCohChunk, c = 0..chunks
-    const uint16_t* col_jump = nullptr;
-    const uint16_t* row_jump = nullptr;
+    const int32_t* step_block = nullptr;  // per band and step: the last block that starts before it (-1: none)
+    const uint32_t* ent = nullptr;
     const void* val = nullptr;
+    const CohRows* pieces = nullptr;
+    int64_t n_pieces = 0;
+    double* ysum = nullptr;  // rows of atomic bands, zero between two SpMVs
     int vtype = 0;
     int32_t lds_rows = 0;  // LDS window of the kernel: rows of the largest LDS-accumulated band
-    int32_t occ8 = 0;      // 1: the kernel instance capped to 8 waves per SIMD
 };
 
 // part: 0 = the whole SpMV, 1 = the slab kernel only, 2 = the column-group
@@ -126,7 +145,6 @@ hipError_t launch_csb(const CsbArgs& a, const void* x, void* y, const pwmk::Powe
                       int part = 0);
 // workgroups of the CSB column-group reduction (= its power-method partials)
 int csb_reduce_blocks(int64_t nor);
-hipError_t launch_coh(const CohArgs& a, const int32_t* atomic_bands, int n_atomic, const void* x, void* y,
-                      const pwmk::PowerArgs* pw, hipStream_t s);
+hipError_t launch_coh(const CohArgs& a, const void* x, void* y, const pwmk::PowerArgs* pw, hipStream_t s);
 
 }  // namespace blocked

@@ -580,25 +580,48 @@ static void coh_bands(int64_t nor, int64_t nnz, const int32_t* rs, int threads, 
 }
 
 // Work list: one LDS task per band whose rows fit the LDS window and whose
-// entries fit one task, atomic tasks of at most kCohTaskChunks chunks
-// otherwise (decode states left zero for the caller to fill).
+// entries fit one task (and are not many times the others'), atomic tasks of
+// kCohAtomicSteps steps otherwise.
 void coh_plan_tasks(const std::vector<CohBandMeta>& B, int64_t lds_rows, std::vector<blocked::CohTask>& tasks,
-                    std::vector<int32_t>& atomic_bands, int32_t* max_lds_rows) {
+                    std::vector<blocked::CohRows>& pieces, std::vector<blocked::CohBand>& table,
+                    int32_t* max_lds_rows) {
     tasks.clear();
-    atomic_bands.clear();
+    pieces.clear();
+    // What one workgroup may be left with: a band closes before the row that
+    // would exceed its share, so the last band holds what the others left, on
+    // power-law rows 3 to 20 times their size (100 K rows: 18 us with that band
+    // cut, 25 without; 500 K: 64 and 69).
+    int32_t sum = 0;
+    int64_t nnz = 0;
+    for (const CohBandMeta& m : B) nnz += m.nnz;
+    const int64_t most = std::min<int64_t>(blocked::kCohTaskSteps * (int64_t)blocked::kCohStep,
+                                           std::max<int64_t>(8192, 2 * nnz / std::max<int64_t>(1, (int64_t)B.size())));
     *max_lds_rows = 0;
     for (int p = 0; p < (int)B.size(); ++p) {
         const CohBandMeta& m = B[p];
-        const int64_t nch = (m.nnz + blocked::kCohChunk - 1) / blocked::kCohChunk;
-        if (m.rows <= lds_rows && nch <= blocked::kCohTaskChunks) {
-            if (m.rows > 0) tasks.push_back({p, 0, (int32_t)nch, 0, 0, 0});
+        const int64_t steps = blocked::coh_steps(m.off_nz, m.nnz);
+        if (m.rows <= lds_rows && m.nnz <= most) {
+            if (m.rows > 0) tasks.push_back({p, 0, (int32_t)steps, 0});
             *max_lds_rows = std::max(*max_lds_rows, (int32_t)m.rows);
             continue;
         }
-        atomic_bands.push_back(p);
-        for (int64_t c0 = 0; c0 < nch; c0 += blocked::kCohTaskChunks)
-            tasks.push_back({p, (int32_t)c0, (int32_t)std::min<int64_t>(blocked::kCohTaskChunks, nch - c0), 1, 0, 0});
+        table[p].sum = sum;
+        for (int64_t r = 0; r < m.rows; r += blocked::kCohPieceRows) {
+            const int32_t n = (int32_t)std::min<int64_t>(blocked::kCohPieceRows, m.rows - r);
+            pieces.push_back({(int32_t)(m.start + r), n, sum});
+            sum += n;
+        }
+        for (int64_t s0 = 0; s0 < steps; s0 += blocked::kCohAtomicSteps)
+            tasks.push_back({p, (int32_t)s0, (int32_t)std::min<int64_t>(blocked::kCohAtomicSteps, steps - s0), 1});
     }
+}
+
+hipError_t coh_clear_sums(pwm_matrix* h, const std::vector<blocked::CohRows>& pieces) {
+    h->coh.n_pieces = (int64_t)pieces.size();
+    if (pieces.empty()) return hipSuccess;
+    const size_t bytes = ((size_t)pieces.back().sum + pieces.back().rows) * sizeof(double);
+    const hipError_t e = h->coh.ysum.alloc(bytes);
+    return e == hipSuccess ? hipMemsetAsync(h->coh.ysum.p, 0, bytes, h->stream) : e;
 }
 
 // rs: host row_start; ci / vals: host CRS arrays, needed only by the host
@@ -618,9 +641,9 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
         return t < 1 ? 1 : t;
     };
     // the caller's thread count, else about 16K entries per band and at
-    // least 640 bands (2.5 per CU: a 5M-entry Poisson matrix runs in 40 us
-    // with 639 bands against 57 us with 319); bands the LDS window or one
-    // task cannot hold are split into atomic tasks below
+    // least 640 bands (2.5 per CU: a 5M-entry Poisson matrix runs in 18.9 us
+    // with 640 bands, 20.0 with 319, 55.6 with 160); bands the LDS window or
+    // one task cannot hold are split into atomic tasks below
     threads = threads > 0 ? clamp(threads)
                           : clamp((int)std::min<int64_t>(INT32_MAX, std::max<int64_t>(640, nnz / 16384)));
     coh_bands(nor, nnz, rs, threads, bstart, bnnz);
@@ -645,11 +668,12 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
     if (device) return coh_layout_device(h, lds_rows);
     // Per band: Hilbert order of blocks (hilbert_size/beta grid), ICRS inside
     // each block, BICRS jumps between blocks.
-    std::vector<uint16_t> col_jump(std::max<int64_t>(nnz, 1)), row_jump(std::max<int64_t>(nnz, 1));
+    std::vector<uint32_t> ent(nnz + 64, 0);
     std::vector<double> data(std::max<int64_t>(nnz, 1));
     std::vector<std::vector<int16_t>> rjb(threads), cjb(threads);
     std::vector<std::vector<int32_t>> bnz(threads);
     std::vector<std::vector<blocked::CohBlock>> blocks(threads);
+    std::vector<std::vector<int64_t>> bfirst(threads);  // first entry of each block in its band
     std::vector<int64_t> nrj(threads, 0);
     parallel_for(threads, 1, [&](int64_t p0, int64_t p1, int) {
         std::vector<int64_t> key_of_block, order, rank, cnt;
@@ -696,27 +720,16 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
                 if (s == t) continue;
                 const int64_t blk = order[q], br = blk / H, bc = blk % H;
                 blocked::CohBlock cb;
-                cb.entry = (int32_t)s;
-                cb.row_jump = (int32_t)rj;
-                cb.brow = (int32_t)br;
-                cb.bcol = (int32_t)bc;
-                // ICRS (TripletToCRS.hpp:402-452)
-                int64_t pr = -1, pc = -1;
+                cb.row = (int32_t)(br * beta);
+                cb.col = (int32_t)(bc * beta);
+                int64_t pr = -1;
                 for (int64_t i = s; i < t; ++i) {
                     const int64_t e = perm[i];
                     const int64_t r = lrow[i] % beta, cc = ci[e] % beta;
                     data[e0 + i] = vals[e];
-                    if (i == s) {
-                        row_jump[e0 + rj++] = (uint16_t)r;
-                        col_jump[e0 + i] = (uint16_t)cc;
-                    } else if (r != pr) {
-                        col_jump[e0 + i] = (uint16_t)(cc + beta - pc);
-                        row_jump[e0 + rj++] = (uint16_t)(r - pr);
-                    } else {
-                        col_jump[e0 + i] = (uint16_t)(cc - pc);
-                    }
+                    ent[e0 + i] = blocked::coh_pack((uint32_t)r, (uint32_t)cc, i == s);
+                    rj += i == s || r != pr;
                     pr = r;
-                    pc = cc;
                 }
                 // block-level BICRS (BlockCOH.hpp:433-439)
                 if (blocks[p].empty()) {
@@ -730,40 +743,35 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
                 }
                 bnz[p].push_back((int32_t)(t - s));
                 blocks[p].push_back(cb);
+                bfirst[p].push_back(s);
                 prev_br = br;
                 prev_bc = bc;
             }
             nrj[p] = rj;
         }
     });
-    // concatenate: row_jump entries of band p start at its entry offset (a
-    // band has at most nnz row segments), block tables band after band
+    // concatenate the block tables band after band
     std::vector<blocked::CohBlock> allb;
     std::vector<blocked::CohBand> table(threads);
     std::vector<int16_t> all_rjb, all_cjb;
-    std::vector<int32_t> all_bnz, ctab;
+    std::vector<int32_t> all_bnz, stab;
     for (int p = 0; p < threads; ++p) {
-        // chunk c of the kernel decodes entries [c*kCohChunk, (c+1)*kCohChunk):
-        // ctab[c] = block holding its first entry, ctab[chunks] = last block
-        table[p].chunk_table = (int32_t)ctab.size();
-        const int64_t nch = (B[p].nnz + blocked::kCohChunk - 1) / blocked::kCohChunk;
+        // step i of the kernel: the last block that starts before its first entry
+        table[p].step_table = (int32_t)stab.size();
+        const int64_t base = B[p].off_nz & 3;
         int64_t b = 0;
-        for (int64_t c = 0; c < nch; ++c) {
-            const int64_t e = c * blocked::kCohChunk;
-            while (b + 1 < (int64_t)blocks[p].size() && blocks[p][b + 1].entry <= e) ++b;
-            ctab.push_back((int32_t)b);
+        for (int64_t i = 0; i < blocked::coh_steps(B[p].off_nz, B[p].nnz); ++i) {
+            while (b < (int64_t)bfirst[p].size() && bfirst[p][b] + base < i * blocked::kCohStep) ++b;
+            stab.push_back((int32_t)b - 1);
         }
-        ctab.push_back((int32_t)std::max<int64_t>(0, (int64_t)blocks[p].size() - 1));
         CohBandMeta& m = B[p];
         m.blocks = (int64_t)blocks[p].size();
         m.row_jumps = nrj[p];
         m.block_row_jumps = (int64_t)rjb[p].size();
-        m.off_rj = m.off_nz;
         m.off_blk = (int64_t)allb.size();
         m.off_rjb = (int64_t)all_rjb.size();
         table[p].start = (int32_t)m.start;
         table[p].rows = (int32_t)m.rows;
-        table[p].beta_bits = m.beta_bits;
         table[p].first_block = (int32_t)m.off_blk;
         table[p].blocks = (int32_t)m.blocks;
         table[p].entry = (int32_t)m.off_nz;
@@ -774,54 +782,22 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
         all_bnz.insert(all_bnz.end(), bnz[p].begin(), bnz[p].end());
     }
     c.total_blocks = (int64_t)allb.size();
-    // work list; each atomic task starts from the decode state (S, R) of the
-    // entry before its first one
     std::vector<blocked::CohTask> tasks;
-    std::vector<int32_t> atomic_bands;
-    coh_plan_tasks(B, lds_rows, tasks, atomic_bands, &c.lds_rows);
-    for (size_t t0 = 0; t0 < tasks.size();) {
-        size_t t1 = t0 + 1;
-        while (t1 < tasks.size() && tasks[t1].band == tasks[t0].band) ++t1;
-        if (tasks[t0].atomic) {
-            const int p = tasks[t0].band;
-            const CohBandMeta& m = B[p];
-            const uint16_t* cj = col_jump.data() + m.off_nz;
-            const uint16_t* rj = row_jump.data() + m.off_nz;
-            const std::vector<blocked::CohBlock>& bl = blocks[p];
-            int64_t S = 0, R = 0, b = 0, e = 0;
-            for (size_t t = t0; t < t1; ++t) {
-                // decode up to the entry before the task's first one
-                const int64_t stop = (int64_t)tasks[t].chunk0 * blocked::kCohChunk;
-                for (; e < stop; ++e) {
-                    while (b + 1 < (int64_t)bl.size() && bl[b + 1].entry <= e) ++b;
-                    if (bl[b].entry == e) {
-                        S = cj[e];
-                        R = rj[bl[b].row_jump];
-                    } else {
-                        S += cj[e];
-                        if ((S >> m.beta_bits) != ((S - cj[e]) >> m.beta_bits)) R += rj[bl[b].row_jump + (S >> m.beta_bits)];
-                    }
-                }
-                tasks[t].carry_s = (int32_t)S;
-                tasks[t].carry_r = (int32_t)R;
-            }
-        }
-        t0 = t1;
-    }
-    c.n_atomic = (int64_t)atomic_bands.size();
+    std::vector<blocked::CohRows> pieces;
+    coh_plan_tasks(B, lds_rows, tasks, pieces, table, &c.lds_rows);
     hipError_t e;
-    if ((e = upload(c.col_jump, col_jump.data(), nnz * 2)) != hipSuccess ||
-        (e = upload(c.row_jump, row_jump.data(), nnz * 2)) != hipSuccess ||
+    if ((e = upload(c.ent, ent.data(), ent.size() * 4)) != hipSuccess ||
         (e = upload(c.row_jump_block, all_rjb.data(), all_rjb.size() * 2)) != hipSuccess ||
         (e = upload(c.col_jump_block, all_cjb.data(), all_cjb.size() * 2)) != hipSuccess ||
         (e = upload(c.block_nnz, all_bnz.data(), all_bnz.size() * 4)) != hipSuccess ||
         (e = upload(c.block_coords, allb.data(), allb.size() * sizeof(blocked::CohBlock))) != hipSuccess ||
         (e = upload(c.band_table, table.data(), table.size() * sizeof(blocked::CohBand))) != hipSuccess ||
-        (e = upload(c.tasks, ctab.data(), ctab.size() * 4)) != hipSuccess ||
+        (e = upload(c.tasks, stab.data(), stab.size() * 4)) != hipSuccess ||
         (e = upload(c.task_list, tasks.data(), tasks.size() * sizeof(blocked::CohTask))) != hipSuccess ||
-        (e = upload(c.atomic_bands, atomic_bands.data(), atomic_bands.size() * 4)) != hipSuccess)
+        (e = upload(c.row_pieces, pieces.data(), pieces.size() * sizeof(blocked::CohRows))) != hipSuccess ||
+        (e = coh_clear_sums(h, pieces)) != hipSuccess)
         return hip_fail(h, e, "BlockCOH upload");
-    data.resize(nnz);
+    data.resize(nnz + 64);  // the kernel reads whole quads
     rc = upload_blocked_values(h, c.data, data);
     if (rc != PWM_OK) return rc;
     c.n_tasks = (int64_t)tasks.size();
@@ -834,7 +810,7 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
 int64_t csb_partials(const pwm_matrix* h) {
     return h->csb.groups > 1 && !h->csb.sweep ? blocked::csb_reduce_blocks(h->nor) : h->csb.n_tasks;
 }
-int64_t coh_partials(const pwm_matrix* h) { return h->coh.n_tasks + h->coh.n_atomic; }
+int64_t coh_partials(const pwm_matrix* h) { return h->coh.n_tasks + h->coh.n_pieces; }
 
 hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw, int part) {
     blocked::CsbArgs a;
@@ -879,69 +855,30 @@ hipError_t csb_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
 hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerArgs* pw) {
     blocked::CohArgs a;
     a.nor = h->nor;
-    a.noc = h->noc;
-    a.n_bands = (int64_t)h->coh.bands.size();
     a.n_tasks = h->coh.n_tasks;
     a.tasks = h->coh.task_list.as<blocked::CohTask>();
     a.bands = h->coh.band_table.as<blocked::CohBand>();
     a.blocks = h->coh.block_coords.as<blocked::CohBlock>();
-    a.chunk_block = h->coh.tasks.as<int32_t>();
-    a.col_jump = h->coh.col_jump.as<uint16_t>();
-    a.row_jump = h->coh.row_jump.as<uint16_t>();
+    a.step_block = h->coh.tasks.as<int32_t>();
+    a.ent = h->coh.ent.as<uint32_t>();
     a.val = h->coh.data.p;
     a.vtype = h->vtype;
     a.lds_rows = h->coh.lds_rows;
-    a.occ8 = h->coh.occ8;
-    hipError_t e = blocked::launch_coh(a, h->coh.atomic_bands.as<int32_t>(), (int)h->coh.n_atomic, x, y, pw, h->stream);
+    a.pieces = h->coh.row_pieces.as<blocked::CohRows>();
+    a.n_pieces = h->coh.n_pieces;
+    a.ysum = h->coh.ysum.as<double>();
+    hipError_t e = blocked::launch_coh(a, x, y, pw, h->stream);
     if (e == hipSuccess && pw)
         e = pwmk::launch_power_reduce(*pw, coh_partials(h), h->stream);
     return e;
 }
 
-// Mean milliseconds of 5 BlockCOH SpMVs (after 2 warm-up ones) on x = 1.
-static int time_coh(pwm_matrix* h, float* ms) {
-    DevBuf tx, ty;
-    const size_t vs = vector_size(h->vtype);
-    hipError_t e;
-    if ((e = tx.alloc(std::max<int64_t>(h->noc, 1) * vs)) != hipSuccess ||
-        (e = ty.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess)
-        return hip_fail(h, e, "BlockCOH autotune vectors");
-    e = pwmk::launch_fill(tx.p, h->noc, h->vtype == PWM_VALUES_F64, 1.0, h->stream);
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (e == hipSuccess) e = hipEventCreate(&e0);
-    if (e == hipSuccess) e = hipEventCreate(&e1);
-    for (int w = 0; w < 2 && e == hipSuccess; ++w) e = coh_launch(h, tx.p, ty.p, nullptr);
-    if (e == hipSuccess) e = hipEventRecord(e0, h->stream);
-    for (int r = 0; r < 5 && e == hipSuccess; ++r) e = coh_launch(h, tx.p, ty.p, nullptr);
-    if (e == hipSuccess) e = hipEventRecord(e1, h->stream);
-    if (e == hipSuccess) e = hipEventSynchronize(e1);
-    float t = 0.0f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    if (e != hipSuccess) return hip_fail(h, e, "BlockCOH autotune");
-    *ms = t / 5.0f;
-    return PWM_OK;
-}
-
-// The BlockCOH layout, then the kernel instance: the compiler's register
-// budget (FP64: 66 VGPRs, 7 waves per SIMD, 3 workgroups of 8 waves per CU)
-// or one capped for 8 waves per SIMD (4 workgroups when the LDS window
-// allows), the faster of the two on x = 1 unless the option coh_occ8 fixes it.
+// The BlockCOH layout.  One kernel, at 8 waves per SIMD; the option coh_occ8 is
+// kept and reported.
 int build_blockcoh(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals) {
-    int rc = build_blockcoh_layout(h, rs, ci, vals);
-    if (rc != PWM_OK) return rc;
-    if (h->coh_occ8 >= 0 || h->coh.n_tasks <= 0) {
-        h->coh.occ8 = h->coh_occ8 > 0 ? 1 : 0;
-        return PWM_OK;
-    }
-    float ms0 = 0.0f, ms1 = 0.0f;
-    h->coh.occ8 = 0;
-    if ((rc = time_coh(h, &ms0)) != PWM_OK) return rc;
-    h->coh.occ8 = 1;
-    if ((rc = time_coh(h, &ms1)) != PWM_OK) return rc;
-    h->coh.occ8 = ms1 < ms0 ? 1 : 0;
-    return PWM_OK;
+    const int rc = build_blockcoh_layout(h, rs, ci, vals);
+    if (rc == PWM_OK) h->coh.occ8 = h->coh_occ8 != 0;
+    return rc;
 }
 
 }  // namespace pwm_impl
@@ -1121,8 +1058,19 @@ extern "C" int pwm_blockcoh_band(pwm_matrix* h, int band, int64_t* counts, int32
     meta[2] = m.V;
     if (!row_jump || !col_jump || !data || !row_jump_block || !col_jump_block || !block_nnz) return PWM_OK;
     hipError_t e = hipSuccess;
-    if (m.row_jumps) e = hipMemcpy(row_jump, h->coh.row_jump.as<uint16_t>() + m.off_rj, m.row_jumps * 2, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && m.nnz) e = hipMemcpy(col_jump, h->coh.col_jump.as<uint16_t>() + m.off_nz, m.nnz * 2, hipMemcpyDeviceToHost);
+    std::vector<uint32_t> ent(m.nnz);
+    if (m.nnz) e = hipMemcpy(ent.data(), h->coh.ent.as<uint32_t>() + m.off_nz, m.nnz * 4, hipMemcpyDeviceToHost);
+    // ICRS jumps (TripletToCRS.hpp:402-452): the first entry of a block gives
+    // its row and column; within it a column jump is the distance to the next
+    // column, plus beta where the row changes (then a row jump too).
+    for (int64_t i = 0, rj = 0; i < m.nnz && e == hipSuccess; ++i) {
+        const int32_t row = ent[i] >> 15 & 0x7fff, col = ent[i] & 0x7fff;
+        const bool first = ent[i] & blocked::kCohFirst;
+        const int32_t prow = first ? 0 : ent[i - 1] >> 15 & 0x7fff, pcol = first ? 0 : ent[i - 1] & 0x7fff;
+        const bool next = !first && row != prow;
+        col_jump[i] = (uint16_t)(col - pcol + (next ? 1 << m.beta_bits : 0));
+        if ((first || next) && rj < m.row_jumps) row_jump[rj++] = (uint16_t)(row - prow);
+    }
     if (e == hipSuccess && m.block_row_jumps)
         e = hipMemcpy(row_jump_block, h->coh.row_jump_block.as<int16_t>() + m.off_rjb, m.block_row_jumps * 2, hipMemcpyDeviceToHost);
     if (e == hipSuccess && m.blocks) {

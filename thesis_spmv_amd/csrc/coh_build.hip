@@ -10,17 +10,15 @@
 //  2. a stable radix sort of (key, payload) puts each band's blocks in
 //     Hilbert order with the entries of a block in CRS order -- the stable
 //     counting sort of the host build;
-//  3. per sorted entry, a block-start flag and a row-start flag (new block,
-//     or another row than the entry before it in the same block); col_jump
-//     and the gathered value follow from the entry and its predecessor;
-//  4. one inclusive scan of the packed flags numbers the row jumps and the
-//     blocks, so every row start writes its row_jump and every block start
-//     its block record in place;
+//  3. per sorted entry, the packed position and the gathered value, and two
+//     flags, block start and row start (new block, or another row than the entry
+//     before it in the same block: the format's row jumps);
+//  4. one inclusive scan of the packed flags numbers the row starts and the
+//     blocks, so every block start writes its block in place;
 //  5. per block, the block-level BICRS jumps (BlockCOH.hpp:433-439), a flag
 //     for each block that starts a block row, and a second scan that places
 //     row_jump_block;
-//  6. per band, the chunk -> block table, and per atomic task the decode
-//     state (S, R) of the entry before its first one.
+//  6. per band, the step -> block table.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
@@ -101,62 +99,39 @@ __global__ void k_coh_keys(CohKeyArgs a, const CohBuildBand* __restrict__ bands,
 __device__ __forceinline__ uint32_t pay_row(uint64_t p) { return (uint32_t)(p >> 16) & 0xffffu; }
 __device__ __forceinline__ uint32_t pay_col(uint64_t p) { return (uint32_t)p & 0xffffu; }
 
-// step 3: flags (row start << 32 | block start), col_jump and the value
+// step 3: flags (row start << 32 | block start), the packed position and the value
 template <typename E>
-__global__ void k_coh_entries(CohKeyArgs a, const CohBuildBand* __restrict__ bands, const uint64_t* __restrict__ keys,
-                              const uint64_t* __restrict__ pay, const E* __restrict__ val,
-                              uint64_t* __restrict__ flags, uint16_t* __restrict__ col_jump, E* __restrict__ data) {
+__global__ void k_coh_entries(CohKeyArgs a, const uint64_t* __restrict__ keys, const uint64_t* __restrict__ pay,
+                              const E* __restrict__ val, uint64_t* __restrict__ flags, uint32_t* __restrict__ ent,
+                              E* __restrict__ data) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nnz; q += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t key = keys[q], p = pay[q];
         const bool bs = q == 0 || keys[q - 1] != key;
-        const uint64_t pp = bs ? 0 : pay[q - 1];
-        const bool rsf = bs || pay_row(pp) != pay_row(p);
-        const uint32_t lc = pay_col(p);
-        uint32_t cj = lc;
-        if (!bs) {
-            const uint32_t beta = 1u << bands[key >> a.hb2].beta_bits;
-            cj = rsf ? lc + beta - pay_col(pp) : lc - pay_col(pp);
-        }
-        col_jump[q] = (uint16_t)cj;
+        const bool rsf = bs || pay_row(pay[q - 1]) != pay_row(p);
+        ent[q] = (bs ? blocked::kCohFirst : 0u) | pay_row(p) << 15 | pay_col(p);
         data[q] = val[p >> 32];
         flags[q] = ((uint64_t)rsf << 32) | (uint64_t)bs;
     }
 }
 
-// step 4: row jumps and block records.  With s = inclusive scan of the flags,
-// the row segment of entry q is number (s[q] >> 32) - 1 overall and
-// (s[q] >> 32) - (s[q0] >> 32) inside its band (q0 = the band's first entry);
-// its block is number (s[q] & 0xffffffff) - 1.
+// step 4: blocks.  With s = inclusive scan of the flags, the block of entry q
+// is number (s[q] & 0xffffffff) - 1.
 __global__ void k_coh_scatter(CohKeyArgs a, const CohBuildBand* __restrict__ bands, const int32_t* __restrict__ rs,
                               const int32_t* __restrict__ ci, const uint64_t* __restrict__ keys,
                               const uint64_t* __restrict__ pay, const uint64_t* __restrict__ flags,
-                              const uint64_t* __restrict__ scan, uint16_t* __restrict__ row_jump,
-                              blocked::CohBlock* __restrict__ blocks, int32_t* __restrict__ block_q,
-                              int32_t* __restrict__ block_band) {
+                              const uint64_t* __restrict__ scan, blocked::CohBlock* __restrict__ blocks,
+                              int32_t* __restrict__ block_q, int32_t* __restrict__ block_band) {
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.nnz; q += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t f = flags[q];
-        if (!(f >> 32)) continue;  // block starts are row starts too
-        const uint64_t key = keys[q], p = pay[q];
-        const int64_t band = (int64_t)(key >> a.hb2);
+        if (!(flags[q] & 1)) continue;
+        const int64_t band = (int64_t)(keys[q] >> a.hb2);
         const CohBuildBand b = bands[band];
-        const uint64_t s = scan[q], s0 = scan[b.off_nz];
-        const int64_t rj = (int64_t)(s >> 32) - (int64_t)(s0 >> 32);
-        if (f & 1) {
-            row_jump[b.off_nz + rj] = (uint16_t)pay_row(p);
-            const int64_t e = (int64_t)(p >> 32);
-            const int64_t r = coh_row_of(rs, a.nor, e);
-            const int64_t blk = (int64_t)(s & 0xffffffffu) - 1;
-            blocked::CohBlock cb;
-            cb.entry = (int32_t)(q - b.off_nz);
-            cb.row_jump = (int32_t)rj;
-            cb.brow = (int32_t)((r - b.start) >> b.beta_bits);
-            cb.bcol = (int32_t)(ci[e] >> b.beta_bits);
-            blocks[blk] = cb;
-            block_q[blk] = (int32_t)q;
-            block_band[blk] = (int32_t)band;
-        } else {
-            row_jump[b.off_nz + rj] = (uint16_t)(pay_row(p) - pay_row(pay[q - 1]));
-        }
+        const int64_t e = (int64_t)(pay[q] >> 32);
+        const int64_t r = coh_row_of(rs, a.nor, e);
+        const int64_t blk = (int64_t)(scan[q] & 0xffffffffu) - 1;
+        blocks[blk] = blocked::CohBlock{(int32_t)((r - b.start) >> b.beta_bits << b.beta_bits),
+                                        (int32_t)(ci[e] >> b.beta_bits << b.beta_bits)};
+        block_q[blk] = (int32_t)q;
+        block_band[blk] = (int32_t)band;
     }
 }
 
@@ -169,20 +144,20 @@ __global__ void k_coh_blocks(int64_t total, int64_t nnz, const CohBuildBand* __r
     for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < total; b += (int64_t)gridDim.x * blockDim.x) {
         const CohBuildBand bd = bands[block_band[b]];
         const int64_t first = (int64_t)(scan[bd.off_nz] & 0xffffffffu) - 1;
-        const blocked::CohBlock cur = blocks[b];
+        const int64_t brow = blocks[b].row >> bd.beta_bits, bcol = blocks[b].col >> bd.beta_bits;
         int64_t cj, rj = 0;
         uint32_t fl = 1;
         if (b == first) {
-            rj = cur.brow;
-            cj = cur.bcol;
+            rj = brow;
+            cj = bcol;
         } else {
-            const blocked::CohBlock prev = blocks[b - 1];
-            if (cur.brow == prev.brow) {
+            const int64_t prow = blocks[b - 1].row >> bd.beta_bits, pcol = blocks[b - 1].col >> bd.beta_bits;
+            if (brow == prow) {
                 fl = 0;
-                cj = (int64_t)cur.bcol - prev.bcol;
+                cj = bcol - pcol;
             } else {
-                rj = (int64_t)cur.brow - prev.brow;
-                cj = (int64_t)cur.bcol - prev.bcol + bd.H;
+                rj = brow - prow;
+                cj = bcol - pcol + bd.H;
             }
         }
         col_jump_block[b] = (int16_t)cj;
@@ -218,52 +193,26 @@ __global__ void k_coh_band_counts(int64_t n_bands, const CohBuildBand* __restric
     }
 }
 
-// step 6: chunk c of band p starts in the band's last block whose first entry
-// is <= c * kCohChunk; entry `chunks` is the band's last block (0 if none)
-__global__ void k_coh_chunks(int64_t n_bands, const blocked::CohBand* __restrict__ table,
-                             const blocked::CohBlock* __restrict__ blocks, int32_t* __restrict__ ctab) {
+// step 6: the last block of band p that starts before step i of the band (-1:
+// none)
+__global__ void k_coh_steps(int64_t n_bands, const blocked::CohBand* __restrict__ table,
+                            const int32_t* __restrict__ block_q, int32_t* __restrict__ stab) {
     for (int64_t p = blockIdx.x; p < n_bands; p += gridDim.x) {
         const blocked::CohBand bd = table[p];
-        const int64_t nch = ((int64_t)bd.nnz + blocked::kCohChunk - 1) / blocked::kCohChunk;
-        const blocked::CohBlock* __restrict__ bl = blocks + bd.first_block;
-        for (int64_t c = threadIdx.x; c <= nch; c += blockDim.x) {
-            int32_t v;
-            if (c == nch) {
-                v = bd.blocks > 0 ? bd.blocks - 1 : 0;
-            } else {
-                const int64_t e = c * blocked::kCohChunk;
-                int64_t lo = 0, hi = bd.blocks - 1;
-                while (lo < hi) {
-                    const int64_t mid = (lo + hi + 1) >> 1;
-                    if (bl[mid].entry <= e)
-                        lo = mid;
-                    else
-                        hi = mid - 1;
-                }
-                v = (int32_t)lo;
+        const int64_t steps = blocked::coh_steps(bd.entry, bd.nnz);
+        const int32_t* __restrict__ bq = block_q + bd.first_block;
+        for (int64_t i = threadIdx.x; i < steps; i += blockDim.x) {
+            const int64_t q = (bd.entry & ~3) + i * blocked::kCohStep;
+            int64_t lo = 0, hi = bd.blocks;  // blocks starting before q: in [lo, hi]
+            while (lo < hi) {
+                const int64_t mid = (lo + hi) >> 1;
+                if (bq[mid] < q)
+                    lo = mid + 1;
+                else
+                    hi = mid;
             }
-            ctab[bd.chunk_table + c] = v;
+            stab[bd.step_table + i] = (int32_t)lo - 1;
         }
-    }
-}
-
-// decode state after the entries before an atomic task's first one: the row
-// inside the block (R) and S = column + beta * (row changes since the block
-// started)
-__global__ void k_coh_carries(int64_t n_tasks, const blocked::CohBand* __restrict__ table,
-                              const uint64_t* __restrict__ pay, const uint64_t* __restrict__ scan,
-                              const int32_t* __restrict__ block_q, blocked::CohTask* __restrict__ tasks) {
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n_tasks; t += (int64_t)gridDim.x * blockDim.x) {
-        blocked::CohTask tk = tasks[t];
-        if (!tk.atomic || tk.chunk0 == 0) continue;
-        const blocked::CohBand bd = table[tk.band];
-        const int64_t q = (int64_t)bd.entry + (int64_t)tk.chunk0 * blocked::kCohChunk - 1;
-        const uint64_t s = scan[q];
-        const int64_t qb = block_q[(int64_t)(s & 0xffffffffu) - 1];
-        const int64_t changes = (int64_t)(s >> 32) - (int64_t)(scan[qb] >> 32);
-        tk.carry_s = (int32_t)(pay_col(pay[q]) + (changes << bd.beta_bits));
-        tk.carry_r = (int32_t)pay_row(pay[q]);
-        tasks[t] = tk;
     }
 }
 
@@ -301,11 +250,9 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
     pwmk::CohKeyArgs ka{nor, nnz, P, 2 * hbits};
 
     const int64_t zpad = std::max<int64_t>(nnz, 1) + 64;
-    if ((e = c.col_jump.alloc(zpad * 2)) != hipSuccess || (e = c.row_jump.alloc(zpad * 2)) != hipSuccess ||
-        (e = c.data.alloc(zpad * vs)) != hipSuccess)
+    if ((e = c.ent.alloc(zpad * 4)) != hipSuccess || (e = c.data.alloc(zpad * vs)) != hipSuccess)
         return hip_fail(h, e, "BlockCOH allocation");
-    if ((e = hipMemsetAsync(c.col_jump.p, 0, zpad * 2, h->stream)) != hipSuccess ||
-        (e = hipMemsetAsync(c.row_jump.p, 0, zpad * 2, h->stream)) != hipSuccess ||
+    if ((e = hipMemsetAsync(c.ent.p, 0, zpad * 4, h->stream)) != hipSuccess ||
         (e = hipMemsetAsync(c.data.p, 0, zpad * vs, h->stream)) != hipSuccess)
         return hip_fail(h, e, "BlockCOH allocation");
 
@@ -337,17 +284,17 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
         uint64_t* flags = keys.as<uint64_t>();
         uint64_t* scan = pay.as<uint64_t>();
         if (vs == 8)
-            hipLaunchKernelGGL(pwmk::k_coh_entries<uint64_t>, g, t, 0, h->stream, ka,
-                               d_bands.as<pwmk::CohBuildBand>(), keys_out.as<uint64_t>(), pay_out.as<uint64_t>(),
-                               h->val.as<uint64_t>(), flags, c.col_jump.as<uint16_t>(), c.data.as<uint64_t>());
+            hipLaunchKernelGGL(pwmk::k_coh_entries<uint64_t>, g, t, 0, h->stream, ka, keys_out.as<uint64_t>(),
+                               pay_out.as<uint64_t>(), h->val.as<uint64_t>(), flags, c.ent.as<uint32_t>(),
+                               c.data.as<uint64_t>());
         else if (vs == 4)
-            hipLaunchKernelGGL(pwmk::k_coh_entries<uint32_t>, g, t, 0, h->stream, ka,
-                               d_bands.as<pwmk::CohBuildBand>(), keys_out.as<uint64_t>(), pay_out.as<uint64_t>(),
-                               h->val.as<uint32_t>(), flags, c.col_jump.as<uint16_t>(), c.data.as<uint32_t>());
+            hipLaunchKernelGGL(pwmk::k_coh_entries<uint32_t>, g, t, 0, h->stream, ka, keys_out.as<uint64_t>(),
+                               pay_out.as<uint64_t>(), h->val.as<uint32_t>(), flags, c.ent.as<uint32_t>(),
+                               c.data.as<uint32_t>());
         else
-            hipLaunchKernelGGL(pwmk::k_coh_entries<uint16_t>, g, t, 0, h->stream, ka,
-                               d_bands.as<pwmk::CohBuildBand>(), keys_out.as<uint64_t>(), pay_out.as<uint64_t>(),
-                               h->val.as<uint16_t>(), flags, c.col_jump.as<uint16_t>(), c.data.as<uint16_t>());
+            hipLaunchKernelGGL(pwmk::k_coh_entries<uint16_t>, g, t, 0, h->stream, ka, keys_out.as<uint64_t>(),
+                               pay_out.as<uint64_t>(), h->val.as<uint16_t>(), flags, c.ent.as<uint32_t>(),
+                               c.data.as<uint16_t>());
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail(h, e, "BlockCOH entries");
         tb = 0;
         e = rocprim::inclusive_scan(nullptr, tb, flags, scan, (size_t)nnz, rocprim::plus<uint64_t>(), h->stream);
@@ -372,7 +319,7 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
             return hip_fail(h, e, "BlockCOH block allocation");
         hipLaunchKernelGGL(pwmk::k_coh_scatter, g, t, 0, h->stream, ka, d_bands.as<pwmk::CohBuildBand>(),
                            h->rs.as<int32_t>(), h->ci.as<int32_t>(), keys_out.as<uint64_t>(), pay_out.as<uint64_t>(),
-                           flags, scan, c.row_jump.as<uint16_t>(), c.block_coords.as<blocked::CohBlock>(),
+                           flags, scan, c.block_coords.as<blocked::CohBlock>(),
                            block_q.as<int32_t>(), block_band.as<int32_t>());
         const dim3 gb(pwmk::grid_of(total));
         hipLaunchKernelGGL(pwmk::k_coh_blocks, gb, t, 0, h->stream, total, nnz, d_bands.as<pwmk::CohBuildBand>(),
@@ -403,15 +350,14 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         if (e != hipSuccess) return hip_fail(h, e, "BlockCOH band counts");
     }
-    // band metadata, the kernel's band table and the chunk-table offsets
+    // band metadata, the kernel's band table and the step-table offsets
     std::vector<blocked::CohBand> table(P);
-    int64_t off_blk = 0, off_rjb = 0, off_ctab = 0;
+    int64_t off_blk = 0, off_rjb = 0, off_stab = 0;
     for (int64_t p = 0; p < P; ++p) {
         CohBandMeta& m = B[p];
         m.blocks = counts[3 * p];
         m.row_jumps = counts[3 * p + 1];
         m.block_row_jumps = counts[3 * p + 2];
-        m.off_rj = m.off_nz;
         m.off_blk = off_blk;
         m.off_rjb = off_rjb;
         off_blk += m.blocks;
@@ -419,40 +365,36 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
         blocked::CohBand& t = table[p];
         t.start = (int32_t)m.start;
         t.rows = (int32_t)m.rows;
-        t.beta_bits = m.beta_bits;
         t.first_block = (int32_t)m.off_blk;
         t.blocks = (int32_t)m.blocks;
         t.entry = (int32_t)m.off_nz;
         t.nnz = (int32_t)m.nnz;
-        t.chunk_table = (int32_t)off_ctab;
-        off_ctab += (m.nnz + blocked::kCohChunk - 1) / blocked::kCohChunk + 1;
+        t.step_table = (int32_t)off_stab;
+        off_stab += blocked::coh_steps(m.off_nz, m.nnz);
     }
     if (off_blk != total) return fail(h, PWM_ERR_HIP, "BlockCOH build: band block counts disagree");
     std::vector<blocked::CohTask> tasks;
-    std::vector<int32_t> atomic_bands;
-    coh_plan_tasks(B, lds_rows, tasks, atomic_bands, &c.lds_rows);
-    c.n_atomic = (int64_t)atomic_bands.size();
+    std::vector<blocked::CohRows> pieces;
+    coh_plan_tasks(B, lds_rows, tasks, pieces, table, &c.lds_rows);
     c.n_tasks = (int64_t)tasks.size();
     if ((e = c.band_table.alloc(P * sizeof(blocked::CohBand))) != hipSuccess ||
         (e = hipMemcpy(c.band_table.p, table.data(), P * sizeof(blocked::CohBand), hipMemcpyHostToDevice)) !=
             hipSuccess ||
-        (e = c.tasks.alloc(off_ctab * 4)) != hipSuccess ||
+        (e = c.tasks.alloc(off_stab * 4)) != hipSuccess ||
         (e = c.task_list.alloc(tasks.size() * sizeof(blocked::CohTask))) != hipSuccess ||
         (!tasks.empty() && (e = hipMemcpy(c.task_list.p, tasks.data(), tasks.size() * sizeof(blocked::CohTask),
                                           hipMemcpyHostToDevice)) != hipSuccess) ||
-        (e = c.atomic_bands.alloc(atomic_bands.size() * 4)) != hipSuccess ||
-        (!atomic_bands.empty() && (e = hipMemcpy(c.atomic_bands.p, atomic_bands.data(), atomic_bands.size() * 4,
-                                                 hipMemcpyHostToDevice)) != hipSuccess))
+        (e = c.row_pieces.alloc(pieces.size() * sizeof(blocked::CohRows))) != hipSuccess ||
+        (!pieces.empty() && (e = hipMemcpy(c.row_pieces.p, pieces.data(), pieces.size() * sizeof(blocked::CohRows),
+                                           hipMemcpyHostToDevice)) != hipSuccess) ||
+        (e = coh_clear_sums(h, pieces)) != hipSuccess)
         return hip_fail(h, e, "BlockCOH tables");
-    hipLaunchKernelGGL(pwmk::k_coh_chunks, dim3((unsigned)std::min<int64_t>(std::max<int64_t>(P, 1), 8192)),
-                       dim3(256), 0, h->stream, P, c.band_table.as<blocked::CohBand>(),
-                       c.block_coords.as<blocked::CohBlock>(), c.tasks.as<int32_t>());
-    if (nnz > 0 && !tasks.empty())
-        hipLaunchKernelGGL(pwmk::k_coh_carries, dim3(pwmk::grid_of((int64_t)tasks.size())), dim3(256), 0, h->stream,
-                           (int64_t)tasks.size(), c.band_table.as<blocked::CohBand>(), pay_out.as<uint64_t>(),
-                           pay.as<uint64_t>(), block_q.as<int32_t>(), c.task_list.as<blocked::CohTask>());
+    if (nnz > 0)
+        hipLaunchKernelGGL(pwmk::k_coh_steps, dim3((unsigned)std::min<int64_t>(std::max<int64_t>(P, 1), 8192)), dim3(256),
+                           0, h->stream, P, c.band_table.as<blocked::CohBand>(), block_q.as<int32_t>(),
+                           c.tasks.as<int32_t>());
     if ((e = hipGetLastError()) == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return hip_fail(h, e, "BlockCOH chunk tables");
+    if (e != hipSuccess) return hip_fail(h, e, "BlockCOH step tables");
     h->rs.release();
     h->ci.release();
     h->val.release();

@@ -65,48 +65,6 @@ __device__ __forceinline__ int block_excl_scan(int v, int* tmp, int* total) {
     return before + incl - v;
 }
 
-// Block-wide segmented scan.  Each thread brings the sum `v` of its entries
-// after its last segment start and `f` = 1 if it holds a segment start.  The
-// result is the value that flows into the thread's first entry: the sum over
-// earlier threads back to the most recent segment start, plus `carry` if no
-// segment starts before this thread.  `tv`/`tf` hold kWaves values each.
-__device__ __forceinline__ int block_seg_excl(int v, int f, int carry, int* tv, int* tf) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int iv = v, ifl = f;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int uv = __shfl_up(iv, d);
-        const int uf = __shfl_up(ifl, d);
-        if (lane >= d) {
-            if (!ifl) iv += uv;
-            ifl |= uf;
-        }
-    }
-    if (lane == 63) {
-        tv[wave] = iv;
-        tf[wave] = ifl;
-    }
-    __syncthreads();
-    // prefix of the earlier waves, seeded with the chunk carry
-    int pv = carry;
-    for (int w = 0; w < wave; ++w) {
-        if (tf[w]) {
-            pv = tv[w];
-        } else {
-            pv += tv[w];
-        }
-    }
-    __syncthreads();
-    // exclusive value of this lane: inclusive of the previous lane in the wave
-    int ev = __shfl_up(iv, 1);
-    int ef = __shfl_up(ifl, 1);
-    if (lane == 0) {
-        ev = 0;
-        ef = 0;
-    }
-    return ef ? ev : ev + pv;
-}
-
 // ---------------------------------------------------------------- CSB
 
 // workgroup -> (slab task t, column group g).  With a multiple of 8 groups the
@@ -617,32 +575,37 @@ int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32) {
 
 // ---------------------------------------------------------------- BlockCOH
 
-// One workgroup per task (CohTask): chunks of kCohChunk consecutive entries
-// of one band, decoded (ICRS, TripletToCRS.hpp:402-452 / BlockCOH.hpp:235-256)
-// with two segmented scans that restart at every block:
-//   S = running sum of col_jump: column = S mod beta, row changes = S div beta
-//   (a row change adds exactly beta, so S = col + beta * changes);
-//   R = running sum of the row_jump entered at each row change: the row.
-// LDS tasks own their band (rows <= LDS window) and write it once; atomic
-// tasks add into y (zeroed by k_coh_zero) with global atomics.
-// OCC8: registers capped so that 8 waves per SIMD fit (4 workgroups per CU
-// when the LDS window allows it) instead of the compiler's 7.
-template <typename VT, bool POWER, bool OCC8>
-__global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
-                                             typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
+// One workgroup per task (CohTask); its waves take the task's steps of
+// kCohStep entries in turn, each on its own: no barrier between the first zero
+// and the last sum.  A lane holds 4 consecutive entries and adds them up while
+// the row stays the same (equal rows in many lanes would take turns: an LDS add
+// of 64 lanes takes 16 clocks on random rows, 56 on runs of 5, 192 on one row);
+// a step within one long row is added up by the wave.  The sums go to the
+// band's y-slice in LDS (LDS tasks, which write it once) or to the band's rows
+// of ysum with global atomics, FP64 both.  The block of an entry is the number
+// of block starts before it: four ballots and a table of the blocks at the
+// steps.
+//
+// Bound by the gathers (FP64 9-point stencil with 2 random entries per row, 1 M
+// rows: 215 G/s of the 213-233 G/s that the L2 serves) or, on a matrix of few
+// blocks, by HBM.  Mean of back-to-back SpMVs on rotating copies, us, against
+// workgroups that decode the stored jumps with two segmented scans per 2048
+// entries: that stencil 88 -> 51, on 90 K rows 18.6 -> 8.2; Poisson 1024^2
+// 39.8 -> 18, 3000^2 283 -> 145; power-law rows, 100 K 67 -> 18, 500 K 315 ->
+// 64, 2 M 687 -> 278.  Tried: 2 or 4 steps at once (the same or slower),
+// non-temporal entry loads (18 -> 22 on the Poisson matrix, 281 -> 275 on the
+// largest), the step table read after the entries (278 -> 302).
+template <typename VT, bool POWER>
+__global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
+                                                typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     // the LDS window holds the rows of the largest band accumulated in LDS
     // (at most coh_lds_rows), sized at launch
     extern __shared__ __align__(16) unsigned char coh_smem[];
     double* ylds = (double*)coh_smem;
-    __shared__ int32_t bstart[kCohChunk + 2];  // up to kCohChunk+1 blocks and a sentinel
-    // the records of the chunk's blocks when there are at most kCohStage of
-    // them (the usual case), so the decode reads them from LDS
-    constexpr int kCohStage = 256;
+    constexpr int kCohStage = 256;  // blocks of a band kept in LDS, where a band has no more
     __shared__ CohBlock bstage[kCohStage];
-    __shared__ int tv[kWaves], tf[kWaves];
-    __shared__ int carry_s, carry_r;
     __shared__ double red[16];
 
     const X* __restrict__ x = x_arg;
@@ -655,135 +618,97 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
         scale = pwmk::step_scale(pw, k);
     }
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const CohTask task = a.tasks[blockIdx.x];
     const CohBand band = a.bands[task.band];
-    const VT* __restrict__ val = (const VT*)a.val + band.entry;
-    const uint16_t* __restrict__ cjmp = a.col_jump + band.entry;
-    const uint16_t* __restrict__ rjmp = a.row_jump + band.entry;
     const CohBlock* __restrict__ blocks = a.blocks + band.first_block;
-    const int32_t* __restrict__ ctab = a.chunk_block + band.chunk_table;
-    const int bits = band.beta_bits;
-    const int64_t beta = (int64_t)1 << bits;
-    const int nnz = band.nnz;
+    typedef const int32_t __attribute__((address_space(4))) * ScalarTable;
+    const ScalarTable stab = (ScalarTable)(a.step_block + band.step_table);
     const bool lds = task.atomic == 0;
+    double* __restrict__ ysum = a.ysum + band.sum;
 
+    const bool staged = band.blocks <= kCohStage;
     if (lds)
         for (int i = tid; i < band.rows; i += kBS) ylds[i] = 0;
-    if (tid == 0) {
-        carry_s = task.carry_s;
-        carry_r = task.carry_r;
+    if (staged)
+        for (int i = tid; i < band.blocks; i += kBS) bstage[i] = blocks[i];
+    __syncthreads();
+    const int64_t first = band.entry, end = first + band.nnz, base = first & ~(int64_t)3;
+    for (int s = task.step0 + wave; s < task.step0 + task.nsteps; s += kWaves) {
+        int b = stab[s];  // a scalar load, ahead of the entries
+        const int64_t q = base + (int64_t)s * kCohStep + 4 * lane;
+        // lanes beyond the band load its last quad (the arrays are padded)
+        const int64_t qc = q < end ? q : (end - 1) & ~(int64_t)3;
+        const pwmk::vi4 quad = *pwmk::G((const pwmk::vi4*)(a.ent + qc));
+        const uint32_t en[4] = {(uint32_t)quad[0], (uint32_t)quad[1], (uint32_t)quad[2], (uint32_t)quad[3]};
+        pwmk::Quad<VT> v;
+        v.load((const VT*)a.val + qc);
+        bool ok[4];
+        uint64_t m[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            ok[j] = q + j >= first && q + j < end;
+            m[j] = __ballot(ok[j] && (en[j] & kCohFirst));
+        }
+        CohBlock blk[4];
+        if ((m[0] | m[1] | m[2] | m[3]) == 0) {  // the wave's entries lie in one block
+            const CohBlock one = staged ? bstage[b] : blocks[b];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) blk[j] = one;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                b = __builtin_amdgcn_mbcnt_hi((uint32_t)(m[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[j], b));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                b += (int)((m[j] >> lane) & 1);
+                const int bi = b > 0 ? b : 0;  // -1 before the band's first entry
+                blk[j] = staged ? bstage[bi] : blocks[bi];
+            }
+        }
+        int row[4];
+        Acc xv[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            row[j] = ok[j] ? blk[j].row + (int)(en[j] >> 15 & 0x7fff) : -1;
+            xv[j] = (Acc)x[(int64_t)blk[j].col + (ok[j] ? en[j] & 0x7fff : 0)];
+        }
+        // (the products come after this test, which runs while the gathers are under way)
+        double sum = 0.0;
+        const int row0 = __builtin_amdgcn_readfirstlane(row[0]);
+        if (row0 >= 0 && __ballot(row[1] != row0 || row[2] != row0 || row[3] != row0 || row[0] != row0) == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum += (double)((Acc)v.get(j) * xv[j]);
+            sum = pwmk::group_sum<64>(sum);
+            if (lane == 0) {
+                if (lds)
+                    atomicAdd(&ylds[row0], sum);
+                else
+                    atomicAdd(&ysum[row0], sum);
+            }
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const Acc p = (Acc)v.get(j) * xv[j];
+            sum += (double)p;
+            if (j < 3 && row[j + 1] == row[j]) continue;
+            if (row[j] >= 0) {
+                if (lds)
+                    atomicAdd(&ylds[row[j]], sum);
+                else
+                    atomicAdd(&ysum[row[j]], sum);
+            }
+            sum = 0.0;
+        }
     }
-    for (int c = task.chunk0; c < task.chunk0 + task.nchunks; ++c) {
-        const int base = c * kCohChunk;
-        const int b_lo = ctab[c], b_hi = ctab[c + 1];  // blocks touching this chunk
-        const int nbl = b_hi - b_lo + 1;
-        __syncthreads();
-        const bool staged = nbl <= kCohStage;
-        for (int i = tid; i < nbl; i += kBS) {
-            const CohBlock cb = blocks[b_lo + i];
-            bstart[i] = cb.entry;
-            if (staged) bstage[i] = cb;
-        }
-        if (tid == 0) bstart[nbl] = 0x7fffffff;
-        __syncthreads();
-        const int e0 = base + tid * kCohIPT;
-        // block of my first entry: last block start <= e0
-        int lo = 0, hi = nbl;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (bstart[mid] <= e0) lo = mid;
-            else hi = mid;
-        }
-        int bj[kCohIPT], cj[kCohIPT], rst[kCohIPT];
-        Acc vv[kCohIPT];
-        int b = lo;
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) {
-            const int e = e0 + j;
-            if (e < nnz) {
-                while (bstart[b + 1] <= e) ++b;
-                bj[j] = b;
-                rst[j] = bstart[b] == e;
-                cj[j] = cjmp[e];
-                vv[j] = (Acc)widen(val[e]);
-            } else {
-                bj[j] = b;
-                rst[j] = 0;
-                cj[j] = 0;
-                vv[j] = 0;
-            }
-        }
-        // scan 1: S
-        int run = 0, anyr = 0;
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) {
-            run = rst[j] ? cj[j] : run + cj[j];
-            anyr |= rst[j];
-        }
-        const int sin = block_seg_excl(run, anyr, carry_s, tv, tf);
-        int S[kCohIPT];
-        run = sin;
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) {
-            run = rst[j] ? cj[j] : run + cj[j];
-            S[j] = run;
-        }
-        // row deltas at every row change
-        CohBlock blk[kCohIPT];
-        int dl[kCohIPT];
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) {
-            const int e = e0 + j;
-            dl[j] = 0;
-            if (e < nnz) {
-                blk[j] = staged ? bstage[bj[j]] : blocks[b_lo + bj[j]];
-                const int kk = S[j] >> bits;
-                const bool newrow = rst[j] || (kk != ((S[j] - cj[j]) >> bits));
-                // a band holds at most nnz row segments: the clamp keeps a
-                // decode error an error in y, never a read outside the band
-                int ri = blk[j].row_jump + kk;
-                ri = ri < nnz ? ri : nnz - 1;
-                if (newrow) dl[j] = rjmp[ri];
-            } else {
-                blk[j] = CohBlock{0, 0, 0, 0};
-            }
-        }
-        // scan 2: R
-        run = 0;
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) run = rst[j] ? dl[j] : run + dl[j];
-        const int rin = block_seg_excl(run, anyr, carry_r, tv, tf);
-        run = rin;
-#pragma unroll
-        for (int j = 0; j < kCohIPT; ++j) {
-            run = rst[j] ? dl[j] : run + dl[j];
-            const int e = e0 + j;
-            if (e < nnz) {
-                const int col = S[j] & (int)(beta - 1);
-                const int row = (int)(blk[j].brow * beta) + run;  // row inside the band
-                if (row >= 0 && row < band.rows) {
-                    int64_t xi = (int64_t)blk[j].bcol * beta + col;
-                    xi = xi < a.noc ? xi : a.noc - 1;
-                    const Acc p = vv[j] * (Acc)x[xi];
-                    if (lds) {
-                        atomicAdd(&ylds[row], (double)p);
-                    } else {
-                        // atomic tasks add the scaled product: y rows of big
-                        // bands are final once every task has finished
-                        atomicAdd(&y[(int64_t)band.start + row], POWER ? (X)((double)p * scale) : (X)p);
-                    }
-                }
-            }
-            // the entry that closes the chunk leaves its S and R for the next chunk
-            if (e == base + kCohChunk - 1 || e == nnz - 1) {
-                carry_s = S[j];
-                carry_r = run;
-            }
-        }
+    if (!lds) {
+        if constexpr (POWER)  // k_coh_finish sums these rows
+            if (tid < 3) pw.partials[3 * blockIdx.x + tid] = 0.0;
+        return;
     }
     __syncthreads();
-    if (!lds) return;
     double yy = 0.0, xy = 0.0, xx = 0.0;
     for (int i = tid; i < band.rows; i += kBS) {
         const int64_t row = (int64_t)band.start + i;
@@ -810,57 +735,50 @@ __global__ __launch_bounds__(kBS, OCC8 ? 8 : 1) void k_coh(CohArgs a, const type
     }
 }
 
-// Zero the rows of the bands that atomic tasks accumulate into (one workgroup
-// per such band), and in power mode clear the atomic tasks' partial slots.
+// The rows of atomic bands (one workgroup per piece): their sums to y, and back
+// to zero for the next SpMV.  Power mode: also |y|^2, x^T y, x^T x, into the
+// partial slots after the tasks' (slot n_tasks + i for piece i).
 template <typename VT, bool POWER>
-__global__ __launch_bounds__(kBS) void k_coh_zero(CohArgs a, const int32_t* __restrict__ atomic_bands,
-                                                  typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
+__global__ __launch_bounds__(kBS) void k_coh_finish(CohArgs a, typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
+    __shared__ double red[16];
+    const X* x = nullptr;
     X* y = y_arg;
+    double scale = 1.0;
     if constexpr (POWER) {
         if (pwmk::power_done(pw)) return;
         const int64_t k = pw.k;
+        x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
+        scale = pwmk::step_scale(pw, k);
     }
-    const CohBand band = a.bands[atomic_bands[blockIdx.x]];
-    for (int i = threadIdx.x; i < band.rows; i += kBS) y[(int64_t)band.start + i] = (X)0;
-    if constexpr (POWER)
-        for (int64_t t = (int64_t)blockIdx.x * kBS + threadIdx.x; t < a.n_tasks; t += (int64_t)gridDim.x * kBS)
-            if (a.tasks[t].atomic) {
-                pw.partials[3 * t + 0] = 0.0;
-                pw.partials[3 * t + 1] = 0.0;
-                pw.partials[3 * t + 2] = 0.0;
-            }
-}
-
-// Power mode: |y|^2, x^T y, x^T x over the rows of atomic bands, into the
-// partial slots after the tasks' (slot n_tasks + i for atomic band i).
-template <typename VT>
-__global__ __launch_bounds__(kBS) void k_coh_stats(CohArgs a, const int32_t* __restrict__ atomic_bands, PowerArgs pw) {
-    using X = typename Arith<VT>::X;
-    __shared__ double red[16];
-    if (pwmk::power_done(pw)) return;
-    const int64_t k = pw.k;
-    const X* x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
-    const X* y = (const X*)((k & 1) ? pw.buf0 : pw.buf1);
-    const double scale = pwmk::step_scale(pw, k);
-    const CohBand band = a.bands[atomic_bands[blockIdx.x]];
+    const CohRows piece = a.pieces[blockIdx.x];
     double yy = 0.0, xy = 0.0, xx = 0.0;
-    for (int i = threadIdx.x; i < band.rows; i += kBS) {
-        const int64_t row = (int64_t)band.start + i;
-        const double yd = (double)y[row], xd = (double)x[row] * scale;
-        yy += yd * yd;
-        xy += xd * yd;
-        xx += xd * xd;
+    for (int i = threadIdx.x; i < piece.rows; i += kBS) {
+        const int64_t row = (int64_t)piece.start + i;
+        const double sum = a.ysum[(int64_t)piece.sum + i];
+        a.ysum[(int64_t)piece.sum + i] = 0.0;
+        if constexpr (POWER) {
+            const X out = (X)(sum * scale);
+            y[row] = out;
+            const double yd = (double)out, xd = (double)x[row] * scale;
+            yy += yd * yd;
+            xy += xd * yd;
+            xx += xd * xd;
+        } else {
+            y[row] = (X)sum;
+        }
     }
-    const double ra = pwmk::block_sum<kBS>(yy, red);
-    const double rb = pwmk::block_sum<kBS>(xy, red);
-    const double rc = pwmk::block_sum<kBS>(xx, red);
-    if (threadIdx.x == 0) {
-        const int64_t slot = a.n_tasks + blockIdx.x;
-        pw.partials[3 * slot + 0] = ra;
-        pw.partials[3 * slot + 1] = rb;
-        pw.partials[3 * slot + 2] = rc;
+    if constexpr (POWER) {
+        const double ra = pwmk::block_sum<kBS>(yy, red);
+        const double rb = pwmk::block_sum<kBS>(xy, red);
+        const double rc = pwmk::block_sum<kBS>(xx, red);
+        if (threadIdx.x == 0) {
+            const int64_t slot = a.n_tasks + blockIdx.x;
+            pw.partials[3 * slot + 0] = ra;
+            pw.partials[3 * slot + 1] = rb;
+            pw.partials[3 * slot + 2] = rc;
+        }
     }
 }
 
@@ -943,36 +861,22 @@ hipError_t launch_csb(const CsbArgs& a, const void* x, void* y, const PowerArgs*
     return hipErrorInvalidValue;
 }
 
-template <typename VT>
-static hipError_t coh_t(const CohArgs& a, const int32_t* atomic_bands, int n_atomic, const void* x, void* y,
-                        const PowerArgs* pw, hipStream_t s) {
+template <typename VT, bool POWER>
+static hipError_t coh_t(const CohArgs& a, const void* x, void* y, const PowerArgs& pw, hipStream_t s) {
     using X = typename Arith<VT>::X;
     if (a.n_tasks <= 0) return hipSuccess;
     const size_t lds = (size_t)std::max<int32_t>(a.lds_rows, 1) * sizeof(double);
-    if (pw) {
-        if (n_atomic > 0)
-            hipLaunchKernelGGL((k_coh_zero<VT, true>), dim3(n_atomic), dim3(kBS), 0, s, a, atomic_bands, (X*)nullptr,
-                               *pw);
-        auto kp = a.occ8 ? k_coh<VT, true, true> : k_coh<VT, true, false>;
-        hipLaunchKernelGGL(kp, dim3((unsigned)a.n_tasks), dim3(kBS), lds, s, a, (const X*)nullptr, (X*)nullptr, *pw);
-        if (n_atomic > 0)
-            hipLaunchKernelGGL((k_coh_stats<VT>), dim3(n_atomic), dim3(kBS), 0, s, a, atomic_bands, *pw);
-    } else {
-        if (n_atomic > 0)
-            hipLaunchKernelGGL((k_coh_zero<VT, false>), dim3(n_atomic), dim3(kBS), 0, s, a, atomic_bands, (X*)y,
-                               PowerArgs{});
-        auto kf = a.occ8 ? k_coh<VT, false, true> : k_coh<VT, false, false>;
-        hipLaunchKernelGGL(kf, dim3((unsigned)a.n_tasks), dim3(kBS), lds, s, a, (const X*)x, (X*)y, PowerArgs{});
-    }
+    hipLaunchKernelGGL((k_coh<VT, POWER>), dim3((unsigned)a.n_tasks), dim3(kBS), lds, s, a, (const X*)x, (X*)y, pw);
+    if (a.n_pieces > 0)
+        hipLaunchKernelGGL((k_coh_finish<VT, POWER>), dim3((unsigned)a.n_pieces), dim3(kBS), 0, s, a, (X*)y, pw);
     return hipGetLastError();
 }
 
-hipError_t launch_coh(const CohArgs& a, const int32_t* atomic_bands, int n_atomic, const void* x, void* y,
-                      const PowerArgs* pw, hipStream_t s) {
+hipError_t launch_coh(const CohArgs& a, const void* x, void* y, const PowerArgs* pw, hipStream_t s) {
     switch (a.vtype) {
-        case 0: return coh_t<double>(a, atomic_bands, n_atomic, x, y, pw, s);
-        case 1: return coh_t<float>(a, atomic_bands, n_atomic, x, y, pw, s);
-        case 2: return coh_t<bf16_t>(a, atomic_bands, n_atomic, x, y, pw, s);
+        case 0: return pw ? coh_t<double, true>(a, x, y, *pw, s) : coh_t<double, false>(a, x, y, PowerArgs{}, s);
+        case 1: return pw ? coh_t<float, true>(a, x, y, *pw, s) : coh_t<float, false>(a, x, y, PowerArgs{}, s);
+        case 2: return pw ? coh_t<bf16_t, true>(a, x, y, *pw, s) : coh_t<bf16_t, false>(a, x, y, PowerArgs{}, s);
     }
     return hipErrorInvalidValue;
 }
