@@ -646,13 +646,11 @@ static hipError_t time_crs_kernel(pwm_matrix* h, int which, const void* x, void*
 
 constexpr int64_t kXcdL2 = (int64_t)4 << 20;  // an XCD's L2
 
-// Whether the columns are scattered: x beyond one XCD's L2, and 256
-// consecutive entries touch more than 128 lines of x on average (banded
-// matrices and stencils some 20 to 60, uniformly random columns all 256).  A
-// sweep in row order then fetches about one 128-byte line per entry from
-// beyond the L2.
-static hipError_t columns_scattered(pwm_matrix* h, bool* scattered) {
-    *scattered = false;
+// Distinct 128-byte lines of x that 256 consecutive entries touch, on average;
+// 0 where x fits one XCD's L2.  Stencils and banded matrices have some 10 to
+// 20, with 2 random entries per row about 55, uniformly random columns all 256.
+static hipError_t column_lines(pwm_matrix* h, double* per_group) {
+    *per_group = 0.0;
     const int64_t xb = (int64_t)vector_size(h->vtype);
     if (h->noc * xb <= kXcdL2 || h->nnz < 256) return hipSuccess;
     const int64_t groups = std::min<int64_t>(h->nnz / 256, 2048);
@@ -664,9 +662,17 @@ static hipError_t columns_scattered(pwm_matrix* h, bool* scattered) {
         e = pwmk::launch_scatter(h->ci.as<int32_t>(), h->nnz, groups, xb == 8 ? 4 : 5, lines.as<unsigned>(), h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(&n, lines.p, 4, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    *scattered = n > 128 * (uint64_t)groups;
+    *per_group = (double)n / (double)groups;
     return e;
 }
+
+// Entry loads of the wave tiles: non-temporal, so that the entries leave the L2
+// to x, where x is beyond one L2 and some of its lines are far apart.  9-point
+// stencil with 2 random entries per row, us, plain and non-temporal: FP64 1001^2
+// 45.9 44.1, 1448^2 103 99.5, 2000^2 205 201, FP32 1448^2 76.0 70.0; 500^2 (2 MB
+// of x) 10.2 12.8.  Poisson: FP64 1024^2 13.7 17.0, 3000^2 123 140, 5000^2 335
+// 381; FP32 5000^2 231 238.
+static int rows_nt(const pwm_matrix* h, double lines) { return h->crs_nt >= 0 ? h->crs_nt : lines > 32.0; }
 
 // Average time of 5 SpMVs (after 2 warm-up ones) of the swept slabs beside the
 // CRS arrays, entry loads plain or non-temporal, the faster kept.
@@ -697,40 +703,46 @@ static hipError_t time_swept(pwm_matrix* h, const void* x, void* y, float* best)
     return e;
 }
 
-// Swept slabs for scattered columns (k_csb_sweep, turns): built beside the CRS
-// arrays and timed into *ms, on a vector of ones x; *ms < 0 when not built.
-// csb_layout = 4 builds them for any columns and returns 0 ms (always the
+// Swept slabs for scattered columns (k_csb_sweep, turns), more than 128 lines
+// per 256 entries: a sweep in row order then fetches about one 128-byte line per
+// entry from beyond the L2.  Built beside the CRS arrays and timed into *ms, on a
+// vector of ones x; *ms < 0 when not built.  csb_layout = 4 builds them for any columns and returns 0 ms (always the
 // faster), 1 to 3 never.  Power-law rows of 16 entries, warm: FP64 1.2 M rows
 // 228 -> 76 us, 2.1 M 487 -> 161; FP32 3 M 586 -> 159; below 4 MB of x the row
 // order is at most a third slower (FP64 600 000 rows, 4.8 MB: 85 -> 60 us) and
 // the build is not worth its time (8 ms at 1.2 M rows).
-static int plan_swept(pwm_matrix* h, const void* x, void* y, float* ms) {
+// CRS_MERGE, which times nothing otherwise, takes them from 8 MB of x on: its load
+// becomes half as long again (6.2 M entries: 6.5 -> 9.8 ms), which 33 SpMVs bring
+// back at 9.6 MB of x (250 -> 108 us each) and 130 at 6.2 MB (65 -> 40).  A CRS
+// load times its kernels in any case (11.0 ms, with the slabs 10.0).
+static bool wants_swept(const pwm_matrix* h, double lines) {
+    if (h->csb_layout == 4) return h->nnz > 0;
+    const int64_t xbytes = h->noc * (int64_t)vector_size(h->vtype);
+    return h->csb_layout == 0 && lines > 128.0 && (h->format == PWM_FORMAT_CRS || xbytes > 2 * kXcdL2);
+}
+static int plan_swept(pwm_matrix* h, double lines, const void* x, void* y, float* ms) {
     *ms = -1.0f;
     h->csb.clear();
     const bool asked = h->csb_layout == 4;
-    bool scattered = asked && h->nnz > 0;
-    hipError_t e = hipSuccess;
-    if (h->csb_layout == 0 && (e = columns_scattered(h, &scattered)) != hipSuccess)
-        return hip_fail(h, e, "column scatter");
-    if (!scattered) return PWM_OK;
+    if (!wants_swept(h, lines)) return PWM_OK;
     const int rc = build_swept_beside_crs(h);
     if (rc != PWM_OK || !h->csb.sweep) return rc;
+    hipError_t e;
     if ((e = time_swept(h, x, y, ms)) != hipSuccess) return hip_fail(h, e, "swept slabs");
     if (asked) *ms = 0.0f;
     return PWM_OK;
 }
 
 // The faster of plain and non-temporal entry loads (the caller's choice, else
-// both are timed) for a CRS kernel that has them, and its time.
-static hipError_t time_entry_loads(pwm_matrix* h, int which, const void* x, void* y, float* best) {
+// both are timed) for the CRS tiles, and its time.
+static hipError_t time_entry_loads(pwm_matrix* h, const void* x, void* y, float* best) {
     int best_nt = 0;
     *best = -1.0f;
     for (int nt : {0, 1}) {
-        if (which == 0 && nt) continue;  // the merge kernel has only plain ones
-        if (which && h->crs_nt >= 0 && nt != h->crs_nt) continue;
+        if (h->crs_nt >= 0 && nt != h->crs_nt) continue;
         h->crs_nt_used = nt;
         float ms = 0.0f;
-        const hipError_t e = time_crs_kernel(h, which, x, y, &ms);
+        const hipError_t e = time_crs_kernel(h, 2, x, y, &ms);
         if (e != hipSuccess) return e;
         if (*best < 0.0f || ms < *best) {
             *best = ms;
@@ -838,7 +850,7 @@ static int plan_crs_rows(pwm_matrix* h) {
 // tiles (k_rows.hip): the kernels below were slower or equal on every such
 // matrix (FP64, us: Poisson 300 x 301 2.7 against 3.4, 5000 x 5000 332 against
 // 441, 9-point stencil with 2 random entries per row, 1448 x 1448, 100 against
-// 100); only the kind of entry load is timed.  Otherwise, or when the caller
+// 100).  Otherwise, or when the caller
 // named a kernel or set up the vector kernel: candidates are that one with the
 // rows-per-wave heuristic G0 = pow2(avg row length / 2) in [2, 32] and with
 // G0/2 and 2 G0 when the longest row fills them (only G0 when the caller
@@ -872,9 +884,15 @@ int plan_crs(pwm_matrix* h) {
     }
     if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
     h->crs_nt_used = h->crs_nt > 0 ? 1 : 0;
-    if (rows && h->crs_nt >= 0) {
+    hipError_t e;
+    double lines = 0.0;
+    if (automatic && (rows || h->csb_layout == 0) && (e = column_lines(h, &lines)) != hipSuccess)
+        return hip_fail(h, e, "column lines");
+    const bool sweep = automatic && h->crs_nt < 0 && wants_swept(h, lines);
+    if (rows) {
+        h->crs_nt_used = rows_nt(h, lines);
         h->crs_used = 3;
-        return PWM_OK;
+        if (!sweep) return PWM_OK;
     }
     if (!rows && (int)gs.size() + (tiles ? 1 : 0) == 1 && (!tiles || h->crs_nt >= 0)) {
         h->crs_used = tiles ? 2 : 1;
@@ -882,7 +900,6 @@ int plan_crs(pwm_matrix* h) {
     }
     const size_t vs = vector_size(h->vtype);
     DevBuf x, y;
-    hipError_t e;
     if ((e = x.alloc(std::max<int64_t>(h->noc, 1) * vs)) != hipSuccess ||
         (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess)
         return hip_fail(h, e, "CRS autotune vectors");
@@ -890,11 +907,11 @@ int plan_crs(pwm_matrix* h) {
     if (e != hipSuccess) return hip_fail(h, e, "CRS autotune vectors");
     float best = -1.0f, swept = -1.0f;
     int best_kernel = 1, best_g = G0;
-    if (automatic && h->crs_nt < 0 && (rc = plan_swept(h, x.p, y.p, &swept)) != PWM_OK) return rc;
+    if (sweep && (rc = plan_swept(h, lines, x.p, y.p, &swept)) != PWM_OK) return rc;
     if (rows || tiles) {
         best_kernel = rows ? 3 : 2;
-        if ((e = time_entry_loads(h, best_kernel, x.p, y.p, &best)) != hipSuccess)
-            return hip_fail(h, e, "CRS autotune");
+        e = rows ? time_crs_kernel(h, 3, x.p, y.p, &best) : time_entry_loads(h, x.p, y.p, &best);
+        if (e != hipSuccess) return hip_fail(h, e, "CRS autotune");
     }
     // the vector kernel gathers in row order like the tiles and was never a
     // third faster than they: it is not timed against a sweep that is
@@ -945,7 +962,6 @@ int plan_merge(pwm_matrix* h) {
     h->mp.carry_row = h->carry_row.as<int32_t>();
     h->mp.carry_val = h->carry_val.p;
     e = pwmk::launch_merge_splits(crs_of(h), h->mp, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "merge split search");
     // Unless the caller chose the partition or the tile size, the SpMV takes
     // the CRS format's wave tiles when the rows are short (Poisson 80 x 80: 8.0
@@ -955,23 +971,31 @@ int plan_merge(pwm_matrix* h) {
     h->csb.clear();
     h->rp = pwmk::RowsPlan{};
     h->crs_used = 0;
-    if ((h->threads > 0 && P == h->threads) || h->ipt != 8) return PWM_OK;
-    int rc = plan_crs_rows(h);
+    const bool chosen = (h->threads > 0 && P == h->threads) || h->ipt != 8;
+    int rc = chosen ? PWM_OK : plan_crs_rows(h);
     if (rc != PWM_OK) return rc;
     const bool rows = h->rp.nt > 0;
+    double lines = 0.0;
+    if (!chosen && (rows || h->csb_layout == 0) && (e = column_lines(h, &lines)) != hipSuccess)
+        return hip_fail(h, e, "column lines");
+    if (rows) {
+        h->crs_used = 3;
+        h->crs_nt_used = rows_nt(h, lines);
+    }
+    if (chosen || !wants_swept(h, lines)) {
+        e = rows ? hipSuccess : hipStreamSynchronize(h->stream);
+        return e == hipSuccess ? PWM_OK : hip_fail(h, e, "merge split search");
+    }
     const size_t vs = vector_size(h->vtype);
-    const bool sweep = h->csb_layout == 4 || h->noc * (int64_t)vs > kXcdL2;
-    if (!rows && !sweep) return PWM_OK;
     DevBuf x, y;
     if ((e = x.alloc(h->noc * vs)) != hipSuccess || (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess ||
         (e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream)) != hipSuccess)
         return hip_fail(h, e, "merge plan vectors");
     float swept = -1.0f, best = -1.0f;
-    if (sweep && (rc = plan_swept(h, x.p, y.p, &swept)) != PWM_OK) return rc;
-    if (!rows && swept < 0.0f) return PWM_OK;
-    h->crs_used = rows ? 3 : 0;
-    if ((e = time_entry_loads(h, h->crs_used, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "merge plan");
-    if (swept >= 0.0f && swept >= best) h->csb.clear();
+    if ((rc = plan_swept(h, lines, x.p, y.p, &swept)) != PWM_OK) return rc;
+    if (swept < 0.0f) return PWM_OK;
+    if ((e = time_crs_kernel(h, h->crs_used, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "merge plan");
+    if (swept >= best) h->csb.clear();
     return PWM_OK;
 }
 

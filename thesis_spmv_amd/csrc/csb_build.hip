@@ -438,35 +438,44 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
     int64_t stored = nnz;  // entries stored (order 1: every run padded to whole blocks of 256)
     if (nnz > 0) {
         pwmk::SweepKeyArgs a{nor, nnz, T, W, wb, (uint32_t)ww, order};
-        DevBuf keys, keys_out, pos, pos_out, tmp, roff;
-        if ((e = keys.alloc(nnz * 8)) != hipSuccess || (e = keys_out.alloc(nnz * 8)) != hipSuccess ||
-            (e = pos.alloc(nnz * 4)) != hipSuccess || (e = pos_out.alloc(nnz * 4)) != hipSuccess)
-            return hip_fail(h, e, "CSB sweep build allocation");
-        const dim3 g(pwmk::grid_of(nnz));
-        hipLaunchKernelGGL(pwmk::k_sweep_keys, g, dim3(256), 0, h->stream, a, h->rs.as<int32_t>(),
-                           h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys.as<uint64_t>(), pos.as<uint32_t>());
-        if ((e = hipGetLastError()) != hipSuccess) return hip_fail(h, e, "CSB sweep keys");
         unsigned end_bit = 1;
         while (end_bit < 64 && ((uint64_t)1 << end_bit) < (uint64_t)cells) ++end_bit;
         if (order) end_bit = std::min(64u, end_bit + (unsigned)wb);
+        // one allocation for all temporaries: freeing a large one takes 0.3 ms
         size_t tb = 0;
-        e = rocprim::radix_sort_pairs(nullptr, tb, keys.as<uint64_t>(), keys_out.as<uint64_t>(), pos.as<uint32_t>(),
-                                      pos_out.as<uint32_t>(), (size_t)nnz, 0u, end_bit, h->stream);
-        if (e == hipSuccess) e = tmp.alloc(std::max<size_t>(tb, 4));
-        if (e == hipSuccess)
-            e = rocprim::radix_sort_pairs(tmp.p, tb, keys.as<uint64_t>(), keys_out.as<uint64_t>(),
-                                          pos.as<uint32_t>(), pos_out.as<uint32_t>(), (size_t)nnz, 0u, end_bit,
-                                          h->stream);
+        e = rocprim::radix_sort_pairs(nullptr, tb, (uint64_t*)nullptr, (uint64_t*)nullptr, (uint32_t*)nullptr,
+                                      (uint32_t*)nullptr, (size_t)nnz, 0u, end_bit, h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "CSB sweep sort");
+        DevBuf all;
+        size_t used = 0;
+        auto part = [&](size_t bytes) {
+            const size_t at = used;
+            used += (bytes + 255) & ~(size_t)255;
+            return at;
+        };
+        const size_t o_keys = part(nnz * 8), o_keys_out = part(nnz * 8), o_pos = part(nnz * 4), o_pos_out = part(nnz * 4),
+                     o_tmp = part(tb), o_roff = part((cells + 1) * 4);
+        if ((e = all.alloc(used)) != hipSuccess) return hip_fail(h, e, "CSB sweep build allocation");
+        uint64_t* keys = (uint64_t*)((char*)all.p + o_keys);
+        uint64_t* keys_out = (uint64_t*)((char*)all.p + o_keys_out);
+        uint32_t* pos = (uint32_t*)((char*)all.p + o_pos);
+        uint32_t* pos_out = (uint32_t*)((char*)all.p + o_pos_out);
+        int32_t* roff = (int32_t*)((char*)all.p + o_roff);
+        const dim3 g(pwmk::grid_of(nnz));
+        hipLaunchKernelGGL(pwmk::k_sweep_keys, g, dim3(256), 0, h->stream, a, h->rs.as<int32_t>(),
+                           h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys, pos);
+        if ((e = hipGetLastError()) != hipSuccess) return hip_fail(h, e, "CSB sweep keys");
+        e = rocprim::radix_sort_pairs((char*)all.p + o_tmp, tb, keys, keys_out, pos, pos_out, (size_t)nnz, 0u, end_bit,
+                                      h->stream);
         if (e != hipSuccess) return hip_fail(h, e, "CSB sweep sort");
         // run starts; order 1 pads every run to whole blocks of 256 entries
-        DevBuf& runs = order ? roff : c.soff;
-        if (order && (e = roff.alloc((cells + 1) * 4)) != hipSuccess) return hip_fail(h, e, "CSB sweep allocation");
+        int32_t* runs = order ? roff : c.soff.as<int32_t>();
         hipLaunchKernelGGL(pwmk::k_csb_soff, dim3(pwmk::grid_of(cells)), dim3(256), 0, h->stream,
-                           keys_out.as<uint64_t>(), nnz, cells, order ? wb : 0, runs.as<int32_t>());
+                           keys_out, nnz, cells, order ? wb : 0, runs);
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail(h, e, "CSB sweep runs");
         if (order) {
             std::vector<int32_t> r(cells + 1), pr(cells + 1);
-            if ((e = hipMemcpyAsync(r.data(), roff.p, cells * 4, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
+            if ((e = hipMemcpyAsync(r.data(), roff, cells * 4, hipMemcpyDeviceToHost, h->stream)) != hipSuccess ||
                 (e = hipStreamSynchronize(h->stream)) != hipSuccess)
                 return hip_fail(h, e, "CSB sweep runs");
             r[cells] = (int32_t)nnz;
@@ -480,13 +489,13 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
             }
             pr[cells] = (int32_t)acc;
             stored = acc;
-            if ((e = hipMemcpyAsync(roff.p, r.data(), (cells + 1) * 4, hipMemcpyHostToDevice, h->stream)) !=
+            if ((e = hipMemcpyAsync(roff, r.data(), (cells + 1) * 4, hipMemcpyHostToDevice, h->stream)) !=
                     hipSuccess ||
                 (e = hipMemcpyAsync(c.soff.p, pr.data(), (cells + 1) * 4, hipMemcpyHostToDevice, h->stream)) !=
                     hipSuccess ||
                 (e = hipStreamSynchronize(h->stream)) != hipSuccess)
                 return hip_fail(h, e, "CSB sweep runs");
-            a.roff = roff.as<int32_t>();
+            a.roff = roff;
             a.poff = c.soff.as<int32_t>();
         }
         const int64_t zpad = ((stored + 3) & ~(int64_t)3) + 4;
@@ -498,18 +507,18 @@ int csb_sweep_device(pwm_matrix* h, const int32_t* rs, int64_t target_slabs, int
             return hip_fail(h, e, "CSB sweep allocation");
         if (vs == 8)
             hipLaunchKernelGGL(pwmk::k_sweep_gather<uint64_t>, g, dim3(256), 0, h->stream, a, h->rs.as<int32_t>(),
-                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out.as<uint64_t>(),
-                               pos_out.as<uint32_t>(), h->val.as<uint64_t>(), c.ind.as<uint32_t>(),
+                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out,
+                               pos_out, h->val.as<uint64_t>(), c.ind.as<uint32_t>(),
                                c.data.as<uint64_t>());
         else if (vs == 4)
             hipLaunchKernelGGL(pwmk::k_sweep_gather<uint32_t>, g, dim3(256), 0, h->stream, a, h->rs.as<int32_t>(),
-                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out.as<uint64_t>(),
-                               pos_out.as<uint32_t>(), h->val.as<uint32_t>(), c.ind.as<uint32_t>(),
+                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out,
+                               pos_out, h->val.as<uint32_t>(), c.ind.as<uint32_t>(),
                                c.data.as<uint32_t>());
         else
             hipLaunchKernelGGL(pwmk::k_sweep_gather<uint16_t>, g, dim3(256), 0, h->stream, a, h->rs.as<int32_t>(),
-                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out.as<uint64_t>(),
-                               pos_out.as<uint32_t>(), h->val.as<uint16_t>(), c.ind.as<uint32_t>(),
+                               h->ci.as<int32_t>(), c.sweep_start.as<int32_t>(), keys_out,
+                               pos_out, h->val.as<uint16_t>(), c.ind.as<uint32_t>(),
                                c.data.as<uint16_t>());
         if ((e = hipGetLastError()) == hipSuccess) e = hipStreamSynchronize(h->stream);  // before the temporaries go
         if (e != hipSuccess) return hip_fail(h, e, "CSB sweep build");
