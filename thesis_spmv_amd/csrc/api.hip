@@ -1017,7 +1017,7 @@ int spmv_launch(pwm_matrix* h, const void* x, void* y, const PowerArgs* pw) {
     return PWM_OK;
 }
 
-static int64_t partials_needed(const pwm_matrix* h) {
+static int64_t partial_slots(const pwm_matrix* h) {
     switch (swept_crs(h) ? PWM_FORMAT_CSB : h->format) {
         case PWM_FORMAT_CRS:
             if (h->crs_used == 3) return pwmk::rows_power_blocks(h->rp.nt);
@@ -1029,6 +1029,21 @@ static int64_t partials_needed(const pwm_matrix* h) {
     }
     return 0;
 }
+
+// Whether a fixed number of power steps defers the norms: few slots, and kernels
+// that can add them up (wave tiles, slab streams that write y, swept slabs,
+// BlockCOH).
+static bool defers_norms(const pwm_matrix* h) {
+    bool can = h->crs_used == 3;
+    if (swept_crs(h) || h->format == PWM_FORMAT_CSB)
+        can = h->csb.sweep || (h->csb.stream && h->csb.groups == 1);
+    else if (h->format == PWM_FORMAT_BLOCKCOH)
+        can = true;
+    return can && !h->power_small && partial_slots(h) <= pwmk::kDeferSlots;
+}
+
+// deferred norms: two steps' slots
+static int64_t partials_needed(const pwm_matrix* h) { return partial_slots(h) * (defers_norms(h) ? 2 : 1); }
 
 }  // namespace pwm_impl
 
@@ -1622,6 +1637,10 @@ static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, doub
     pw.max_it = max_it;
     pw.tol = tol;
     pw.k = 0;
+    const int64_t slots = partial_slots(h);
+    pw.defer = tol < 0 && defers_norms(h);
+    pw.prev = nullptr;
+    pw.prev_n = 0;
     // what the loop leaves in ctrl: the step count, the done flag, and the
     // last step's lambda and |y|^2
     struct {
@@ -1647,12 +1666,24 @@ static int run_power(pwm_matrix* h, void* buf0, void* buf1, int64_t max_it, doub
             if (e != hipSuccess) return hip_fail(h, e, "power loop");
             pw.k = end;
         }
-        for (; pw.k < end; ++pw.k)
+        for (; pw.k < end; ++pw.k) {
             if ((rc = spmv_launch(h, nullptr, nullptr, &pw)) != PWM_OK) return rc;
+            if (pw.defer) {
+                pw.prev = pw.partials;
+                pw.prev_n = slots;
+                pw.partials = ws->partials + (pw.k & 1 ? 0 : 3 * slots);
+            }
+        }
         if (tol >= 0 && end < max_it) {
             if (!read_back()) return hip_fail(h, e, "power loop");
             if (out.done) break;
         }
+    }
+    if (pw.defer) {  // the last step's norms
+        pw.k = max_it - 1;
+        e = pwmk::launch_power_final(pw, pw.prev, slots, 1, h->stream);
+        if (e != hipSuccess) return hip_fail(h, e, "power norms");
+        pw.k = max_it;
     }
     if (!h->power_small) {
         e = pwmk::launch_power_finish(pw, h->nor, h->vtype == PWM_VALUES_F64, h->stream);

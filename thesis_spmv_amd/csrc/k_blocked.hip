@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kBS) void k_csb(CsbArgs a, const typename Arith<VT>
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = pwmk::recorded_scale(pw);
     }
     const VT* __restrict__ val = (const VT*)a.val;
     const uint32_t* __restrict__ ind = a.ind;
@@ -231,10 +231,11 @@ __global__ __launch_bounds__(kBS) void k_csb(CsbArgs a, const typename Arith<VT>
 // so the loads carry no branch.
 constexpr int kSBS = 256;
 
+// POWER: 1 a power step, 2 one that adds up the last step's norms (deferred);
 // kSU: groups of 4 entries per thread per step (2 or 4); NT: non-temporal
 // entry loads and partial-slab stores; WIDE: ind holds the column and srows
 // the row in the slab.
-template <typename VT, bool POWER, int kSU, bool NT, bool WIDE>
+template <typename VT, int POWER, int kSU, bool NT, bool WIDE>
 __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
                                                      typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename A
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = POWER == 2 ? 1.0 / sqrt(pwmk::last_norm<kSBS>(pw, red)) : pwmk::recorded_scale(pw);
     }
     const VT* __restrict__ val = (const VT*)a.val;
     const uint32_t* __restrict__ ind = a.ind;
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kSBS) void k_csb_stream(CsbArgs a, const typename A
     __syncthreads();
     const int64_t beta = (int64_t)1 << a.bits;
     const int64_t row0 = (t / a.slabs) * beta + (t % a.slabs) * (int64_t)h;
-    csb_write_slab<X, Acc, kSBS, POWER, NT>(a, ylds, h, row0, g, t, x, y, scale, pw, red);
+    csb_write_slab<X, Acc, kSBS, (POWER > 0), NT>(a, ylds, h, row0, g, t, x, y, scale, pw, red);
 }
 
 // y[r] = sum over the column groups of ypart[g][r], groups in order (and the
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(kBS) void k_csb_reduce(CsbArgs a, typename Arith<VT
                                                     PowerArgs pw) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
-    __shared__ double red[16];
+    __shared__ double red[48];
     X* __restrict__ y = y_arg;
     const X* __restrict__ x = nullptr;
     double scale = 1.0;
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(kBS) void k_csb_reduce(CsbArgs a, typename Arith<VT
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = pwmk::recorded_scale(pw);
     }
     const Acc* __restrict__ yp = (const Acc*)a.ypart;
     double yy = 0.0, xy = 0.0, xx = 0.0;
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(kSwBS) void k_csb_sweep(CsbArgs a, const typename A
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = 1.0 / sqrt(pwmk::last_norm<kSwBS>(pw, red));
     }
     const VT* __restrict__ val = (const VT*)a.val;
     const uint32_t* __restrict__ ind = a.ind;
@@ -606,7 +607,7 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
     double* ylds = (double*)coh_smem;
     constexpr int kCohStage = 256;  // blocks of a band kept in LDS, where a band has no more
     __shared__ CohBlock bstage[kCohStage];
-    __shared__ double red[16];
+    __shared__ double red[48];
 
     const X* __restrict__ x = x_arg;
     X* __restrict__ y = y_arg;
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = 1.0 / sqrt(pwmk::last_norm<kBS>(pw, red));
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -741,7 +742,7 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
 template <typename VT, bool POWER>
 __global__ __launch_bounds__(kBS) void k_coh_finish(CohArgs a, typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
-    __shared__ double red[16];
+    __shared__ double red[48];
     const X* x = nullptr;
     X* y = y_arg;
     double scale = 1.0;
@@ -750,7 +751,7 @@ __global__ __launch_bounds__(kBS) void k_coh_finish(CohArgs a, typename Arith<VT
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = pwmk::step_scale(pw, k);
+        scale = 1.0 / sqrt(pwmk::last_norm<kBS>(pw, red));
     }
     const CohRows piece = a.pieces[blockIdx.x];
     double yy = 0.0, xy = 0.0, xx = 0.0;
@@ -822,19 +823,19 @@ static hipError_t csb_t(const CsbArgs& a, const void* x, void* y, const PowerArg
     } else if (a.stream) {
         const size_t lds = (size_t)a.slab_rows * sizeof(double);
         const dim3 grid((unsigned)a.n_tasks);
-        // kernel instance for (power step, unroll, non-temporal)
+        // kernel instance for (power step, width, unroll, non-temporal)
         auto pick = [&](auto power, auto wide) {
-            constexpr bool P = decltype(power)::value, W = decltype(wide)::value;
+            constexpr int P = decltype(power)::value;
+            constexpr bool W = decltype(wide)::value;
             if (a.unroll == 4) return a.nt ? k_csb_stream<VT, P, 4, true, W> : k_csb_stream<VT, P, 4, false, W>;
             return a.nt ? k_csb_stream<VT, P, 2, true, W> : k_csb_stream<VT, P, 2, false, W>;
         };
-        if (pw)
-            hipLaunchKernelGGL(a.wide ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{}),
-                               grid, dim3(kSBS), lds, s, a, (const X*)nullptr, (X*)nullptr, *pw);
-        else
-            hipLaunchKernelGGL(a.wide ? pick(std::false_type{}, std::true_type{})
-                                      : pick(std::false_type{}, std::false_type{}),
-                               grid, dim3(kSBS), lds, s, a, (const X*)x, (X*)y, PowerArgs{});
+        auto pick_wide = [&](auto power) { return a.wide ? pick(power, std::true_type{}) : pick(power, std::false_type{}); };
+        auto k = !pw         ? pick_wide(std::integral_constant<int, 0>{})
+                 : pw->defer ? pick_wide(std::integral_constant<int, 2>{})
+                             : pick_wide(std::integral_constant<int, 1>{});
+        hipLaunchKernelGGL(k, grid, dim3(kSBS), lds, s, a, pw ? (const X*)nullptr : (const X*)x,
+                           pw ? (X*)nullptr : (X*)y, pw ? *pw : PowerArgs{});
     } else if (pw) {
         hipLaunchKernelGGL((k_csb<VT, true>), dim3((unsigned)a.n_tasks), dim3(kBS), 0, s, a, (const X*)nullptr,
                            (X*)nullptr, *pw);

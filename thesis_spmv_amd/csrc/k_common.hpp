@@ -165,16 +165,16 @@ struct PowerArgs {
     int64_t max_it;
     double tol;        // < 0: never stop early
     int64_t k;         // this step
+    // Deferred norms (tol < 0, few slots): a step leaves its partial sums, and
+    // the blocks of the next step add up the previous step's prev_n slots
+    // themselves (prev_n = 0: its record is complete).
+    bool defer;
+    const double* prev;
+    int64_t prev_n;
 };
 
 // An earlier step met the stop test: this one does nothing.
 __device__ __forceinline__ bool power_done(const PowerArgs& p) { return p.tol >= 0.0 && p.k > 0 && p.ctrl[1]; }
-
-// FP64 scale applied to step k's output: 1/|y_{k-1}| (1 for the first step,
-// which multiplies the caller's unnormalised start vector).
-__device__ __forceinline__ double step_scale(const PowerArgs& p, int64_t k) {
-    return k == 0 ? 1.0 : 1.0 / sqrt(p.rec[4 * (k - 1)]);
-}
 
 // Step k's record, stop test and step count, from its |y|^2, x^T y and x^T x
 // (one thread).
@@ -194,6 +194,57 @@ __device__ __forceinline__ void power_record(const PowerArgs& pw, int64_t k, dou
     double* result = (double*)(pw.ctrl + 4);
     result[0] = lam;
     result[1] = yy;
+}
+
+constexpr int kPsU = 4;  // slots a thread loads together
+
+// Sum of the slots i0, i0 + stride, ... < end of this thread, in that order.
+__device__ __forceinline__ void slot_sum(const double* slots, int64_t i0, int64_t stride, int64_t end, double& yy,
+                                         double& xy, double& xx) {
+    for (int64_t i = i0; i < end; i += kPsU * stride) {
+        double a[kPsU], b[kPsU], c[kPsU];
+#pragma unroll
+        for (int u = 0; u < kPsU; ++u) {
+            const int64_t j = i + u * stride;
+            const bool ok = j < end;
+            a[u] = ok ? slots[3 * j + 0] : 0.0;
+            b[u] = ok ? slots[3 * j + 1] : 0.0;
+            c[u] = ok ? slots[3 * j + 2] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kPsU; ++u) {
+            yy += a[u];
+            xy += b[u];
+            xx += c[u];
+        }
+    }
+}
+
+// |y_{k-1}|^2 (1 for the first step, which multiplies the caller's unnormalised
+// start vector; the step's output is divided by the root of it): from the record
+// of step k-1 or, deferred, from its slots, which every block adds up (in the
+// same order); block 0 then writes the record.  All BS threads of the block call
+// it; `scratch` holds >= 48 doubles.
+template <int BS>
+__device__ __forceinline__ double last_norm(const PowerArgs& p, double* scratch) {
+    if (p.prev_n == 0) return p.k == 0 ? 1.0 : p.rec[4 * (p.k - 1)];
+    double yy = 0.0, xy = 0.0, xx = 0.0;
+    slot_sum(p.prev, threadIdx.x, BS, p.prev_n, yy, xy, xx);
+    if (blockIdx.x == 0) {
+        block_sum3<BS>(yy, xy, xx, scratch);
+        if (threadIdx.x == 0) power_record(p, p.k - 1, yy, xy, xx);
+    } else {
+        yy = block_sum<BS>(yy, scratch);
+    }
+    return yy;
+}
+
+// The scale from the record, for steps that do not defer their norms.  (Kernels
+// of many short workgroups have an instance of their own for deferred steps: the
+// choice at run time, with its barrier, held up the first loads of every
+// workgroup, FP64 Poisson 5000 x 5000 in CRS 358 -> 376 us a step.)
+__device__ __forceinline__ double recorded_scale(const PowerArgs& p) {
+    return p.k == 0 ? 1.0 : 1.0 / sqrt(p.rec[4 * (p.k - 1)]);
 }
 
 }  // namespace pwmk

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(kBS) void k_crs_vector(CrsDev A, int n_vec_blocks, 
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = step_scale(pw, k);
+        scale = recorded_scale(pw);
     }
     const int32_t* __restrict__ rs = A.rs;
     const int32_t* __restrict__ ci = A.ci;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kFinBS) void k_crs_finalize(CrsDev A, int n_partial
         k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = step_scale(pw, k);
+        scale = recorded_scale(pw);
     }
     double yy = 0.0, xy = 0.0, xx = 0.0;
     const double* part = (const double*)lr.chunk_partial;

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kMBS) void k_merge_spmv(CrsDev A, MergePlan mp, con
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = step_scale(pw, k);
+        scale = recorded_scale(pw);
     }
     const int64_t p = xcd_remap(blockIdx.x, mp.P);
     const int64_t a1 = mp.split_a[p + 1];
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(ONE ? kFixOneBS : kFixBS) void k_merge_fixup_power1
     const int64_t k = pw.k;
     const X* __restrict__ x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
     X* __restrict__ y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-    const double scale = step_scale(pw, k);
+    const double scale = recorded_scale(pw);
     const Acc* cv = (const Acc*)mp.carry_val;
     const int64_t nrows = A.nrows;
     const int64_t p0 = (int64_t)blockIdx.x * per;

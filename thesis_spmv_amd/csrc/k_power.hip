@@ -168,30 +168,6 @@ __global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArg
 
 constexpr int kFinBS = 1024;
 constexpr int kSumBS = 256;
-constexpr int kPsU = 4;  // slots a thread loads together
-
-// Sum of the slots i0, i0 + stride, ... < end of this thread, in that order.
-__device__ __forceinline__ void slot_sum(const double* slots, int64_t i0, int64_t stride, int64_t end, double& yy,
-                                         double& xy, double& xx) {
-    for (int64_t i = i0; i < end; i += kPsU * stride) {
-        double a[kPsU], b[kPsU], c[kPsU];
-#pragma unroll
-        for (int u = 0; u < kPsU; ++u) {
-            const int64_t j = i + u * stride;
-            const bool ok = j < end;
-            a[u] = ok ? slots[3 * j + 0] : 0.0;
-            b[u] = ok ? slots[3 * j + 1] : 0.0;
-            c[u] = ok ? slots[3 * j + 2] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kPsU; ++u) {
-            yy += a[u];
-            xy += b[u];
-            xx += c[u];
-        }
-    }
-}
-
 // Many slots: workgroup b leaves the sum of slots [b*per, (b+1)*per) in slot
 // b*per.
 __global__ __launch_bounds__(kSumBS) void k_power_sum(PowerArgs pw, int64_t n, int64_t per) {
@@ -230,6 +206,7 @@ hipError_t launch_power_final(const PowerArgs& pw, const double* slots, int64_t 
 // One workgroup reads kPsU slots per thread in one go; beyond two such rounds
 // a launch that spreads the reading costs less than a third.
 hipError_t launch_power_reduce(const PowerArgs& pw, int64_t n, hipStream_t s) {
+    if (pw.defer) return hipSuccess;
     if (n <= 2 * kPsU * kFinBS) return launch_power_final(pw, pw.partials, n, 1, s);
     const int64_t per = std::max<int64_t>(kPsU * kSumBS, (n + kFinBS - 1) / kFinBS);
     const int64_t nb = (n + per - 1) / per;

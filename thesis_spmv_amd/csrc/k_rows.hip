@@ -31,9 +31,13 @@ constexpr int kRwChunk = 256;     // consecutive tiles per XCD in the block orde
 constexpr int kRwBS = 64;         // threads per block of an SpMV
 
 // Threads per block of a power step, one partial-sum slot a block: 256 (FP32
-// 3000 x 3000: 92.7 us a step against 99.9 with 512), but at most 200 000
-// slots, which the fixed workspace of the no-allocation power method holds.
-static int rows_power_bs(int64_t nt) { return (nt + 3) / 4 <= 200000 ? 256 : 512; }
+// 3000 x 3000: 92.7 us a step against 99.9 with 512, 100 x 100 4.2 against
+// 4.7), but 512 where that brings the slots down to what the next step adds up
+// itself (k_power.hip; FP64 600 x 600: 11.1 -> 8.5 us) and, for the largest, to
+// 200 000, which the fixed workspace of the no-allocation power method holds.
+static int rows_power_bs(int64_t nt) {
+    return (nt > 2048 && (nt + 7) / 8 <= kDeferSlots) || (nt + 3) / 4 > 200000 ? 512 : 256;
+}
 
 // First row whose entries start at or after p * step (n from the last cut on).
 __device__ __forceinline__ int64_t rows_cut(const int32_t* __restrict__ rs, int64_t n, int64_t nt, int64_t step,
@@ -60,13 +64,15 @@ __global__ void k_rows_plan(const int32_t* __restrict__ rs, int64_t n, int64_t s
     if (t < nt && rows_cut(rs, n, nt, step, t + 1) - a > 64 * kRwSlots) *too_many_rows = 1;
 }
 
+// POWER: 1 a power step, 2 one that adds up the last step's norms (deferred).
 // NT: non-temporal entry loads (the entries, read once, leave the L2 to x).
-template <typename VT, int BS, bool POWER, bool NT>
+template <typename VT, int BS, int POWER, bool NT>
 __global__ __launch_bounds__(BS) void k_rows(CrsDev A, RowsPlan rp, const typename Arith<VT>::X* __restrict__ x_arg,
                                              typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     __shared__ __align__(16) Acc prods[BS / 64][kRwEntries];
+    __shared__ double red[POWER ? 48 : 1];
     const X* __restrict__ x = x_arg;
     X* __restrict__ y = y_arg;
     double scale = 1.0;
@@ -75,7 +81,7 @@ __global__ __launch_bounds__(BS) void k_rows(CrsDev A, RowsPlan rp, const typena
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = step_scale(pw, k);
+        scale = POWER == 2 ? 1.0 / sqrt(last_norm<BS>(pw, red)) : recorded_scale(pw);
     }
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -154,7 +160,6 @@ __global__ __launch_bounds__(BS) void k_rows(CrsDev A, RowsPlan rp, const typena
         }
     }
     if constexpr (POWER) {
-        __shared__ double red[48];
         block_sum3<BS>(yy, xy, xx, red);
         if (threadIdx.x == 0) {
             pw.partials[3 * blockIdx.x + 0] = yy;
@@ -185,9 +190,10 @@ hipError_t launch_rows_plan(const CrsDev& A, int64_t step, int64_t nt, int2* cut
 template <typename VT, int BS>
 static void launch_rows_power(const CrsDev& A, const RowsPlan& rp, const PowerArgs& pw, hipStream_t s) {
     using X = typename Arith<VT>::X;
-    hipLaunchKernelGGL((A.nt ? k_rows<VT, BS, true, true> : k_rows<VT, BS, true, false>),
-                       dim3((unsigned)rows_power_blocks(rp.nt)), dim3(BS), 0, s, A, rp, (const X*)nullptr, (X*)nullptr,
-                       pw);
+    auto k = pw.defer ? (A.nt ? k_rows<VT, BS, 2, true> : k_rows<VT, BS, 2, false>)
+                      : (A.nt ? k_rows<VT, BS, 1, true> : k_rows<VT, BS, 1, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)rows_power_blocks(rp.nt)), dim3(BS), 0, s, A, rp, (const X*)nullptr,
+                       (X*)nullptr, pw);
 }
 
 template <typename VT>
@@ -199,7 +205,7 @@ static hipError_t launch_rows_t(const CrsDev& A, const RowsPlan& rp, const void*
     else if (pw)
         launch_rows_power<VT, 512>(A, rp, *pw, s);
     else
-        hipLaunchKernelGGL((A.nt ? k_rows<VT, kRwBS, false, true> : k_rows<VT, kRwBS, false, false>),
+        hipLaunchKernelGGL((A.nt ? k_rows<VT, kRwBS, 0, true> : k_rows<VT, kRwBS, 0, false>),
                            dim3((unsigned)((rp.nt + kRwBS / 64 - 1) / (kRwBS / 64))), dim3(kRwBS), 0, s, A, rp,
                            (const X*)x, (X*)y, PowerArgs{});
     return hipGetLastError();

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kTBS) void k_tiles_spmv(CrsDev A, const ETile* __re
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = step_scale(pw, k);
+        scale = recorded_scale(pw);
     }
     const int64_t p = xcd_remap(blockIdx.x, mp.P);
     const ETile T = tiles[p];

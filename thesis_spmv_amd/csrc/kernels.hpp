@@ -91,7 +91,15 @@ inline int merge_fix_blocks(int64_t P) {
 }
 
 // ---- power method: norms of a step, and small matrices (k_power.hip) --------
-// The n partial-sum slots of step pw.k into its record (slots are overwritten).
+// A step of at most kDeferSlots slots can leave its norms to the next one, whose
+// blocks add the slots up before they scale.  A launch for it costs about 3 us of
+// a step; n blocks that read n slots of 24 bytes each cost nothing that shows up
+// to 500 slots and 2 us at 1200.  FP64 Poisson in CRS, us per step: 100 x 100 6.3
+// -> 4.3, 300 x 300 7.4 -> 5.0, 600 x 600 11.3 -> 8.5, 700 x 700 (1229 slots)
+// 13.0 -> 11.8.
+constexpr int64_t kDeferSlots = 1280;
+// The n partial-sum slots of step pw.k into its record (slots are overwritten);
+// nothing for a step that defers its norms.
 hipError_t launch_power_reduce(const PowerArgs& pw, int64_t n, hipStream_t s);
 // The slots 0, step, 2 step, ... (n of them) of `slots`, by one workgroup.
 hipError_t launch_power_final(const PowerArgs& pw, const double* slots, int64_t n, int64_t step, hipStream_t s);
