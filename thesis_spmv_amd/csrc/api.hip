@@ -332,6 +332,13 @@ static hipError_t window_upload(void* dst, size_t bytes, hipStream_t s, Fill fil
 // for the work queued on s.  b: the buffer to begin with.
 template <typename Empty>
 static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, Empty empty, int b = 0) {
+    if (bytes <= kInlineBytes) {  // (an event costs 5 us more than the stream)
+        hipError_t e = pwmk::launch_copy_bytes(g_stage[b], src, bytes, true, s);
+        const hipError_t e2 = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = e2;
+        if (e == hipSuccess) empty((const char*)g_stage[b], 0, bytes);
+        return e;
+    }
     auto issue = [&](size_t off, int to) {
         const Window W(std::min(kStageBytes, bytes - off), bytes);
         hipError_t e = hipSuccess;
@@ -347,11 +354,6 @@ static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, 
         if (off + kStageBytes < bytes && (e = issue(off + kStageBytes, b ^ 1)) != hipSuccess) break;
         const size_t n = std::min(kStageBytes, bytes - off);
         const char* stage = (const char*)g_stage[b];
-        if (n <= kInlineBytes) {
-            e = hipEventSynchronize(g_ring_ev[b * kRingChunks]);
-            if (e == hipSuccess) empty(stage, off, off + n);
-            continue;
-        }
         const Window W(n, bytes);
         std::atomic<size_t> ready{0};  // chunks that have arrived
         std::atomic<bool> bad{false};
