@@ -627,23 +627,36 @@ static hipError_t crs_kernel_launch(pwm_matrix* h, int which, const void* x, voi
     return e;
 }
 
-// Average time of 5 SpMVs (after 2 warm-up ones) of CRS kernel `which` on
-// the device vectors x, y.
-static hipError_t time_crs_kernel(pwm_matrix* h, int which, const void* x, void* y, float* ms) {
-    hipEvent_t a, b;
-    (void)hipEventCreate(&a);
-    (void)hipEventCreate(&b);
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < 2 && e == hipSuccess; ++i) e = crs_kernel_launch(h, which, x, y, nullptr);
-    (void)hipEventRecord(a, h->stream);
-    for (int i = 0; i < 5 && e == hipSuccess; ++i) e = crs_kernel_launch(h, which, x, y, nullptr);
-    (void)hipEventRecord(b, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    *ms = 0.0f;
-    (void)hipEventElapsedTime(ms, a, b);
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
+// Mean of 5 SpMVs after 2 warm-up ones.  From 4 M entries on (25 us a run and
+// more: one run pages everything in, two give its time to a few percent) 2 after
+// 1, unless these 2 took less than 0.1 ms.  Loading power-law rows in CSB, which
+// times 13 layouts: 6.4 M entries 16.6 -> 13.7 ms, 48 M 87 -> 56; in CRS 6.4 ->
+// 5.3 and 38 -> 30.
+hipError_t time_launches(pwm_matrix* h, const std::function<hipError_t()>& launch, float* ms) {
+    hipEvent_t a = nullptr, b = nullptr;
+    hipError_t e = hipEventCreate(&a);
+    if (e == hipSuccess) e = hipEventCreate(&b);
+    auto run = [&](int warm, int timed) {
+        float t = 0.0f;
+        for (int i = 0; i < warm && e == hipSuccess; ++i) e = launch();
+        if (e == hipSuccess) e = hipEventRecord(a, h->stream);
+        for (int i = 0; i < timed && e == hipSuccess; ++i) e = launch();
+        if (e == hipSuccess) e = hipEventRecord(b, h->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(b);
+        if (e == hipSuccess) e = hipEventElapsedTime(&t, a, b);
+        return t / timed;
+    };
+    const bool large = h->nnz >= ((int64_t)4 << 20);
+    *ms = large ? run(1, 2) : run(2, 5);
+    if (large && e == hipSuccess && 2 * *ms < 0.1f) *ms = run(0, 5);
+    if (a) (void)hipEventDestroy(a);
+    if (b) (void)hipEventDestroy(b);
     return e;
+}
+
+// Time of an SpMV by CRS kernel `which` on the device vectors x, y.
+static hipError_t time_crs_kernel(pwm_matrix* h, int which, const void* x, void* y, float* ms) {
+    return time_launches(h, [&] { return crs_kernel_launch(h, which, x, y, nullptr); }, ms);
 }
 
 constexpr int64_t kXcdL2 = (int64_t)4 << 20;  // an XCD's L2
@@ -676,39 +689,30 @@ static hipError_t column_lines(pwm_matrix* h, double* per_group) {
 // 381; FP32 5000^2 231 238.
 static int rows_nt(const pwm_matrix* h, double lines) { return h->crs_nt >= 0 ? h->crs_nt : lines > 32.0; }
 
-// Average time of 5 SpMVs (after 2 warm-up ones) of the swept slabs beside the
-// CRS arrays, entry loads plain or non-temporal, the faster kept.
+// Time of an SpMV by the swept slabs beside the CRS arrays, entry loads plain or
+// non-temporal, the faster kept.
 static hipError_t time_swept(pwm_matrix* h, const void* x, void* y, float* best) {
-    hipEvent_t a, b;
-    (void)hipEventCreate(&a);
-    (void)hipEventCreate(&b);
     hipError_t e = hipSuccess;
     int best_nt = 0;
     *best = -1.0f;
     for (int nt = 0; nt < 2 && e == hipSuccess; ++nt) {
         h->csb.nt = nt;
-        for (int i = 0; i < 2 && e == hipSuccess; ++i) e = csb_launch(h, x, y, nullptr);
-        (void)hipEventRecord(a, h->stream);
-        for (int i = 0; i < 5 && e == hipSuccess; ++i) e = csb_launch(h, x, y, nullptr);
-        (void)hipEventRecord(b, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, a, b);
+        e = time_launches(h, [&] { return csb_launch(h, x, y, nullptr); }, &ms);
         if (*best < 0.0f || ms < *best) {
             *best = ms;
             best_nt = nt;
         }
     }
     h->csb.nt = best_nt;
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
     return e;
 }
 
 // Swept slabs for scattered columns (k_csb_sweep, turns), more than 128 lines
 // per 256 entries: a sweep in row order then fetches about one 128-byte line per
 // entry from beyond the L2.  Built beside the CRS arrays and timed into *ms, on a
-// vector of ones x; *ms < 0 when not built.  csb_layout = 4 builds them for any columns and returns 0 ms (always the
+// vector of ones x; *ms < 0 when not built.  csb_layout = 4 builds them for any
+// columns and returns 0 ms (always the
 // faster), 1 to 3 never.  Power-law rows of 16 entries, warm: FP64 1.2 M rows
 // 228 -> 76 us, 2.1 M 487 -> 161; FP32 3 M 586 -> 159; below 4 MB of x the row
 // order is at most a third slower (FP64 600 000 rows, 4.8 MB: 85 -> 60 us) and
@@ -858,7 +862,7 @@ static int plan_crs_rows(pwm_matrix* h) {
 // G0/2 and 2 G0 when the longest row fills them (only G0 when the caller
 // fixed group_size), and the tiles kernel (unless crs_kernel excludes
 // either).  With more than one candidate,
-// each is timed on x = 1 (2 warm-up + 5 timed SpMVs) and the fastest is kept.
+// each is timed on x = 1 and the fastest is kept.
 int plan_crs(pwm_matrix* h) {
     const double avg = h->nor > 0 ? (double)h->nnz / (double)h->nor : 0.0;
     const int G0 = h->group_opt > 0 ? h->group_opt : std::min(32, std::max(2, pow2_ceil((int64_t)ceil(avg / 2.0))));

@@ -270,6 +270,9 @@ hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt,
 // then complete but must not be used)
 hipError_t upload_indices_staged(void* dst, const int32_t* src, int64_t n, int64_t bound, bool* out_of_range,
                                  hipStream_t s, const std::function<void()>* between = nullptr);
+// Time of an SpMV of h as `launch` queues it on h->stream, on the caller's
+// vectors, for the plans that are chosen at load.
+hipError_t time_launches(pwm_matrix* h, const std::function<hipError_t()>& launch, float* ms);
 // n device values (FP64 or FP32), as doubles on the host, the same way (after
 // the work queued on s).
 hipError_t download_doubles(double* dst, const void* src, int64_t n, bool f64, hipStream_t s);

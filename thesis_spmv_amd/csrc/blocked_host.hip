@@ -164,8 +164,7 @@ static int download_crs(pwm_matrix* h, std::vector<int32_t>& ci, std::vector<dou
     return PWM_OK;
 }
 
-// Mean milliseconds of 5 SpMVs (after 2 warm-up ones) of the handle's CSB
-// layout as it stands, on x = 1.
+// Time of an SpMV of the handle's CSB layout as it stands, on x = 1.
 static int time_csb(pwm_matrix* h, float* ms) {
     DevBuf tx, ty;
     const size_t vs = vector_size(h->vtype);
@@ -174,21 +173,8 @@ static int time_csb(pwm_matrix* h, float* ms) {
         (e = ty.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess)
         return hip_fail(h, e, "CSB autotune vectors");
     e = pwmk::launch_fill(tx.p, h->noc, h->vtype == PWM_VALUES_F64, 1.0, h->stream);
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (e == hipSuccess) e = hipEventCreate(&e0);
-    if (e == hipSuccess) e = hipEventCreate(&e1);
-    for (int w = 0; w < 2 && e == hipSuccess; ++w) e = csb_launch(h, tx.p, ty.p, nullptr);
-    if (e == hipSuccess) e = hipEventRecord(e0, h->stream);
-    for (int r = 0; r < 5 && e == hipSuccess; ++r) e = csb_launch(h, tx.p, ty.p, nullptr);
-    if (e == hipSuccess) e = hipEventRecord(e1, h->stream);
-    if (e == hipSuccess) e = hipEventSynchronize(e1);
-    float t = 0.0f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&t, e0, e1);
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    if (e != hipSuccess) return hip_fail(h, e, "CSB autotune");
-    *ms = t / 5.0f;
-    return PWM_OK;
+    if (e == hipSuccess) e = time_launches(h, [&] { return csb_launch(h, tx.p, ty.p, nullptr); }, ms);
+    return e == hipSuccess ? PWM_OK : hip_fail(h, e, "CSB autotune");
 }
 
 // Swept-slab layout: as many nnz-balanced slabs as the chip has CUs (one
@@ -485,9 +471,6 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
         if ((e = tx.alloc(noc * vs)) != hipSuccess || (e = ty.alloc(nor * vs)) != hipSuccess)
             return hip_fail(h, e, "CSB autotune vectors");
         (void)pwmk::launch_fill(tx.p, noc, h->vtype == PWM_VALUES_F64, 1.0, h->stream);
-        hipEvent_t e0, e1;
-        (void)hipEventCreate(&e0);
-        (void)hipEventCreate(&e1);
         float best = 1e30f;
         int32_t best_g = cands[0], best_u = unrolls[0], best_nt = nts[0];
         for (int32_t gc : cands)
@@ -497,13 +480,9 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
                     c.unroll = uc;
                     c.nt = ntc;
                     c.n_tasks = units * gc;
-                    for (int w = 0; w < 2; ++w) (void)csb_launch(h, tx.p, ty.p, nullptr);
-                    (void)hipEventRecord(e0, h->stream);
-                    for (int r = 0; r < 5; ++r) (void)csb_launch(h, tx.p, ty.p, nullptr);
-                    (void)hipEventRecord(e1, h->stream);
-                    (void)hipEventSynchronize(e1);
                     float ms = 0;
-                    (void)hipEventElapsedTime(&ms, e0, e1);
+                    e = time_launches(h, [&] { return csb_launch(h, tx.p, ty.p, nullptr); }, &ms);
+                    if (e != hipSuccess) return hip_fail(h, e, "CSB autotune");
                     if (ms < best) {
                         best = ms;
                         best_g = gc;
@@ -511,8 +490,6 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
                         best_nt = ntc;
                     }
                 }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
         c.groups = best_g;
         c.unroll = best_u;
         c.nt = best_nt;
