@@ -687,7 +687,8 @@ static hipError_t column_lines(pwm_matrix* h, double* per_group) {
 // 45.9 44.1, 1448^2 103 99.5, 2000^2 205 201, FP32 1448^2 76.0 70.0; 500^2 (2 MB
 // of x) 10.2 12.8.  Poisson: FP64 1024^2 13.7 17.0, 3000^2 123 140, 5000^2 335
 // 381; FP32 5000^2 231 238.
-static int rows_nt(const pwm_matrix* h, double lines) { return h->crs_nt >= 0 ? h->crs_nt : lines > 32.0; }
+constexpr double kSpreadLines = 32.0;
+static int rows_nt(const pwm_matrix* h, double lines) { return h->crs_nt >= 0 ? h->crs_nt : lines > kSpreadLines; }
 
 // Time of an SpMV by the swept slabs beside the CRS arrays, entry loads plain or
 // non-temporal, the faster kept.
@@ -856,8 +857,10 @@ static int plan_crs_rows(pwm_matrix* h) {
 // tiles (k_rows.hip): the kernels below were slower or equal on every such
 // matrix (FP64, us: Poisson 300 x 301 2.7 against 3.4, 5000 x 5000 332 against
 // 441, 9-point stencil with 2 random entries per row, 1448 x 1448, 100 against
-// 100).  Otherwise, or when the caller
-// named a kernel or set up the vector kernel: candidates are that one with the
+// 100), but where x has far lines and more than 24 MB (that stencil on 2896 x
+// 2896: FP64 441 against 434, FP32, 33.5 MB of x, 369 against 364; on 2200 x 2200
+// in FP32, 19 MB, 197 against 196).  Otherwise, or when the caller named a kernel
+// or set up the vector kernel: candidates are that one with the
 // rows-per-wave heuristic G0 = pow2(avg row length / 2) in [2, 32] and with
 // G0/2 and 2 G0 when the longest row fills them (only G0 when the caller
 // fixed group_size), and the tiles kernel (unless crs_kernel excludes
@@ -881,25 +884,24 @@ int plan_crs(pwm_matrix* h) {
     h->rp = pwmk::RowsPlan{};
     h->csb.clear();
     const bool automatic = h->crs_kernel == 0 && h->group_opt == 0 && h->vec_blocks_opt == 0 && h->long_row == 0;
-    if (automatic && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
+    hipError_t e;
+    double lines = 0.0;
+    if (automatic && (e = column_lines(h, &lines)) != hipSuccess) return hip_fail(h, e, "column lines");
+    const int64_t xbytes = h->noc * (int64_t)vector_size(h->vtype);
+    if (automatic && !(lines > kSpreadLines && xbytes > 6 * kXcdL2) && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
     const bool rows = h->rp.nt > 0;
     const bool tiles = !rows && h->crs_kernel != 1;
+    const bool sweep = automatic && h->crs_nt < 0 && wants_swept(h, lines);
     if (rows) {
         gs.clear();
         h->lr = pwmk::LongRows{};
-    }
-    if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
-    h->crs_nt_used = h->crs_nt > 0 ? 1 : 0;
-    hipError_t e;
-    double lines = 0.0;
-    if (automatic && (rows || h->csb_layout == 0) && (e = column_lines(h, &lines)) != hipSuccess)
-        return hip_fail(h, e, "column lines");
-    const bool sweep = automatic && h->crs_nt < 0 && wants_swept(h, lines);
-    if (rows) {
         h->crs_nt_used = rows_nt(h, lines);
         h->crs_used = 3;
         if (!sweep) return PWM_OK;
+    } else {
+        h->crs_nt_used = h->crs_nt > 0 ? 1 : 0;
     }
+    if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
     if (!rows && (int)gs.size() + (tiles ? 1 : 0) == 1 && (!tiles || h->crs_nt >= 0)) {
         h->crs_used = tiles ? 2 : 1;
         return plan_crs_vector(h, tiles ? G0 : gs[0]);
