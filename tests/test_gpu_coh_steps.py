@@ -3,7 +3,8 @@
 Cases where the steps' bookkeeping can go wrong: bands that begin off a multiple
 of 4 entries, a step within one row, more blocks than are kept in LDS, a band cut
 into atomic tasks (rows beyond the window, or many times the others' entries),
-empty bands.  y is the FP64 sum of the products, rounded once; the products are
+empty bands, bands of one wave each (scattered columns, x beyond 10 MB in FP64).
+y is the FP64 sum of the products, rounded once; the products are
 formed in the vectors' type, so against exact products each adds its own
 rounding: |err| <= u_x (|y| + sum |a x|) + L 2^-52 sum |a x|, with u_x = 2^-24 for
 FP32 vectors (BF16 storage too) and 2^-53 for FP64."""
@@ -27,11 +28,12 @@ def _lens(kind, rng):
         lens = np.zeros(6000, np.int64)
         lens[5::50] = rng.integers(1, 700, 120)
         return lens
-    return np.full({"tiny": 9, "blocks": 700, "wide": 120000}[kind], {"tiny": 3, "blocks": 11, "wide": 4}[kind])
+    return np.full({"tiny": 9, "blocks": 700, "wide": 120000, "waves": 66000}[kind],
+                   {"tiny": 3, "blocks": 11, "wide": 4, "waves": 9}[kind])
 
 
 CASES = [("tiny", 7, -1), ("blocks", 10000000, 1), ("wide", 300000, 1), ("wide", 300000, 3), ("last_band", 30011, -1),
-         ("one_row", 60000, -1), ("one_row", 60000, 2), ("gaps", 4099, -1), ("gaps", 4099, 5)]
+         ("one_row", 60000, -1), ("one_row", 60000, 2), ("gaps", 4099, -1), ("gaps", 4099, 5), ("waves", 1500000, 1100)]
 
 
 @pytest.mark.parametrize("values", ["f64", "f32", "bf16"])

@@ -661,10 +661,9 @@ static hipError_t time_crs_kernel(pwm_matrix* h, int which, const void* x, void*
 
 constexpr int64_t kXcdL2 = (int64_t)4 << 20;  // an XCD's L2
 
-// Distinct 128-byte lines of x that 256 consecutive entries touch, on average;
-// 0 where x fits one XCD's L2.  Stencils and banded matrices have some 10 to
-// 20, with 2 random entries per row about 55, uniformly random columns all 256.
-static hipError_t column_lines(pwm_matrix* h, double* per_group) {
+// Stencils and banded matrices have some 10 to 20, with 2 random entries per row
+// about 55, uniformly random columns all 256.
+hipError_t column_lines(pwm_matrix* h, double* per_group) {
     *per_group = 0.0;
     const int64_t xb = (int64_t)vector_size(h->vtype);
     if (h->noc * xb <= kXcdL2 || h->nnz < 256) return hipSuccess;

@@ -159,6 +159,7 @@ struct CohDev {
     DevBuf ysum;           // their sums
     int64_t n_tasks = 0, total_blocks = 0, n_pieces = 0;
     int32_t lds_rows = 0;  // rows of the largest band accumulated in LDS (the kernel's LDS window)
+    int32_t one_wave = 0;  // tasks of one wave each
     int32_t occ8 = 0;      // reported: 8 waves per SIMD unless the option coh_occ8 says 0
     void clear() {
         bands.clear();
@@ -167,7 +168,7 @@ struct CohDev {
             b->release();
         n_tasks = total_blocks = n_pieces = 0;
         lds_rows = 0;
-        occ8 = 0;
+        occ8 = one_wave = 0;
     }
 };
 
@@ -270,6 +271,9 @@ hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt,
 // then complete but must not be used)
 hipError_t upload_indices_staged(void* dst, const int32_t* src, int64_t n, int64_t bound, bool* out_of_range,
                                  hipStream_t s, const std::function<void()>* between = nullptr);
+// Distinct 128-byte lines of x that 256 consecutive entries of the device CRS
+// touch, on average; 0 where x fits one XCD's L2.
+hipError_t column_lines(pwm_matrix* h, double* per_group);
 // Time of an SpMV of h as `launch` queues it on h->stream, on the caller's
 // vectors, for the plans that are chosen at load.
 hipError_t time_launches(pwm_matrix* h, const std::function<hipError_t()>& launch, float* ms);

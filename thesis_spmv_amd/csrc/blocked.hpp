@@ -137,6 +137,7 @@ struct CohArgs {
     double* ysum = nullptr;  // rows of atomic bands, zero between two SpMVs
     int vtype = 0;
     int32_t lds_rows = 0;  // LDS window of the kernel: rows of the largest LDS-accumulated band
+    int32_t one_wave = 0;  // 1: a task is one wave's, not a workgroup's of 8
 };
 
 // part: 0 = the whole SpMV, 1 = the slab kernel only, 2 = the column-group

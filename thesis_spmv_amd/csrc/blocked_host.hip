@@ -841,6 +841,7 @@ hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     a.val = h->coh.data.p;
     a.vtype = h->vtype;
     a.lds_rows = h->coh.lds_rows;
+    a.one_wave = h->coh.one_wave;
     a.pieces = h->coh.row_pieces.as<blocked::CohRows>();
     a.n_pieces = h->coh.n_pieces;
     a.ysum = h->coh.ysum.as<double>();
@@ -850,12 +851,22 @@ hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     return e;
 }
 
-// The BlockCOH layout.  One kernel, at 8 waves per SIMD; the option coh_occ8 is
-// kept and reported.
+// The BlockCOH layout, and whether its tasks run one wave each: more than 128
+// lines of x per 256 entries, x beyond 10 MB and enough tasks for 4 waves per
+// CU.  Power-law rows, us with 8 waves and with one: FP64 1 M (8 MB of x) 129 147,
+// 2 M 282 263, 3 M 536 419, FP32 3 M (12 MB) 360 338; the 9-point stencil with 2
+// random entries per row (55 lines) on 2000^2 225 266.  The option coh_occ8 is
+// kept and reported; both instances run at 8 waves per SIMD.
 int build_blockcoh(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals) {
+    double lines = 0.0;
+    const hipError_t e = column_lines(h, &lines);
+    if (e != hipSuccess) return hip_fail(h, e, "column lines");
     const int rc = build_blockcoh_layout(h, rs, ci, vals);
-    if (rc == PWM_OK) h->coh.occ8 = h->coh_occ8 != 0;
-    return rc;
+    if (rc != PWM_OK) return rc;
+    h->coh.occ8 = h->coh_occ8 != 0;
+    h->coh.one_wave = lines > 128.0 && h->noc * (int64_t)vector_size(h->vtype) > ((int64_t)10 << 20) &&
+                      h->coh.n_tasks >= 1024;
+    return PWM_OK;
 }
 
 }  // namespace pwm_impl

@@ -587,18 +587,24 @@ int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32) {
 // of block starts before it: four ballots and a table of the blocks at the
 // steps.
 //
+// BS: 512, or 64 where x is far beyond an L2 and the columns are scattered
+// (blocked_host.hip): 8 waves that take a band's steps in turn are 2048 entries
+// apart, some 30 blocks, 4 MB of x; a wave per band keeps to a few blocks, the
+// bands of an XCD walk x in the same order and meet in its L2.
+//
 // Bound by the gathers (FP64 9-point stencil with 2 random entries per row, 1 M
 // rows: 215 G/s of the 213-233 G/s that the L2 serves) or, on a matrix of few
 // blocks, by HBM.  Mean of back-to-back SpMVs on rotating copies, us, against
 // workgroups that decode the stored jumps with two segmented scans per 2048
 // entries: that stencil 88 -> 51, on 90 K rows 18.6 -> 8.2; Poisson 1024^2
 // 39.8 -> 18, 3000^2 283 -> 145; power-law rows, 100 K 67 -> 18, 500 K 315 ->
-// 64, 2 M 687 -> 278.  Tried: 2 or 4 steps at once (the same or slower),
-// non-temporal entry loads (18 -> 22 on the Poisson matrix, 281 -> 275 on the
-// largest), the step table read after the entries (278 -> 302).
-template <typename VT, bool POWER>
-__global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
-                                                typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
+// 64, 2 M 687 -> 261 (with 8 waves per band 278), 3 M 871 -> 411 (536).  Tried: 2
+// or 4 steps at once (the same or slower), non-temporal entry loads (18 -> 22 on
+// the Poisson matrix, 281 -> 275 on the 2 M rows), the step table read after the
+// entries (278 -> 302).
+template <typename VT, bool POWER, int BS>
+__global__ __launch_bounds__(BS) void k_coh(CohArgs a, const typename Arith<VT>::X* __restrict__ x_arg,
+                                            typename Arith<VT>::X* __restrict__ y_arg, PowerArgs pw) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     // the LDS window holds the rows of the largest band accumulated in LDS
@@ -617,7 +623,7 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = 1.0 / sqrt(pwmk::last_norm<kBS>(pw, red));
+        scale = 1.0 / sqrt(pwmk::last_norm<BS>(pw, red));
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -631,12 +637,12 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
 
     const bool staged = band.blocks <= kCohStage;
     if (lds)
-        for (int i = tid; i < band.rows; i += kBS) ylds[i] = 0;
+        for (int i = tid; i < band.rows; i += BS) ylds[i] = 0;
     if (staged)
-        for (int i = tid; i < band.blocks; i += kBS) bstage[i] = blocks[i];
+        for (int i = tid; i < band.blocks; i += BS) bstage[i] = blocks[i];
     __syncthreads();
     const int64_t first = band.entry, end = first + band.nnz, base = first & ~(int64_t)3;
-    for (int s = task.step0 + wave; s < task.step0 + task.nsteps; s += kWaves) {
+    for (int s = task.step0 + wave; s < task.step0 + task.nsteps; s += (BS / 64)) {
         int b = stab[s];  // a scalar load, ahead of the entries
         const int64_t q = base + (int64_t)s * kCohStep + 4 * lane;
         // lanes beyond the band load its last quad (the arrays are padded)
@@ -711,7 +717,7 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
     }
     __syncthreads();
     double yy = 0.0, xy = 0.0, xx = 0.0;
-    for (int i = tid; i < band.rows; i += kBS) {
+    for (int i = tid; i < band.rows; i += BS) {
         const int64_t row = (int64_t)band.start + i;
         if constexpr (POWER) {
             const X out = (X)(ylds[i] * scale);
@@ -725,9 +731,9 @@ __global__ __launch_bounds__(kBS) void k_coh(CohArgs a, const typename Arith<VT>
         }
     }
     if constexpr (POWER) {
-        const double ra = pwmk::block_sum<kBS>(yy, red);
-        const double rb = pwmk::block_sum<kBS>(xy, red);
-        const double rc = pwmk::block_sum<kBS>(xx, red);
+        const double ra = pwmk::block_sum<BS>(yy, red);
+        const double rb = pwmk::block_sum<BS>(xy, red);
+        const double rc = pwmk::block_sum<BS>(xx, red);
         if (tid == 0) {
             pw.partials[3 * blockIdx.x + 0] = ra;
             pw.partials[3 * blockIdx.x + 1] = rb;
@@ -867,7 +873,8 @@ static hipError_t coh_t(const CohArgs& a, const void* x, void* y, const PowerArg
     using X = typename Arith<VT>::X;
     if (a.n_tasks <= 0) return hipSuccess;
     const size_t lds = (size_t)std::max<int32_t>(a.lds_rows, 1) * sizeof(double);
-    hipLaunchKernelGGL((k_coh<VT, POWER>), dim3((unsigned)a.n_tasks), dim3(kBS), lds, s, a, (const X*)x, (X*)y, pw);
+    auto k = a.one_wave ? k_coh<VT, POWER, 64> : k_coh<VT, POWER, kBS>;
+    hipLaunchKernelGGL(k, dim3((unsigned)a.n_tasks), dim3(a.one_wave ? 64 : kBS), lds, s, a, (const X*)x, (X*)y, pw);
     if (a.n_pieces > 0)
         hipLaunchKernelGGL((k_coh_finish<VT, POWER>), dim3((unsigned)a.n_pieces), dim3(kBS), 0, s, a, (X*)y, pw);
     return hipGetLastError();
