@@ -79,7 +79,7 @@ typedef struct {
     int32_t non_temporal;      /* CSB slab streams / CRS tiles: 1 = non-temporal entry loads */
     int32_t layout;            /* CSB: 1 slab pieces, 2 slab streams, 3 wide slab streams, 4 swept slabs */
     int32_t kernels;           /* kernel launches of one pwm_mv_device */
-    int32_t high_occupancy;    /* BlockCOH: 1 when the kernel instance with registers capped for 8 waves per SIMD runs */
+    int32_t high_occupancy;    /* BlockCOH: 0 with the option coh_occ8 = 0, else 1 */
 } pwm_info_t;
 
 /* Constructor SparseMatrix(int threads) (Matrix/SparseMatrix.hpp:30) through
