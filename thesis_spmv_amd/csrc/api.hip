@@ -1046,7 +1046,8 @@ static bool defers_norms(const pwm_matrix* h) {
         can = h->csb.sweep || (h->csb.stream && h->csb.groups == 1);
     else if (h->format == PWM_FORMAT_BLOCKCOH)
         can = true;
-    return can && !h->power_small && partial_slots(h) <= pwmk::kDeferSlots;
+    const int64_t slots = partial_slots(h);
+    return can && !h->power_small && slots > 0 && slots <= pwmk::kDeferSlots;
 }
 
 // deferred norms: two steps' slots
