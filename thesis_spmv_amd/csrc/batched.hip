@@ -319,6 +319,15 @@ static void batch_add_jobs(pwm_batch* b, int64_t max_it, double tol) {
     }
 }
 
+// Start vector of instance i: hash stream i of `seed`.
+static hipError_t batch_start_vectors(pwm_batch* b, uint64_t seed) {
+    std::vector<pwmk::EVec> v;
+    v.reserve(b->inst.size());
+    for (size_t i = 0; i < b->inst.size(); ++i)
+        v.push_back({b->arena.at(b->inst[i].o_vec), b->inst[i].n, (uint64_t)i, 1.0});
+    return pwmk::engine_start_vectors(v.data(), (int)v.size(), b->vtype, seed, b->stream);
+}
+
 static void batch_release_jobs(pwm_batch* b) {
     for (BatchInst& I : b->inst) {
         b->eng->release(I.slot);
@@ -342,9 +351,7 @@ static int batch_autotune(pwm_batch* b) {
         cands.push_back({ipt, 0});
         if (!b->bf16_exact) cands.push_back({ipt, 1});  // the mixed-storage engine has no persistent grid
     }
-    hipError_t e = hipSuccess;
-    for (size_t i = 0; i < b->inst.size() && e == hipSuccess; ++i)
-        e = pwmk::engine_start_vector(b->arena.at(b->inst[i].o_vec), b->inst[i].n, b->vtype, 0, (uint64_t)i, b->stream);
+    hipError_t e = batch_start_vectors(b, 0);
     if (e != hipSuccess) return bhip(b, e, "batch autotune start vectors");
     hipEvent_t e0, e1;
     if ((e = hipEventCreate(&e0)) != hipSuccess) return bhip(b, e, "batch autotune");
@@ -420,12 +427,7 @@ extern "C" int pwm_batch_solve(pwm_batch* b, int64_t max_it, double tol, uint64_
     if (b->autotune && !b->tuned && (rc = batch_autotune(b)) != PWM_OK) return rc;
     if (E.ipt() != b->ipt && (rc = E.set_ipt(b->ipt)) != PWM_OK) return bfail(b, rc, "pwm_batch_solve: items_per_thread");
     E.persistent = b->persistent != 0;
-    pwm_impl::Arena& A = b->arena;
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < ni && e == hipSuccess; ++i) {
-        BatchInst& I = b->inst[i];
-        e = pwmk::engine_start_vector(A.at(I.o_vec), I.n, b->vtype, seed, (uint64_t)i, b->stream);
-    }
+    hipError_t e = batch_start_vectors(b, seed);
     if (e != hipSuccess) return bhip(b, e, "batch start vectors");
     hipEvent_t e0, e1;
     (void)hipEventCreate(&e0);
@@ -445,11 +447,13 @@ extern "C" int pwm_batch_solve(pwm_batch* b, int64_t max_it, double tol, uint64_
             break;
         }
     }
-    if (rc == PWM_OK)
-        for (int i = 0; i < ni && e == hipSuccess; ++i) {
-            const BatchInst& I = b->inst[i];
-            e = pwmk::engine_normalize(E.last_buffer(I.slot), I.n, b->vtype, 1.0 / sqrt(E.state(I.slot).yy), b->stream);
-        }
+    if (rc == PWM_OK) {
+        std::vector<pwmk::EVec> v;
+        v.reserve(ni);
+        for (const BatchInst& I : b->inst)
+            v.push_back({E.last_buffer(I.slot), I.n, 0, 1.0 / sqrt(E.state(I.slot).yy)});
+        e = pwmk::engine_scale_vectors(v.data(), ni, b->vtype, b->stream);
+    }
     (void)hipEventRecord(e1, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     float t = 0;
@@ -485,7 +489,7 @@ extern "C" int pwm_batch_solve(pwm_batch* b, int64_t max_it, double tol, uint64_
 }
 
 // The start vector the solver used for instance `id` with `seed` (host
-// restatement of k_eng_start with stream id = instance id).
+// restatement of k_eng_start with id = instance id).
 extern "C" int pwm_batch_start_vector(pwm_batch* b, int32_t id, uint64_t seed, double* out) {
     if (!b || !out || id < 0 || id >= (int32_t)b->inst.size()) return bfail(b, PWM_ERR_INVALID, "pwm_batch_start_vector");
     const int64_t n = b->inst[id].n;

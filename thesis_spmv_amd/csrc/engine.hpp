@@ -108,8 +108,17 @@ constexpr int VT_MIXED16 = 3;
 
 int32_t engine_tiles_for(int64_t n, int64_t nnz, int ipt);
 hipError_t engine_plan_tiles(const int32_t* rs, int64_t n, int64_t nnz, int ipt, ETile* tiles, hipStream_t s);
-hipError_t engine_start_vector(void* x, int64_t n, int vtype, uint64_t seed, uint64_t stream_id, hipStream_t s);
-hipError_t engine_normalize(void* v, int64_t n, int vtype, double inv_norm, hipStream_t s);
+// One vector of a group launch: its start values come from hash stream `id`,
+// its final iterate is multiplied by `scale`.
+struct EVec {
+    void* p;
+    int64_t n;
+    uint64_t id;
+    double scale;
+};
+constexpr int kVecGroup = 64;  // vectors per launch
+hipError_t engine_start_vectors(const EVec* v, int count, int vtype, uint64_t seed, hipStream_t s);
+hipError_t engine_scale_vectors(const EVec* v, int count, int vtype, hipStream_t s);
 // grid_persist > 0: persistent tile kernel with that many workgroups.
 hipError_t engine_step(const EArgs& a, int vtype, int ipt, int grid_work, int grid_persist, int grid_slots,
                        hipStream_t s);

@@ -460,7 +460,8 @@ static int stage(pwm_server* s, size_t max_jobs, size_t max_new, int* staged) {
         J.has_block = true;
         ++s->staged_front;
         ++*staged;
-        const hipError_t e = pwmk::engine_start_vector(s->arena.at(J.off), M.n, s->vtype, J.seed, 0, s->ustream);
+        const pwmk::EVec v = {s->arena.at(J.off), M.n, 0, 1.0};
+        const hipError_t e = pwmk::engine_start_vectors(&v, 1, s->vtype, J.seed, s->ustream);
         if (e != hipSuccess) {
             rc = shp(s, e, "job start vector");
             break;
@@ -526,7 +527,8 @@ static int admit(pwm_server* s) {
 // Record the finished slots' results (appended to last_finished), normalise
 // their final iterates and free their engine slots.
 static int retire(pwm_server* s, const std::vector<int>& fin) {
-    hipError_t e = hipSuccess;
+    std::vector<pwmk::EVec> v;
+    v.reserve(fin.size());
     for (int slot : fin) {
         const int64_t id = s->slot_job[slot];
         s->last_finished.push_back(id);
@@ -537,12 +539,13 @@ static int retire(pwm_server* s, const std::vector<int>& fin) {
         J.iters = S.it;
         J.last = s->eng->last_buffer(slot);
         J.state = 2;
-        if (e == hipSuccess) e = pwmk::engine_normalize(J.last, s->mats[J.mat].n, s->vtype, 1.0 / J.ynorm, s->stream);
+        v.push_back({J.last, s->mats[J.mat].n, 0, 1.0 / J.ynorm});
         s->eng->release(slot);
         s->slot_job[slot] = -1;
         s->mats[J.mat].refs--;
         ++s->finished_total;
     }
+    hipError_t e = pwmk::engine_scale_vectors(v.data(), (int)v.size(), s->vtype, s->stream);
     if (e == hipSuccess && !fin.empty()) e = hipStreamSynchronize(s->stream);
     if (e != hipSuccess) return shp(s, e, "job retirement");
     return PWM_OK;
