@@ -37,3 +37,24 @@ def test_group_edges(values, tol, count, long_at):
             xr, _ = oracle.crs_power_iteration(A, b.start_vector(i, A.nor, seed=seed), 2)
             v, _ = b.vector(i, A.nor)
             assert np.max(np.abs(v - xr)) <= tol, (values, count, i, m, n)
+
+
+@pytest.mark.parametrize("its", [1, 31, 32, 33, 64, 70])
+def test_tail_of_a_chunk(its):
+    """Steps around multiples of the 32-step chunk: full chunks replay a graph,
+    a shorter last one is launched step by step; the same bits either way, with
+    other work between the solves."""
+    out = []
+    for graph in (1, 0):
+        b = pw.Batch("f32", graph=graph)
+        sizes = [(3, 4), (70, 61), (300, 9)]
+        for m, n in sizes:
+            b.add_poisson(m, n)
+        for rep in range(3):
+            lam, k, _ = b.solve(its, -1.0, seed=7)
+            assert np.all(k == its)
+            out.append((lam, [b.vector(i, m * n)[0] for i, (m, n) in enumerate(sizes)]))
+    for lam, vecs in out[1:]:
+        assert np.array_equal(lam, out[0][0])
+        for v, w in zip(vecs, out[0][1]):
+            assert np.array_equal(v, w)

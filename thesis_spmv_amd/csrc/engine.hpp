@@ -22,7 +22,8 @@
 // device and both kernels read the list lengths from device memory, so every
 // step of a chunk has the same launch arguments: a chunk of steps is
 // captured once in a hipGraph (grids sized to the list capacities) and
-// replayed until a list outgrows its capacity or shrinks below a quarter.
+// replayed until a list outgrows its capacity or shrinks below a quarter; a
+// chunk cut short by max_it is launched step by step.
 #pragma once
 
 #include <hip/hip_runtime.h>
