@@ -172,27 +172,27 @@ __device__ __forceinline__ bool eng_view(const EJob* __restrict__ jobs, const ES
 
 // Stage (after tile_load), barrier, compute, carry and FP64 partials of one
 // tile.  `after_stage` runs right after the staging barrier.
-template <typename VT, int ITEMS, typename F>
+template <typename VT, int BS, int ITEMS, typename F>
 __device__ __forceinline__ void eng_tile(const EWork& W, const EView<typename Arith<VT>::X>& v,
                                          const TileRegs<VT, ITEMS>& R,
-                                         MergeTileSmem<typename Arith<VT>::A, kEngBS, ITEMS>& sm, double* red,
+                                         MergeTileSmem<typename Arith<VT>::A, BS, ITEMS>& sm, double* red,
                                          F&& after_stage) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
     const int na = W.a1 - W.a0;
     X xr[ITEMS];
-    if (W.stream) stream_xrows<VT, kEngBS, ITEMS>(v.x, W.a0, na, xr);
-    tile_stage<VT, kEngBS, ITEMS>(R, W.rs, v.x, W.a0, na, W.b0, W.b1, sm);
+    if (W.stream) stream_xrows<VT, BS, ITEMS>(v.x, W.a0, na, xr);
+    tile_stage<VT, BS, ITEMS>(R, W.rs, v.x, W.a0, na, W.b0, W.b1, sm);
     __syncthreads();
     after_stage();
     double yy = 0.0, xy = 0.0, xx = 0.0;
     Acc c = 0;
     if (W.stream)
-        stream_compute<VT, kEngBS, ITEMS, true>(v.y, xr, W.a0, W.a1, W.b0, v.scale, sm, yy, xy, xx);
+        stream_compute<VT, BS, ITEMS, true>(v.y, xr, W.a0, W.a1, W.b0, v.scale, sm, yy, xy, xx);
     else
-        c = merge_compute<VT, kEngBS, ITEMS, true>(W.rs, v.x, v.y, W.a0, W.a1, W.b0, W.b1, v.scale, sm, yy, xy, xx);
-    if (threadIdx.x == kEngBS - 1) G((Acc*)v.carry)[W.tile] = c;
-    block_sum3<kEngBS>(yy, xy, xx, red);  // its closing barrier also frees the LDS tile
+        c = merge_compute<VT, BS, ITEMS, true>(W.rs, v.x, v.y, W.a0, W.a1, W.b0, W.b1, v.scale, sm, yy, xy, xx);
+    if (threadIdx.x == BS - 1) G((Acc*)v.carry)[W.tile] = c;
+    block_sum3<BS>(yy, xy, xx, red);  // its closing barrier also frees the LDS tile
     if (threadIdx.x == 0) {
         const auto p = G(v.partials + 3 * (int64_t)W.tile);
         p[0] = yy;
@@ -206,34 +206,42 @@ __device__ __forceinline__ void eng_tile(const EWork& W, const EView<typename Ar
 // list out for that.
 // The tile kernels take their read-only arrays as restrict parameters, so the
 // compiler reads the uniform work entry, job and state with scalar loads.
-// They are compiled for 8 waves per SIMD (256 x 8-item FP32 tiles: 62
+// They are compiled for 8 waves per SIMD (8 FP32 items per thread: 62
 // instead of 68 VGPRs), which keeps more tiles in flight when few jobs are
 // left in a solve.
-template <typename VT, int ITEMS>
-__global__ __launch_bounds__(kEngBS, 8) void k_eng_tiles(const EWork* __restrict__ work, const EJob* __restrict__ jobs,
+// A thread takes at most 8 items: what bounds the step is gathers in flight,
+// and 16 items per thread need the registers of 4 FP32 waves per SIMD (3 FP64),
+// where 512 threads of 8 on the same tile run 8 (4 FP64).  24 FP32 instances
+// of up to 300 000 rows, 100 steps: 11 840 -> 10 270 us, with BF16 values
+// where exact 12 090 -> 10 720; 22 of up to 6 435 rows, 45 steps: 708 -> 588; 24
+// FP64 of up to 300 000 rows, 50 steps: 8 170 -> 8 110; 4 of up to 5 000: 820 -> 682.
+// (1024 threads of 4 items are held to 64 registers and spill: three to six
+// times slower on the large batches.)
+template <typename VT, int BS, int ITEMS>
+__global__ __launch_bounds__(BS, 8) void k_eng_tiles(const EWork* __restrict__ work, const EJob* __restrict__ jobs,
                                                       const EState* __restrict__ st, const ECtl* __restrict__ ctl) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
-    __shared__ MergeTileSmem<Acc, kEngBS, ITEMS> sm;
+    __shared__ MergeTileSmem<Acc, BS, ITEMS> sm;
     __shared__ double red[48];
     if ((int)blockIdx.x >= ctl->n_work) return;
     const EWork W = work[blockIdx.x];
     EView<X> v;
     if (!eng_view(jobs, st, W.slot, v)) return;
     TileRegs<VT, ITEMS> R;
-    tile_load<VT, kEngBS, ITEMS>(R, W.ci, (const VT*)W.val, W.b0, W.b1);
-    eng_tile<VT, ITEMS>(W, v, R, sm, red, [] {});
+    tile_load<VT, BS, ITEMS>(R, W.ci, (const VT*)W.val, W.b0, W.b1);
+    eng_tile<VT, BS, ITEMS>(W, v, R, sm, red, [] {});
 }
 
 // FP32 vectors, each tile's values FP32 or BF16 by its job (a branch that is
 // uniform over the workgroup); the accumulator and LDS tile are FP32 either
 // way.
-template <int ITEMS>
-__global__ __launch_bounds__(kEngBS, 8) void k_eng_tiles_mixed(const EWork* __restrict__ work,
+template <int BS, int ITEMS>
+__global__ __launch_bounds__(BS, 8) void k_eng_tiles_mixed(const EWork* __restrict__ work,
                                                             const EJob* __restrict__ jobs,
                                                             const EState* __restrict__ st,
                                                             const ECtl* __restrict__ ctl) {
-    __shared__ MergeTileSmem<float, kEngBS, ITEMS> sm;
+    __shared__ MergeTileSmem<float, BS, ITEMS> sm;
     __shared__ double red[48];
     if ((int)blockIdx.x >= ctl->n_work) return;
     const EWork W = work[blockIdx.x];
@@ -241,12 +249,12 @@ __global__ __launch_bounds__(kEngBS, 8) void k_eng_tiles_mixed(const EWork* __re
     if (!eng_view(jobs, st, W.slot, v)) return;
     if (W.vt16) {
         TileRegs<bf16_t, ITEMS> R;
-        tile_load<bf16_t, kEngBS, ITEMS>(R, W.ci, (const bf16_t*)W.val, W.b0, W.b1);
-        eng_tile<bf16_t, ITEMS>(W, v, R, sm, red, [] {});
+        tile_load<bf16_t, BS, ITEMS>(R, W.ci, (const bf16_t*)W.val, W.b0, W.b1);
+        eng_tile<bf16_t, BS, ITEMS>(W, v, R, sm, red, [] {});
     } else {
         TileRegs<float, ITEMS> R;
-        tile_load<float, kEngBS, ITEMS>(R, W.ci, (const float*)W.val, W.b0, W.b1);
-        eng_tile<float, ITEMS>(W, v, R, sm, red, [] {});
+        tile_load<float, BS, ITEMS>(R, W.ci, (const float*)W.val, W.b0, W.b1);
+        eng_tile<float, BS, ITEMS>(W, v, R, sm, red, [] {});
     }
 }
 
@@ -255,12 +263,12 @@ __global__ __launch_bounds__(kEngBS, 8) void k_eng_tiles_mixed(const EWork* __re
 // its own XCD).  The next entry is read while the current tile is staged,
 // and its col_ind/value loads are issued right after the staging barrier, so
 // they are in flight while the current tile is computed.
-template <typename VT, int ITEMS>
-__global__ __launch_bounds__(kEngBS) void k_eng_tiles_p(const EWork* __restrict__ work, const EJob* __restrict__ jobs,
+template <typename VT, int BS, int ITEMS>
+__global__ __launch_bounds__(BS) void k_eng_tiles_p(const EWork* __restrict__ work, const EJob* __restrict__ jobs,
                                                         const EState* __restrict__ st, const ECtl* __restrict__ ctl) {
     using X = typename Arith<VT>::X;
     using Acc = typename Arith<VT>::A;
-    __shared__ MergeTileSmem<Acc, kEngBS, ITEMS> sm;
+    __shared__ MergeTileSmem<Acc, BS, ITEMS> sm;
     __shared__ double red[48];
     const int nw = ctl->n_work;
     const int Gs = gridDim.x;
@@ -268,7 +276,7 @@ __global__ __launch_bounds__(kEngBS) void k_eng_tiles_p(const EWork* __restrict_
     if (e >= nw) return;
     EWork W = work[e];
     TileRegs<VT, ITEMS> R;
-    if (W.slot >= 0) tile_load<VT, kEngBS, ITEMS>(R, W.ci, (const VT*)W.val, W.b0, W.b1);
+    if (W.slot >= 0) tile_load<VT, BS, ITEMS>(R, W.ci, (const VT*)W.val, W.b0, W.b1);
     for (;;) {
         const int en = e + Gs;
         EWork Wn;
@@ -276,11 +284,11 @@ __global__ __launch_bounds__(kEngBS) void k_eng_tiles_p(const EWork* __restrict_
         if (en < nw) Wn = work[en];
         EView<X> v;
         if (eng_view(jobs, st, W.slot, v)) {
-            eng_tile<VT, ITEMS>(W, v, R, sm, red, [&] {
-                if (Wn.slot >= 0) tile_load<VT, kEngBS, ITEMS>(R, Wn.ci, (const VT*)Wn.val, Wn.b0, Wn.b1);
+            eng_tile<VT, BS, ITEMS>(W, v, R, sm, red, [&] {
+                if (Wn.slot >= 0) tile_load<VT, BS, ITEMS>(R, Wn.ci, (const VT*)Wn.val, Wn.b0, Wn.b1);
             });
         } else if (Wn.slot >= 0) {
-            tile_load<VT, kEngBS, ITEMS>(R, Wn.ci, (const VT*)Wn.val, Wn.b0, Wn.b1);
+            tile_load<VT, BS, ITEMS>(R, Wn.ci, (const VT*)Wn.val, Wn.b0, Wn.b1);
         }
         if (en >= nw) break;
         e = en;
@@ -383,34 +391,35 @@ __global__ __launch_bounds__(kFinBS) void k_eng_finish(EArgs a) {
     }
 }
 
-template <typename VT, int ITEMS>
+template <typename VT, int BS, int ITEMS>
 static hipError_t step_t(const EArgs& a, int gw, int gp, int gs, hipStream_t s) {
     if (gp > 0)
-        hipLaunchKernelGGL((k_eng_tiles_p<VT, ITEMS>), dim3(gp), dim3(kEngBS), 0, s, a.work, a.jobs,
+        hipLaunchKernelGGL((k_eng_tiles_p<VT, BS, ITEMS>), dim3(gp), dim3(BS), 0, s, a.work, a.jobs,
                            (const EState*)a.st, a.ctl);
     else
-        hipLaunchKernelGGL((k_eng_tiles<VT, ITEMS>), dim3(gw), dim3(kEngBS), 0, s, a.work, a.jobs,
+        hipLaunchKernelGGL((k_eng_tiles<VT, BS, ITEMS>), dim3(gw), dim3(BS), 0, s, a.work, a.jobs,
                            (const EState*)a.st, a.ctl);
     hipLaunchKernelGGL((k_eng_finish<VT>), dim3(gs), dim3(kFinBS), 0, s, a);
     return hipGetLastError();
 }
 
-template <typename VT, int ITEMS>
+template <typename VT, int BS, int ITEMS>
 static int resident_t() {
     int per_cu = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eng_tiles_p<VT, ITEMS>, kEngBS, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_eng_tiles_p<VT, BS, ITEMS>, BS, 0) != hipSuccess)
         return 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     return per_cu * cus / 8 * 8;
 }
 
+// Threads and items per thread of a 256 x ipt tile: see k_eng_tiles.
 template <typename VT>
 static hipError_t step_v(const EArgs& a, int ipt, int gw, int gp, int gs, hipStream_t s) {
     switch (ipt) {
-        case 4: return step_t<VT, 4>(a, gw, gp, gs, s);
-        case 8: return step_t<VT, 8>(a, gw, gp, gs, s);
-        case 16: return step_t<VT, 16>(a, gw, gp, gs, s);
+        case 4: return step_t<VT, 256, 4>(a, gw, gp, gs, s);
+        case 8: return step_t<VT, 256, 8>(a, gw, gp, gs, s);
+        case 16: return step_t<VT, 512, 8>(a, gw, gp, gs, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -418,16 +427,16 @@ static hipError_t step_v(const EArgs& a, int ipt, int gw, int gp, int gs, hipStr
 template <typename VT>
 static int resident_v(int ipt) {
     switch (ipt) {
-        case 4: return resident_t<VT, 4>();
-        case 8: return resident_t<VT, 8>();
-        case 16: return resident_t<VT, 16>();
+        case 4: return resident_t<VT, 256, 4>();
+        case 8: return resident_t<VT, 256, 8>();
+        case 16: return resident_t<VT, 512, 8>();
         default: return 0;
     }
 }
 
-template <int ITEMS>
+template <int BS, int ITEMS>
 static hipError_t step_mixed(const EArgs& a, int gw, int gs, hipStream_t s) {
-    hipLaunchKernelGGL((k_eng_tiles_mixed<ITEMS>), dim3(gw), dim3(kEngBS), 0, s, a.work, a.jobs, (const EState*)a.st,
+    hipLaunchKernelGGL((k_eng_tiles_mixed<BS, ITEMS>), dim3(gw), dim3(BS), 0, s, a.work, a.jobs, (const EState*)a.st,
                        a.ctl);
     hipLaunchKernelGGL((k_eng_finish<float>), dim3(gs), dim3(kFinBS), 0, s, a);
     return hipGetLastError();
@@ -436,9 +445,9 @@ static hipError_t step_mixed(const EArgs& a, int gw, int gs, hipStream_t s) {
 hipError_t engine_step(const EArgs& a, int vtype, int ipt, int gw, int gp, int gs, hipStream_t s) {
     if (vtype == VT_MIXED16) {  // no persistent variant
         switch (ipt) {
-            case 4: return step_mixed<4>(a, gw, gs, s);
-            case 8: return step_mixed<8>(a, gw, gs, s);
-            case 16: return step_mixed<16>(a, gw, gs, s);
+            case 4: return step_mixed<256, 4>(a, gw, gs, s);
+            case 8: return step_mixed<256, 8>(a, gw, gs, s);
+            case 16: return step_mixed<512, 8>(a, gw, gs, s);
             default: return hipErrorInvalidValue;
         }
     }

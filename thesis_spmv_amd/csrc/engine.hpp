@@ -102,7 +102,7 @@ struct EArgs {
     const ECtl* ctl;
 };
 
-constexpr int kEngBS = 256;
+constexpr int kEngBS = 256;  // a tile holds kEngBS * items_per_thread merge items
 // Engine value type for FP32 vectors with per-job FP32 or BF16 values
 // (EJob::vt16), beside VT_F64 / VT_F32 / VT_BF16.
 constexpr int VT_MIXED16 = 3;
