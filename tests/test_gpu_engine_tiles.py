@@ -1,5 +1,5 @@
 """The batch engine's tiles of 256 x 16 merge items, run by 512 threads of 8
-items each: instances whose items end just before, at and after a tile, rows
+items each (FP64: 256 of 16): instances whose items end just before, at and after a tile, rows
 around the 64 entries up to which a tile is summed row by row, and rows around
 the 1024 entries from which a tile's cut may split them.
 

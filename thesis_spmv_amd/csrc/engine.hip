@@ -209,14 +209,23 @@ __device__ __forceinline__ void eng_tile(const EWork& W, const EView<typename Ar
 // They are compiled for 8 waves per SIMD (8 FP32 items per thread: 62
 // instead of 68 VGPRs), which keeps more tiles in flight when few jobs are
 // left in a solve.
-// A thread takes at most 8 items: what bounds the step is gathers in flight,
-// and 16 items per thread need the registers of 4 FP32 waves per SIMD (3 FP64),
-// where 512 threads of 8 on the same tile run 8 (4 FP64).  24 FP32 instances
-// of up to 300 000 rows, 100 steps: 11 840 -> 10 270 us, with BF16 values
-// where exact 12 090 -> 10 720; 22 of up to 6 435 rows, 45 steps: 708 -> 588; 24
-// FP64 of up to 300 000 rows, 50 steps: 8 170 -> 8 110; 4 of up to 5 000: 820 -> 682.
-// (1024 threads of 4 items are held to 64 registers and spill: three to six
-// times slower on the large batches.)
+// Tiles of 256 x 16 FP32 items are run by 512 threads of 8 items: what bounds
+// the step is gathers in flight, and 16 items per thread need the registers of
+// 4 waves per SIMD, where 512 threads of 8 on the same tile run 8.  24
+// instances of up to 300 000 rows, 100 steps: 11 840 -> 10 280 us, with BF16
+// values where exact 12 060 -> 10 670; 22 of up to 6 435 rows, 45 steps: 709 ->
+// 597.  Only many large grids, which stream, lose a little: 256 Poisson grids
+// of sides up to 1024, a step: 892 -> 899 us in FP32, 871 -> 898 in BF16.
+// In FP64 two workgroups of 512 fit a CU against three of 256, and the same
+// grids take 1 486 us a step against 1 301: 256 threads of 16 there.  (1024
+// threads of 4 items are held to 64 registers and spill: three to six times
+// slower on the large batches.)
+template <typename VT>
+struct Tile16 {
+    static constexpr int threads = sizeof(typename Arith<VT>::A) == 8 ? 256 : 512;
+    static constexpr int items = kEngBS * 16 / threads;
+};
+
 template <typename VT, int BS, int ITEMS>
 __global__ __launch_bounds__(BS, 8) void k_eng_tiles(const EWork* __restrict__ work, const EJob* __restrict__ jobs,
                                                       const EState* __restrict__ st, const ECtl* __restrict__ ctl) {
@@ -413,13 +422,12 @@ static int resident_t() {
     return per_cu * cus / 8 * 8;
 }
 
-// Threads and items per thread of a 256 x ipt tile: see k_eng_tiles.
 template <typename VT>
 static hipError_t step_v(const EArgs& a, int ipt, int gw, int gp, int gs, hipStream_t s) {
     switch (ipt) {
         case 4: return step_t<VT, 256, 4>(a, gw, gp, gs, s);
         case 8: return step_t<VT, 256, 8>(a, gw, gp, gs, s);
-        case 16: return step_t<VT, 512, 8>(a, gw, gp, gs, s);
+        case 16: return step_t<VT, Tile16<VT>::threads, Tile16<VT>::items>(a, gw, gp, gs, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -429,7 +437,7 @@ static int resident_v(int ipt) {
     switch (ipt) {
         case 4: return resident_t<VT, 256, 4>();
         case 8: return resident_t<VT, 256, 8>();
-        case 16: return resident_t<VT, 512, 8>();
+        case 16: return resident_t<VT, Tile16<VT>::threads, Tile16<VT>::items>();
         default: return 0;
     }
 }
@@ -447,7 +455,7 @@ hipError_t engine_step(const EArgs& a, int vtype, int ipt, int gw, int gp, int g
         switch (ipt) {
             case 4: return step_mixed<256, 4>(a, gw, gs, s);
             case 8: return step_mixed<256, 8>(a, gw, gs, s);
-            case 16: return step_mixed<512, 8>(a, gw, gs, s);
+            case 16: return step_mixed<Tile16<float>::threads, Tile16<float>::items>(a, gw, gs, s);
             default: return hipErrorInvalidValue;
         }
     }
