@@ -528,10 +528,10 @@ static CrsDev crs_of(const pwm_matrix* h) {
 }
 
 // The CRS arrays the one-workgroup power method reads: the handle's own, or
-// the copy a blocked format keeps of a small matrix.
+// those a blocked format keeps of a small matrix.
 static CrsDev small_crs_of(const pwm_matrix* h) {
     CrsDev A = crs_of(h);
-    if (h->format == PWM_FORMAT_CSB || h->format == PWM_FORMAT_BLOCKCOH) {
+    if (h->sm_rs.p) {
         A.rs = h->sm_rs.as<int32_t>();
         A.ci = h->sm_ci.as<int32_t>();
         A.val = h->sm_val.p;
@@ -1230,32 +1230,10 @@ static void reset_matrix(pwm_matrix* h) {
     h->sm_val.release();
 }
 
-// A blocked format drops the CRS arrays once it is built; the one-workgroup
-// power method of a small matrix keeps its own copy (at most 200 KB).
-static int keep_small_crs(pwm_matrix* h) {
-    const size_t vb = value_size(h->vtype);
-    hipError_t e;
-    if ((e = h->sm_rs.alloc((h->nor + 1) * 4)) != hipSuccess ||
-        (e = h->sm_ci.alloc(std::max<int64_t>(h->nnz, 1) * 4)) != hipSuccess ||
-        (e = h->sm_val.alloc(std::max<int64_t>(h->nnz, 1) * vb)) != hipSuccess)
-        return hip_fail(h, e, "small-matrix copy");
-    e = hipMemcpyAsync(h->sm_rs.p, h->rs.p, (h->nor + 1) * 4, hipMemcpyDeviceToDevice, h->stream);
-    if (e == hipSuccess && h->nnz)
-        e = hipMemcpyAsync(h->sm_ci.p, h->ci.p, h->nnz * 4, hipMemcpyDeviceToDevice, h->stream);
-    if (e == hipSuccess && h->nnz)
-        e = hipMemcpyAsync(h->sm_val.p, h->val.p, h->nnz * vb, hipMemcpyDeviceToDevice, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);  // before the build frees the originals
-    if (e != hipSuccess) return hip_fail(h, e, "small-matrix copy");
-    return PWM_OK;
-}
-
 static int finish_load(pwm_matrix* h, const int32_t* hrs, const int32_t* hci, const double* hval) {
     int rc = compute_matrix_stats(h);
     if (rc != PWM_OK) return rc;
     h->power_small = wants_power_small(h);
-    if (h->power_small && (h->format == PWM_FORMAT_CSB || h->format == PWM_FORMAT_BLOCKCOH) &&
-        (rc = keep_small_crs(h)) != PWM_OK)
-        return rc;
     switch (h->format) {
         case PWM_FORMAT_CRS: rc = plan_crs(h); break;
         case PWM_FORMAT_CRS_MERGE: rc = plan_merge(h); break;

@@ -235,7 +235,7 @@ struct pwm_matrix {
     pwm_impl::CohDev coh;
 
     // small matrices: the power loop runs in one workgroup (k_power.hip); the
-    // blocked formats keep a copy of their CRS arrays for it
+    // blocked formats keep their CRS arrays for it (at most 200 KB)
     bool power_small = false;
     pwm_impl::DevBuf sm_rs, sm_ci, sm_val;
 
@@ -323,6 +323,9 @@ size_t vector_size(int vtype);
 // per-format planning after the CRS arrays are on the device
 int plan_crs(pwm_matrix* h);
 int plan_merge(pwm_matrix* h);
+// A blocked format drops the CRS arrays once it is built; those of a small matrix
+// stay for its power method.
+void drop_crs(pwm_matrix* h);
 int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals);
 int build_blockcoh(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals);
 // one SpMV of the loaded format on device vectors; pw != nullptr: power step

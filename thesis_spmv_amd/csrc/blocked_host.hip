@@ -228,6 +228,17 @@ int build_swept_beside_crs(pwm_matrix* h) {
     return rc == PWM_ERR_UNSUPPORTED || rc == PWM_ERR_NOMEM ? PWM_OK : rc;
 }
 
+void drop_crs(pwm_matrix* h) {
+    if (h->power_small) {
+        h->sm_rs.swap(h->rs);
+        h->sm_ci.swap(h->ci);
+        h->sm_val.swap(h->val);
+    }
+    h->rs.release();
+    h->ci.release();
+    h->val.release();
+}
+
 // rs: host row_start; ci / vals: host CRS arrays, or NULL (values already
 // validated for the storage type) -- they are then downloaded only if the
 // host-built slab-piece layout is used.
@@ -298,9 +309,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
         if (rc == PWM_OK) {
             if (h->csb_layout == 4) {
                 // the CRS arrays are not needed by the CSB kernels
-                h->rs.release();
-                h->ci.release();
-                h->val.release();
+                drop_crs(h);
                 return PWM_OK;
             }
             if ((rc = time_csb(h, &swept_ms)) != PWM_OK) return rc;
@@ -510,9 +519,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
         }
     }
     // the CRS arrays are not needed by the CSB kernels
-    h->rs.release();
-    h->ci.release();
-    h->val.release();
+    drop_crs(h);
     return PWM_OK;
 }
 
@@ -778,9 +785,7 @@ static int build_blockcoh_layout(pwm_matrix* h, const int32_t* rs, const int32_t
     rc = upload_blocked_values(h, c.data, data);
     if (rc != PWM_OK) return rc;
     c.n_tasks = (int64_t)tasks.size();
-    h->rs.release();
-    h->ci.release();
-    h->val.release();
+    drop_crs(h);
     return PWM_OK;
 }
 

@@ -395,9 +395,7 @@ int coh_layout_device(pwm_matrix* h, int64_t lds_rows) {
                            c.tasks.as<int32_t>());
     if ((e = hipGetLastError()) == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "BlockCOH step tables");
-    h->rs.release();
-    h->ci.release();
-    h->val.release();
+    drop_crs(h);
     return PWM_OK;
 }
 
