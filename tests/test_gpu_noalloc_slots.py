@@ -1,0 +1,29 @@
+"""Matrices near the partial-sum slots of the no-allocation power method's fixed
+workspace (PWM_NOALLOC_MAX_SLOTS) stay within them.
+
+CRS_MERGE, rows of 60 entries: a slot of the merge kernels is a tile of 2048
+merge items, 208 496 slots for the 420 M entries here; the wave tiles that such
+rows take must not need more than the workspace holds."""
+import numpy as np
+import pytest
+
+pw = pytest.importorskip("thesis_spmv_amd")
+pytestmark = pytest.mark.gpu
+
+
+def test_short_rows():
+    n, L = 7_000_000, 60
+    ci = (np.minimum(np.arange(n), n - L)[:, None] + np.arange(L)).astype(np.int32).ravel()
+    rs = (np.arange(n + 1, dtype=np.int64) * L).astype(np.int32)
+    m = pw.CRSMergeHip(values="f32")
+    m.loadCRS(n, n, rs, ci, np.ones(n * L))
+    assert m.info()["kernels"] == 1  # the wave tiles
+    x, y = (pw.DeviceVector(n, np.float32) for _ in range(2))
+    x.fill(1.0)
+    lam, norm, k = m.power_method_device_noalloc(x, y, 1)
+    # every row sums to 60; one rounding of the norm's square root
+    assert k == 1 and lam == 60.0 and abs(norm - 60.0 * np.sqrt(n)) <= 2.0 ** -52 * norm
+    ref = (x.download(), y.download())
+    x.fill(1.0)
+    assert (lam, norm, k) == m.power_method_device(x, y, 1)
+    assert np.array_equal(x.download(), ref[0]) and np.array_equal(y.download(), ref[1])

@@ -19,6 +19,7 @@
 // plain read reaches 6.1).  1024 x 1024 over three copies: 16.0 -> 13.7 us.
 // Two groups per lane (339 us), two or more tiles per wave with the next one's
 // loads in flight (353 us) and resident waves (412 us) are slower.
+#include "../../include/pwm_hip.h"
 #include "kernels.hpp"
 #include "merge_tile.hpp"
 
@@ -33,9 +34,13 @@ constexpr int kRwBS = 64;         // threads per block of an SpMV
 // Threads per block of a power step, one partial-sum slot a block: 256 (FP32
 // 3000 x 3000: 92.7 us a step against 99.9 with 512, 100 x 100 4.2 against
 // 4.7), but 512 where that brings the slots down to what the next step adds up
-// itself (k_power.hip; FP64 600 x 600: 11.1 -> 8.5 us) and, for the largest, to
-// 200 000, which the fixed workspace of the no-allocation power method holds.
+// itself (k_power.hip; FP64 600 x 600: 11.1 -> 8.5 us) or to 200 000, and 1024
+// where 512 leave more slots than the fixed workspace of the no-allocation power
+// method holds: 16 tiles a block are at least 3040 entries, more than the 2048
+// merge items a slot of CRS_MERGE's merge kernels stands for, so it takes every
+// matrix here that it takes there.
 static int rows_power_bs(int64_t nt) {
+    if ((nt + 7) / 8 > PWM_NOALLOC_MAX_SLOTS) return 1024;
     return (nt > 2048 && (nt + 7) / 8 <= kDeferSlots) || (nt + 3) / 4 > 200000 ? 512 : 256;
 }
 
@@ -200,10 +205,13 @@ template <typename VT>
 static hipError_t launch_rows_t(const CrsDev& A, const RowsPlan& rp, const void* x, void* y, const PowerArgs* pw,
                                 hipStream_t s) {
     using X = typename Arith<VT>::X;
-    if (pw && rows_power_bs(rp.nt) == 256)
+    const int bs = pw ? rows_power_bs(rp.nt) : 0;
+    if (bs == 256)
         launch_rows_power<VT, 256>(A, rp, *pw, s);
-    else if (pw)
+    else if (bs == 512)
         launch_rows_power<VT, 512>(A, rp, *pw, s);
+    else if (bs == 1024)
+        launch_rows_power<VT, 1024>(A, rp, *pw, s);
     else
         hipLaunchKernelGGL((A.nt ? k_rows<VT, kRwBS, 0, true> : k_rows<VT, kRwBS, 0, false>),
                            dim3((unsigned)((rp.nt + kRwBS / 64 - 1) / (kRwBS / 64))), dim3(kRwBS), 0, s, A, rp,
