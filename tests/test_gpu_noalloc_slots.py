@@ -3,7 +3,10 @@ workspace (PWM_NOALLOC_MAX_SLOTS) stay within them.
 
 CRS_MERGE, rows of 60 entries: a slot of the merge kernels is a tile of 2048
 merge items, 208 496 slots for the 420 M entries here; the wave tiles that such
-rows take must not need more than the workspace holds."""
+rows take must not need more than the workspace holds.
+
+BlockCOH in one band: 32 768 entries a task would make 23 463 slots of the 769 M
+entries here; tasks of 4096 entries and pieces of 2048 rows make 263 K."""
 import numpy as np
 import pytest
 
@@ -27,3 +30,18 @@ def test_short_rows():
     x.fill(1.0)
     assert (lam, norm, k) == m.power_method_device(x, y, 1)
     assert np.array_equal(x.download(), ref[0]) and np.array_equal(y.download(), ref[1])
+
+
+def test_one_band():
+    m, n = 12400, 12400
+    A = pw.BlockCOHHip(1, "bf16")
+    A.generatePoissonMatrix(m, n)
+    assert A.info()["threads"] == 1
+    x, y = (pw.DeviceVector(m * n, np.float32) for _ in range(2))
+    x.fill(1.0)
+    lam, norm, k = A.power_method_device_noalloc(x, y, 1)
+    # A 1 is the number of missing neighbours: 1 on the edges, 2 in the corners
+    assert k == 1 and lam == 2.0 * (m + n) / (m * n)
+    assert abs(norm ** 2 - (2 * (m + n - 4) + 16)) <= 1e-12 * norm ** 2
+    g = y.download().reshape(n, m)  # divided by its norm: the power method's result
+    assert not g[1:-1, 1:-1].any() and np.allclose(g[0, 1:-1] * norm, 1.0, rtol=1e-6)

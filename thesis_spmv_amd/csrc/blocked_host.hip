@@ -565,38 +565,64 @@ static void coh_bands(int64_t nor, int64_t nnz, const int32_t* rs, int threads, 
 
 // Work list: one LDS task per band whose rows fit the LDS window and whose
 // entries fit one task (and are not many times the others'), atomic tasks of
-// kCohAtomicSteps steps otherwise.
+// kCohAtomicSteps steps otherwise, whose rows are finished in pieces of
+// kCohPieceRows.
 void coh_plan_tasks(const std::vector<CohBandMeta>& B, int64_t lds_rows, std::vector<blocked::CohTask>& tasks,
                     std::vector<blocked::CohRows>& pieces, std::vector<blocked::CohBand>& table,
                     int32_t* max_lds_rows) {
-    tasks.clear();
-    pieces.clear();
     // What one workgroup may be left with: a band closes before the row that
     // would exceed its share, so the last band holds what the others left, on
     // power-law rows 3 to 20 times their size (100 K rows: 18 us with that band
     // cut, 25 without; 500 K: 64 and 69).
-    int32_t sum = 0;
+    constexpr int64_t kTask = blocked::kCohTaskSteps * (int64_t)blocked::kCohStep;
     int64_t nnz = 0;
     for (const CohBandMeta& m : B) nnz += m.nnz;
-    const int64_t most = std::min<int64_t>(blocked::kCohTaskSteps * (int64_t)blocked::kCohStep,
-                                           std::max<int64_t>(8192, 2 * nnz / std::max<int64_t>(1, (int64_t)B.size())));
+    const int64_t cut = std::min(kTask, std::max<int64_t>(8192, 2 * nnz / std::max<int64_t>(1, (int64_t)B.size())));
+    int64_t most = cut, steps = blocked::kCohAtomicSteps, rows = blocked::kCohPieceRows;
+    auto in_lds = [&](const CohBandMeta& m) { return m.rows <= lds_rows && m.nnz <= most; };
+    auto slots = [&] {
+        int64_t n = 0;
+        for (const CohBandMeta& m : B)
+            n += in_lds(m) ? m.rows > 0
+                           : (blocked::coh_steps(m.off_nz, m.nnz) + steps - 1) / steps + (m.rows + rows - 1) / rows;
+        return n;
+    };
+    // Each task and each piece has a partial-sum slot in a power step.  Beyond
+    // what the no-allocation power method's workspace holds, tasks and pieces
+    // grow, and at the last fewer bands are cut (500 K power-law rows: 88 us with
+    // atomic tasks of 32 steps, 84 with 16, 145 with 128).
+    while (slots() > PWM_NOALLOC_MAX_SLOTS && rows < (int64_t)1 << 30) {
+        rows *= 2;
+        if (steps < blocked::kCohTaskSteps)
+            steps *= 2;
+        else
+            most = kTask;
+    }
+    if (slots() > PWM_NOALLOC_MAX_SLOTS) {  // too many bands for it in any case
+        most = cut;
+        steps = blocked::kCohAtomicSteps;
+        rows = blocked::kCohPieceRows;
+    }
+    tasks.clear();
+    pieces.clear();
+    int32_t sum = 0;
     *max_lds_rows = 0;
     for (int p = 0; p < (int)B.size(); ++p) {
         const CohBandMeta& m = B[p];
-        const int64_t steps = blocked::coh_steps(m.off_nz, m.nnz);
-        if (m.rows <= lds_rows && m.nnz <= most) {
-            if (m.rows > 0) tasks.push_back({p, 0, (int32_t)steps, 0});
+        const int64_t n_steps = blocked::coh_steps(m.off_nz, m.nnz);
+        if (in_lds(m)) {
+            if (m.rows > 0) tasks.push_back({p, 0, (int32_t)n_steps, 0});
             *max_lds_rows = std::max(*max_lds_rows, (int32_t)m.rows);
             continue;
         }
         table[p].sum = sum;
-        for (int64_t r = 0; r < m.rows; r += blocked::kCohPieceRows) {
-            const int32_t n = (int32_t)std::min<int64_t>(blocked::kCohPieceRows, m.rows - r);
+        for (int64_t r = 0; r < m.rows; r += rows) {
+            const int32_t n = (int32_t)std::min<int64_t>(rows, m.rows - r);
             pieces.push_back({(int32_t)(m.start + r), n, sum});
             sum += n;
         }
-        for (int64_t s0 = 0; s0 < steps; s0 += blocked::kCohAtomicSteps)
-            tasks.push_back({p, (int32_t)s0, (int32_t)std::min<int64_t>(blocked::kCohAtomicSteps, steps - s0), 1});
+        for (int64_t s0 = 0; s0 < n_steps; s0 += steps)
+            tasks.push_back({p, (int32_t)s0, (int32_t)std::min<int64_t>(steps, n_steps - s0), 1});
     }
 }
 
