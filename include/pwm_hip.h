@@ -79,7 +79,7 @@ typedef struct {
     int32_t non_temporal;      /* CSB slab streams / CRS tiles: 1 = non-temporal entry loads */
     int32_t layout;            /* CSB: 1 slab pieces, 2 slab streams, 3 wide slab streams, 4 swept slabs */
     int32_t kernels;           /* kernel launches of one pwm_mv_device */
-    int32_t high_occupancy;    /* BlockCOH: 0 with the option coh_occ8 = 0, else 1 */
+    int32_t high_occupancy;    /* BlockCOH: 1 when workgroups of 8 waves run, 0 when waves run on their own */
 } pwm_info_t;
 
 /* Constructor SparseMatrix(int threads) (Matrix/SparseMatrix.hpp:30) through
@@ -174,9 +174,10 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * "csb_build" (CSB slab-piece layout built on the device, 0, or on the host,
  * 1; both give the same arrays; the slab streams are always built on the
  * device), "coh_build" (BlockCOH layout built on the device, 0, or on the
- * host, 1; both give the same arrays), "coh_occ8" (-1, 0 or 1, reported
- * as high_occupancy, -1 as 1; one BlockCOH kernel, at 8 waves per SIMD,
- * serves all three), "crs_kernel" (CRS: 0 = one wave per tile of short
+ * host, 1; both give the same arrays), "coh_occ8" (BlockCOH: 1 = a
+ * workgroup of 8 waves per task, 0 = one wave per task, -1 = 8 waves, or the
+ * faster of the two in a load-time timing where the columns are scattered over
+ * more than 10 MB of x, the default), "crs_kernel" (CRS: 0 = one wave per tile of short
  * rows when no row has more than 64 entries, else time the vector kernel at
  * three lane counts and the row-aligned tiles kernel at load and keep the
  * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =

@@ -1153,7 +1153,7 @@ extern "C" int pwm_set_option(pwm_matrix* h, const char* key, int64_t value) {
         if (value < 1 || value > 8) return fail(h, PWM_ERR_INVALID, "csb_sweep_waves must be 1..8");
         h->csb_sweep_waves = (int32_t)value;
     } else if (k == "coh_occ8") {
-        if (value < -1 || value > 1) return fail(h, PWM_ERR_INVALID, "coh_occ8 must be -1 (timed), 0 or 1");
+        if (value < -1 || value > 1) return fail(h, PWM_ERR_INVALID, "coh_occ8 must be -1 (automatic), 0 or 1");
         h->coh_occ8 = (int32_t)value;
     } else if (k == "csb_unroll") {
         if (value != 0 && value != 2 && value != 4) return fail(h, PWM_ERR_INVALID, "csb_unroll must be 0, 2 or 4");
@@ -1443,7 +1443,7 @@ extern "C" int pwm_info(const pwm_matrix* h, pwm_info_t* out) {
     }
     if (swept_crs(h)) out->kernels = 1;
     if (h->format == PWM_FORMAT_CSB && h->csb.n_tasks <= 0) out->kernels = 0;
-    out->high_occupancy = h->format == PWM_FORMAT_BLOCKCOH ? h->coh.occ8 : 0;
+    out->high_occupancy = h->format == PWM_FORMAT_BLOCKCOH ? !h->coh.one_wave : 0;
     out->non_temporal = h->format == PWM_FORMAT_CSB || swept_crs(h)         ? h->csb.nt
                         : (h->format == PWM_FORMAT_CRS && h->crs_used == 2) || h->crs_used == 3 ? h->crs_nt_used
                                                                            : 0;

@@ -159,8 +159,7 @@ struct CohDev {
     DevBuf ysum;           // their sums
     int64_t n_tasks = 0, total_blocks = 0, n_pieces = 0;
     int32_t lds_rows = 0;  // rows of the largest band accumulated in LDS (the kernel's LDS window)
-    int32_t one_wave = 0;  // tasks of one wave each
-    int32_t occ8 = 0;      // reported: 8 waves per SIMD unless the option coh_occ8 says 0
+    int32_t one_wave = 0;  // tasks of one wave each (else workgroups of 8)
     void clear() {
         bands.clear();
         for (DevBuf* b : {&ent, &data, &row_jump_block, &col_jump_block, &block_nnz, &block_coords, &band_table, &tasks, &task_list, &row_pieces,
@@ -168,7 +167,7 @@ struct CohDev {
             b->release();
         n_tasks = total_blocks = n_pieces = 0;
         lds_rows = 0;
-        occ8 = one_wave = 0;
+        one_wave = 0;
     }
 };
 
@@ -226,7 +225,7 @@ struct pwm_matrix {
     int32_t csb_sweep_unroll = 2; // swept slabs: groups of 4 entries per lane per chunk (1, 2 or 4)
     int32_t csb_sweep_waves = 1;  // swept slabs: slabs per CU (workgroups run in that many waves)
     int32_t csb_sweep_order = 1;  // swept slabs: 0 = rows inside a window's run, 1 = columns (lanes share x lines)
-    int32_t coh_occ8 = -1;        // BlockCOH: reported as high_occupancy (-1 or 1: yes); one kernel serves all
+    int32_t coh_occ8 = -1;        // BlockCOH tasks: 1 = workgroups of 8 waves, 0 = one wave, -1 = by rule and timing
     int32_t csb_unroll = 0;  // stream kernel groups of 4 per thread per step (0 = default)
     int32_t csb_nt = -1;     // slab streams: non-temporal entry loads / partial stores (-1 = timed)
     int32_t csb_build = 0;   // CSB slab pieces: 0 = built on the device, 1 = on the host

@@ -882,22 +882,49 @@ hipError_t coh_launch(pwm_matrix* h, const void* x, void* y, const pwmk::PowerAr
     return e;
 }
 
-// The BlockCOH layout, and whether its tasks run one wave each: more than 128
-// lines of x per 256 entries, x beyond 10 MB and enough tasks for 4 waves per
-// CU.  Power-law rows, us with 8 waves and with one: FP64 1 M (8 MB of x) 129 147,
-// 2 M 282 263, 3 M 536 419, FP32 3 M (12 MB) 360 338; the 9-point stencil with 2
-// random entries per row (55 lines) on 2000^2 225 266.  The option coh_occ8 is
-// kept and reported; both instances run at 8 waves per SIMD.
+// Whether the tasks run one wave each (k_coh): the option coh_occ8 = 0 or 1 says
+// so (0: one wave); otherwise both are timed where one wave can win, with more
+// than 128 lines of x per 256 entries, x beyond 10 MB and enough tasks for 4 waves
+// per CU.  What decides there is not known from the sizes: a wave per band stays
+// within a few blocks of x, but 24 M entries are 1464 bands, and their LDS windows
+// let more (short ones, which crowd on some CUs) or fewer of them share a CU.
+// Rows of L random columns, 24 M entries, us with 8 waves and with one: FP64 L = 6
+// 281 195, 8 239 191, 12 197 184, 16 194 228; FP32 3 273 204, 6 173 128, 8 147 123.
+// Power-law rows: FP64 1 M (8 MB of x) 129 147, 2 M 282 263, 3 M 536 419, FP32
+// 3 M (12 MB) 360 338; the 9-point stencil with 2 random entries per row (55
+// lines) on 2000^2 225 266.
+static int choose_coh_waves(pwm_matrix* h, double lines) {
+    CohDev& c = h->coh;
+    c.one_wave = h->coh_occ8 == 0;
+    if (h->coh_occ8 >= 0 || lines <= 128.0 || h->noc * (int64_t)vector_size(h->vtype) <= ((int64_t)10 << 20) ||
+        c.n_tasks < 1024)
+        return PWM_OK;
+    DevBuf x, y;
+    const size_t vs = vector_size(h->vtype);
+    hipError_t e = x.alloc(h->noc * vs);
+    if (e == hipSuccess) e = y.alloc(h->nor * vs);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return PWM_OK;
+    }
+    if (e == hipSuccess) e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64, 1.0, h->stream);
+    float ms[2] = {0.0f, 0.0f};
+    for (int one = 0; one < 2 && e == hipSuccess; ++one) {
+        c.one_wave = one;
+        e = time_launches(h, [&] { return coh_launch(h, x.p, y.p, nullptr); }, &ms[one]);
+    }
+    if (e != hipSuccess) return hip_fail(h, e, "BlockCOH autotune");
+    c.one_wave = ms[1] < ms[0];
+    return PWM_OK;
+}
+
 int build_blockcoh(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double* vals) {
     double lines = 0.0;
     const hipError_t e = column_lines(h, &lines);
     if (e != hipSuccess) return hip_fail(h, e, "column lines");
-    const int rc = build_blockcoh_layout(h, rs, ci, vals);
-    if (rc != PWM_OK) return rc;
-    h->coh.occ8 = h->coh_occ8 != 0;
-    h->coh.one_wave = lines > 128.0 && h->noc * (int64_t)vector_size(h->vtype) > ((int64_t)10 << 20) &&
-                      h->coh.n_tasks >= 1024;
-    return PWM_OK;
+    int rc = build_blockcoh_layout(h, rs, ci, vals);
+    if (rc == PWM_OK) rc = choose_coh_waves(h, lines);
+    return rc;
 }
 
 }  // namespace pwm_impl

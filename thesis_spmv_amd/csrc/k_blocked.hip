@@ -587,10 +587,13 @@ int csb_sweep_blocks_per_cu(int vtype, int rows, bool acc32) {
 // of block starts before it: four ballots and a table of the blocks at the
 // steps.
 //
-// BS: 512, or 64 where x is far beyond an L2 and the columns are scattered
-// (blocked_host.hip): 8 waves that take a band's steps in turn are 2048 entries
-// apart, some 30 blocks, 4 MB of x; a wave per band keeps to a few blocks, the
-// bands of an XCD walk x in the same order and meet in its L2.
+// BS: 512, or 64 where that times faster at load (blocked_host.hip): 8 waves
+// that take a band's steps in turn are 2048 entries apart, on x far beyond an L2
+// and scattered columns some 30 blocks, 4 MB of x; a wave per band keeps to a few
+// blocks, the bands of an XCD walk x in the same order and meet in its L2.  Every
+// workgroup reserves the LDS window of the largest band whatever its size, so
+// waves on their own are as many per CU as their windows let in: 11 at 1542 rows,
+// 6 at 3084, 3 at 6168.
 //
 // Bound by the gathers (FP64 9-point stencil with 2 random entries per row, 1 M
 // rows: 215 G/s of the 213-233 G/s that the L2 serves) or, on a matrix of few
