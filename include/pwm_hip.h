@@ -56,9 +56,10 @@ extern "C" {
 
 /* ---- device storage precision of the matrix values ---------------------
  * F64: values and vectors FP64, FP64 accumulation (parity mode).
- * F32: values and vectors FP32, FP32 accumulation per row.
+ * F32: values, vectors and products FP32, a row's sum FP32 or FP64 by the
+ *       kernel.
  * BF16: values BF16 (accepted only when every value is exact in BF16, e.g.
- *       the Poisson stencil's 4/-1), vectors FP32, FP32 accumulation.
+ *       the Poisson stencil's 4/-1), vectors FP32, sums as for F32.
  * Norms, Rayleigh quotients and convergence tests are FP64 in every mode. */
 #define PWM_VALUES_F64  0
 #define PWM_VALUES_F32  1

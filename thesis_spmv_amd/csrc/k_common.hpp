@@ -129,6 +129,43 @@ __device__ __forceinline__ void block_sum3(double& a, double& b, double& c, doub
     c = tc;
 }
 
+// Sum of the products prod[k], prod[k + stride], ... below e, in LDS, by one lane
+// with four reads in flight.  FP64: left to right.  FP32 products are summed in
+// FP64, but 16 at a time as four FP32 sums of four, since the conversions and FP64
+// adds of a long row show (FP32 SpMV of rows of 64, us, all in FP64, so, and left
+// to right in FP32: 20 000 rows 7.4 6.6 6.8, 300 000 rows 84.2 83.4 83.9; Poisson
+// 3000 x 3000 84.9 86.7 84.8, 5000 x 5000 230 230 231; 100 power steps of one
+// workgroup at 37 x 29 195 195 190).  A left-to-right FP32 sum is less exact than
+// the lane trees of the vector and merge kernels: rms error over sum |a x| of a row
+// of 8 / 16 / 64 3.1e-8 / 3.0e-8 / 2.9e-8, there 2.5e-8 / 2.1e-8 / 1.3e-8 and
+// 2.9e-8 / 2.5e-8 / 1.5e-8; here 1.8e-8 / 2.0e-8 / 1.0e-8.
+template <typename Acc>
+__device__ __forceinline__ double row_sum(const Acc* prod, int k, int e, int stride) {
+    double sum = 0.0;
+    if constexpr (sizeof(Acc) == 4) {
+        for (; k + 15 * stride < e; k += 16 * stride) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const Acc* p = prod + k + 4 * u * stride;
+                sum += (double)((p[0] + p[stride]) + (p[2 * stride] + p[3 * stride]));
+            }
+        }
+    }
+    for (; k + 3 * stride < e; k += 4 * stride) {
+        const Acc p0 = prod[k], p1 = prod[k + stride], p2 = prod[k + 2 * stride], p3 = prod[k + 3 * stride];
+        if constexpr (sizeof(Acc) == 4) {
+            sum += ((double)p0 + (double)p1) + ((double)p2 + (double)p3);
+        } else {
+            sum += p0;
+            sum += p1;
+            sum += p2;
+            sum += p3;
+        }
+    }
+    for (; k < e; k += stride) sum += (double)prod[k];
+    return sum;
+}
+
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs, each
 // with its own 4 MB L2.  Renumber blocks so that XCD j works on the j-th
 // contiguous eighth of the work items: neighbouring rows (which share x

@@ -9,7 +9,7 @@
 // step's products in LDS, and a step is
 //   products   every thread multiplies its entries by x from LDS, products to
 //              LDS;                                                 barrier
-//   row sums   G lanes per row sum the row's products (G = 1: left to right),
+//   row sums   G lanes per row sum the row's products (row_sum, then the lanes'),
 //              scale, write the new iterate to LDS and add up |y|^2, x.y, x.x;
 //              wave sums to LDS;                                    barrier
 // so nothing but LDS is touched between the first load and the last store:
@@ -17,9 +17,9 @@
 // needed only in the next step's row sums: wave 0 computes the scale (an FP64
 // square root and division) while the others already multiply.
 //
-// The arithmetic is the general path's: products and row sums in the
-// accumulator type, out = sum / |y_previous| and the norms in FP64, every sum
-// in a fixed order.  A step takes 1.1 us at 10 x 10, 1.7 us at 37 x 29 (15.9
+// The arithmetic is the general path's: products in the accumulator type, row
+// sums (row_sum), out = sum / |y_previous| and the norms in FP64, every sum in a
+// fixed order.  A step takes 1.1 us at 10 x 10, 1.7 us at 37 x 29 (15.9
 // before) and 2.6 us at 52 x 51, FP64; 100 steps at 37 x 29 take 0.20 ms.
 #include <algorithm>
 
@@ -82,24 +82,11 @@ __global__ __launch_bounds__(kPsBS) void k_power_small(CrsDev A, int G, PowerArg
         double yy = 0.0, xy = 0.0, xx = 0.0;
         for (int r0 = 0; r0 < n; r0 += ngrp) {
             const int r = r0 + grp;
-            Acc s = 0;
-            if (r < n) {
-                // in order, four LDS reads in flight
-                const int e1 = rs[r + 1];
-                int e = rs[r] + gl;
-                for (; e + 3 * G < e1; e += 4 * G) {
-                    const Acc p0 = prod[e], p1 = prod[e + G], p2 = prod[e + 2 * G], p3 = prod[e + 3 * G];
-                    s += p0;
-                    s += p1;
-                    s += p2;
-                    s += p3;
-                }
-                for (; e < e1; e += G) s += prod[e];
-            }
+            double s = r < n ? row_sum(prod, rs[r] + gl, rs[r + 1], G) : 0.0;
             for (int off = 1; off < G; off <<= 1) s += __shfl_xor(s, off);
             if (gl == 0 && r < n) {
                 const double xd = (double)x[r] * scale;
-                const X out = (X)((double)s * scale);
+                const X out = (X)(s * scale);
                 y[r] = out;
                 const double yd = (double)out;
                 yy += yd * yd;

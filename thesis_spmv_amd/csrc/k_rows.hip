@@ -4,7 +4,7 @@
 // apart, moved up to the next row start, so that a tile is at most 256 entries
 // (one aligned group of 4 per lane of a wave) and 128 rows.  One wave a tile:
 // it loads its group with 128-bit loads, gathers x, leaves the products in its
-// own slice of LDS and sums the rows, a lane per row and left to right.  No
+// own slice of LDS and sums the rows, a lane per row (row_sum).  No
 // wave waits for another, the only chain is cut -> entries -> x, and the many
 // short waves keep enough loads in flight to run at the rate a plain read of
 // the arrays reaches.
@@ -138,21 +138,10 @@ __global__ __launch_bounds__(BS) void k_rows(CrsDev A, RowsPlan rp, const typena
         for (int s = 0; s < kRwSlots; ++s) {
             const int r = lane + 64 * s;
             if (r < nr) {
-                int k = beg[s] - off;
-                const int e = end[s] - off;
-                // left to right, four LDS reads in flight at a time
-                Acc sum = 0;
-                for (; k + 4 <= e; k += 4) {
-                    const Acc p0 = prod[k], p1 = prod[k + 1], p2 = prod[k + 2], p3 = prod[k + 3];
-                    sum += p0;
-                    sum += p1;
-                    sum += p2;
-                    sum += p3;
-                }
-                for (; k < e; ++k) sum += prod[k];
+                const double sum = row_sum(prod, beg[s] - off, end[s] - off, 1);
                 if constexpr (POWER) {
                     const double xd = (double)xr[s] * scale;
-                    const X out = (X)((double)sum * scale);
+                    const X out = (X)(sum * scale);
                     G(y)[a0 + r] = out;
                     const double yd = (double)out;
                     yy += yd * yd;
