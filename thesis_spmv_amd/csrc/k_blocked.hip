@@ -760,7 +760,9 @@ __global__ __launch_bounds__(kBS) void k_coh_finish(CohArgs a, typename Arith<VT
         const int64_t k = pw.k;
         x = (const X*)((k & 1) ? pw.buf1 : pw.buf0);
         y = (X*)((k & 1) ? pw.buf0 : pw.buf1);
-        scale = 1.0 / sqrt(pwmk::last_norm<kBS>(pw, red));
+        // with deferred norms k_coh, before this in the step, wrote the record: one
+        // scale for all rows (its blocks may add the slots up in another order)
+        scale = pwmk::recorded_scale(pw);
     }
     const CohRows piece = a.pieces[blockIdx.x];
     double yy = 0.0, xy = 0.0, xx = 0.0;

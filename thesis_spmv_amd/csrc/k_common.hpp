@@ -259,9 +259,10 @@ __device__ __forceinline__ void slot_sum(const double* slots, int64_t i0, int64_
 
 // |y_{k-1}|^2 (1 for the first step, which multiplies the caller's unnormalised
 // start vector; the step's output is divided by the root of it): from the record
-// of step k-1 or, deferred, from its slots, which every block adds up (in the
-// same order); block 0 then writes the record.  All BS threads of the block call
-// it; `scratch` holds >= 48 doubles.
+// of step k-1 or, deferred, from its slots, which every block of the kernel adds up
+// in the same order (BS decides it: a step's other kernels take the record); block 0
+// then writes the record.  All BS threads of the block call it; `scratch` holds >=
+// 48 doubles.
 template <int BS>
 __device__ __forceinline__ double last_norm(const PowerArgs& p, double* scratch) {
     if (p.prev_n == 0) return p.k == 0 ? 1.0 : p.rec[4 * (p.k - 1)];
