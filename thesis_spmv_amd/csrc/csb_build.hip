@@ -270,6 +270,8 @@ int csb_stream_device(pwm_matrix* h, int rb, int cb, int64_t S, bool wide) {
             e = hipMemcpyAsync(soff.data(), c.soff.p, cells * 4, hipMemcpyDeviceToHost, h->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         if (e != hipSuccess) return hip_fail(h, e, "CSB build");
+    } else if ((e = hipMemsetAsync(c.soff.p, 0, cells * 4, h->stream)) != hipSuccess) {
+        return hip_fail(h, e, "CSB build");
     }
     soff[cells] = (int32_t)nnz;
     // the stored order's blk_ptr: block (br, bc) holds the runs of its S slabs
