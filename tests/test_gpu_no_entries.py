@@ -1,5 +1,6 @@
 """Matrices without entries, and with long stretches of rows without any: y is
-written, with zeros."""
+written, with zeros, on every format (BlockCOH puts more empty rows than its LDS
+window holds into bands that have no task of their own)."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("values", ["f64", "f32"])
 @pytest.mark.parametrize("nor,full", [(4096, 0), (4097, 0), (8193, 0), (30000, 0), (30000, 5), (30000, 29995)])
-@pytest.mark.parametrize("cls,threads", [(pw.CRSHip, -1), (pw.CRSMergeHip, -1), (pw.CSBHip, -1)], ids=lambda v: getattr(v, "__name__", str(v)))
+@pytest.mark.parametrize("cls,threads", [(pw.CRSHip, -1), (pw.CRSMergeHip, -1), (pw.CSBHip, -1), (pw.BlockCOHHip, -1),
+                                         (pw.BlockCOHHip, 1)], ids=lambda v: getattr(v, "__name__", str(v)))
 def test_rows_without_entries(cls, threads, nor, full, values):
     noc = 700
     lens = np.zeros(nor, np.int64)

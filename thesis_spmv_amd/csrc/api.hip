@@ -1045,7 +1045,7 @@ static bool defers_norms(const pwm_matrix* h) {
     if (swept_crs(h) || h->format == PWM_FORMAT_CSB)
         can = h->csb.sweep || (h->csb.stream && h->csb.groups == 1);
     else if (h->format == PWM_FORMAT_BLOCKCOH)
-        can = true;
+        can = h->coh.n_tasks > 0;
     const int64_t slots = partial_slots(h);
     return can && !h->power_small && slots > 0 && slots <= pwmk::kDeferSlots;
 }

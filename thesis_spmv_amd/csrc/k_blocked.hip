@@ -876,10 +876,11 @@ hipError_t launch_csb(const CsbArgs& a, const void* x, void* y, const PowerArgs*
 template <typename VT, bool POWER>
 static hipError_t coh_t(const CohArgs& a, const void* x, void* y, const PowerArgs& pw, hipStream_t s) {
     using X = typename Arith<VT>::X;
-    if (a.n_tasks <= 0) return hipSuccess;
     const size_t lds = (size_t)std::max<int32_t>(a.lds_rows, 1) * sizeof(double);
     auto k = a.one_wave ? k_coh<VT, POWER, 64> : k_coh<VT, POWER, kBS>;
-    hipLaunchKernelGGL(k, dim3((unsigned)a.n_tasks), dim3(a.one_wave ? 64 : kBS), lds, s, a, (const X*)x, (X*)y, pw);
+    // no tasks: one band without entries, too tall for the LDS; its rows are pieces
+    if (a.n_tasks > 0)
+        hipLaunchKernelGGL(k, dim3((unsigned)a.n_tasks), dim3(a.one_wave ? 64 : kBS), lds, s, a, (const X*)x, (X*)y, pw);
     if (a.n_pieces > 0)
         hipLaunchKernelGGL((k_coh_finish<VT, POWER>), dim3((unsigned)a.n_pieces), dim3(kBS), 0, s, a, (X*)y, pw);
     return hipGetLastError();
