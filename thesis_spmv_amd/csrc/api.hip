@@ -152,8 +152,8 @@ void parallel_run(int64_t n, int64_t chunk, const LoopFn& fn, const LeadFn* lead
     p->cv_done.wait(lk, [&] { return p->pending == 0; });
 }
 
-// Pinned staging for host -> device uploads: two process-wide buffers of
-// kStageBytes, held until the process ends; one upload at a time uses them.
+// Pinned staging for transfers: two process-wide buffers of kStageBytes, held
+// until the process ends; one transfer at a time uses them.
 namespace {
 constexpr size_t kStageBytes = (size_t)64 << 20;
 std::mutex g_stage_mu;
@@ -162,6 +162,40 @@ hipEvent_t g_stage_ev[2] = {nullptr, nullptr};
 constexpr size_t kRingChunks = 16;  // most chunks per buffer
 hipEvent_t g_ring_ev[2 * kRingChunks] = {};
 bool g_stage_failed = false;
+
+// Vectors of at most kInlineBytes go through a piece of their own, one per call
+// under way: they wait for nobody's transfer.  At most kShortSlots pieces, each
+// allocated when first needed and kept for the process.
+constexpr size_t kInlineBytes = (size_t)1 << 20;
+constexpr int kShortSlots = 16;
+std::mutex g_short_mu;
+char* g_short_free[kShortSlots];
+int g_short_n = 0, g_short_made = 0;  // free ones, all
+
+struct ShortSlot {
+    char* p = nullptr;  // nullptr: none to be had
+    ShortSlot() {
+        std::lock_guard<std::mutex> lk(g_short_mu);
+        if (g_short_n > 0) {
+            p = g_short_free[--g_short_n];
+        } else if (g_short_made < kShortSlots) {
+            void* q = nullptr;
+            if (hipHostMalloc(&q, kInlineBytes, hipHostMallocCoherent | hipHostMallocPortable) == hipSuccess) {
+                p = (char*)q;
+                ++g_short_made;
+            } else {
+                (void)hipGetLastError();
+            }
+        }
+    }
+    ~ShortSlot() {
+        if (!p) return;
+        std::lock_guard<std::mutex> lk(g_short_mu);
+        g_short_free[g_short_n++] = p;
+    }
+    ShortSlot(const ShortSlot&) = delete;
+    ShortSlot& operator=(const ShortSlot&) = delete;
+};
 }  // namespace
 
 // Chunk of one staged transfer: about an eighth of it (whole MB, at least
@@ -257,11 +291,9 @@ static auto floats_out(double* dst) {
 // 999 575 -> 450, 5000 x 5000 as before; FP32, which used to convert in separate
 // loops, 1000 x 999 590 -> 280 and 4000 x 3000 9300 -> 2170.
 namespace {
-// Short transfers are copied by the calling thread: waking the others costs
-// more (mv of 0.7 MB vectors takes 75 us, through the threads 97; of 1.4 MB 143
-// through the threads, without them 155).
-constexpr size_t kInlineBytes = (size_t)1 << 20;
-
+// Transfers of at most kInlineBytes are copied by the calling thread: waking the
+// others costs more (mv of 0.7 MB vectors takes 75 us, through the threads 97; of
+// 1.4 MB 143 through the threads, without them 155).
 struct Window {
     size_t bytes, chunk, piece, nch;
     int64_t pieces;
@@ -329,9 +361,13 @@ static hipError_t window_upload(void* dst, size_t bytes, hipStream_t s, Fill fil
 }
 
 // Device -> host: empty(stage, a0, a1) takes bytes [a0, a1) from `stage`.  Waits
-// for the work queued on s.  b: the buffer to begin with.
+// for the work queued on s.  The caller holds g_stage_mu and stage_ready() is
+// true.  b: the buffer to begin with.  The host threads are woken when the work
+// before the copies has ended, or (soon) at once, where that is over before they
+// are awake: waking takes some 40 us (mv of 2 MB vectors 150 us, with the threads
+// woken behind the SpMV 189; of 8 MB 449 and 453).
 template <typename Empty>
-static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, Empty empty, int b = 0) {
+static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, Empty empty, int b = 0, bool soon = true) {
     if (bytes <= kInlineBytes) {  // (an event costs 5 us more than the stream)
         hipError_t e = pwmk::launch_copy_bytes(g_stage[b], src, bytes, true, s);
         const hipError_t e2 = hipStreamSynchronize(s);
@@ -349,7 +385,9 @@ static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, 
         }
         return e;
     };
-    hipError_t e = issue(0, b);
+    hipError_t e = soon ? hipSuccess : hipEventRecord(g_stage_ev[b], s);
+    if (e == hipSuccess) e = issue(0, b);
+    if (e == hipSuccess && !soon) e = hipEventSynchronize(g_stage_ev[b]);
     for (size_t off = 0; off < bytes && e == hipSuccess; off += kStageBytes, b ^= 1) {
         if (off + kStageBytes < bytes && (e = issue(off + kStageBytes, b ^ 1)) != hipSuccess) break;
         const size_t n = std::min(kStageBytes, bytes - off);
@@ -476,10 +514,22 @@ hipError_t upload_values_staged(void* dst, const double* src, int64_t n, int vt,
 hipError_t download_doubles(double* dst, const void* src, int64_t n, bool f64, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const size_t bytes = (size_t)n * (f64 ? 8 : 4);
+    if (bytes <= kInlineBytes) {
+        ShortSlot slot;
+        if (slot.p) {
+            hipError_t e = pwmk::launch_copy_bytes(slot.p, src, bytes, true, s);
+            const hipError_t e2 = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = e2;
+            if (e == hipSuccess) f64 ? bytes_out(dst)(slot.p, 0, bytes) : floats_out(dst)(slot.p, 0, bytes);
+            return e;
+        }
+    }
+    hipError_t e = hipStreamSynchronize(s);  // before the lock
+    if (e != hipSuccess) return e;
     std::lock_guard<std::mutex> lk(g_stage_mu);
     if (!stage_ready()) {  // no pinned memory: a plain copy to pageable memory
         std::vector<float> f(f64 ? 0 : n);
-        hipError_t e = hipMemcpyAsync(f64 ? (void*)dst : f.data(), src, bytes, hipMemcpyDeviceToHost, s);
+        e = hipMemcpyAsync(f64 ? (void*)dst : f.data(), src, bytes, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         for (size_t i = 0; i < f.size() && e == hipSuccess; ++i) dst[i] = f[i];
         return e;
@@ -1537,15 +1587,37 @@ static int download_vec(pwm_matrix* h, const void* src, double* dst, int64_t n) 
     return e == hipSuccess ? PWM_OK : hip_fail(h, e, "vector download");
 }
 
-// y = A x on host vectors of at most one staging buffer each: x goes through
-// one, y through the other, and the host waits once, for y.
+// y = A x on short host vectors: x and y go through one piece of pinned memory,
+// in the stream's order, and the host waits once, for y.
+static int mv_short(pwm_matrix* h, const double* x, double* y, char* stage) {
+    const bool f64 = h->vtype == PWM_VALUES_F64;
+    const size_t vs = vector_size(h->vtype), nx = (size_t)h->noc * vs, ny = (size_t)h->nor * vs;
+    f64 ? bytes_in(x)(stage, 0, nx) : values_in(x, PWM_VALUES_F32)(stage, 0, nx);
+    hipError_t e = pwmk::launch_copy_bytes(h->hx.p, stage, nx, false, h->stream);
+    int rc = e == hipSuccess ? spmv_launch(h, h->hx.p, h->hy.p, nullptr) : hip_fail(h, e, "vector upload");
+    if (rc == PWM_OK && (e = pwmk::launch_copy_bytes(stage, h->hy.p, ny, true, h->stream)) != hipSuccess)
+        rc = hip_fail(h, e, "vector download");
+    e = hipStreamSynchronize(h->stream);
+    if (rc == PWM_OK && e != hipSuccess) rc = hip_fail(h, e, "SpMV on host vectors");
+    if (rc == PWM_OK) f64 ? bytes_out(y)(stage, 0, ny) : floats_out(y)(stage, 0, ny);
+    return rc;
+}
+
+// y = A x on host vectors of at most one staging buffer each: x goes through one,
+// y through the other, y's copies are queued behind the SpMV and the host waits
+// once, for y.  Without that an FP64 call on a 1000 x 999 grid takes 482 instead of
+// 453 us, an FP32 one 320 instead of 280.  g_stage_mu is held meanwhile, so only for
+// SpMVs that are short beside their transfers.
+constexpr int64_t kShortSpmv = (int64_t)1 << 26;  // entries, some 0.2 to 0.5 ms
+constexpr int64_t kSoonSpmv = (int64_t)1 << 23;   // some 40 us
 static int mv_staged(pwm_matrix* h, const double* x, double* y, bool* done) {
     const bool f64 = h->vtype == PWM_VALUES_F64;
     const size_t vs = vector_size(h->vtype);
-    if ((size_t)std::max(h->nor, h->noc) * vs > kStageBytes) return PWM_OK;
+    if (h->nnz > kShortSpmv || (size_t)std::max(h->nor, h->noc) * vs > kStageBytes) return PWM_OK;
     std::lock_guard<std::mutex> lk(g_stage_mu);
     if (!stage_ready()) return PWM_OK;  // no pinned memory: the general path
     *done = true;
+    const bool soon = h->nnz <= kSoonSpmv;
     hipError_t e = f64 ? window_upload(h->hx.p, (size_t)h->noc * vs, h->stream, bytes_in(x), false)
                        : window_upload(h->hx.p, (size_t)h->noc * vs, h->stream, values_in(x, PWM_VALUES_F32), false);
     const int rc = e == hipSuccess ? spmv_launch(h, h->hx.p, h->hy.p, nullptr) : hip_fail(h, e, "vector upload");
@@ -1553,8 +1625,8 @@ static int mv_staged(pwm_matrix* h, const double* x, double* y, bool* done) {
         (void)hipStreamSynchronize(h->stream);
         return rc;
     }
-    e = f64 ? window_download(h->hy.p, (size_t)h->nor * vs, h->stream, bytes_out(y), 1)
-            : window_download(h->hy.p, (size_t)h->nor * vs, h->stream, floats_out(y), 1);
+    e = f64 ? window_download(h->hy.p, (size_t)h->nor * vs, h->stream, bytes_out(y), 1, soon)
+            : window_download(h->hy.p, (size_t)h->nor * vs, h->stream, floats_out(y), 1, soon);
     return e == hipSuccess ? PWM_OK : hip_fail(h, e, "vector download");
 }
 
@@ -1564,8 +1636,13 @@ extern "C" int pwm_mv(pwm_matrix* h, const double* x, double* y) {
     if (!x || !y) return fail(h, PWM_ERR_INVALID, "pwm_mv: NULL vector");
     if (x < y + h->nor && y < x + h->noc) return fail(h, PWM_ERR_INVALID, "pwm_mv: x and y overlap");
     int rc = stage_vectors(h);
+    if (rc != PWM_OK) return rc;
+    if ((size_t)std::max(h->nor, h->noc) * vector_size(h->vtype) <= kInlineBytes) {
+        ShortSlot slot;
+        if (slot.p) return mv_short(h, x, y, slot.p);
+    }
     bool done = false;
-    if (rc == PWM_OK) rc = mv_staged(h, x, y, &done);
+    rc = mv_staged(h, x, y, &done);
     if (done) return rc;
     if (rc == PWM_OK) rc = upload_vec(h, x, h->hx.p, h->noc);
     if (rc == PWM_OK) rc = spmv_launch(h, h->hx.p, h->hy.p, nullptr);
