@@ -158,7 +158,9 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * runs faster in the load-time timing; on CRS and CRS_MERGE handles: 0 = swept
  * slabs are kept beside the CRS arrays and swept in a fixed order when x
  * exceeds 4 MB (CRS_MERGE: 8 MB), the columns are scattered and they run faster
- * in the load-time timing, 4 = always when they fit, 1 to 3 = never), "csb_window_bits" (swept slabs: log2 of the
+ * in the load-time timing, 4 = always when they fit, 1 to 3 = never; never where
+ * crs_kernel, group_size, vec_blocks, long_row or crs_nt, on CRS_MERGE the
+ * thread count or items_per_thread, choose the kernel), "csb_window_bits" (swept slabs: log2 of the
  * columns per window, 0 = 1 MB of x), "csb_sync_every" (swept slabs: windows
  * between workgroup barriers, 1, 2, 4 or 8, default 2), "csb_sweep_unroll"
  * (swept slabs: groups of 4 entries per lane per chunk, 1, 2 or 4, default 2),
@@ -183,7 +185,9 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * three lane counts and the row-aligned tiles kernel at load and keep the
  * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =
  * non-temporal col_ind/value loads, 0 = plain, -1 = time both at load, for the
- * wave tiles by the spread of the columns, the default).  Must be set before the matrix is loaded unless noted. */
+ * wave tiles by the spread of the columns, the default; 0 and 1 on a CRS handle
+ * also keep the tiles, wave tiles and vector kernels for SpMV and power method:
+ * no swept slabs, no power method in one workgroup).  Must be set before the matrix is loaded unless noted. */
 int pwm_set_option(pwm_matrix* h, const char* key, int64_t value);
 
 /* ---- device-resident additions ----------------------------------------

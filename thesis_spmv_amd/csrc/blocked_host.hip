@@ -220,8 +220,15 @@ static int build_swept(pwm_matrix* h, const int32_t* rs, bool ord) {
 }
 
 int build_swept_beside_crs(pwm_matrix* h) {
-    if ((int64_t)h->h_rs.size() != h->nor + 1) return PWM_OK;
-    const int rc = build_swept(h, h->h_rs.data(), true);
+    // the slabs are cut on the host; a matrix generated on the device keeps no host
+    // row offsets
+    std::vector<int32_t> rs;
+    if ((int64_t)h->h_rs.size() != h->nor + 1) {
+        rs.resize(h->nor + 1);
+        const hipError_t e = hipMemcpy(rs.data(), h->rs.p, (h->nor + 1) * 4, hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return hip_fail(h, e, "swept slabs: row offsets");
+    }
+    const int rc = build_swept(h, rs.empty() ? h->h_rs.data() : rs.data(), true);
     if (rc == PWM_OK) return PWM_OK;
     h->csb.clear();
     (void)hipGetLastError();
