@@ -157,8 +157,8 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * rows pack, else 3, replaced by 4 when x exceeds 2 MB, the slabs fit and 4
  * runs faster in the load-time timing; on CRS and CRS_MERGE handles: 0 = swept
  * slabs are kept beside the CRS arrays and swept in a fixed order when x
- * exceeds 4 MB (CRS_MERGE: 8 MB), the columns are scattered and they run faster
- * in the load-time timing, 4 = always when they fit, 1 to 3 = never; never where
+ * exceeds 4 MB (CRS_MERGE: 8 MB), the columns are scattered, three quarters of
+ * the device memory stay free and they run faster in the load-time timing, 4 = always when they fit, 1 to 3 = never; never where
  * crs_kernel, group_size, vec_blocks, long_row or crs_nt, on CRS_MERGE the
  * thread count or items_per_thread, choose the kernel), "csb_window_bits" (swept slabs: log2 of the
  * columns per window, 0 = 1 MB of x), "csb_sync_every" (swept slabs: windows

@@ -771,10 +771,22 @@ static hipError_t time_swept(pwm_matrix* h, const void* x, void* y, float* best)
 // becomes half as long again (6.2 M entries: 6.5 -> 9.8 ms), which 33 SpMVs bring
 // back at 9.6 MB of x (250 -> 108 us each) and 130 at 6.2 MB (65 -> 40).  A CRS
 // load times its kernels in any case (11.0 ms, with the slabs 10.0).
+//
+// The slabs are a second copy of the matrix, which nobody asked for: they are kept
+// only while three quarters of the device memory stay free, so that all handles'
+// slabs together take about an eighth of it at most.
+static bool leaves_room(const pwm_matrix* h) {
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return free >= total / 4 * 3 + (size_t)h->nnz * (4 + value_size(h->vtype));
+}
 static bool wants_swept(const pwm_matrix* h, double lines) {
     if (h->csb_layout == 4) return h->nnz > 0;
     const int64_t xbytes = h->noc * (int64_t)vector_size(h->vtype);
-    return h->csb_layout == 0 && lines > 128.0 && (h->format == PWM_FORMAT_CRS || xbytes > 2 * kXcdL2);
+    return h->csb_layout == 0 && lines > 128.0 && (h->format == PWM_FORMAT_CRS || xbytes > 2 * kXcdL2) && leaves_room(h);
 }
 static int plan_swept(pwm_matrix* h, double lines, const void* x, void* y, float* ms) {
     *ms = -1.0f;
@@ -1045,7 +1057,13 @@ int plan_merge(pwm_matrix* h) {
     }
     const size_t vs = vector_size(h->vtype);
     DevBuf x, y;
-    if ((e = x.alloc(h->noc * vs)) != hipSuccess || (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) != hipSuccess ||
+    if ((e = x.alloc(h->noc * vs)) == hipErrorOutOfMemory ||
+        (e == hipSuccess && (e = y.alloc(std::max<int64_t>(h->nor, 1) * vs)) == hipErrorOutOfMemory)) {
+        (void)hipGetLastError();  // nothing to time on: the kernel chosen so far stays
+        e = hipStreamSynchronize(h->stream);
+        return e == hipSuccess ? PWM_OK : hip_fail(h, e, "merge split search");
+    }
+    if (e != hipSuccess ||
         (e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream)) != hipSuccess)
         return hip_fail(h, e, "merge plan vectors");
     float swept = -1.0f, best = -1.0f;
