@@ -282,6 +282,7 @@ hipError_t download_doubles(double* dst, const void* src, int64_t n, bool f64, h
 // CSB slab-stream layout built on the device from the device CRS arrays
 // (csb_build.hip); h->csb.bits/H/V set.  csb_key_bits: bits of its sort key.
 int csb_key_bits(int64_t cells, int bits);
+int csb_lds_bits(int vtype, int64_t nor);
 int csb_stream_device(pwm_matrix* h, int rb, int cb, int64_t S, bool wide);
 // CSB slab-piece layout (the stored order, blk_ptr and the pieces of slabs of
 // beta >> k rows) built on the device the same way; h->csb.bits/H/V set.

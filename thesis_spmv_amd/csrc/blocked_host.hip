@@ -246,6 +246,15 @@ void drop_crs(pwm_matrix* h) {
     h->val.release();
 }
 
+// Most rows of a slab of the slab streams, as a power of two: 4096 (32 KB of LDS);
+// for FP32 vectors beyond 2^29 rows 8192, since neither the 64-bit sort key (slab,
+// block column, Z-Morton code) of square matrices beyond 2^30 rows nor the
+// no-allocation power method's partial-sum slots hold twice the slabs.
+int csb_lds_bits(int vtype, int64_t nor) {
+    static_assert(blocked::kCsbLdsRows == 1 << 12, "the slab pieces' LDS rows");
+    return vtype != PWM_VALUES_F64 && nor > (int64_t)1 << 29 ? 13 : 12;
+}
+
 // rs: host row_start; ci / vals: host CRS arrays, or NULL (values already
 // validated for the storage type) -- they are then downloaded only if the
 // host-built slab-piece layout is used.
@@ -286,8 +295,7 @@ int build_csb(pwm_matrix* h, const int32_t* rs, const int32_t* ci, const double*
     // key (slab, block column, Z-Morton code) would need more than 64 bits;
     // they are sorted on the device too (key: block, Z-Morton code), or
     // built on the host with csb_build = 1.
-    const int lds_bits = 12;
-    static_assert(blocked::kCsbLdsRows == 1 << 12, "slabs of 2^lds_bits rows fill the LDS rows");
+    const int lds_bits = csb_lds_bits(h->vtype, nor);
     int cb = 0;
     while (((int64_t)1 << cb) < noc) ++cb;
     // no longer than needed for about 4096 slabs (16 workgroups per CU),
