@@ -1,9 +1,9 @@
 """Matrices near the partial-sum slots of the no-allocation power method's fixed
 workspace (PWM_NOALLOC_MAX_SLOTS) stay within them.
 
-CRS_MERGE, rows of 60 entries: a slot of the merge kernels is a tile of 2048
-merge items, 208 496 slots for the 420 M entries here; the wave tiles that such
-rows take must not need more than the workspace holds.
+CRS_MERGE, rows of 27 entries and one of 64: a slot of the merge kernels is a tile
+of 2048 merge items, 211 919 slots for the 419 M entries here; the wave tiles that
+such rows take must not need more than the workspace holds.
 
 BlockCOH in one band: 32 768 entries a task would make 23 463 slots of the 769 M
 entries here; tasks of 4096 entries and pieces of 2048 rows make 263 K."""
@@ -15,17 +15,20 @@ pytestmark = pytest.mark.gpu
 
 
 def test_short_rows():
-    n, L = 7_000_000, 60
-    ci = (np.minimum(np.arange(n), n - L)[:, None] + np.arange(L)).astype(np.int32).ravel()
-    rs = (np.arange(n + 1, dtype=np.int64) * L).astype(np.int32)
+    n, L = 15_500_000, 27
+    lens = np.full(n, L)
+    lens[0] = 64
+    rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([np.arange(64), (np.minimum(np.arange(1, n), n - L)[:, None] + np.arange(L)).ravel()])
     m = pw.CRSMergeHip(values="f32")
-    m.loadCRS(n, n, rs, ci, np.ones(n * L))
+    m.loadCRS(n, n, rs, ci.astype(np.int32), np.ones(len(ci)))
     assert m.info()["kernels"] == 1  # the wave tiles
     x, y = (pw.DeviceVector(n, np.float32) for _ in range(2))
     x.fill(1.0)
     lam, norm, k = m.power_method_device_noalloc(x, y, 1)
-    # every row sums to 60; one rounding of the norm's square root
-    assert k == 1 and lam == 60.0 and abs(norm - 60.0 * np.sqrt(n)) <= 2.0 ** -52 * norm
+    # whole row sums; one rounding of the norm's square root
+    assert k == 1 and lam == len(ci) / n
+    assert abs(norm - np.sqrt(float(L * L * (n - 1) + 64 * 64))) <= 2.0 ** -52 * norm
     ref = (x.download(), y.download())
     x.fill(1.0)
     assert (lam, norm, k) == m.power_method_device(x, y, 1)

@@ -914,9 +914,35 @@ static int plan_crs_rows(pwm_matrix* h) {
     return PWM_OK;
 }
 
-// CRS planning and the autotuner.  Rows of at most 64 entries take the wave
-// tiles (k_rows.hip): the kernels below were slower or equal on every such
-// matrix (FP64, us: Poisson 300 x 301 2.7 against 3.4, 5000 x 5000 332 against
+// Where the wave tiles need no timing: up to `mean` entries per row, and on small
+// matrices (0.5 M entries), whose kernels differ by less than a microsecond of a
+// call.  A lane sums a row alone, and of longer rows a tile has few.  Rows of L
+// columns near the diagonal, FP64 SpMV in us, wave tiles, CRS tiles, vector and merge
+// kernel: 150 000 rows L = 12 5.2 5.5 6.1 11.4, 20 8.0 9.6 10.3 15.6, 28 10.7 11.9
+// 11.4 18.6, 48 26.9 20.5 17.1 23.6, 64 39.8 25.8 19.3 28.4; 1 M rows L = 12 23.8 25.2
+// 29.8 35.9, 16 40.7 37.5 34.2 43.7, 28 68 72 88 80, 48 153 123 160 129.  Random
+// columns hide it: 150 000 rows L = 64 49 48 50 54.
+constexpr int64_t kRowsMeanCrs = 12, kRowsMeanMerge = 28;
+static bool rows_untimed(const pwm_matrix* h, int64_t mean) {
+    return h->nnz <= mean * h->nor || h->nnz < (int64_t)1 << 19;
+}
+
+// Time of an SpMV by the wave tiles.  Less 1.5 us where their power steps defer the
+// norms, half of what that saves a step: the other kernels' do not.
+static hipError_t time_rows(pwm_matrix* h, const void* x, void* y, float* ms) {
+    const hipError_t e = time_crs_kernel(h, 3, x, y, ms);
+    if (pwmk::rows_power_blocks(h->rp.nt) <= pwmk::kDeferSlots) *ms -= 0.0015f;
+    return e;
+}
+
+static void drop_rows(pwm_matrix* h) {
+    h->rp = pwmk::RowsPlan{};
+    h->rows_cut.release();
+}
+
+// CRS planning and the autotuner.  Where no row has more than 64 entries the wave
+// tiles (k_rows.hip) run, on a mean of at most 12 by rule (FP64, us, against the
+// fastest of the others: Poisson 300 x 301 2.7 against 3.4, 5000 x 5000 332 against
 // 441, 9-point stencil with 2 random entries per row, 1448 x 1448, 100 against
 // 100), but where x has far lines and more than 24 MB (that stencil on 2896 x
 // 2896: FP64 441 against 434, FP32, 33.5 MB of x, 369 against 364; on 2200 x 2200
@@ -924,8 +950,8 @@ static int plan_crs_rows(pwm_matrix* h) {
 // or set up the vector kernel: candidates are that one with the
 // rows-per-wave heuristic G0 = pow2(avg row length / 2) in [2, 32] and with
 // G0/2 and 2 G0 when the longest row fills them (only G0 when the caller
-// fixed group_size), and the tiles kernel (unless crs_kernel excludes
-// either).  With more than one candidate,
+// fixed group_size), the tiles kernel (unless crs_kernel excludes
+// either) and the wave tiles.  With more than one candidate,
 // each is timed on x = 1 and the fastest is kept.
 int plan_crs(pwm_matrix* h) {
     const double avg = h->nor > 0 ? (double)h->nnz / (double)h->nor : 0.0;
@@ -942,7 +968,7 @@ int plan_crs(pwm_matrix* h) {
         }
     }
     int rc;
-    h->rp = pwmk::RowsPlan{};
+    drop_rows(h);
     h->csb.clear();
     const bool automatic = h->crs_kernel == 0 && h->group_opt == 0 && h->vec_blocks_opt == 0 && h->long_row == 0;
     hipError_t e;
@@ -950,10 +976,10 @@ int plan_crs(pwm_matrix* h) {
     if (automatic && (e = column_lines(h, &lines)) != hipSuccess) return hip_fail(h, e, "column lines");
     const int64_t xbytes = h->noc * (int64_t)vector_size(h->vtype);
     if (automatic && !(lines > kSpreadLines && xbytes > 6 * kXcdL2) && (rc = plan_crs_rows(h)) != PWM_OK) return rc;
-    const bool rows = h->rp.nt > 0;
-    const bool tiles = !rows && h->crs_kernel != 1;
+    const bool rows = h->rp.nt > 0, rows_only = rows && rows_untimed(h, kRowsMeanCrs);
+    bool tiles = !rows_only && h->crs_kernel != 1;
     const bool sweep = automatic && h->crs_nt < 0 && wants_swept(h, lines);
-    if (rows) {
+    if (rows_only) {
         gs.clear();
         h->lr = pwmk::LongRows{};
         h->crs_nt_used = rows_nt(h, lines);
@@ -962,8 +988,8 @@ int plan_crs(pwm_matrix* h) {
     } else {
         h->crs_nt_used = h->crs_nt > 0 ? 1 : 0;
     }
-    if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
     if (!rows && (int)gs.size() + (tiles ? 1 : 0) == 1 && (!tiles || h->crs_nt >= 0)) {
+        if (tiles && (rc = plan_crs_tiles(h)) != PWM_OK) return rc;
         h->crs_used = tiles ? 2 : 1;
         return plan_crs_vector(h, tiles ? G0 : gs[0]);
     }
@@ -975,12 +1001,27 @@ int plan_crs(pwm_matrix* h) {
     e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream);
     if (e != hipSuccess) return hip_fail(h, e, "CRS autotune vectors");
     float best = -1.0f, swept = -1.0f;
-    int best_kernel = 1, best_g = G0;
+    int best_kernel = 1, best_g = G0, best_nt = 0;
     if (sweep && (rc = plan_swept(h, lines, x.p, y.p, &swept)) != PWM_OK) return rc;
-    if (rows || tiles) {
-        best_kernel = rows ? 3 : 2;
-        e = rows ? time_crs_kernel(h, 3, x.p, y.p, &best) : time_entry_loads(h, x.p, y.p, &best);
-        if (e != hipSuccess) return hip_fail(h, e, "CRS autotune");
+    if (rows) {
+        best_kernel = 3;
+        best_nt = h->crs_nt_used = rows_nt(h, lines);
+        if ((e = time_rows(h, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
+        // those below gather in row order too
+        if (swept >= 0.0f && swept < 0.7f * best) {
+            tiles = false;
+            gs.clear();
+        }
+    }
+    if (tiles) {
+        float ms = 0.0f;
+        if ((rc = plan_crs_tiles(h)) != PWM_OK) return rc;
+        if ((e = time_entry_loads(h, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
+        if (!rows || ms < best) {
+            best = ms;
+            best_kernel = 2;
+            best_nt = h->crs_nt_used;
+        }
     }
     // the vector kernel gathers in row order like the tiles and was never a
     // third faster than they: it is not timed against a sweep that is
@@ -989,16 +1030,17 @@ int plan_crs(pwm_matrix* h) {
         if ((rc = plan_crs_vector(h, g)) != PWM_OK) return rc;
         float ms = 0.0f;
         if ((e = time_crs_kernel(h, 1, x.p, y.p, &ms)) != hipSuccess) return hip_fail(h, e, "CRS autotune");
-        if (best < 0.0f || ms < best) {
+        if ((!rows && !tiles && best < 0.0f) || ms < best) {
             best = ms;
             best_kernel = 1;
             best_g = g;
         }
     }
     h->crs_used = best_kernel;
+    if (best_kernel != 1) h->crs_nt_used = best_nt;
     if (swept >= 0.0f && swept >= best) h->csb.clear();
-    if (rows) return PWM_OK;
-    if (h->csb.sweep) {
+    if (best_kernel != 3) drop_rows(h);
+    if (best_kernel == 3 || h->csb.sweep) {
         h->lr = pwmk::LongRows{};
         h->vec_blocks = 0;
         return PWM_OK;
@@ -1035,15 +1077,16 @@ int plan_merge(pwm_matrix* h) {
     // Unless the caller chose the partition or the tile size, the SpMV takes
     // the CRS format's wave tiles when the rows are short (Poisson 80 x 80: 8.0
     // -> 3.0 us, 1024 x 1024: 23.2 -> 13.8, 5000 x 5000: 405 -> 338, FP64; the
-    // merge of each thread's items is what they save) and its swept slabs when
+    // merge of each thread's items is what they save; timed against the merge
+    // kernel above a mean of 28 entries) and its swept slabs when
     // the columns are scattered and the slabs time faster.
     h->csb.clear();
-    h->rp = pwmk::RowsPlan{};
+    drop_rows(h);
     h->crs_used = 0;
     const bool chosen = (h->threads > 0 && P == h->threads) || h->ipt != 8;
     int rc = chosen ? PWM_OK : plan_crs_rows(h);
     if (rc != PWM_OK) return rc;
-    const bool rows = h->rp.nt > 0;
+    const bool rows = h->rp.nt > 0, contest = rows && !rows_untimed(h, kRowsMeanMerge);
     double lines = 0.0;
     if (!chosen && (rows || h->csb_layout == 0) && (e = column_lines(h, &lines)) != hipSuccess)
         return hip_fail(h, e, "column lines");
@@ -1051,7 +1094,7 @@ int plan_merge(pwm_matrix* h) {
         h->crs_used = 3;
         h->crs_nt_used = rows_nt(h, lines);
     }
-    if (chosen || !wants_swept(h, lines)) {
+    if (chosen || (!contest && !wants_swept(h, lines))) {
         e = rows ? hipSuccess : hipStreamSynchronize(h->stream);
         return e == hipSuccess ? PWM_OK : hip_fail(h, e, "merge split search");
     }
@@ -1067,9 +1110,20 @@ int plan_merge(pwm_matrix* h) {
         (e = pwmk::launch_fill(x.p, h->noc, h->vtype == PWM_VALUES_F64 ? 1 : 0, 1.0, h->stream)) != hipSuccess)
         return hip_fail(h, e, "merge plan vectors");
     float swept = -1.0f, best = -1.0f;
+    if (contest) {
+        float merge = 0.0f;
+        if ((e = time_rows(h, x.p, y.p, &best)) != hipSuccess ||
+            (e = time_crs_kernel(h, 0, x.p, y.p, &merge)) != hipSuccess)
+            return hip_fail(h, e, "merge plan");
+        if (merge < best) {
+            best = merge;
+            h->crs_used = 0;
+            drop_rows(h);
+        }
+    }
     if ((rc = plan_swept(h, lines, x.p, y.p, &swept)) != PWM_OK) return rc;
     if (swept < 0.0f) return PWM_OK;
-    if ((e = time_crs_kernel(h, h->crs_used, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "merge plan");
+    if (!contest && (e = time_crs_kernel(h, h->crs_used, x.p, y.p, &best)) != hipSuccess) return hip_fail(h, e, "merge plan");
     if (swept >= best) h->csb.clear();
     return PWM_OK;
 }
