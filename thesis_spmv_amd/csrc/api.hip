@@ -363,9 +363,9 @@ static hipError_t window_upload(void* dst, size_t bytes, hipStream_t s, Fill fil
 // Device -> host: empty(stage, a0, a1) takes bytes [a0, a1) from `stage`.  Waits
 // for the work queued on s.  The caller holds g_stage_mu and stage_ready() is
 // true.  b: the buffer to begin with.  The host threads are woken when the work
-// before the copies has ended, or (soon) at once, where that is over before they
-// are awake: waking takes some 40 us (mv of 2 MB vectors 150 us, with the threads
-// woken behind the SpMV 189; of 8 MB 449 and 453).
+// before the copies has ended, or (soon) at once, where that is short: waking takes
+// some 40 us (mv of 2 MB vectors 150 us, with the threads woken behind the SpMV 189;
+// of 8 MB 449 and 453, of 32 MB 1425 and 1440).
 template <typename Empty>
 static hipError_t window_download(const void* src, size_t bytes, hipStream_t s, Empty empty, int b = 0, bool soon = true) {
     if (bytes <= kInlineBytes) {  // (an event costs 5 us more than the stream)
@@ -1681,7 +1681,7 @@ static int mv_short(pwm_matrix* h, const double* x, double* y, char* stage) {
 // 453 us, an FP32 one 320 instead of 280.  g_stage_mu is held meanwhile, so only for
 // SpMVs that are short beside their transfers.
 constexpr int64_t kShortSpmv = (int64_t)1 << 26;  // entries, some 0.2 to 0.5 ms
-constexpr int64_t kSoonSpmv = (int64_t)1 << 23;   // some 40 us
+constexpr int64_t kSoonSpmv = (int64_t)1 << 25;   // at most 0.1 ms or so
 static int mv_staged(pwm_matrix* h, const double* x, double* y, bool* done) {
     const bool f64 = h->vtype == PWM_VALUES_F64;
     const size_t vs = vector_size(h->vtype);
