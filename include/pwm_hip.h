@@ -180,10 +180,10 @@ int pwm_matrix_stats(const pwm_matrix* h, pwm_stats_t* out);
  * host, 1; both give the same arrays), "coh_occ8" (BlockCOH: 1 = a
  * workgroup of 8 waves per task, 0 = one wave per task, -1 = 8 waves, or the
  * faster of the two in a load-time timing where the columns are scattered over
- * more than 10 MB of x, the default), "crs_kernel" (CRS: 0 = one wave per tile of short
- * rows when no row has more than 64 entries, else time the vector kernel at
- * three lane counts and the row-aligned tiles kernel at load and keep the
- * fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =
+ * more than 10 MB of x, the default), "crs_kernel" (CRS: 0 = one wave per tile of rows
+ * when none has more than 64 entries and they are few on average, else time
+ * these, the vector kernel at three lane counts and the row-aligned tiles kernel
+ * at load and keep the fastest, 1 = vector, 2 = tiles), "crs_nt" (CRS tiles kernels: 1 =
  * non-temporal col_ind/value loads, 0 = plain, -1 = time both at load, for the
  * wave tiles by the spread of the columns, the default; 0 and 1 on a CRS handle
  * also keep the tiles, wave tiles and vector kernels for SpMV and power method:

@@ -356,9 +356,9 @@ class SparseMatrixHip:
 
 class CRSHip(SparseMatrixHip):
     """CRS (beside CRS / CRSOMP, Matrix/CRS.hpp, Env_Implementations/CRSOMP.hpp): one
-    wave per tile of short rows (no row above 64 entries), else the vector
-    kernel or the row-aligned tiles kernel, whichever timed faster at load
-    (option crs_kernel: 1 vector, 2 tiles)."""
+    wave per tile of short rows (none above 64 entries, few on average), else
+    that, the vector kernel or the row-aligned tiles kernel, whichever timed
+    fastest at load (option crs_kernel: 1 vector, 2 tiles), or swept slabs."""
     FORMAT = FORMAT_CRS
 
 

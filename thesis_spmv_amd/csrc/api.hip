@@ -1995,7 +1995,7 @@ extern "C" int pwm_power_method_device_noalloc(pwm_matrix* h, void* x, void* y, 
     if (int rc0 = check_device_xy(h, x, h->nor, y, h->nor, "pwm_power_method_device_noalloc")) return rc0;
     char* base = nullptr;
     if (int rc0 = noalloc_scratch(h, &base)) return rc0;
-    // the step control is reset by the power loop's first kernel; records
+    // the first step ignores the step control that another call left; records
     // and partial sums are written before they are read
     const PowerWs ws{(int*)base, (double*)(base + kNoAllocRecOff), (double*)(base + kNoAllocPartOff)};
     int64_t steps = 0;

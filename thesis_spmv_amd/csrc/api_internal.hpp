@@ -197,7 +197,8 @@ struct pwm_matrix {
     pwmk::LongRows lr;
     pwm_impl::DevBuf lr_chunks, lr_rows, lr_begin, lr_partial;
     // CRS kernel: 0 = wave tiles when the rows are short, else time the vector
-    // and tiles kernels at load and keep the faster, 1 = vector, 2 = tiles
+    // and tiles kernels (and the wave tiles, up to 64 entries a row) at load and
+    // keep the fastest, 1 = vector, 2 = tiles
     // (row-aligned tiles, carries through the merge fix-up; the tiles plan
     // lives in mp / split_* / carry_*).  crs_used: 1, 2, or 3 for wave tiles.
     // Swept slabs in csb (csb.sweep = 1) replace any of them, and the merge
@@ -207,7 +208,7 @@ struct pwm_matrix {
     pwmk::RowsPlan rp;
     pwm_impl::DevBuf rows_cut;
     pwm_impl::DevBuf tiles;
-    int crs_nt = -1;          // tiles and wave tiles: non-temporal entry loads (-1 = timed at load)
+    int crs_nt = -1;          // tiles and wave tiles: non-temporal entry loads (-1 = tiles timed, wave tiles by rule)
     int crs_nt_used = 0;
     bool tiles_carry = true;  // some tile is a merge tile (its carry needs the fix-up)
 
